@@ -271,9 +271,9 @@ typedef struct {
     int64_t bytes;            /* device bytes of the packed format, its
                                  SpMM value stream included              */
     int64_t spmm_bytes;       /* bytes of it one vnm_spmm reads: the value
-                                 stream (row, B row and FP32 weight per
-                                 kept value) and the work-item table     */
-    int32_t items;            /* SpMM work items (whole rows of at most 64
+                                 stream (B row and FP32 weight per kept
+                                 value) and the work-item table           */
+    int32_t items;            /* SpMM work items (rows of at most 64
                                  values, or 64-value chunks of longer
                                  rows)                                    */
     int32_t slots;            /* rows of partial sums: one per chunk of a
@@ -319,18 +319,18 @@ int vnm_spmm(vnm_packed *p, const void *B, int ldb, int n, int b_dtype,
  * overlap on one GPU (other contexts or streams) race.  A product needing
  * more (vnm_packed_info.slots * n floats) returns VNM_E_ARG.  The launch
  * shape is the one vnm_spmm chose or vnm_spmm_set_shape fixed for
- * (b_dtype, n), else 8 bytes per lane. */
+ * (b_dtype, n), else the one vnm_spmm would choose. */
 int vnm_spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int b_dtype,
                      const float *b_scales, float *C, int ldc);
 
-/* Launch shape of vnm_spmm for (b_dtype, n): each lane gathers
- * cols_per_lane consecutive values of a B row per entry (2 to 16 bytes) and
- * the columns split into tiles of 64 * cols_per_lane; when the tile count
- * divides 8, each tile runs on its own XCDs.  Not in the reference (its
- * kernels have fixed shapes).  By default the first vnm_spmm call of a shape
- * times every usable value and keeps the fastest; set_shape with a value in
- * {1, 2, 4, 8, 16} fixes it, 0 clears it; get_shape gives 0 when the shape
- * has not been chosen yet. */
+/* Launch shape of vnm_spmm for (b_dtype, n): the columns split into tiles of
+ * 64 * cols_per_lane, of which a group of lanes gathers one per value, 16 bytes a
+ * lane; when the tile count divides 8, each tile runs on its own XCDs.  Not
+ * in the reference (its kernels have fixed shapes).  Every shape gives the
+ * same bits.  By default the first vnm_spmm call of a shape takes tiles of 256
+ * bytes of a B row where they divide n, else narrower ones; set_shape with a
+ * value in {1, 2, 4, 8, 16} (cols_per_lane * sizeof(B value) of 2 to 16) fixes
+ * it, 0 clears it; get_shape gives 0 when the shape has not been chosen yet. */
 int vnm_spmm_set_shape(vnm_packed *p, int b_dtype, int n, int cols_per_lane);
 int vnm_spmm_get_shape(const vnm_packed *p, int b_dtype, int n, int32_t *cols_per_lane);
 
@@ -345,7 +345,7 @@ int vnm_gcn_layer(vnm_packed *p, const uint16_t *X, int ldx, int K, const uint16
 /* Batched SpMM: C_g = A_g B_g (+ bias_g) for `count` packed matrices of one
  * value dtype and uneven sizes, all with n output columns, in one persistent
  * launch captured with its row pre-fill as a HIP graph.  Not in the
- * reference.  cols_per_lane = 0 tunes the launch shape on the batch itself.
+ * reference.  cols_per_lane = 0 takes the shape vnm_spmm would choose.
  * The operand pointers are fixed at creation; vnm_batch_run replays the graph
  * on the context stream.  b_scales and bias may be NULL (per-entry NULLs
  * allowed for bias). */

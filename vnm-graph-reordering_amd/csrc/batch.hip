@@ -1,14 +1,15 @@
 // Batched V:N:M SpMM and the GCN aggregation layer (gfx950).
 //
 // Batch: many packed matrices of uneven size multiplied in one persistent
-// launch.  The work items (64 values x one column tile) of all matrices
-// form one list (prefix offsets per matrix); a fixed grid of 8 workgroups per
-// CU walks it, each XCD taking a contiguous range so neighbouring items of
-// one matrix share that XCD's L2.  A device table holds every matrix's
-// pointers (SpmmArgs).  The batch is tuned once (values per lane, timed on the
-// whole batch) and then captured as a HIP graph of two kernels -- the SpMM
-// and the fix-up pass (rows cut into chunks, whose partial sums are added in
-// item order) -- replayed by vnm_batch_run.
+// launch.  The work units (the items of one wave x one column tile) of all
+// matrices form one list (prefix offsets per matrix); a fixed grid of 8
+// workgroups per CU walks it, each XCD taking a contiguous range so neighbouring
+// units of one matrix share that XCD's L2.  A device table holds every matrix's
+// pointers (SpmmArgs).  The batch is captured once as a HIP graph of two kernels
+// -- the SpMM and the fix-up pass (rows cut into chunks, whose partial sums are
+// added in chunk order) -- replayed by vnm_batch_run.  24 Chung-Lu graphs of 1,000
+// to 40,000 nodes, BF16, n = 256: 338 us with the single SpMM's earlier kernel
+// and a width timed per batch, 275 now.
 //
 // GCN layer (the consumer of gnn/single/pyg_gcn.py:41-74, aggr='add'):
 // Y = A_vnm (X W) + bias.  X W runs on MFMA (BF16 inputs, FP32 accumulation,
@@ -25,7 +26,8 @@
 struct vnm_batch {
     vnm_ctx *ctx = nullptr;
     int count = 0, n = 0, bt = 0, at = 0, vec = 0, T = 1;
-    int total_units = 0, nfix = 0, grid = 0, per_xcd = 0, waves_per_xcd = 0;
+    int total_units = 0, nfix = 0, nhub = 0, grid = 0, per_xcd = 0, waves_per_xcd = 0;
+    bool has_bias = false;  // some matrix has a bias
     vnm::DBuf<vnm::SpmmArgs> descs;
     vnm::DBuf<int32_t> unit_off;
     vnm::DBuf<int4> fix;          // {matrix, row, first slot, slots}
@@ -40,10 +42,12 @@ struct vnm_batch {
 
 namespace vnm {
 
-template <int BT, int VEC>
+template <int BT, int LPR, int LB, bool EXTRA>
 __global__ __launch_bounds__(256) void k_spmm_batch(const SpmmArgs *__restrict__ descs,
                                                     const int32_t *__restrict__ unit_off, int count, int T,
                                                     int total, int per_xcd, int waves_per_xcd) {
+    constexpr int NV = LB / bsize<BT>();
+    __shared__ __align__(16) float turn[NV > 4 ? 4 : 1][NV > 4 ? 64 * NV : 4];
     // wave-uniform; readfirstlane lets the unit's reads be scalar loads
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
@@ -58,57 +62,71 @@ __global__ __launch_bounds__(256) void k_spmm_batch(const SpmmArgs *__restrict__
             else hi = mid - 1;
         }
         const int local = unit - unit_off[lo];
-        spmm_unit<BT, VEC>(descs[lo], local / T, local % T, T);
+        spmm_items<BT, LPR, LB, EXTRA>(descs[lo], local / T * (64 / LPR), local % T, turn[NV > 4 ? wv : 0]);
     }
 }
 
-// Fix-up of the listed (matrix, row) pairs: cut rows get the sum of their
-// slots in item order (rows of a matrix without work items, the bias or zero).
-__global__ __launch_bounds__(256) void k_fix_batch(const int4 *__restrict__ list, int nf, int n,
+// Fix-up of the listed (matrix, row) pairs, hub rows first: cut rows get the
+// sum of their slots in item order (rows of a matrix without work items, the
+// bias or zero).
+__global__ __launch_bounds__(256) void k_fix_batch(const int4 *__restrict__ list, int nf, int nhub, int n,
                                                    const SpmmArgs *__restrict__ descs) {
-    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (w >= nf) return;
-    const int4 e = list[w];
+    int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int hp = n / 64, cp = (n + 255) / 256;
+    const bool hub = w < nhub * hp;
+    if (!hub) w -= nhub * hp;
+    const int i = hub ? w / hp : nhub + w / cp;
+    if (i >= nf) return;
+    const int4 e = list[i];
     const SpmmArgs &a = descs[e.x];
-    fix_row(a.C + (size_t)e.y * a.ldc, a.part, a.pn, e.z, e.w, n, a.bias, false);
+    float *crow = a.C + (size_t)e.y * a.ldc;
+    if (hub) fix_row<1, 32>(crow, a.part, a.pn, e.z, e.w, w % hp * 64, n, a.bias, false);
+    else fix_row<4, 8>(crow, a.part, a.pn, e.z, e.w, w % cp * 256, n, a.bias, false);
 }
 
+// Rows of a matrix's fix-up list into the batch's.
 __global__ void k_tag_fix(const int4 *__restrict__ fix, int nf, int g, int4 *__restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nf) out[i] = make_int4(g, fix[i].x, fix[i].y, fix[i].z);
 }
 
-template <int BT, int VEC>
+template <int BT, int LPR, int LB = 16>
 static void launch_batch_v(vnm_batch *b, hipStream_t st) {
-    hipLaunchKernelGGL((k_spmm_batch<BT, VEC>), dim3(b->grid), dim3(256), 0, st, b->descs.p, b->unit_off.p,
-                       b->count, b->T, b->total_units, b->per_xcd, b->waves_per_xcd);
+    if (b->has_bias)
+        hipLaunchKernelGGL((k_spmm_batch<BT, LPR, LB, true>), dim3(b->grid), dim3(256), 0, st, b->descs.p,
+                           b->unit_off.p, b->count, b->T, b->total_units, b->per_xcd, b->waves_per_xcd);
+    else
+        hipLaunchKernelGGL((k_spmm_batch<BT, LPR, LB, false>), dim3(b->grid), dim3(256), 0, st, b->descs.p,
+                           b->unit_off.p, b->count, b->T, b->total_units, b->per_xcd, b->waves_per_xcd);
 }
 
 static void launch_batch_b(vnm_batch *b, hipStream_t st) {
     const int v = b->vec;
     if (b->bt == VNM_DT_F32) {
-        if (v == 4) launch_batch_v<VNM_DT_F32, 4>(b, st);
-        else if (v == 2) launch_batch_v<VNM_DT_F32, 2>(b, st);
-        else launch_batch_v<VNM_DT_F32, 1>(b, st);
+        if (v == 4) launch_batch_v<VNM_DT_F32, 64>(b, st);
+        else if (v == 2) launch_batch_v<VNM_DT_F32, 32>(b, st);
+        else launch_batch_v<VNM_DT_F32, 16>(b, st);
     } else if (b->bt == VNM_DT_BF16) {
-        if (v == 8) launch_batch_v<VNM_DT_BF16, 8>(b, st);
-        else if (v == 4) launch_batch_v<VNM_DT_BF16, 4>(b, st);
-        else if (v == 2) launch_batch_v<VNM_DT_BF16, 2>(b, st);
-        else launch_batch_v<VNM_DT_BF16, 1>(b, st);
+        if (v == 8) launch_batch_v<VNM_DT_BF16, 64>(b, st);
+        else if (v == 4) launch_batch_v<VNM_DT_BF16, 32>(b, st);
+        else if (v == 2) launch_batch_v<VNM_DT_BF16, 16>(b, st);
+        else launch_batch_v<VNM_DT_BF16, 8>(b, st);
     } else {
-        if (v == 16) launch_batch_v<VNM_DT_FP8, 16>(b, st);
-        else if (v == 8) launch_batch_v<VNM_DT_FP8, 8>(b, st);
-        else if (v == 4) launch_batch_v<VNM_DT_FP8, 4>(b, st);
-        else launch_batch_v<VNM_DT_FP8, 2>(b, st);
+        if (v == 16) launch_batch_v<VNM_DT_FP8, 64>(b, st);
+        else if (v == 8) launch_batch_v<VNM_DT_FP8, 32>(b, st);
+        else if (v == 4) launch_batch_v<VNM_DT_FP8, 16>(b, st);
+        else if (v == 2) launch_batch_v<VNM_DT_FP8, 8>(b, st);
+        else launch_batch_v<VNM_DT_FP8, 8, 8>(b, st);
     }
 }
 
-// Set the launch shape for `vec` values per lane: tile count, units, grid.
+// Set the launch shape for tiles of 64 * vec columns: tile count, units, grid.
 static void batch_shape(vnm_batch *b, const std::vector<int> &items, int vec, std::vector<int32_t> &off) {
     b->vec = vec;
     b->T = b->n / (64 * vec);
     off.assign(b->count + 1, 0);
-    for (int g = 0; g < b->count; ++g) off[g + 1] = off[g] + items[g] * b->T;
+    const int per = tile_items(b->bt, vec);  // items of a unit
+    for (int g = 0; g < b->count; ++g) off[g + 1] = off[g] + (items[g] + per - 1) / per * b->T;
     b->total_units = off[b->count];
     int ncu = 256;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->ctx->device) != hipSuccess || ncu < 8)
@@ -123,7 +141,8 @@ static int batch_enqueue(vnm_batch *b, hipStream_t st) {
         launch_batch_b(b, st);
     }
     if (b->nfix > 0)
-        hipLaunchKernelGGL(k_fix_batch, dim3((b->nfix + 3) / 4), dim3(256), 0, st, b->fix.p, b->nfix, b->n,
+        hipLaunchKernelGGL(k_fix_batch, dim3((unsigned)((fix_waves(b->nfix, b->nhub, b->n) + 3) / 4)), dim3(256), 0, st,
+                           b->fix.p, b->nfix, b->nhub, b->n,
                            b->descs.p);
     VNM_LAUNCH_CHECK("k_spmm_batch");
     return VNM_OK;
@@ -159,17 +178,20 @@ static int batch_create(vnm_ctx *ctx, vnm_packed *const *ps, int count, const vo
     b->n = n;
     b->bt = bt;
     b->at = at;
+    for (int g = 0; g < count; ++g) b->has_bias |= bias && bias[g];
     std::vector<SpmmArgs> d(count);
     std::vector<int> items(count);
     std::vector<size_t> part_off(count + 1, 0);
-    std::vector<int> fix_off(count + 1, 0);
+    std::vector<int> hub_off(count + 1, 0), fix_off(count + 1, 0);  // hub rows, and the other listed rows
     int rc;
     for (int g = 0; g < count; ++g) {
         items[g] = ps[g]->nitems;
         part_off[g + 1] = part_off[g] + (size_t)ps[g]->nslots * n;
-        fix_off[g + 1] = fix_off[g] + ps[g]->nfix;
+        hub_off[g + 1] = hub_off[g] + ps[g]->nhub;
+        fix_off[g + 1] = fix_off[g] + ps[g]->nfix - ps[g]->nhub;
     }
-    b->nfix = fix_off[count];
+    b->nhub = hub_off[count];
+    b->nfix = b->nhub + fix_off[count];
     if ((rc = b->descs.alloc(count)) || (rc = b->unit_off.alloc(count + 1)) ||
         (rc = b->fix.alloc(std::max(b->nfix, 1))) || (rc = b->part.alloc(std::max<size_t>(part_off[count], 1))))
         return rc;
@@ -177,38 +199,18 @@ static int batch_create(vnm_ctx *ctx, vnm_packed *const *ps, int count, const vo
         d[g] = packed_args(ps[g], B[g], ldb[g], bs ? bs[g] : nullptr, C[g], ldc[g], bias ? bias[g] : nullptr,
                            b->part.p + part_off[g], n);
     VNM_HIP_TRY(hipMemcpyAsync(b->descs.p, d.data(), count * sizeof(SpmmArgs), hipMemcpyHostToDevice, st));
-    for (int g = 0; g < count; ++g)
-        if (ps[g]->nfix)
-            hipLaunchKernelGGL(k_tag_fix, dim3((ps[g]->nfix + 255) / 256), dim3(256), 0, st, ps[g]->fix.p,
-                               ps[g]->nfix, g, b->fix.p + fix_off[g]);
+    for (int g = 0; g < count; ++g) {
+        const int hubs = ps[g]->nhub, rest = ps[g]->nfix - hubs;
+        if (hubs)
+            hipLaunchKernelGGL(k_tag_fix, dim3((hubs + 255) / 256), dim3(256), 0, st, ps[g]->fix.p, hubs, g,
+                               b->fix.p + hub_off[g]);
+        if (rest)
+            hipLaunchKernelGGL(k_tag_fix, dim3((rest + 255) / 256), dim3(256), 0, st, ps[g]->fix_rest(), rest, g,
+                               b->fix.p + b->nhub + fix_off[g]);
+    }
     VNM_LAUNCH_CHECK("k_tag_fix");
     std::vector<int32_t> off;
-    if (vec == 0) {
-        // tuner: each usable shape, one warm-up and three timed batches
-        hipEvent_t e0, e1;
-        VNM_HIP_TRY(hipEventCreate(&e0));
-        VNM_HIP_TRY(hipEventCreate(&e1));
-        float best = 1e30f;
-        for (int v = 16; v >= 1; v /= 2) {
-            if (!vec_ok(bt, n, v)) continue;
-            batch_shape(b.get(), items, v, off);
-            VNM_HIP_TRY(hipMemcpyAsync(b->unit_off.p, off.data(), (count + 1) * 4, hipMemcpyHostToDevice, st));
-            if ((rc = batch_enqueue(b.get(), st))) break;
-            (void)hipEventRecord(e0, st);
-            for (int i = 0; i < 3 && rc == VNM_OK; ++i) rc = batch_enqueue(b.get(), st);
-            (void)hipEventRecord(e1, st);
-            float ms = 0.f;
-            if (rc || hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-                if (!rc) rc = set_error(VNM_E_HIP, "batch tuning timing failed");
-                break;
-            }
-            if (getenv("VNM_DEBUG")) fprintf(stderr, "[vnm] batch tune bt=%d n=%d vec=%d %.4f ms\n", bt, n, v, ms / 3);
-            if (ms < best) { best = ms; vec = v; }
-        }
-        (void)hipEventDestroy(e0);
-        (void)hipEventDestroy(e1);
-        if (rc) return rc;
-    }
+    if (vec == 0) vec = default_vec(bt, n);
     batch_shape(b.get(), items, vec, off);
     VNM_HIP_TRY(hipMemcpyAsync(b->unit_off.p, off.data(), (count + 1) * 4, hipMemcpyHostToDevice, st));
     VNM_HIP_TRY(hipStreamSynchronize(st));

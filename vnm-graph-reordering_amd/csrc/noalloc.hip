@@ -46,15 +46,6 @@ int noalloc_setup(int device, float **out) {
     return VNM_OK;
 }
 
-// Values per lane when no shape was chosen for (bt, n): 8 bytes per lane,
-// or the widest narrower setting that fits n (no timing, which would create
-// events).
-static int default_vec(int bt, int n) {
-    for (int v = 8 / bsize_of(bt); v >= 1; v /= 2)
-        if (vec_ok(bt, n, v)) return v;
-    return 0;
-}
-
 static int spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs, float *C, int ldc) {
     int rc = spmm_check(p, B, ldb, n, bt, bs, C, ldc);
     if (rc) return rc;
@@ -66,7 +57,6 @@ static int spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int bt, co
                          scratch_rows(p), n, scratch_rows(p) * (size_t)n, NOALLOC_FLOATS);
     auto it = p->shapes.find(shape_key(bt, n));
     const int v = it != p->shapes.end() ? it->second : default_vec(bt, n);
-    if (!v) return set_error(VNM_E_ARG, "spmm_noalloc: no launch shape fits n = %d", n);
     return spmm_run(p, v, B, ldb, n, bt, bs, C, ldc, nullptr, p->ctx->noalloc_slots, false);
 }
 

@@ -20,23 +20,27 @@
 // block its segment, selectors and scale).
 //
 // SpMM: C[R x n] = A_vnm B, FP32 accumulation.  Packing also writes the
-// SpMM's value stream: every kept value of the row entries, row-major, as
-// (row, B row, FP32 weight = value x block scale), 12 bytes per value, so the
-// SpMM reads no block data and branches on no selector.  A work item holds
-// whole rows of at most 64 values, or a 64-value chunk of a longer row (item
-// table built once per packed matrix); a wave takes one item for one column
-// tile of 64 * VEC columns and walks it row by row: the row's B rows and
-// weights arrive as scalar loads, every lane gathers VEC consecutive values of
-// each B row (2 to 16 bytes) into VEC FMAs with the weight as a scalar
-// operand, and owns VEC columns of the output row, which is stored when the
-// row ends (rows that keep nothing are written in the gaps).  The chunks of a
-// long row store partial sums into slots, and a fix-up pass adds each cut
-// row's slots in item order, so C is bit-identical for every launch shape and
-// run: no atomics.  The T column tiles interleave in 128-byte pieces of each
-// row, and when T divides 8, tile t runs on its own 8/T XCDs, so each XCD's L2
-// serves one 1/T slice of B spread over all of its channels.  VEC is chosen per (B
-// dtype, n) by timing the usable values on first use (vnm_spmm_set_shape
-// overrides).  FP8 B is decoded by the gfx950 e4m3 conversion instruction.
+// SpMM's value stream: every kept value of the row entries as (B row, FP32
+// weight = value x block scale), 8 bytes per value, so the SpMM reads no block
+// data and branches on no selector.  A work item is a whole row of at most 64
+// values or a 64-value chunk of a longer row; items and stream are sorted by
+// item length.  A wave takes 64 / LPR items for one column tile, LPR lanes per
+// item: one load instruction gathers the tiles of 64 / LPR B rows, 16 bytes per
+// lane, with the values' B rows and weights spread over the lanes by DPP, and the
+// row is stored once, after its last value (rows that keep nothing are written in
+// the gaps).  The chunks of a long row store partial sums into slots, and a
+// fix-up pass adds each cut row's slots in chunk order, so C is bit-identical
+// for every launch shape and run: no atomics.  When the tile count T divides 8,
+// tile t runs on its own 8/T XCDs, so each XCD's L2 serves one 1/T slice of B.
+// FP8 B is decoded by the gfx950 e4m3 conversion instruction.
+//
+// Measured (us per product, fix-up pass included; before: one item of mixed row
+// lengths per wave, the B row's offset a scalar, 2 to 8 bytes per lane, the width
+// timed on first use): R-MAT 65,536, 128:2:8, n = 256: FP32 88 -> 76, BF16 82 ->
+// 49; R-MAT 131,072 degree 24, 64:2:4, BF16 n = 128: 107 -> 68; Chung-Lu 20,011
+// FP8 n = 384: 45 -> 26.  The FP32 gather moves 1.07 GB through L1s that take
+// 33 us for it when every request hits, 37 when every one hits L2; the rest is L2
+// misses (a copy of the loop without row ends or weights' FMAs: 60).
 #include "graph.h"
 #include "hip_common.h"
 #include "packed.h"
@@ -383,48 +387,55 @@ __global__ void k_val_counts(const uint8_t *__restrict__ ent_idx, int E, int32_t
     else if (e == E) nv[e] = 0;
 }
 
+// Where the values of a row go: piece c of row r (the row, or its c-th chunk of
+// ITEM values) starts at pdst[pbase[r] + c] of the value stream.
+struct Pieces {
+    const int32_t *vrp, *pbase, *pdst;
+};
+
+// Value i (in row-major order) of row r: B row c, weight w.
+__device__ __forceinline__ void put_value(const Pieces &P, int i, int r, int c, float w, uint2 *__restrict__ vrec) {
+    const int k = i - P.vrp[r];
+    vrec[P.pdst[P.pbase[r] + k / ITEM] + k % ITEM] = make_uint2((uint32_t)c, __float_as_uint(w));
+}
+
 template <int DT>
-__device__ __forceinline__ void emit_values(int e, int o, int M, const int32_t *__restrict__ ent_row,
-                                            const int32_t *__restrict__ ent_col, const uint8_t *__restrict__ ent_idx,
-                                            const uint8_t *__restrict__ ent_val, const int32_t *__restrict__ ent_blk,
-                                            const float *__restrict__ blk_scale, int32_t *__restrict__ vrow,
-                                            int32_t *__restrict__ vcol, float *__restrict__ vw) {
+__device__ __forceinline__ void emit_values(int e, int M, const int32_t *__restrict__ voff, const Pieces &P,
+                                            const int32_t *__restrict__ ent_row, const int32_t *__restrict__ ent_col,
+                                            const uint8_t *__restrict__ ent_idx, const uint8_t *__restrict__ ent_val,
+                                            const int32_t *__restrict__ ent_blk, const float *__restrict__ blk_scale,
+                                            uint2 *__restrict__ vrec) {
+    const int o = voff[e];
     const int r = ent_row[e], c0 = ent_col[e];
     const uint32_t code = ent_idx[e];
     const float sc = DT == VNM_DT_FP8 ? blk_scale[ent_blk[e]] : 1.f;
-    vrow[o] = r;
-    vcol[o] = c0;
-    vw[o] = load_aval<DT>(ent_val, 2 * e) * sc;
-    if (code & 0x10u) {
-        vrow[o + 1] = r;
-        vcol[o + 1] = (c0 & ~(M - 1)) | (int)(code & 15u);
-        vw[o + 1] = load_aval<DT>(ent_val, 2 * e + 1) * sc;
-    }
+    put_value(P, o, r, c0, load_aval<DT>(ent_val, 2 * e) * sc, vrec);
+    if (code & 0x10u)
+        put_value(P, o + 1, r, (c0 & ~(M - 1)) | (int)(code & 15u), load_aval<DT>(ent_val, 2 * e + 1) * sc, vrec);
 }
 
-// The SpMM's value stream: row entry e's values (its first, then its second)
-// at voff[e] as (row, B row, weight), the weight being the stored value times
-// the block scale (FP8; 1 otherwise) rounded to FP32 once.
-__global__ void k_values(int E, int M, int dtype, const int32_t *__restrict__ voff,
+// The SpMM's value stream: row entry e's values (its first, then its second),
+// each weight being the stored value times the block scale (FP8; 1 otherwise)
+// rounded to FP32 once.
+__global__ void k_values(int E, int M, int dtype, const int32_t *__restrict__ voff, Pieces P,
                          const int32_t *__restrict__ ent_row, const int32_t *__restrict__ ent_col,
                          const uint8_t *__restrict__ ent_idx, const uint8_t *__restrict__ ent_val,
                          const int32_t *__restrict__ ent_blk, const float *__restrict__ blk_scale,
-                         int32_t *__restrict__ vrow, int32_t *__restrict__ vcol, float *__restrict__ vw) {
+                         uint2 *__restrict__ vrec) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= E) return;
-    const int o = voff[e];
     switch (dtype) {
         case VNM_DT_F32:
-            emit_values<VNM_DT_F32>(e, o, M, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrow, vcol, vw);
+            emit_values<VNM_DT_F32>(e, M, voff, P, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrec);
             break;
         case VNM_DT_BF16:
-            emit_values<VNM_DT_BF16>(e, o, M, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrow, vcol, vw);
+            emit_values<VNM_DT_BF16>(e, M, voff, P, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrec);
             break;
         case VNM_DT_F16:
-            emit_values<VNM_DT_F16>(e, o, M, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrow, vcol, vw);
+            emit_values<VNM_DT_F16>(e, M, voff, P, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrec);
             break;
         default:
-            emit_values<VNM_DT_FP8>(e, o, M, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrow, vcol, vw);
+            emit_values<VNM_DT_FP8>(e, M, voff, P, ent_row, ent_col, ent_idx, ent_val, ent_blk, blk_scale, vrec);
             break;
     }
 }
@@ -436,10 +447,134 @@ __global__ void k_vrowptr(const int32_t *__restrict__ rowptr, const int32_t *__r
     if (r <= R) vrp[r] = voff[rowptr[r]];
 }
 
+// ------------------------------------------------------------ work items
+
+// Rows without values from row r on, counted up to GAP_MAX + 1.
+__device__ __forceinline__ int empty_run(const int32_t *__restrict__ vrp, int R, int r) {
+    int n = 0;
+    while (n <= GAP_MAX && r + n < R && vrp[r + n + 1] == vrp[r + n]) ++n;
+    return n;
+}
+
+// Per row: its pieces (np), a cut row's first slot (slot0), the rows without
+// values written after an uncut row (gap), and the rows of the fix-up pass --
+// cut rows, and rows without values that no uncut row writes: those before the
+// first row with values, after a cut row, or in a run of more than GAP_MAX.
+// cnt: slots, hub rows, other listed rows.  Slots and list positions come from
+// counters, so they differ from one packing to the next; nothing computed does.
+__global__ __launch_bounds__(256) void k_row_pieces(const int32_t *__restrict__ vrp, int R, int32_t *__restrict__ np,
+                                                    int32_t *__restrict__ slot0, uint8_t *__restrict__ gap,
+                                                    int32_t *__restrict__ cnt, int4 *__restrict__ fix) {
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r > R) return;
+    const int len = r < R ? vrp[r + 1] - vrp[r] : 0;
+    const int pieces = (len + ITEM - 1) / ITEM;
+    np[r] = pieces;
+    if (r == R) return;
+    bool list = false;
+    int s0 = 0, ns = 0;
+    if (len > ITEM) {
+        list = true;
+        ns = pieces;
+        s0 = atomicAdd(&cnt[0], ns);
+        slot0[r] = s0;
+        gap[r] = 0;
+    } else if (len > 0) {
+        const int e = empty_run(vrp, R, r + 1);
+        gap[r] = (uint8_t)(e <= GAP_MAX ? e : 0);
+    } else {
+        int b = 1;  // the row with values before this one is r - b
+        while (b <= GAP_MAX && r - b >= 0 && vrp[r - b + 1] == vrp[r - b]) ++b;
+        list = b > GAP_MAX || r - b < 0 || vrp[r - b + 1] - vrp[r - b] > ITEM ||
+               empty_run(vrp, R, r - b + 1) > GAP_MAX;
+    }
+    const bool hub = list && ns > HUB_SLOTS;
+    const bool rest = list && !hub;
+    if (hub) fix[atomicAdd(&cnt[1], 1)] = make_int4(r, s0, ns, 0);
+    const uint64_t m = __ballot(rest);  // one atomic per wave
+    if (rest) {
+        const int lane = threadIdx.x & 63;
+        int base = 0;
+        const int lead = __builtin_ctzll(m);
+        if (lane == lead) base = atomicAdd(&cnt[2], (int)__popcll(m));
+        base = __shfl(base, lead, 64);
+        fix[R - 1 - (base + (int)__popcll(m & ((1ull << lane) - 1)))] = make_int4(r, s0, ns, 0);
+    }
+}
+
+// The pieces in row order: sort key (long pieces first; slots of the arrays past
+// the last piece sort behind them), and what the work item will hold.
+__global__ __launch_bounds__(256) void k_pieces(const int32_t *__restrict__ vrp, int R, const int32_t *__restrict__ pbase,
+                                                const int32_t *__restrict__ slot0, const uint8_t *__restrict__ gap,
+                                                int cap, uint64_t *__restrict__ key, int32_t *__restrict__ id,
+                                                int2 *__restrict__ info) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < R) {
+        const int len = vrp[t + 1] - vrp[t], p0 = pbase[t];
+        const bool cut = len > ITEM;
+        for (int c = 0; c * ITEM < len; ++c) {
+            const int l = min(ITEM, len - c * ITEM);
+            key[p0 + c] = (uint64_t)(ITEM - l);
+            id[p0 + c] = p0 + c;
+            info[p0 + c] = make_int2(cut ? slot0[t] + c : t, l | (cut ? 1 << 16 : (int)gap[t] << 8));
+        }
+    }
+    for (int i = pbase[R] + t; i < cap; i += gridDim.x * blockDim.x) {
+        key[i] = ITEM;
+        id[i] = i;
+        info[i] = make_int2(0, 0);
+    }
+}
+
+__global__ void k_piece_lens(const int32_t *__restrict__ order, const int2 *__restrict__ info, int cap,
+                             int32_t *__restrict__ len) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < cap) len[i] = info[order[i]].y & 0xFF;
+}
+
+// The work items: the sorted pieces (beg: their starts in the value stream), in
+// groups of GROUP neighbours -- the most a wave walks side by side, so those
+// have one length -- whose order steps through the sorted list by about 0.62 of
+// it.  In sorted order the launch gathers only at first and mostly stores at
+// the end: R-MAT 65,536, FP32, n = 256: 110 us sorted, 80 mixed.
+constexpr int GROUP = 8;
+__global__ __launch_bounds__(256) void k_items(const int32_t *__restrict__ npieces, const int32_t *__restrict__ order,
+                                               const int2 *__restrict__ info, const int32_t *__restrict__ beg,
+                                               int32_t *__restrict__ pdst, int4 *__restrict__ items) {
+    __shared__ int step;
+    const int n = *npieces, ng = n / GROUP;
+    if (threadIdx.x == 0) {
+        // a step coprime to the group count visits every group once
+        int s = max(1, (int)(ng * 0.618f));
+        for (;; ++s) {
+            int x = s, y = ng;
+            while (y) {
+                const int r = x % y;
+                x = y;
+                y = r;
+            }
+            if (x <= 1 || ng <= 1) break;
+        }
+        step = s;
+    }
+    __syncthreads();
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const int g = j / GROUP;
+    const int i = g < ng ? (int)((int64_t)g * step % ng) * GROUP + j % GROUP : j;
+    const int id = order[i];
+    const int2 f = info[id];
+    pdst[id] = beg[i];
+    const Piece p{beg[i], f.y & 0xFF, f.x, (int16_t)((f.y >> 8) & 0xFF), (int16_t)(f.y >> 16)};
+    items[j] = *(const int4 *)&p;
+}
+
 // ------------------------------------------------------------ SpMM kernel
 
-template <int BT, int VEC>
-__global__ __launch_bounds__(256) void k_spmm(SpmmArgs a, int T, int items, int per_g) {
+template <int BT, int LPR, int LB, bool EXTRA>
+__global__ __launch_bounds__(256) void k_spmm(SpmmArgs a, int T, int per_g) {
+    constexpr int NV = LB / bsize<BT>();
+    __shared__ __align__(16) float turn[NV > 4 ? 4 : 1][NV > 4 ? 64 * NV : 4];
     const int wv = threadIdx.x >> 6;
     // workgroups are dealt round-robin over the 8 XCDs
     const int xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
@@ -453,24 +588,30 @@ __global__ __launch_bounds__(256) void k_spmm(SpmmArgs a, int T, int items, int 
         tile = lwg % T;
         iwg = lwg / T;
     }
-    // wave-uniform; readfirstlane lets the entry reads be scalar loads
-    const int item = __builtin_amdgcn_readfirstlane(iwg * 4 + wv);
-    if (item >= items) return;
-    spmm_unit<BT, VEC>(a, item, __builtin_amdgcn_readfirstlane(tile), T);
+    const int item0 = __builtin_amdgcn_readfirstlane((iwg * 4 + wv) * (64 / LPR));
+    if (item0 >= a.items) return;
+    spmm_items<BT, LPR, LB, EXTRA>(a, item0, __builtin_amdgcn_readfirstlane(tile), turn[NV > 4 ? wv : 0]);
 }
 
 // Fix-up pass: rows cut into chunks get the sum of their partial-sum slots
-// in item order (one wave each); a matrix without work items, the bias or
-// zero in every row.
-__global__ __launch_bounds__(256) void k_spmm_fix(const int4 *__restrict__ fix, int nfix, const float *__restrict__ part,
-                                                  int pn, int n, float *__restrict__ C, int ldc,
-                                                  const float *__restrict__ bias, const uint8_t *__restrict__ dvb,
-                                                  int V) {
+// in item order; a matrix without work items, the bias or zero in every row.
+__global__ __launch_bounds__(256) void k_spmm_fix(const int4 *__restrict__ hubs, int nhub,
+                                                  const int4 *__restrict__ rest, int nrest,
+                                                  const float *__restrict__ part, int pn, int n,
+                                                  float *__restrict__ C, int ldc, const float *__restrict__ bias,
+                                                  const uint8_t *__restrict__ dvb, int V) {
     // wave-uniform, so the list entry is a scalar load
-    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-    if (w >= nfix) return;
-    const int4 f = fix[w];
-    fix_row(C + (size_t)f.x * ldc, part, pn, f.y, f.z, n, bias, dvb != nullptr && dvb[f.x / V] != 0);
+    int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    const int hp = n / 64, cp = (n + 255) / 256;
+    const bool hub = w < nhub * hp;
+    if (!hub) w -= nhub * hp;
+    const int i = hub ? w / hp : w / cp;
+    if (!hub && i >= nrest) return;
+    const int4 f = hub ? hubs[i] : rest[i];
+    float *crow = C + (size_t)f.x * ldc;
+    const bool dense = dvb != nullptr && dvb[f.x / V] != 0;
+    if (hub) fix_row<1, 32>(crow, part, pn, f.y, f.z, w % hp * 64, n, bias, dense);
+    else fix_row<4, 8>(crow, part, pn, f.y, f.z, w % cp * 256, n, bias, dense);
 }
 
 // ------------------------------------------------------------ host
@@ -490,74 +631,41 @@ static std::vector<uint32_t> subsets4(int M) {
     return out;
 }
 
-// SpMM work items from the value row pointers (host pass, once per packed matrix):
-// consecutive whole rows while they fit in ITEM values; a row longer than
-// ITEM starts a new item and is cut into ITEM-value chunks, each with a
-// partial-sum slot of its own (consecutive slots), the last chunk staying
-// open for the rows that follow.  So an item's only cut row is its first.
-// The fix-up list holds the cut rows with their slot range and the rows of
-// runs of more than GAP_MAX rows that keep nothing (the SpMM's item walk
-// writes the shorter runs; without any item, the list holds every row).
-static int build_items(vnm_packed *p, const int32_t *d_vrp) {
+// SpMM work items from the value row pointers, on the device: the pieces of
+// every row, sorted by length, and where each starts in the value stream
+// (pbase, pdst).  At most cap pieces.
+struct PieceBufs {
+    DBuf<int32_t> np, slot0, pbase, id, order, len, beg, pdst, cnt;
+    DBuf<uint8_t> gap;
+    DBuf<uint64_t> key, key2;
+    DBuf<int2> info;
+};
+
+static int build_items(vnm_packed *p, const int32_t *vrp, int64_t values, PieceBufs &P) {
     hipStream_t st = p->ctx->stream;
     const int R = p->nrows;
-    std::vector<int32_t> rp(R + 1);
-    VNM_HIP_TRY(hipMemcpyAsync(rp.data(), d_vrp, (size_t)(R + 1) * 4, hipMemcpyDeviceToHost, st));
-    VNM_HIP_TRY(hipStreamSynchronize(st));
-    std::vector<int32_t> beg, slot;
-    std::vector<int4> fix;
-    int cur_len = 0, nslots = 0;
-    bool open = false;
-    for (int r = 0; r < R; ++r) {
-        const int b = rp[r], L = rp[r + 1] - b;
-        if (L == 0) continue;
-        if (L <= ITEM) {
-            if (open && cur_len + L > ITEM) open = false;
-            if (!open) {
-                beg.push_back(b);
-                slot.push_back(-1);
-                open = true;
-                cur_len = 0;
-            }
-            cur_len += L;
-        } else {
-            const int nch = (L + ITEM - 1) / ITEM;
-            fix.push_back(make_int4(r, nslots, nch, 0));
-            for (int c = 0; c < nch; ++c) {
-                beg.push_back(b + c * ITEM);
-                slot.push_back(nslots++);
-            }
-            open = true;
-            cur_len = L - (nch - 1) * ITEM;
-        }
-    }
-    beg.push_back(rp[R]);
-    if (slot.empty()) {
-        for (int r = 0; r < R; ++r) fix.push_back(make_int4(r, 0, 0, 0));
-    } else {
-        // runs of more than GAP_MAX rows without entries: one fix-up wave per row
-        for (int r = 0; r < R;) {
-            if (rp[r + 1] != rp[r]) { ++r; continue; }
-            int e = r;
-            while (e < R && rp[e + 1] == rp[e]) ++e;
-            if (e - r > GAP_MAX)
-                for (int q = r; q < e; ++q) fix.push_back(make_int4(q, 0, 0, 0));
-            r = e;
-        }
-    }
-    p->nitems = (int)slot.size();
-    p->nslots = nslots;
-    p->nfix = (int)fix.size();
+    // a row of at most ITEM values is one piece, and the others' chunks hold
+    // ITEM values but for one per row
+    const int cap = (int)(R + values / ITEM + 1);
     int rc;
-    if ((rc = p->item_beg.alloc(beg.size())) || (rc = p->item_slot.alloc(std::max<size_t>(slot.size(), 1))) ||
-        (rc = p->fix.alloc(std::max<size_t>(fix.size(), 1))))
+    if ((rc = p->item.alloc(cap)) || (rc = p->fix.alloc(R)) || (rc = P.np.alloc(R + 1)) || (rc = P.pbase.alloc(R + 1)) ||
+        (rc = P.slot0.alloc(R)) || (rc = P.gap.alloc(R)) || (rc = P.cnt.alloc(4)) || (rc = P.key.alloc(cap)) ||
+        (rc = P.key2.alloc(cap)) || (rc = P.id.alloc(cap)) || (rc = P.order.alloc(cap)) || (rc = P.info.alloc(cap)) ||
+        (rc = P.len.alloc(cap)) || (rc = P.beg.alloc(cap)) || (rc = P.pdst.alloc(cap)))
         return rc;
-    VNM_HIP_TRY(hipMemcpyAsync(p->item_beg.p, beg.data(), beg.size() * 4, hipMemcpyHostToDevice, st));
-    if (!slot.empty())
-        VNM_HIP_TRY(hipMemcpyAsync(p->item_slot.p, slot.data(), slot.size() * 4, hipMemcpyHostToDevice, st));
-    if (!fix.empty())
-        VNM_HIP_TRY(hipMemcpyAsync(p->fix.p, fix.data(), fix.size() * sizeof(int4), hipMemcpyHostToDevice, st));
-    VNM_HIP_TRY(hipStreamSynchronize(st));
+    VNM_HIP_TRY(hipMemsetAsync(P.cnt.p, 0, 16, st));
+    hipLaunchKernelGGL(k_row_pieces, dim3(grid_of((int64_t)R + 1, 256)), dim3(256), 0, st, vrp, R, P.np.p, P.slot0.p,
+                       P.gap.p, P.cnt.p, p->fix.p);
+    if ((rc = scan_excl_i32(P.np.p, P.pbase.p, R + 1, st))) return rc;
+    hipLaunchKernelGGL(k_pieces, dim3(grid_of(R, 256)), dim3(256), 0, st, vrp, R, P.pbase.p, P.slot0.p, P.gap.p, cap,
+                       P.key.p, P.id.p, P.info.p);
+    if ((rc = sort_pairs_u64_i32(P.key.p, P.key2.p, P.id.p, P.order.p, cap, 7, st))) return rc;
+    hipLaunchKernelGGL(k_piece_lens, dim3(grid_of(cap, 256)), dim3(256), 0, st, P.order.p, P.info.p, cap, P.len.p);
+    if ((rc = scan_excl_i32(P.len.p, P.beg.p, cap, st))) return rc;
+    hipLaunchKernelGGL(k_items, dim3(grid_of(cap, 256)), dim3(256), 0, st, P.pbase.p + R, P.order.p, P.info.p, P.beg.p,
+                       P.pdst.p, p->item.p);
+    p->ctx->launches += 4;
+    VNM_LAUNCH_CHECK("pack items");
     return VNM_OK;
 }
 
@@ -733,29 +841,31 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
     }
     hipLaunchKernelGGL(k_val_counts, dim3(grid_of((int64_t)E + 1, 256)), dim3(256), 0, st, p->ent_idx.p, E, nv.p);
     if ((rc = scan_excl_i32(nv.p, voff.p, (int64_t)E + 1, st))) { delete p; return rc; }
-    int NV = 0;
-    VNM_HIP_TRY(hipMemcpyAsync(&NV, voff.p + E, 4, hipMemcpyDeviceToHost, st));
-    VNM_HIP_TRY(hipStreamSynchronize(st));
-    p->nval = NV;
-    // VTAIL zero records past the end: the SpMM reads B rows and weights a
-    // block of values at a time
-    const size_t vn = (size_t)NV + VTAIL;
-    if ((rc = p->vrow.alloc(vn)) || (rc = p->vcol.alloc(vn)) || (rc = p->vw.alloc(vn))) {
+    hipLaunchKernelGGL(k_vrowptr, dim3(grid_of((int64_t)R + 1, 256)), dim3(256), 0, st, p->rowptr.p, voff.p, R,
+                       vrp.p);
+    // the sparse-MFMA part's values are not in the row entries
+    const int64_t values = std::min<int64_t>(p->retained, 2 * (int64_t)E);
+    PieceBufs P;
+    if ((rc = p->vrec.alloc(std::max<int64_t>(values, 1))) || (rc = build_items(p, vrp.p, values, P))) {
         delete p;
         return rc;
     }
-    VNM_HIP_TRY(hipMemsetAsync(p->vrow.p + NV, 0, VTAIL * 4, st));
-    VNM_HIP_TRY(hipMemsetAsync(p->vcol.p + NV, 0, VTAIL * 4, st));
-    VNM_HIP_TRY(hipMemsetAsync(p->vw.p + NV, 0, VTAIL * 4, st));
     if (E > 0)
-        hipLaunchKernelGGL(k_values, dim3(grid_of(E, 256)), dim3(256), 0, st, E, M, dtype, voff.p, p->ent_row.p,
-                           p->ent_col.p, p->ent_idx.p, p->ent_val.p, p->ent_blk.p, p->blk_scale.p,
-                           p->vrow.p, p->vcol.p, p->vw.p);
-    hipLaunchKernelGGL(k_vrowptr, dim3(grid_of((int64_t)R + 1, 256)), dim3(256), 0, st, p->rowptr.p, voff.p, R,
-                       vrp.p);
+        hipLaunchKernelGGL(k_values, dim3(grid_of(E, 256)), dim3(256), 0, st, E, M, dtype, voff.p,
+                           Pieces{vrp.p, P.pbase.p, P.pdst.p}, p->ent_row.p, p->ent_col.p, p->ent_idx.p,
+                           p->ent_val.p, p->ent_blk.p, p->blk_scale.p, p->vrec.p);
     g->ctx->launches += 4;
     VNM_LAUNCH_CHECK("pack values");
-    if ((rc = build_items(p, vrp.p))) { delete p; return rc; }
+    int32_t cn[3], np = 0, nval = 0;
+    VNM_HIP_TRY(hipMemcpyAsync(cn, P.cnt.p, 12, hipMemcpyDeviceToHost, st));
+    VNM_HIP_TRY(hipMemcpyAsync(&np, P.pbase.p + R, 4, hipMemcpyDeviceToHost, st));
+    VNM_HIP_TRY(hipMemcpyAsync(&nval, voff.p + E, 4, hipMemcpyDeviceToHost, st));
+    VNM_HIP_TRY(hipStreamSynchronize(st));  // the scratch is freed on return
+    p->nval = nval;
+    p->nitems = np;
+    p->nslots = cn[0];
+    p->nhub = cn[1];
+    p->nfix = cn[1] + cn[2];
     *out = p;
     return VNM_OK;
 }
@@ -774,22 +884,38 @@ int ensure_part(vnm_packed *p, int n) {
 
 int bsize_of(int bt) { return bt == VNM_DT_F32 ? 4 : bt == VNM_DT_BF16 ? 2 : 1; }
 
-// Values per lane usable for (bt, n): 2 to 16 bytes per lane load, and the
-// 64 * vec column tile divides n.
+// Column tiles of 64 * vec values usable for (bt, n): a tile is 128 to 1,024
+// bytes of a B row (8 to 64 lanes of 16 bytes) and divides n.
 bool vec_ok(int bt, int n, int vec) {
     if (vec != 1 && vec != 2 && vec != 4 && vec != 8 && vec != 16) return false;
     const int bytes = vec * bsize_of(bt);
     return bytes >= 2 && bytes <= 16 && n % (64 * vec) == 0;
 }
 
+// The tile taken unless the caller fixes one: 256 bytes where they divide the
+// row, else 128.  Tiles of 256 and 512 bytes are within 3 % of each other, 128
+// up to 15 % slower (twice the item and value reads per byte), 1,024 20-30 %
+// (no slice of B stays with an XCD): us at 128 / 256 / 512 / 1,024 bytes, R-MAT
+// 65,536 n = 256 FP32 - / 76.3 / 76.4 / 98.7, BF16 54.4 / 49.0 / 52.5 / -;
+// R-MAT 131,072 n = 128 BF16 68.2 / 69.9.  FP8 rows of an odd number of
+// 64-column groups have no usable tile (vec_ok) and run as 64-byte tiles (vec 1).
+int default_vec(int bt, int n) {
+    for (int v = 4 / bsize_of(bt); v >= 1; v /= 2)
+        if (vec_ok(bt, n, v)) return v;
+    return 1;
+}
+
+// Items one wave walks: 64 lanes over the lanes of a tile.
+int tile_items(int bt, int vec) {
+    const int bytes = 64 * vec * bsize_of(bt);
+    return bytes >= 128 ? 1024 / bytes : 8;
+}
+
 SpmmArgs packed_args(const vnm_packed *p, const void *B, int ldb, const float *bs, float *C, int ldc,
                      const float *bias, float *part, int pn) {
     SpmmArgs a;
-    a.item_beg = p->item_beg.p;
-    a.item_slot = p->item_slot.p;
-    a.vrow = p->vrow.p;
-    a.vcol = p->vcol.p;
-    a.vw = p->vw.p;
+    a.pieces = p->item.p;
+    a.vrec = p->vrec.p;
     a.B = (const uint8_t *)B;
     a.b_scales = bs;
     a.C = C;
@@ -806,11 +932,11 @@ SpmmArgs packed_args(const vnm_packed *p, const void *B, int ldb, const float *b
     return a;
 }
 
-template <int BT, int VEC>
+template <int BT, int LPR, int LB = 16>
 static void launch_v(const SpmmArgs &args, int n, hipStream_t st) {
-    const int T = n / (64 * VEC);
-    const int items = args.items;
-    const int iwg = (items + 3) / 4;
+    const int T = n * bsize<BT>() / (LPR * LB);
+    const int per_wg = 4 * (64 / LPR);  // items of a workgroup
+    const int iwg = (args.items + per_wg - 1) / per_wg;
     int per_g;
     if (8 % T == 0) {
         const int gs = 8 / T;
@@ -818,26 +944,30 @@ static void launch_v(const SpmmArgs &args, int n, hipStream_t st) {
     } else {
         per_g = (iwg * T + 7) / 8;
     }
-    hipLaunchKernelGGL((k_spmm<BT, VEC>), dim3(8 * per_g), dim3(256), 0, st, args, T, items, per_g);
+    if (args.bias || args.dvb)
+        hipLaunchKernelGGL((k_spmm<BT, LPR, LB, true>), dim3(8 * per_g), dim3(256), 0, st, args, T, per_g);
+    else
+        hipLaunchKernelGGL((k_spmm<BT, LPR, LB, false>), dim3(8 * per_g), dim3(256), 0, st, args, T, per_g);
 }
 
 // The value stream carries FP32 weights, so the kernel depends on B's dtype
-// and the values per lane only.
+// and the tile width only.
 static void launch_b(const SpmmArgs &args, int vec, int n, int bt, hipStream_t st) {
     if (bt == VNM_DT_F32) {
-        if (vec == 4) launch_v<VNM_DT_F32, 4>(args, n, st);
-        else if (vec == 2) launch_v<VNM_DT_F32, 2>(args, n, st);
-        else launch_v<VNM_DT_F32, 1>(args, n, st);
+        if (vec == 4) launch_v<VNM_DT_F32, 64>(args, n, st);
+        else if (vec == 2) launch_v<VNM_DT_F32, 32>(args, n, st);
+        else launch_v<VNM_DT_F32, 16>(args, n, st);
     } else if (bt == VNM_DT_BF16) {
-        if (vec == 8) launch_v<VNM_DT_BF16, 8>(args, n, st);
-        else if (vec == 4) launch_v<VNM_DT_BF16, 4>(args, n, st);
-        else if (vec == 2) launch_v<VNM_DT_BF16, 2>(args, n, st);
-        else launch_v<VNM_DT_BF16, 1>(args, n, st);
+        if (vec == 8) launch_v<VNM_DT_BF16, 64>(args, n, st);
+        else if (vec == 4) launch_v<VNM_DT_BF16, 32>(args, n, st);
+        else if (vec == 2) launch_v<VNM_DT_BF16, 16>(args, n, st);
+        else launch_v<VNM_DT_BF16, 8>(args, n, st);
     } else {
-        if (vec == 16) launch_v<VNM_DT_FP8, 16>(args, n, st);
-        else if (vec == 8) launch_v<VNM_DT_FP8, 8>(args, n, st);
-        else if (vec == 4) launch_v<VNM_DT_FP8, 4>(args, n, st);
-        else launch_v<VNM_DT_FP8, 2>(args, n, st);
+        if (vec == 16) launch_v<VNM_DT_FP8, 64>(args, n, st);
+        else if (vec == 8) launch_v<VNM_DT_FP8, 32>(args, n, st);
+        else if (vec == 4) launch_v<VNM_DT_FP8, 16>(args, n, st);
+        else if (vec == 2) launch_v<VNM_DT_FP8, 8>(args, n, st);
+        else launch_v<VNM_DT_FP8, 8, 8>(args, n, st);
     }
 }
 
@@ -857,7 +987,8 @@ int spmm_run(vnm_packed *p, int vec, const void *B, int ldb, int n, int bt, cons
         p->ctx->launches++;
     }
     if (p->nfix > 0) {
-        hipLaunchKernelGGL(k_spmm_fix, dim3((p->nfix + 3) / 4), dim3(256), 0, st, p->fix.p, p->nfix, part, n, n, C,
+        hipLaunchKernelGGL(k_spmm_fix, dim3((unsigned)((fix_waves(p->nfix, p->nhub, n) + 3) / 4)), dim3(256), 0, st,
+                           p->fix.p, p->nhub, p->fix_rest(), p->nfix - p->nhub, part, n, n, C,
                            ldc, bias, args.dvb, p->V);
         p->ctx->launches++;
     }
@@ -874,39 +1005,6 @@ static int spmm_v(vnm_packed *p, int vec, const void *B, int ldb, int n, int bt,
 }
 
 int shape_key(int bt, int n) { return (bt << 24) | n; }
-
-// Autotuner: time every usable values-per-lane setting on this matrix and
-// shape (one warm-up and three timed calls each, HIP events on the context
-// stream) and keep the fastest; the choice stays with the packed matrix.
-static int tune_vec(vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs, float *C, int ldc,
-                    const float *bias, int *best_v) {
-    hipStream_t st = p->ctx->stream;
-    hipEvent_t e0, e1;
-    VNM_HIP_TRY(hipEventCreate(&e0));
-    VNM_HIP_TRY(hipEventCreate(&e1));
-    float best = 1e30f;
-    int bv = 0, rc = VNM_OK;
-    for (int v = 16; v >= 1 && rc == VNM_OK; v /= 2) {
-        if (!vec_ok(bt, n, v)) continue;
-        if ((rc = spmm_v(p, v, B, ldb, n, bt, bs, C, ldc, bias, false))) break;
-        if (hipEventRecord(e0, st) != hipSuccess) { rc = set_error(VNM_E_HIP, "event record failed"); break; }
-        for (int i = 0; i < 3 && rc == VNM_OK; ++i) rc = spmm_v(p, v, B, ldb, n, bt, bs, C, ldc, bias, false);
-        if (rc) break;
-        float ms = 0.f;
-        if (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
-            hipEventElapsedTime(&ms, e0, e1) != hipSuccess) {
-            rc = set_error(VNM_E_HIP, "event timing failed");
-            break;
-        }
-        if (getenv("VNM_DEBUG")) fprintf(stderr, "[vnm] spmm tune bt=%d n=%d vec=%d %.4f ms\n", bt, n, v, ms / 3);
-        if (ms < best) { best = ms; bv = v; }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (rc) return rc;
-    *best_v = bv;
-    return VNM_OK;
-}
 
 int spmm_check(const vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs,
                       const float *C, int ldc) {
@@ -930,14 +1028,8 @@ int spmm(vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs, 
          const float *bias) {
     int rc = spmm_check(p, B, ldb, n, bt, bs, C, ldc);
     if (rc) return rc;
-    int v = 0;
-    auto it = p->shapes.find(shape_key(bt, n));
-    if (it != p->shapes.end()) {
-        v = it->second;
-    } else {
-        if ((rc = tune_vec(p, B, ldb, n, bt, bs, C, ldc, bias, &v))) return rc;
-        p->shapes[shape_key(bt, n)] = v;
-    }
+    // the shape stays with the packed matrix: vnm_spmm_get_shape reports it
+    const int v = p->shapes.emplace(shape_key(bt, n), default_vec(bt, n)).first->second;
     return spmm_v(p, v, B, ldb, n, bt, bs, C, ldc, bias, true);
 }
 
@@ -976,11 +1068,10 @@ int vnm_packed_info_get(const vnm_packed *p, vnm_packed_info *info) {
     const int blk = p->dtype == VNM_DT_FP8 ? 4 : 0;  // per-entry block index for the FP8 scale
     info->bytes = 4ll * (p->nrows + 1) + (int64_t)p->nent * (4 + 4 + 1 + 2 * vs + blk) +
                   (int64_t)p->nblocks * (4 + 2 + 4);
-    // the SpMM's value stream: (row, B row, FP32 weight) per value
-    info->bytes += (int64_t)p->nval * 12;
-    // what k_spmm reads: the value stream and the item table (first value
-    // and slot of each item)
-    info->spmm_bytes = (int64_t)p->nval * 12 + (int64_t)p->nitems * 8;
+    // the SpMM's value stream: (B row, FP32 weight) per value
+    info->bytes += (int64_t)p->nval * 8;
+    // what k_spmm reads: the value stream and the item table
+    info->spmm_bytes = (int64_t)p->nval * 8 + (int64_t)p->nitems * (int64_t)sizeof(Piece);
     info->items = p->nitems;
     info->slots = (int32_t)scratch_rows(p);
     info->dense_blocks = p->ndense;

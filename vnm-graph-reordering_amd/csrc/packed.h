@@ -23,18 +23,18 @@ struct vnm_packed {
     vnm::DBuf<uint8_t> ent_idx, ent_val;                   // values: 2 per entry, dtype-sized
     vnm::DBuf<uint16_t> blk_sel;
     vnm::DBuf<float> blk_scale;
-    // the SpMM's value stream: every value of the row entries, row-major, as
-    // (row, B row, FP32 weight), and VTAIL zero records past its end
+    // the SpMM's value stream: every value of the row entries as (B row, FP32
+    // weight), in the order of the work items -- pieces: whole rows of at most
+    // ITEM values, and the ITEM-value chunks of longer rows, whose partial sums go
+    // to slots -- which are sorted by length
     int32_t nval = 0;
-    vnm::DBuf<int32_t> vrow, vcol;
-    vnm::DBuf<float> vw;
-    // SpMM work items: whole rows of at most ITEM values, and rows longer
-    // than ITEM cut into ITEM-value chunks whose partial sums go to slots
-    int32_t nitems = 0, nslots = 0, nfix = 0;
-    vnm::DBuf<int32_t> item_beg;                           // nitems + 1 value offsets
-    vnm::DBuf<int32_t> item_slot;                          // slot of the item's first row, or -1
-    vnm::DBuf<int4> fix;                                   // {row, first slot, slots, 0}: rows the
-                                                           // fix-up pass writes (empty or cut)
+    vnm::DBuf<uint2> vrec;
+    int32_t nitems = 0, nslots = 0, nfix = 0, nhub = 0;
+    vnm::DBuf<int4> item;                                  // vnm::Piece
+    // rows the fix-up pass writes (empty or cut), {row, first slot, slots, 0}:
+    // the nhub hub rows from the front, the other nfix - nhub at the end
+    vnm::DBuf<int4> fix;
+    const int4 *fix_rest() const { return fix.p + (fix.n - (size_t)(nfix - nhub)); }
     vnm::DBuf<float> part;                                 // nslots x n partial sums
     // 2:4 sparse-MFMA part (dense.hip): blocks keeping >= dense_min values
     int32_t dense_min = 0, ndense = 0, nchunks = 0, ngroups = 0, nmulti = 0, ndslots = 0;
@@ -50,11 +50,19 @@ struct vnm_packed {
 
 namespace vnm {
 
-constexpr int ITEM = 64;      // values per work item
-constexpr int SBLK = 8;       // values per block of the SpMM's item walk
-constexpr int VTAIL = SBLK;   // zero records past the end of the value stream
-constexpr int GAP_MAX = 8;    // runs of rows without entries up to this long are written by the
-                              // item walk; longer runs by the fix-up pass (one wave per row)
+constexpr int ITEM = 64;      // most values of a work item, and values of a long row's chunk
+constexpr int SBLK = 8;       // gathers in flight per lane group of the SpMM
+constexpr int GAP_MAX = 8;    // runs of rows without entries up to this long, after an uncut row,
+                              // are written with that row; other such rows by the fix-up pass
+
+// A work item of the SpMM: `len` values from `beg` on in the value stream,
+// whose sum goes to row `row` of C (and `gap` rows without values after it get
+// the bias or zero) or, with `slot` set, to partial-sum slot `row`.
+struct Piece {
+    int32_t beg, len, row;
+    int16_t gap, slot;
+};
+static_assert(sizeof(Piece) == 16, "read as one int4");
 
 // ------------------------------------------------------------ value codecs
 
@@ -111,138 +119,94 @@ constexpr int bsize() { return BT == VNM_DT_F32 ? 4 : BT == VNM_DT_BF16 ? 2 : 1;
 
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 
-// VEC consecutive B values (VEC * sizeof(value) bytes, 2..16) of one row.
-template <int BT, int VEC>
+// LB bytes of one B row, as one lane gathers them: NV = LB / sizeof(value)
+// values.
+template <int LB>
 struct BRaw {
-    static constexpr int BYTES = VEC * bsize<BT>();
-    static constexpr int NW = BYTES < 4 ? 1 : BYTES / 4;
-    uint32_t w[NW];
+    uint32_t w[LB / 4];
 };
 
-template <int BT, int VEC>
-__device__ __forceinline__ BRaw<BT, VEC> zero_raw() {
-    BRaw<BT, VEC> r;
-#pragma unroll
-    for (int i = 0; i < BRaw<BT, VEC>::NW; ++i) r.w[i] = 0;
-    return r;
-}
-
 // acc += w * (decoded raw)
-template <int BT, int VEC>
-__device__ __forceinline__ void fma_raw(float (&acc)[VEC], float w, const BRaw<BT, VEC> &raw) {
+template <int BT, int LB>
+__device__ __forceinline__ void fma_raw(float (&acc)[LB / bsize<BT>()], float w, const BRaw<LB> &raw) {
+    constexpr int NV = LB / bsize<BT>();
     if constexpr (BT == VNM_DT_F32) {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) acc[i] = fmaf(w, __uint_as_float(raw.w[i]), acc[i]);
+        for (int i = 0; i < NV; ++i) acc[i] = fmaf(w, __uint_as_float(raw.w[i]), acc[i]);
     } else if constexpr (BT == VNM_DT_BF16) {
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) {
+        for (int i = 0; i < NV; ++i) {
             const uint32_t x = raw.w[i / 2];
             acc[i] = fmaf(w, __uint_as_float((i & 1) ? (x & 0xFFFF0000u) : (x << 16)), acc[i]);
         }
     } else {
         // OCP e4m3 through the gfx950 conversion, two values per call
 #pragma unroll
-        for (int i = 0; i < VEC; i += 4) {
+        for (int i = 0; i < NV; i += 4) {
             const uint32_t x = raw.w[i / 4];
             const f32x2_t lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)x, false);
+            const f32x2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)x, true);
             acc[i] = fmaf(w, lo.x, acc[i]);
             acc[i + 1] = fmaf(w, lo.y, acc[i + 1]);
-            if constexpr (VEC >= 4) {
-                const f32x2_t hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)x, true);
-                acc[i + 2] = fmaf(w, hi.x, acc[i + 2]);
-                acc[i + 3] = fmaf(w, hi.y, acc[i + 3]);
-            }
+            acc[i + 2] = fmaf(w, hi.x, acc[i + 2]);
+            acc[i + 3] = fmaf(w, hi.y, acc[i + 3]);
         }
     }
 }
 
-// Store a finished output row slice (plus the bias slice, when given).
-template <int NV>
-__device__ __forceinline__ void store_vec(float *__restrict__ cp, const float (&acc)[NV],
-                                          const float *__restrict__ bias) {
-    float v[NV];
+// A lane's NB runs of 4 columns, RUN columns apart: partial sums, rows of C
+// (nontemporal, so that the output stream does not push the gathered B rows out
+// of L2), and values added to them.
+template <int NB, int RUN>
+__device__ __forceinline__ void store_runs(float *__restrict__ p, const float (&v)[4 * NB]) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = bias ? acc[i] + bias[i] : acc[i];
-    if constexpr (NV % 4 == 0) {
-#pragma unroll
-        for (int i = 0; i < NV; i += 4) *(float4 *)(cp + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
-    } else if constexpr (NV == 2) {
-        *(float2 *)cp = make_float2(v[0], v[1]);
-    } else {
-        cp[0] = v[0];
-    }
+    for (int i = 0; i < NB; ++i)
+        *(float4 *)(p + i * RUN) = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
 }
 
-// store_vec for rows of C: nontemporal stores, so that the output stream
-// does not push the gathered B rows out of L2 (the same values land)
-template <int NV>
-__device__ __forceinline__ void store_vec_nt(float *__restrict__ cp, const float (&acc)[NV],
-                                             const float *__restrict__ bias) {
-    float v[NV];
+template <int NB, int RUN>
+__device__ __forceinline__ void store_runs_nt(float *__restrict__ p, const float (&v)[4 * NB]) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = bias ? acc[i] + bias[i] : acc[i];
-    if constexpr (NV % 4 == 0) {
-        typedef float f4 __attribute__((ext_vector_type(4)));
-#pragma unroll
-        for (int i = 0; i < NV; i += 4)
-            __builtin_nontemporal_store(f4{v[i], v[i + 1], v[i + 2], v[i + 3]}, (f4 *)(cp + i));
-    } else if constexpr (NV == 2) {
-        typedef float f2 __attribute__((ext_vector_type(2)));
-        __builtin_nontemporal_store(f2{v[0], v[1]}, (f2 *)cp);
-    } else {
-        __builtin_nontemporal_store(v[0], cp);
-    }
+    for (int i = 0; i < NB; ++i)
+        __builtin_nontemporal_store(f4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]}, (f4 *)(p + i * RUN));
 }
 
-template <int NV>
-__device__ __forceinline__ void load_vec(const float *__restrict__ cp, float (&v)[NV]) {
-    if constexpr (NV % 4 == 0) {
+template <int NB, int RUN>
+__device__ __forceinline__ void add_runs(float (&v)[4 * NB], const float *__restrict__ p) {
 #pragma unroll
-        for (int i = 0; i < NV; i += 4) {
-            const float4 x = *(const float4 *)(cp + i);
-            v[i] = x.x; v[i + 1] = x.y; v[i + 2] = x.z; v[i + 3] = x.w;
-        }
-    } else if constexpr (NV == 2) {
-        const float2 x = *(const float2 *)cp;
-        v[0] = x.x; v[1] = x.y;
-    } else {
-        v[0] = cp[0];
+    for (int i = 0; i < NB; ++i) {
+        const float4 x = *(const float4 *)(p + i * RUN);
+        v[4 * i] += x.x; v[4 * i + 1] += x.y; v[4 * i + 2] += x.z; v[4 * i + 3] += x.w;
     }
 }
 
 // One packed matrix as the SpMM kernels see it.
 struct SpmmArgs {
-    const int32_t *item_beg, *item_slot;
-    const int32_t *vrow, *vcol;  // the value stream
-    const float *vw;
+    const int4 *pieces;  // the work items (Piece)
+    const uint2 *vrec;   // the value stream: {B row, weight}
     const uint8_t *B;
     const float *b_scales;
     float *C;
     float *part;        // nslots x pn partial sums of cut rows
     const float *bias;  // nullptr or n floats added to every output row
     const uint8_t *dvb; // nullptr, or per V-row block 1 when C already holds the block's dense sums
-    int items, ldb, ldc, pn;
+    int items, ldb, ldc, pn;  // pn = n, the columns of the product
     int b_rows;         // rows of B (columns of A); b_rows * ldb * sizeof(value) < 2^32
     int c_rows;         // rows of C (of A)
     int V;
 };
 
-// VEC values of one B row for this lane, by a buffer load whose row offset
-// (soff) is a scalar and whose column offset (voff) is fixed per lane.
-template <int BT, int VEC>
-__device__ __forceinline__ BRaw<BT, VEC> load_row(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
-    BRaw<BT, VEC> r;
-    constexpr int BY = BRaw<BT, VEC>::BYTES;
-    if constexpr (BY == 16) {
-        const auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff, (int)soff, 0);
+// LB bytes of one B row for this lane.
+template <int LB>
+__device__ __forceinline__ BRaw<LB> load_row(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
+    BRaw<LB> r;
+    if constexpr (LB == 16) {
+        const auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
         r.w[0] = t[0]; r.w[1] = t[1]; r.w[2] = t[2]; r.w[3] = t[3];
-    } else if constexpr (BY == 8) {
-        const auto t = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)voff, (int)soff, 0);
-        r.w[0] = t[0]; r.w[1] = t[1];
-    } else if constexpr (BY == 4) {
-        r.w[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, (int)soff, 0);
     } else {
-        r.w[0] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)voff, (int)soff, 0);
+        const auto t = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, 0, 0);
+        r.w[0] = t[0]; r.w[1] = t[1];
     }
     return r;
 }
@@ -256,257 +220,177 @@ __device__ __forceinline__ float load_aval(const uint8_t *__restrict__ p, int i)
     else return e4m3_to_f32(p[i]);
 }
 
-__device__ __forceinline__ int lane_bcast(int v, int k) { return __builtin_amdgcn_readlane(v, k); }
-__device__ __forceinline__ float lane_bcast(float v, int k) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+// Value J (< SBLK) of this lane's group, from the lane that holds it: lanes
+// J and 8 + J of every row of 16 hold value J of their group.
+template <int LPR, int J>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
+    constexpr int NEWBCAST = 0x150;  // DPP row_newbcast: one lane of a row of 16 to the whole row
+    if constexpr (LPR >= 16) {
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, NEWBCAST + J, 0xF, 0xF, true);
+    } else {
+        // the two groups of a row of 16 one after the other (bank masks)
+        const int lo = __builtin_amdgcn_update_dpp((int)v, (int)v, NEWBCAST + J, 0xF, 0x3, false);
+        return (uint32_t)__builtin_amdgcn_update_dpp(lo, (int)v, NEWBCAST + 8 + J, 0xF, 0xC, false);
+    }
 }
 
-// C = A_vnm B for one work item (`cnt` <= ITEM values from `beg` on in the
-// value stream) and column tile `tile` of T (64 * VEC columns), one wave.  The
-// value stream holds every kept value of the row entries in row-major order
-// as (row, B row, weight); the weight is the stored value times its block's
-// scale (FP8 A), rounded to FP32 once at packing, as a product formed here
-// would be.  Lane k reads the row of value k and a ballot marks where rows
-// start; the wave then walks the item in blocks of 8 values.  A block's B
-// rows and weights are scalar loads, so per value the wave spends one scalar
-// multiply (the B row's byte offset), one buffer load (VEC consecutive values
-// of the B row per lane, 2 to 16 bytes) and VEC FMAs that take the weight as
-// a scalar operand: no per-value lane broadcasts or branches.  All 8 gathers
-// of a block are in flight before its FMAs, whatever the row lengths; the
-// FMAs go one row segment of the block at a time.  Each lane owns VEC
-// columns of the output row and stores them when the row ends; the rows that
-// keep nothing between it and the next (up to the next item's first row
-// `next_row`; item 0 also from row 0) get the bias or zero.  Items hold whole
-// rows, except chunks of rows longer than ITEM values: such a chunk is the
-// first row of its item, and its sum goes to the item's partial-sum slot
-// (slot >= 0) instead of C; the fix-up pass adds a cut row's slots in item
-// order.  So every output value is one fixed sequence of FP32 operations (the
-// row's values in order), whatever the launch shape.
-template <int BT, int VEC>
-__device__ __forceinline__ void spmm_item(const int32_t *__restrict__ vrow, const int32_t *__restrict__ vcol,
-                                          const float *__restrict__ vw, const float *__restrict__ bsc,
-                                          const uint8_t *__restrict__ B, float *__restrict__ C,
-                                          float *__restrict__ part, const float *__restrict__ bias,
-                                          const uint8_t *__restrict__ dvb, int V, int beg, int cnt, int slot,
-                                          int lead_row, int next_row, int ldb, int ldc, int pn, int b_rows,
-                                          int tile, int T) {
-    constexpr int SB = bsize<BT>();
+// f(integral_constant<int, J>) for J = 0 .. SBLK - 1.
+template <int J = 0, typename F>
+__device__ __forceinline__ void each_step(F &&f) {
+    if constexpr (J < SBLK) {
+        f(std::integral_constant<int, J>());
+        each_step<J + 1>(f);
+    }
+}
+
+// C = A_vnm B for 64 / LPR consecutive work items from item0 on and column
+// tile `tile` (LPR * LB bytes of every B row), one wave: LPR lanes per item, LB
+// bytes of a B row per lane.
+//
+// What bounds it is the gather: every kept value reads one B row's tile
+// through the vector L1, and a CU's L1 takes one 64-byte request a cycle, so
+// loads of 16 bytes per lane are the cheapest per byte.  Groups of lanes that
+// walk items of their own keep 16-byte loads whatever the tile width: one load
+// instruction fetches 64 / LPR tiles, one per item, and a tile can be as
+// narrow as 128 bytes of BF16 or FP8.  (One item per wave, with the B row's
+// offset a scalar, read 2 to 8 bytes per lane there.)
+//
+// Items are sorted by length, so the groups of a wave walk items of one length
+// (but where it changes) and end together.  Lane J of a group reads value J of a
+// block of SBLK: its B row's offset and weight reach the group's lanes by DPP.  The
+// gathers of a block are all in flight before its FMAs; the next block's values
+// are loaded before them.  Every output value is one fixed sequence of FP32
+// operations (the row's values in order; the fix-up pass adds a cut row's
+// chunks in order), whatever the launch shape.
+//
+// EXTRA: there is a bias, or rows that hold a dense part's sum.  turn: 64 NV
+// floats of LDS of the wave's own (NV = values of a lane) when NV > 4.
+template <int BT, int LPR, int LB, bool EXTRA>
+__device__ __forceinline__ void spmm_items(const SpmmArgs &a, int item0, int tile, float *turn) {
+    constexpr int SB = bsize<BT>(), NV = LB / SB;
     const int lane = threadIdx.x & 63;
-    const int rowb = ldb * SB;
-    const __amdgpu_buffer_rsrc_t rs =
-        __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)((uint32_t)b_rows * (uint32_t)rowb), 0x00020000);
-    const int rr = lane < cnt ? vrow[beg + lane] : 0;
-    const int first_row = lane_bcast(rr, 0);
-    // values that start a new row (value 0 does not: cur starts there)
-    const int prev_rr = __shfl_up(rr, 1, 64);
-    const uint64_t starts = __ballot(lane > 0 && lane < cnt && rr != prev_rr);
-    // the T column tiles interleave in 128-byte pieces (one L2 line of a B
-    // row): tile t takes pieces t, t + T, t + 2T, ... of every row, so each
-    // XCD's L2 holds its 1/T of B spread over the whole row
-    constexpr int LB = VEC * SB;  // bytes per lane and B row
-    auto tile_byte = [&](int b) { return ((b >> 7) * T + tile) * 128 + (b & 127); };
-    // 8 bytes per lane: two B rows per load instruction, 16 bytes per lane --
-    // lanes 0-31 read the tile of one row, lanes 32-63 that of the next, and
-    // two lane-half swaps (v_permlane32_swap) then give every lane both rows'
-    // 8 bytes for the columns it owns (lane i and i + 32 own the two halves
-    // of bytes [16i, 16i + 16))
-    constexpr bool PAIR = LB == 8;
-    const int upper = lane >> 5;
-    const int col0 = tile_byte(PAIR ? 16 * (lane & 31) + 8 * upper : lane * LB) / SB;
-    const int voff = PAIR ? tile_byte(16 * (lane & 31)) : col0 * SB;
-    const float *bias_c = bias ? bias + col0 : nullptr;
-    float acc[VEC];
-    int cur = first_row;
-    // rows whose V-row block has a dense part hold its sum already (written by
-    // the dense kernel): row sums add to it
-    auto dense_row = [&](int r) { return dvb != nullptr && dvb[r / V] != 0; };
-    // rows [r0, r1) -- a maximal run without values -- get the bias or zero
-    // (plus a dense sum); runs longer than GAP_MAX are the fix-up pass's, so
-    // no wave walks thousands of empty rows
-    auto fill = [&](int r0, int r1) {
-        if (r1 - r0 > GAP_MAX) return;
-        float z[VEC];
+    const int item = item0 + lane / LPR;
+    int4 pc = make_int4(0, 0, 0, 0);
+    if (item < a.items) pc = a.pieces[item];
+    const int len = pc.y;
+    const uint32_t rowb = (uint32_t)a.ldb * SB;
+    const uint32_t bytes = (uint32_t)(a.b_rows - 1) * rowb + (uint32_t)a.pn * SB;  // B up to its last value
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void *)a.B, 0, (int)bytes, 0x00020000);
+    const uint32_t voff = (uint32_t)(tile * LPR + lane % LPR) * LB;
+    // a lane without a value gathers from past B's end, where a buffer load
+    // reads nothing (or, when B ends within a row of 4 GiB, from some row of
+    // B), and only its own group's sum, which is complete, is kept below
+    const uint32_t none = 0xFFFFFF00u - rowb;
+    const uint2 *__restrict__ vals = a.vrec + pc.x;
+    const int mine = lane % SBLK;
+    float acc[NV];
 #pragma unroll
-        for (int i = 0; i < VEC; ++i) z[i] = 0.f;
-        for (int r = r0; r < r1; ++r) {
-            float *cp = C + (size_t)r * ldc + col0;
-            if (dense_row(r)) {
-                if (bias_c) {
-                    float d[VEC];
-                    load_vec<VEC>(cp, d);
-                    store_vec<VEC>(cp, d, bias_c);
-                }
-            } else {
-                store_vec_nt<VEC>(cp, z, bias_c);
-            }
-        }
-    };
-    fill(lead_row, first_row);
-    // the finished row `cur`: to its slot when it is the item's cut first row
-    auto flush = [&]() {
-        if (slot >= 0 && cur == first_row) {
-            store_vec<VEC>(part + (size_t)slot * pn + col0, acc, nullptr);
+    for (int i = 0; i < NV; ++i) acc[i] = 0.f;
+    uint2 v = mine < len ? vals[mine] : make_uint2(0u, 0u);
+    // one block of values from k0 on: all SBLK of them, or (LAST) the first
+    // `m` only, m uniform over the wave
+    auto block = [&](auto LAST, int k0, int m) {
+        constexpr bool last = decltype(LAST)::value;
+        const bool live = k0 + mine < len;
+        uint32_t off = live ? v.x * rowb : none, w = v.y;
+        if constexpr (BT == VNM_DT_FP8) w = __float_as_uint(__uint_as_float(w) * a.b_scales[v.x >> 7]);
+        if (!last && k0 + SBLK + mine < len) v = vals[k0 + SBLK + mine];
+        BRaw<LB> raw[SBLK];
+        each_step([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            if (!last || j < m) raw[j] = load_row<LB>(rs, voff + group_bcast<LPR, j>(off));
+        });
+        if (!last && k0 + SBLK <= len) {
+            each_step([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                fma_raw<BT, LB>(acc, __uint_as_float(group_bcast<LPR, j>(w)), raw[j]);
+            });
         } else {
-            float *cp = C + (size_t)cur * ldc + col0;
-            if (dense_row(cur)) {
-                float d[VEC];
-                load_vec<VEC>(cp, d);
-#pragma unroll
-                for (int i = 0; i < VEC; ++i) acc[i] += d[i];
-            }
-            store_vec_nt<VEC>(cp, acc, bias_c);
+            each_step([&](auto J) {
+                constexpr int j = decltype(J)::value;
+                if (last && j >= m) return;
+                const float wj = __uint_as_float(group_bcast<LPR, j>(w));
+                if (k0 + j < len) fma_raw<BT, LB>(acc, wj, raw[j]);
+            });
         }
     };
+    // items come in descending length, so the wave's longest is its first
+    const int mlen = __builtin_amdgcn_readfirstlane(len);
+    int k0 = 0;
+    for (; k0 + SBLK <= mlen; k0 += SBLK) block(std::false_type(), k0, SBLK);
+    if (k0 < mlen) block(std::true_type(), k0, mlen - k0);
+    // lane l of a group of BF16 or FP8 lanes holds columns NV l .. NV l + NV - 1
+    // of the tile: through LDS to 4 l .. 4 l + 3 of each run of 4 LPR columns, so
+    // that a store writes whole lines (partial ones cost FP8 4 times the requests)
+    constexpr int NB = NV / 4;
+    const int l = lane % LPR;
+    if constexpr (NB > 1) {
+        float *t = turn + (lane - l) * NV;
 #pragma unroll
-    for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-    const int32_t *__restrict__ cp = vcol + beg;
-    const float *__restrict__ wp = vw + beg;
-    // the B row of one value (the weight picks up the B row's FP8 scale)
-    auto gather = [&](int c, float &w) {
-        if constexpr (BT == VNM_DT_FP8) w *= bsc[c >> 7];
-        return load_row<BT, VEC>(rs, voff, (uint32_t)c * (uint32_t)rowb);
-    };
-    // the B rows of two values (PAIR), each lane's offset in full in the
-    // per-lane operand (in range, like every B row)
-    auto gather2 = [&](int c0, float &w0, int c1, float &w1, BRaw<BT, VEC> &r0, BRaw<BT, VEC> &r1) {
-        if constexpr (BT == VNM_DT_FP8) {
-            w0 *= bsc[c0 >> 7];
-            w1 *= bsc[c1 >> 7];
-        }
-        const uint32_t o0 = __builtin_amdgcn_readfirstlane((uint32_t)c0 * (uint32_t)rowb);
-        const uint32_t o1 = __builtin_amdgcn_readfirstlane((uint32_t)c1 * (uint32_t)rowb);
-        const uint32_t vo = (uint32_t)voff + (upper ? o1 : o0);
-        const auto t = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)vo, 0, 0);
-        const auto s0 = __builtin_amdgcn_permlane32_swap(t[0], t[2], false, false);
-        const auto s1 = __builtin_amdgcn_permlane32_swap(t[1], t[3], false, false);
-        r0.w[0] = s0[0];
-        r0.w[1] = s1[0];
-        r1.w[0] = s0[1];
-        r1.w[1] = s1[1];
-    };
-    // blocks of 8 values (the item's last may hold fewer, m): their B rows and
-    // weights by scalar loads, all gathers in flight, then the FMAs in value
-    // order, one row segment of the block at a time (a block without a row
-    // start is one segment)
-    constexpr int BLK = SBLK;
-    for (int k0 = 0; k0 < cnt; k0 += BLK) {
-        const int m = min(BLK, cnt - k0);
-        int c[BLK];
-        float w[BLK];
+        for (int i = 0; i < NV; i += 4) *(float4 *)(t + l * NV + i) = make_float4(acc[i], acc[i + 1], acc[i + 2], acc[i + 3]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int t = 0; t < BLK; ++t) {  // past the item: later items or the stream's zero tail
-            c[t] = cp[k0 + t];
-            w[t] = wp[k0 + t];
-        }
-        BRaw<BT, VEC> raw[BLK];
-        if constexpr (PAIR) {
-            if (m == BLK) {
-#pragma unroll
-                for (int t = 0; t < BLK; t += 2) gather2(c[t], w[t], c[t + 1], w[t + 1], raw[t], raw[t + 1]);
-            } else {
-                float wd = 0.f;
-                BRaw<BT, VEC> rd;
-#pragma unroll
-                for (int t = 0; t < BLK; t += 2) {
-                    if (t + 1 < m) gather2(c[t], w[t], c[t + 1], w[t + 1], raw[t], raw[t + 1]);
-                    else if (t < m) gather2(c[t], w[t], c[t], wd, raw[t], rd);  // the last, unpaired
-                }
-            }
-        } else if (m == BLK) {
-#pragma unroll
-            for (int t = 0; t < BLK; ++t) raw[t] = gather(c[t], w[t]);
-        } else {
-#pragma unroll
-            for (int t = 0; t < BLK; ++t)
-                if (t < m) raw[t] = gather(c[t], w[t]);
-        }
-        // values of this block that start a row (value 0's bit is clear)
-        uint32_t rem = (uint32_t)(starts >> k0) & ((1u << BLK) - 1u);
-        if (m == BLK && rem == 0) {
-#pragma unroll
-            for (int t = 0; t < BLK; ++t) fma_raw<BT, VEC>(acc, w[t], raw[t]);
-            continue;
-        }
-        for (int t0 = 0;;) {
-            // values [t0, t1) of the block belong to row `cur`
-            const int t1 = rem ? (int)__builtin_ctz(rem) : m;
-            const uint32_t seg = ((1u << t1) - 1u) & ~((1u << t0) - 1u);
-#pragma unroll
-            for (int t = 0; t < BLK; ++t)
-                if ((seg >> t) & 1u) fma_raw<BT, VEC>(acc, w[t], raw[t]);
-            if (!rem) break;
-            // a new row starts at value k0 + t1
-            flush();
-#pragma unroll
-            for (int i = 0; i < VEC; ++i) acc[i] = 0.f;
-            const int nxt = lane_bcast(rr, k0 + t1);
-            fill(cur + 1, nxt);
-            cur = nxt;
-            t0 = t1;
-            rem &= rem - 1u;
+        for (int i = 0; i < NB; ++i) {
+            const float4 x = *(const float4 *)(t + i * 4 * LPR + 4 * l);
+            acc[4 * i] = x.x; acc[4 * i + 1] = x.y; acc[4 * i + 2] = x.z; acc[4 * i + 3] = x.w;
         }
     }
-    flush();
-    fill(cur + 1, next_row);
+    if (len == 0) return;
+    const int c0 = tile * LPR * NV + 4 * l;  // first column of run 0
+    constexpr int RUN = 4 * LPR;
+    if (pc.w >> 16) {
+        store_runs<NB, RUN>(a.part + (size_t)pc.z * a.pn + c0, acc);
+        return;
+    }
+    float *cp = a.C + (size_t)pc.z * a.ldc + c0;
+    const int gap = pc.w & 0xFFFF;
+    for (int i = 0; i <= gap; ++i) {
+        if constexpr (EXTRA) {
+            // rows whose V-row block has a dense part hold its sum already
+            // (written by the dense kernel): row sums add to it
+            if (a.dvb != nullptr && a.dvb[(pc.z + i) / a.V] != 0) add_runs<NB, RUN>(acc, cp);
+            if (a.bias) add_runs<NB, RUN>(acc, a.bias + c0);
+        }
+        store_runs_nt<NB, RUN>(cp, acc);
+#pragma unroll
+        for (int q = 0; q < NV; ++q) acc[q] = 0.f;
+        cp += a.ldc;
+    }
 }
 
-// Work item `item` (wave-uniform), column tile `tile` of T of one packed matrix.
-template <int BT, int VEC>
-__device__ __forceinline__ void spmm_unit(const SpmmArgs &a, int item, int tile, int T) {
-    const int beg = a.item_beg[item];
-    const int end = a.item_beg[item + 1];
-    // rows that keep nothing: item 0 fills those before its first row, every
-    // item those between its rows and after its last, up to the next item's
-    // first row (the last item: up to the row count)
-    const int lead = item == 0 ? 0 : a.c_rows;
-    const int next_row = item + 1 < a.items ? a.vrow[end] : a.c_rows;
-    spmm_item<BT, VEC>(a.vrow, a.vcol, a.vw, a.b_scales, a.B, a.C, a.part, a.bias, a.dvb, a.V, beg, end - beg,
-                       a.item_slot[item], lead, next_row, a.ldb, a.ldc, a.pn, a.b_rows, tile, T);
-}
-
-// Fix-up of one listed row (a wave): the sum of its `ns` partial-sum slots
-// from `s0` on, in slot order, plus the row's dense sum when it has one,
-// plus the bias; a matrix without work items lists every row with ns = 0.  The slots' loads go out
-// 16 at a time before they are added (in order), so a row of many chunks
-// waits for a few round trips rather than one per slot.
+// Fix-up of some columns of one listed row (a wave, W columns per lane from
+// c0 + W lane on): the sum of its `ns` partial-sum slots from `s0` on, in slot
+// order, plus the row's dense sum when it has one, plus the bias.  What bounds it
+// is the chain of round trips: FB slots' loads go out before they are added, in
+// order.  Most cut rows have a few slots: those and the rows without values
+// (ns = 0) take 4 columns per lane and 8 slots at a time; the hub rows, listed
+// first, 1 column per lane and 32 slots.
+constexpr int HUB_SLOTS = 16;  // a row of more slots is a hub row
+template <int W, int FB>
 __device__ __forceinline__ void fix_row(float *__restrict__ crow, const float *__restrict__ part, int pn, int s0,
-                                        int ns, int n, const float *__restrict__ bias, bool dense) {
-    constexpr int FB = 16;
-    const int lane = threadIdx.x & 63;
-    for (int c = lane * 4; c < n; c += 256) {
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        const float *pc = part + (size_t)s0 * pn + c;
-        for (int j0 = 0; j0 < ns; j0 += FB) {
-            float4 v[FB];
+                                        int ns, int c0, int n, const float *__restrict__ bias, bool dense) {
+    typedef float vec __attribute__((ext_vector_type(W)));
+    const int c = c0 + W * (threadIdx.x & 63);
+    if (c >= n) return;
+    vec acc = (vec)0.f;
+    const float *pc = part + (size_t)s0 * pn + c;
+    for (int j0 = 0; j0 < ns; j0 += FB) {
+        vec v[FB];
 #pragma unroll
-            for (int j = 0; j < FB; ++j)
-                v[j] = j0 + j < ns ? *(const float4 *)(pc + (size_t)(j0 + j) * pn) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int j = 0; j < FB; ++j) v[j] = j0 + j < ns ? *(const vec *)(pc + (size_t)(j0 + j) * pn) : (vec)0.f;
 #pragma unroll
-            for (int j = 0; j < FB; ++j) {
-                if (j0 + j < ns) {
-                    acc.x += v[j].x;
-                    acc.y += v[j].y;
-                    acc.z += v[j].z;
-                    acc.w += v[j].w;
-                }
-            }
-        }
-        if (dense) {  // the row's dense sum, written by the dense kernel
-            const float4 d = *(const float4 *)(crow + c);
-            acc.x += d.x;
-            acc.y += d.y;
-            acc.z += d.z;
-            acc.w += d.w;
-        }
-        if (bias) {
-            const float4 b = *(const float4 *)(bias + c);
-            acc.x += b.x;
-            acc.y += b.y;
-            acc.z += b.z;
-            acc.w += b.w;
-        }
-        *(float4 *)(crow + c) = acc;
+        for (int j = 0; j < FB; ++j)
+            if (j0 + j < ns) acc += v[j];
     }
+    if (dense) acc += *(const vec *)(crow + c);  // written by the dense kernel
+    if (bias) acc += *(const vec *)(bias + c);
+    *(vec *)(crow + c) = acc;
+}
+
+// Waves of a fix-up pass over nfix rows, the first nhub of them hub rows, and
+// wave w's row and first column.
+__host__ __device__ inline int64_t fix_waves(int nfix, int nhub, int n) {
+    return (int64_t)nhub * (n / 64) + (int64_t)(nfix - nhub) * ((n + 255) / 256);
 }
 
 // ------------------------------------------------------------ host helpers (pack.hip)
@@ -515,6 +399,8 @@ int ensure_part(vnm_packed *p, int n);
 size_t scratch_rows(const vnm_packed *p);
 int bsize_of(int bt);
 bool vec_ok(int bt, int n, int vec);
+int default_vec(int bt, int n);
+int tile_items(int bt, int vec);
 SpmmArgs packed_args(const vnm_packed *p, const void *B, int ldb, const float *bs, float *C, int ldc,
                      const float *bias, float *part, int pn);
 int spmm(vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs, float *C, int ldc,
