@@ -882,9 +882,10 @@ __global__ void k_lp_pick(LPCtl *ctl, int nseg, int M, int mode0, uint64_t seed0
     dbest[s] = (int8_t)bdi;
     abest[s] = (int8_t)bai;
     // (score descending, segment) in 32 + sbits bits, sbits the bits of the
-    // largest segment index: the keys' order, sorted on those bits only
-    // one array for one sort: donors first, acceptors after them (bit
-    // 32 + sbits set), a segment without a donor the last of the donors
+    // largest segment index.  One array for one sort: donors first, acceptors after
+    // them (bit 32 + sbits set), a segment without a donor the last of the
+    // donors.  Each half is in segment order already, so the (stable) sort compares
+    // the score and the bit above it only.
     const uint64_t low = (1ull << (32 + sbits)) - 1;
     dkey[s] = bdi >= 0 ? ((uint64_t)(~ord_f32(bd)) << sbits) | (uint32_t)s : low;
     akey[s] = (low + 1) | ((uint64_t)(~ord_f32(ba)) << sbits) | (uint32_t)s;
@@ -1376,9 +1377,8 @@ static int build_lists(vnm_graph *g, uint64_t *keys, uint64_t *tmp, int64_t n, i
                        DBuf<int32_t> &ptr, DBuf<int32_t> &idx, std::vector<int32_t> &hptr) {
     hipStream_t st = g->ctx->stream;
     const int R = g->nrows;
-    int bits = 1;
-    while ((1ll << bits) <= R) ++bits;
-    int rc = sort_keys_u64(keys, tmp, n, 32 + bits, st);
+    // members are below R; entries outside the graph have owner R and sort last
+    int rc = sort_keys_u64(keys, tmp, n, key_halves(bits_for(R - 1), bits_for(R)), st);
     if (rc) return rc;
     if ((rc = ptr.alloc(R + 1)) || (rc = idx.alloc(std::max<int64_t>(nvalid, 1)))) return rc;
     VNM_HIP_TRY(hipMemsetAsync(ptr.p, 0, (R + 1) * 4, st));  // stays all zero when nothing is valid
@@ -1747,10 +1747,9 @@ static int lp_run_begin(LPRun &r, vnm_graph *g, const vnm_lp_model *m, int N, in
     r.nnorm = std::max(1, std::min(topk, ns));
     r.ncap = mode == 1 ? r.nnorm : r.nnorm * window;
     // sort keys hold a segment or candidate index in their low bits
-    auto bits_of = [](int64_t x) { int b = 1; while ((1ll << b) <= x) ++b; return b; };
-    r.sbits = bits_of(ns - 1);
-    r.ibits = bits_of(r.ncap - 1);
-    r.gbits = bits_of(2 * (int64_t)g->nrows);
+    r.sbits = bits_for(ns - 1);
+    r.ibits = bits_for(r.ncap - 1);
+    r.gbits = bits_for(2 * (int64_t)g->nrows);
     r.gmax = (uint32_t)((1ull << r.gbits) - 1);
     r.smask = (1ull << r.sbits) - 1;
     r.imask = (1ull << r.ibits) - 1;
@@ -1793,7 +1792,8 @@ static int lp_run_iter(LPRun &r) {
                        c->ptr.p, c->ccls.p, c->segcls.p, c->Y.p, w.dkey.p, w.dkey.p + ns, w.dbest.p, w.abest.p,
                        r.sbits);
     VNM_LAUNCH_CHECK("k_lp_pick");
-    if ((rc = sort_keys_u64_if(w.dkey.p, w.sdkey.p, 2 * (int64_t)ns, 33 + r.sbits, st, &ctl->done))) return rc;
+    if ((rc = sort_keys_u64_if(w.dkey.p, w.sdkey.p, 2 * (int64_t)ns, key_range(r.sbits, 33 + r.sbits), st,
+                               &ctl->done))) return rc;
     hipLaunchKernelGGL(k_lp_ctl_mid, dim3(1), dim3(64), 0, st, ctl, r.topk, r.window, ns);
     hipLaunchKernelGGL(k_lp_match, dim3(grid_of(r.nnorm, 256)), dim3(256), 0, st, ctl, r.window, ns, M, r.mode,
                        r.seed, w.sdkey.p, w.sdkey.p + ns, w.dbest.p, w.abest.p, g->inv.p, c->Y.p, w.cand.p, r.smask);
@@ -1802,7 +1802,8 @@ static int lp_run_iter(LPRun &r) {
     hipLaunchKernelGGL(k_lp_gain_keys, dim3(grid_of(r.ncap, 256)), dim3(256), 0, st, ctl, r.ncap, w.cand.p,
                        w.best.p, w.gkey.p, r.ibits, r.gmax);
     // one candidate per donor: the first nnorm keys; the whole window: ncap
-    const int kbits = r.gbits + r.ibits;
+    // keys come in candidate order, so the sort leaves their low ibits alone
+    const KeyBits kbits = key_range(r.ibits, r.gbits + r.ibits);
     if (r.mode != 2 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.nnorm, kbits, st, &ctl->skip_norm))) return rc;
     if (r.mode != 1 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.ncap, kbits, st, &ctl->skip_exh))) return rc;
     const size_t shm = (size_t)((ns + 31) / 32) * 4;

@@ -1433,7 +1433,8 @@ int build_csc_unique(vnm_graph *g) {
                            k0.p);
         g->ctx->launches++;
         VNM_LAUNCH_CHECK("k_csc_keys");
-        if ((rc = sort_keys_u64(k0.p, k1.p, n, 64, st))) return rc;
+        // ids are below R; the other entries' all-ones keys sort last
+        if ((rc = sort_keys_u64(k0.p, k1.p, n, key_halves(bits_for(R - 1), bits_for(R)), st))) return rc;
         hipLaunchKernelGGL(k_csc_unique, dim3(grid_for(n, 256)), dim3(256), 0, st, k1.p, n, rows.p, flags.p,
                            g->cptr.p);
         g->ctx->launches++;

@@ -62,12 +62,6 @@ static int grid_of(int64_t n, int block) {
     return (int)std::max<int64_t>(1, std::min<int64_t>(g, 1 << 20));
 }
 
-static int bits_for(int64_t x) {
-    int b = 1;
-    while ((1ll << b) <= x) ++b;
-    return b;
-}
-
 // ------------------------------------------------------------ value codecs
 
 // ------------------------------------------------------------ packer kernels
@@ -659,7 +653,7 @@ static int build_items(vnm_packed *p, const int32_t *vrp, int64_t values, PieceB
     if ((rc = scan_excl_i32(P.np.p, P.pbase.p, R + 1, st))) return rc;
     hipLaunchKernelGGL(k_pieces, dim3(grid_of(R, 256)), dim3(256), 0, st, vrp, R, P.pbase.p, P.slot0.p, P.gap.p, cap,
                        P.key.p, P.id.p, P.info.p);
-    if ((rc = sort_pairs_u64_i32(P.key.p, P.key2.p, P.id.p, P.order.p, cap, 7, st))) return rc;
+    if ((rc = sort_pairs_u64_i32(P.key.p, P.key2.p, P.id.p, P.order.p, cap, key_range(0, 7), st))) return rc;
     hipLaunchKernelGGL(k_piece_lens, dim3(grid_of(cap, 256)), dim3(256), 0, st, P.order.p, P.info.p, cap, P.len.p);
     if ((rc = scan_excl_i32(P.len.p, P.beg.p, cap, st))) return rc;
     hipLaunchKernelGGL(k_items, dim3(grid_of(cap, 256)), dim3(256), 0, st, P.pbase.p + R, P.order.p, P.info.p, P.beg.p,
@@ -702,7 +696,11 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
     const int gb = grid_of(nnz, 256);
     hipLaunchKernelGGL(k_nz_keys, dim3(gb), dim3(256), 0, st, g->row.p, g->col.p, g->val.p, nnz,
                        nseg * M, keys.p, idx.p);
-    if ((rc = sort_pairs_u64_i32(keys.p, keys2.p, idx.p, idx2.p, nnz, 64, st))) return rc;
+    // rows are below R and columns below nseg * M; dropped entries' all-ones
+    // keys sort last
+    if ((rc = sort_pairs_u64_i32(keys.p, keys2.p, idx.p, idx2.p, nnz,
+                                 key_halves(bits_for((int64_t)nseg * M - 1), bits_for(R)), st)))
+        return rc;
     // count of nonzero entries = position of the first ~0 key
     std::vector<uint64_t> hk(1);
     int64_t nz = nnz;
@@ -745,8 +743,9 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
         VNM_HIP_TRY(hipMemsetAsync(rlen.p, 0, (size_t)U * 4, st));
         hipLaunchKernelGGL(k_pk_runs, dim3(grid_of(nz, 256)), dim3(256), 0, st, keys2.p, head.p,
                            excl.p, nz, M, V, nblk, bits.p, rstart.p, rlen.p, bkey.p, rid.p);
-        const int kb = 32 + bits_for((int64_t)nseg * nblk);
-        if ((rc = sort_pairs_u64_i32(bkey.p, bkey2.p, rid.p, rid2.p, U, std::min(64, kb), st))) return rc;
+        if ((rc = sort_pairs_u64_i32(bkey.p, bkey2.p, rid.p, rid2.p, U,
+                                     key_halves(bits_for(R - 1), bits_for((int64_t)nseg * nblk)), st)))
+            return rc;
         hipLaunchKernelGGL(k_blk_heads, dim3(grid_of(U, 256)), dim3(256), 0, st, bkey2.p, U, bhead.p);
         if ((rc = scan_excl_i32(bhead.p, bexcl.p, U, st))) return rc;
         int32_t last[2];

@@ -10,13 +10,29 @@
 
 namespace vnm {
 
-// Stable LSD radix sort on bits [0, end_bit) of the keys (the input is not
-// written; out must not alias it).
-int sort_keys_u64(const uint64_t *in, uint64_t *out, int64_t n, int end_bit, hipStream_t st);
+// The bits of a 64-bit key that a sort compares: w0 bits from s0 on, and (w1 >
+// 0, then w0 < 64) w1 more significant ones from s1 on.  Bits in neither range may
+// hold anything; they move with the key.
+struct KeyBits {
+    int s0, w0, s1, w1;
+};
+inline KeyBits key_range(int begin, int end) { return KeyBits{begin, end - begin, 0, 0}; }
+// (hi, lo) keys of two 32-bit halves, the low half below 2^lo, the high half below 2^hi
+inline KeyBits key_halves(int lo, int hi) { return KeyBits{0, lo, 32, hi}; }
+// Bits that hold 0 .. x.
+inline int bits_for(int64_t x) {
+    int b = 1;
+    while ((1ll << b) <= x) ++b;
+    return b;
+}
+
+// Stable LSD radix sort on those bits (the input is not written; out must not
+// alias it).
+int sort_keys_u64(const uint64_t *in, uint64_t *out, int64_t n, KeyBits bits, hipStream_t st);
 // sort_keys_u64 whose kernels all return at once while *skip is nonzero
 // (read on the device when they run: a launch chain enqueued ahead of the
 // decision)
-int sort_keys_u64_if(const uint64_t *in, uint64_t *out, int64_t n, int end_bit, hipStream_t st, const int *skip);
+int sort_keys_u64_if(const uint64_t *in, uint64_t *out, int64_t n, KeyBits bits, hipStream_t st, const int *skip);
 // Grow this host thread's current scratch slot to what a sort of n keys
 // (with values) needs, so that sorts up to that size allocate nothing (as
 // under capture).
@@ -26,7 +42,7 @@ int sort_scratch_reserve(int64_t n);
 // concurrently need separate slots.
 int sort_scratch_slot(int slot);
 int sort_pairs_u64_i32(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t *vout,
-                       int64_t n, int end_bit, hipStream_t st);
+                       int64_t n, KeyBits bits, hipStream_t st);
 int scan_excl_i32(const int32_t *in, int32_t *out, int64_t n, hipStream_t st);
 int scan_incl_max_i32(const int32_t *in, int32_t *out, int64_t n, hipStream_t st);
 // out[j] = in[i] for the j-th i with flags[i] != 0, in order; *d_count = j's.

@@ -3,31 +3,38 @@
 // stable `sorted` over per-row keys), the packer's (row, column) and
 // (block, row) orders and the proposer's adjacency builds.
 //
-// Radix sort: LSD, 8-bit digits, one pass per digit of [0, end_bit).  A tile
-// is 4,096 keys, 1,024 per wave of a 256-thread workgroup.  Per pass:
-//   k_radix_hist     the tile's digit counts (LDS atomics), written
-//                    digit-major (hist[d * tiles + t]);
-//   scan             exclusive sum of the digit-major counts: the output
-//                    offset of (digit d, tile t) -- all smaller digits first,
-//                    then the earlier tiles' keys of digit d;
-//   k_radix_scatter  each wave ranks its 1,024 keys in 16 rounds of 64: the
-//                    lanes of a round holding one digit find each other with
-//                    8 ballots (one per digit bit), the lowest of them adds
-//                    the group's size to the wave's running count of the
-//                    digit (LDS), so a key's rank is its wave's count so far
-//                    plus the lanes below it in the group.  Waves' counts are
-//                    then prefixed in wave order, the tile's keys placed in
-//                    LDS in digit order, and written out with consecutive
-//                    lanes on consecutive output positions.
+// Radix sort: LSD over the key's sorted bits (KeyBits: one or two ranges of the
+// 64, so that the unused bits between a key's fields cost no pass), digits of at
+// most 8 bits, one pass per digit.  A tile is 4,096 keys, 256 per wave of a
+// 1,024-thread workgroup.  Every pass ranks a tile's keys the same way: a wave
+// takes its keys 64 at a time; the lanes holding one digit find each other
+// with a ballot per digit bit, the lowest of them adds the group's size to the
+// wave's running count of the digit (LDS), so a key's rank is its wave's count
+// so far plus the lanes below it in the group.  Waves' counts are then prefixed in
+// wave order, the tile's keys placed in LDS in digit order, and written out with
+// consecutive lanes on consecutive output positions.  A pass is bound by this
+// chain, not by its bytes, so a tile has 16 waves of 4 rounds (4 waves of 16:
+// 12.5 us a pass at 16,384 keys).
+//   up to 4,096 keys  all passes in one launch of one workgroup, the keys in
+//                     registers and LDS (k_sort_one)
+//   up to 65,536      one launch per pass: each tile derives its offsets from
+//                     the pass's count table and counts the next pass's digits
+//                     for its destination tiles (k_radix_fused); up to 16,384
+//                     keys in tiles of 1,024, which spread the ranking's vector
+//                     work over 16 CUs (16,384 keys of 33 bits: 65 us on one CU
+//                     in one launch, 85 in 6 launches of 4-wave tiles of 4,096)
+//   more              three: digit counts per tile (k_radix_hist, digit-major),
+//                     a workgroup per digit scanning its tiles' counts
+//                     (k_digit_scan), k_radix_scatter (1 M pairs: 39 us a pass
+//                     with 4-wave tiles and a three-launch scan, 21 now)
 // Every step keeps input order among equal digits, so each pass -- and the
 // sort -- is stable.  Passes ping-pong between the output and a scratch
 // buffer so the last one lands in the output; the input is never written.
 //
-// Scan: tiles of 4,096 elements; per-tile totals (k_scan_reduce), one
-// workgroup scanning the totals (k_scan_totals), then each tile scanned in
-// LDS with its offset (k_scan_tile).  Sum and max, int32 or uint8 input.
-// Inputs of at most one tile are sorted (k_radix_small) or scanned
-// (k_scan_small) by one workgroup in one launch.
+// Scan: tiles of 4,096 elements; per-tile totals (k_scan_reduce), then each
+// tile scanned in LDS from the sum of the totals before it (k_scan_tile; over
+// SCAN_DIRECT tiles one workgroup scans the totals first, k_scan_totals).  Sum and
+// max, int32 or uint8 input; at most one tile in one launch (k_scan_small).
 // Compaction: exclusive sum of the flags, then a scatter of flagged items.
 #include "sortlib.h"
 
@@ -37,11 +44,16 @@ namespace vnm {
 
 namespace {
 
-constexpr int WG = 256;                 // threads per workgroup
+constexpr int WG = 256;                 // threads per workgroup of the scans
 constexpr int NWAVE = WG / 64;
-constexpr int ROUNDS = 16;              // 64-key rounds per wave and tile
-constexpr int TILE = WG * ROUNDS;       // 4,096 keys per tile
+constexpr int ROUNDS = 16;              // elements per thread of a scan tile
+constexpr int TILE = WG * ROUNDS;       // 4,096 elements per tile
 constexpr int RADIX = 256;
+constexpr int SWG = 1024;               // threads per workgroup of the sort
+constexpr int SWAVE = SWG / 64;
+constexpr int SROUNDS = TILE / SWG;     // 64-key rounds per wave and tile
+constexpr int FWG = 256;                // ... of the fused sort's small tiles
+constexpr int SCAN_DIRECT = 2048;       // scan tiles whose totals each tile sums itself
 
 // Scratch of the calling host thread, grown on demand (one per thread, so
 // concurrent contexts on worker threads do not share it).
@@ -123,183 +135,253 @@ struct OpMax {
 
 // ------------------------------------------------------------ radix sort
 
-__device__ __forceinline__ int digit_of(uint64_t k, int shift, int bits) {
-    return (int)((k >> shift) & ((1u << bits) - 1u));
+// The sorted bits of a key as one number: w0 bits from s0 on, then (w1 > 0) the
+// bits from s1 on.
+__device__ __forceinline__ uint64_t sort_bits(const KeyBits &b, uint64_t k) {
+    uint64_t c = k >> b.s0;
+    if (b.w1) c = (c & ((1ull << b.w0) - 1)) | ((k >> b.s1) << b.w0);
+    return c;
 }
 
-__global__ __launch_bounds__(WG) void k_radix_hist(const uint64_t *__restrict__ keys, int64_t n, int shift,
-                                                   int bits, int tiles, int32_t *__restrict__ hist, const int *__restrict__ skip) {
-    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
-    __shared__ int32_t cnt[RADIX];
-    cnt[threadIdx.x] = 0;
-    __syncthreads();
-    const int64_t t0 = (int64_t)blockIdx.x * TILE;
-#pragma unroll 4
-    for (int j = 0; j < ROUNDS; ++j) {
-        const int64_t i = t0 + j * WG + threadIdx.x;
-        if (i < n) atomicAdd(&cnt[digit_of(keys[i], shift, bits)], 1);
-    }
-    __syncthreads();
-    hist[(int64_t)threadIdx.x * tiles + blockIdx.x] = cnt[threadIdx.x];
-}
+// One pass's digit.
+struct Digit {
+    KeyBits b;
+    int shift, bits;
+    __device__ __forceinline__ int of(uint64_t k) const { return (int)((sort_bits(b, k) >> shift) & ((1u << bits) - 1u)); }
+};
 
-template <bool VALS>
-__global__ __launch_bounds__(WG) void k_radix_scatter(const uint64_t *__restrict__ kin,
-                                                      const int32_t *__restrict__ vin,
-                                                      uint64_t *__restrict__ kout, int32_t *__restrict__ vout,
-                                                      int64_t n, int shift, int bits, int tiles,
-                                                      const int32_t *__restrict__ offs, const int *__restrict__ skip) {
-    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
-    __shared__ int32_t run[NWAVE][RADIX];   // per wave: keys of each digit so far
-    __shared__ int32_t start[RADIX];        // tile position of each digit's first key
-    __shared__ int32_t sh[NWAVE];
-    __shared__ uint64_t sk[TILE];
-    __shared__ int32_t sv[VALS ? TILE : 1];
+// LDS of a tile's ranking.
+template <int T>
+struct RankShared {
+    int32_t run[T / 64][RADIX];  // per wave: keys of each digit so far, then in the waves before
+    int32_t start[RADIX];       // tile position of each digit's first key
+    int32_t sh[RADIX / 64];
+};
+
+// Exclusive prefix of one value per thread over threads 0 .. RADIX - 1; every
+// thread of the workgroup calls it (the others get nothing of use).
+__device__ __forceinline__ int32_t prefix256(int32_t v, int32_t *sh) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < NWAVE * RADIX; i += WG) (&run[0][0])[i] = 0;
+    const int32_t inc = wave_scan_incl(v, [](int32_t a, int32_t b) { return a + b; });
+    if (w < RADIX / 64 && lane == 63) sh[w] = inc;
     __syncthreads();
-    // wave w ranks keys [w * 1024, (w + 1) * 1024) of the tile, 64 per round
-    const int64_t base = (int64_t)blockIdx.x * TILE + (int64_t)w * (64 * ROUNDS);
-    uint64_t key[ROUNDS];
-    int32_t val[ROUNDS];
-    int dig[ROUNDS], rnk[ROUNDS];
+    int32_t base = 0;
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int64_t i = base + r * 64 + lane;
-        const bool ok = i < n;
-        key[r] = ok ? kin[i] : 0ull;
-        if constexpr (VALS) val[r] = ok ? vin[i] : 0;
-        const int d = ok ? digit_of(key[r], shift, bits) : 0;
-        uint64_t peers = __ballot(ok);
-        for (int b = 0; b < bits; ++b) {
+    for (int i = 0; i < RADIX / 64; ++i) base += i < w ? sh[i] : 0;
+    return base + inc - v;
+}
+
+// Tile positions of the R * 64 keys a wave holds (key r of lane l is the wave's
+// key r * 64 + l; those with !ok(r) take none) in digit order, and the digits.
+// Every thread calls it; positions are valid, and S may be read, after it.
+template <int T, int R, typename Ok>
+__device__ __forceinline__ void rank_tile(RankShared<T> &S, const uint64_t (&key)[R], Ok ok, const Digit &dg,
+                                          int (&pos)[R], int (&dig)[R]) {
+    constexpr int NW = T / 64;
+    const int w = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < NW * RADIX; i += T) (&S.run[0][0])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const bool in = ok(r);
+        const int d = in ? dg.of(key[r]) : 0;
+        uint64_t peers = __ballot(in);
+        for (int b = 0; b < dg.bits; ++b) {
             const uint64_t bal = __ballot((d >> b) & 1);
             peers &= ((d >> b) & 1) ? bal : ~bal;
         }
         const int below = __popcll(peers & lanemask_lt());
         int r0 = 0;
-        if (ok) r0 = run[w][d];
+        if (in) r0 = S.run[w][d];
         // the group's lowest lane advances the digit's count after every
         // lane of the group has read it (same wave: LDS order is program order)
-        if (ok && below == 0) run[w][d] = r0 + __popcll(peers);
-        dig[r] = ok ? d : -1;
-        rnk[r] = r0 + below;
+        if (in && below == 0) S.run[w][d] = r0 + __popcll(peers);
+        dig[r] = in ? d : -1;
+        pos[r] = r0 + below;
     }
     __syncthreads();
     // per digit (thread d): prefix over waves in wave order, tile count
-    const int d = threadIdx.x;
     int32_t c = 0;
+    if (threadIdx.x < RADIX) {
+        const int d = threadIdx.x;
+        int32_t x[NW];
 #pragma unroll
-    for (int i = 0; i < NWAVE; ++i) {
-        const int32_t x = run[i][d];
-        run[i][d] = c;
-        c += x;
+        for (int i = 0; i < NW; ++i) x[i] = S.run[i][d];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            S.run[i][d] = c;
+            c += x[i];
+        }
     }
-    int32_t total;
-    const int32_t st = wg_scan_excl<int32_t>(c, OpSum(), 0, sh, &total);
-    start[d] = st;
+    const int32_t st = prefix256(c, S.sh);
+    if (threadIdx.x < RADIX) S.start[threadIdx.x] = st;
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
+    for (int r = 0; r < R; ++r)
+        if (dig[r] >= 0) pos[r] += S.start[dig[r]] + S.run[w][dig[r]];
+}
+
+// Digit counts of every tile, digit-major; `zero` (nz ints) is cleared for the
+// fused passes' tables.
+template <int T>
+__global__ __launch_bounds__(T) void k_radix_hist(const uint64_t *__restrict__ keys, int64_t n, Digit dg, int tiles,
+                                                    int32_t *__restrict__ hist, int32_t *__restrict__ zero, int nz,
+                                                    const int *__restrict__ skip) {
+    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
+    __shared__ int32_t cnt[RADIX];
+    if (threadIdx.x < RADIX) cnt[threadIdx.x] = 0;
+    for (int i = blockIdx.x * T + threadIdx.x; i < nz; i += gridDim.x * T) zero[i] = 0;
+    __syncthreads();
+    const int64_t t0 = (int64_t)blockIdx.x * (T * SROUNDS);
+#pragma unroll
+    for (int j = 0; j < SROUNDS; ++j) {
+        const int64_t i = t0 + j * T + threadIdx.x;
+        if (i < n) atomicAdd(&cnt[dg.of(keys[i])], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < RADIX) hist[(int64_t)threadIdx.x * tiles + blockIdx.x] = cnt[threadIdx.x];
+}
+
+// Digit blockIdx.x's counts become the keys of that digit in the tiles before;
+// its total goes to total[digit].
+__global__ __launch_bounds__(SWG) void k_digit_scan(int32_t *__restrict__ hist, int tiles, int32_t *__restrict__ total,
+                                                    const int *__restrict__ skip) {
+    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
+    __shared__ int32_t sh[SWAVE];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int32_t *h = hist + (int64_t)blockIdx.x * tiles;
+    int32_t carry = 0;
+    for (int b = 0; b < tiles; b += SWG) {
+        const int i = b + threadIdx.x;
+        const int32_t v = i < tiles ? h[i] : 0;
+        const int32_t inc = wave_scan_incl(v, [](int32_t x, int32_t y) { return x + y; });
+        if (lane == 63) sh[w] = inc;
+        __syncthreads();
+        int32_t base = carry, all = 0;
+#pragma unroll
+        for (int q = 0; q < SWAVE; ++q) {
+            base += q < w ? sh[q] : 0;
+            all += sh[q];
+        }
+        if (i < tiles) h[i] = base + inc - v;
+        carry += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) total[blockIdx.x] = carry;
+}
+
+template <bool VALS>
+__global__ __launch_bounds__(SWG) void k_radix_scatter(const uint64_t *__restrict__ kin,
+                                                       const int32_t *__restrict__ vin,
+                                                       uint64_t *__restrict__ kout, int32_t *__restrict__ vout,
+                                                       int64_t n, Digit dg, int tiles,
+                                                       const int32_t *__restrict__ before,
+                                                       const int32_t *__restrict__ total,
+                                                       const int *__restrict__ skip) {
+    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
+    __shared__ RankShared<SWG> S;
+    __shared__ int32_t offs[RADIX], psh[RADIX / 64];
+    __shared__ uint64_t sk[TILE];
+    __shared__ int32_t sv[VALS ? TILE : 1];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t t0 = (int64_t)blockIdx.x * TILE;
+    const int64_t base = t0 + w * (64 * SROUNDS) + lane;
+    uint64_t key[SROUNDS];
+    int32_t val[SROUNDS];
+#pragma unroll
+    for (int r = 0; r < SROUNDS; ++r) {
+        const int64_t i = base + r * 64;
+        key[r] = i < n ? kin[i] : 0ull;
+        if constexpr (VALS) val[r] = i < n ? vin[i] : 0;
+    }
+    int32_t tot = 0, bef = 0;
+    if (threadIdx.x < RADIX) {
+        tot = total[threadIdx.x];
+        bef = before[(int64_t)threadIdx.x * tiles + blockIdx.x];
+    }
+    const int32_t off = prefix256(tot, psh) + bef;
+    if (threadIdx.x < RADIX) offs[threadIdx.x] = off;
+    int pos[SROUNDS], dig[SROUNDS];
+    rank_tile(S, key, [&](int r) { return base + r * 64 < n; }, dg, pos, dig);
+#pragma unroll
+    for (int r = 0; r < SROUNDS; ++r) {
         if (dig[r] >= 0) {
-            const int p = start[dig[r]] + run[w][dig[r]] + rnk[r];
-            sk[p] = key[r];
-            if constexpr (VALS) sv[p] = val[r];
+            sk[pos[r]] = key[r];
+            if constexpr (VALS) sv[pos[r]] = val[r];
         }
     }
     __syncthreads();
     // write out: tile position p holds the key of digit dd at offset
     // p - start[dd] of that digit's run
-    const int64_t t0 = (int64_t)blockIdx.x * TILE;
     const int cnt = (int)std::min<int64_t>(TILE, n - t0);
-    for (int p = threadIdx.x; p < cnt; p += WG) {
+#pragma unroll
+    for (int r = 0; r < SROUNDS; ++r) {
+        const int p = r * SWG + threadIdx.x;
+        if (p >= cnt) break;
         const uint64_t k = sk[p];
-        const int dd = digit_of(k, shift, bits);
-        const int64_t o = (int64_t)offs[(int64_t)dd * tiles + blockIdx.x] + (p - start[dd]);
+        const int dd = dg.of(k);
+        const int64_t o = (int64_t)offs[dd] + (p - S.start[dd]);
         kout[o] = k;
         if constexpr (VALS) vout[o] = sv[p];
     }
 }
 
-// A whole sort of at most TILE keys in one workgroup: every pass ranks the
-// keys as k_radix_scatter does (each wave its 1,024 keys in 16 rounds of
-// 64), places them in LDS in digit order and reads them back in the rank
-// layout for the next pass -- one launch instead of five per pass, for the
-// many small sorts of the VENOM refinement levels and the proposer.
+// Digit widths of a sort of `total` bits in ceil(total / 8) passes.
+__host__ __device__ inline int digit_bits(int total, int shift) {
+    const int left = total - shift;
+    return (left + (left + 7) / 8 - 1) / ((left + 7) / 8);
+}
+
+// A whole sort of at most one tile in one workgroup: every pass ranks the
+// keys as k_radix_scatter does, places them in LDS in
+// digit order and reads them back in the rank layout for the next pass.
 template <bool VALS>
-__global__ __launch_bounds__(WG) void k_radix_small(const uint64_t *__restrict__ kin, const int32_t *__restrict__ vin,
-                                                    uint64_t *__restrict__ kout, int32_t *__restrict__ vout, int n,
-                                                    int end_bit, const int *__restrict__ skip) {
+__global__ __launch_bounds__(SWG) void k_sort_one(const uint64_t *__restrict__ kin, const int32_t *__restrict__ vin,
+                                                  uint64_t *__restrict__ kout, int32_t *__restrict__ vout, int n,
+                                                  KeyBits b, const int *__restrict__ skip) {
     if (skip && *skip) return;  // the caller's flag: this sort is not wanted
-    __shared__ int32_t run[NWAVE][RADIX];
-    __shared__ int32_t start[RADIX];
-    __shared__ int32_t sh[NWAVE];
-    __shared__ uint64_t sk[TILE];
-    __shared__ int32_t sv[VALS ? TILE : 1];
+    __shared__ RankShared<SWG> S;
+    constexpr int R = SROUNDS;
+    __shared__ uint64_t sk[TILE];  // a pass's keys, then its values
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int base = w * (64 * ROUNDS);
-    uint64_t key[ROUNDS];
-    int32_t val[ROUNDS];
+    const int base = w * (64 * R) + lane;
+    uint64_t key[R];
+    int32_t val[R];
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int i = base + r * 64 + lane;
+    for (int r = 0; r < R; ++r) {
+        const int i = base + r * 64;
         key[r] = i < n ? kin[i] : 0ull;
         if constexpr (VALS) val[r] = i < n ? vin[i] : 0;
     }
-    for (int shift = 0; shift < end_bit; shift += 8) {
-        const int bits = min(8, end_bit - shift);
-        for (int i = threadIdx.x; i < NWAVE * RADIX; i += WG) (&run[0][0])[i] = 0;
-        __syncthreads();
-        int dig[ROUNDS], rnk[ROUNDS];
+    const int total = b.w0 + b.w1;
+    for (int shift = 0; shift < total;) {
+        const int bits = digit_bits(total, shift);
+        int pos[R], dig[R];
+        rank_tile(S, key, [&](int r) { return base + r * 64 < n; }, Digit{b, shift, bits}, pos, dig);
+        shift += bits;
 #pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const bool ok = base + r * 64 + lane < n;
-            const int d = ok ? digit_of(key[r], shift, bits) : 0;
-            uint64_t peers = __ballot(ok);
-            for (int b = 0; b < bits; ++b) {
-                const uint64_t bal = __ballot((d >> b) & 1);
-                peers &= ((d >> b) & 1) ? bal : ~bal;
-            }
-            const int below = __popcll(peers & lanemask_lt());
-            int r0 = 0;
-            if (ok) r0 = run[w][d];
-            if (ok && below == 0) run[w][d] = r0 + __popcll(peers);
-            dig[r] = ok ? d : -1;
-            rnk[r] = r0 + below;
-        }
-        __syncthreads();
-        const int d = threadIdx.x;
-        int32_t c = 0;
-#pragma unroll
-        for (int i = 0; i < NWAVE; ++i) {
-            const int32_t x = run[i][d];
-            run[i][d] = c;
-            c += x;
-        }
-        int32_t total;
-        start[d] = wg_scan_excl<int32_t>(c, OpSum(), 0, sh, &total);
+        for (int r = 0; r < R; ++r)
+            if (dig[r] >= 0) sk[pos[r]] = key[r];
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            if (dig[r] >= 0) {
-                const int p = start[dig[r]] + run[w][dig[r]] + rnk[r];
-                sk[p] = key[r];
-                if constexpr (VALS) sv[p] = val[r];
-            }
-        }
+        for (int r = 0; r < R; ++r)
+            if (base + r * 64 < n) key[r] = sk[base + r * 64];
         __syncthreads();
+        if constexpr (VALS) {
+            int32_t *sv = (int32_t *)sk;
 #pragma unroll
-        for (int r = 0; r < ROUNDS; ++r) {
-            const int i = base + r * 64 + lane;
-            if (i < n) {
-                key[r] = sk[i];
-                if constexpr (VALS) val[r] = sv[i];
-            }
+            for (int r = 0; r < R; ++r)
+                if (dig[r] >= 0) sv[pos[r]] = val[r];
+            __syncthreads();
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (base + r * 64 < n) val[r] = sv[base + r * 64];
+            __syncthreads();
         }
-        __syncthreads();
     }
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int i = base + r * 64 + lane;
+    for (int r = 0; r < R; ++r) {
+        const int i = base + r * 64;
         if (i < n) {
             kout[i] = key[r];
             if constexpr (VALS) vout[i] = val[r];
@@ -307,111 +389,80 @@ __global__ __launch_bounds__(WG) void k_radix_small(const uint64_t *__restrict__
     }
 }
 
-// Sorts of 2 to FUSED_TILES tiles: one launch per pass.  Each workgroup
+// Sorts of up to FUSED_TILES tiles: one launch per pass.  Each workgroup
 // derives its tile's offsets itself from the pass's (digit, tile) count
-// table (a scan of at most 256 * FUSED_TILES counts, in (digit, tile)
-// order), ranks and scatters its tile as k_radix_scatter does, and counts
+// table, ranks and scatters its tile as k_radix_scatter does, and counts
 // the next pass's digits of the keys it writes by destination tile (an LDS
 // table, then one atomic add per nonzero count), so no separate histogram
 // or scan launch is needed between passes.
 constexpr int FUSED_TILES = 16;
 
-__global__ void k_fill_zero_i32(int32_t *p, int n, const int *__restrict__ skip) {
+template <bool VALS, int T>
+__global__ __launch_bounds__(T) void k_radix_fused(const uint64_t *__restrict__ kin, const int32_t *__restrict__ vin,
+                                                     uint64_t *__restrict__ kout, int32_t *__restrict__ vout,
+                                                     int n, Digit dg, int tiles, const int32_t *__restrict__ hist,
+                                                     Digit ndg, int32_t *__restrict__ next_hist,
+                                                     const int *__restrict__ skip) {
     if (skip && *skip) return;  // the caller's flag: this sort is not wanted
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
-}
-
-template <bool VALS>
-__global__ __launch_bounds__(WG) void k_radix_fused(const uint64_t *__restrict__ kin, const int32_t *__restrict__ vin,
-                                                    uint64_t *__restrict__ kout, int32_t *__restrict__ vout,
-                                                    int n, int shift, int bits, int tiles,
-                                                    const int32_t *__restrict__ hist, int next_shift,
-                                                    int next_bits, int32_t *__restrict__ next_hist, const int *__restrict__ skip) {
-    if (skip && *skip) return;  // the caller's flag: this sort is not wanted
-    __shared__ int32_t run[NWAVE][RADIX];
-    __shared__ int32_t start[RADIX];
-    __shared__ int32_t offs[RADIX];
-    __shared__ int32_t sh[NWAVE];
-    __shared__ uint64_t sk[TILE];
-    __shared__ int32_t sv[VALS ? TILE : 1];
+    constexpr int TL = T * SROUNDS;  // keys of a tile
+    __shared__ RankShared<T> S;
+    __shared__ int32_t offs[RADIX], psh[RADIX / 64];
+    __shared__ uint64_t sk[TL];
+    __shared__ int32_t sv[VALS ? TL : 1];
     __shared__ int32_t nh[FUSED_TILES * RADIX];  // next pass: counts per (destination tile, digit)
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int tile = blockIdx.x;
-    for (int i = threadIdx.x; i < NWAVE * RADIX; i += WG) (&run[0][0])[i] = 0;
+    const int base = tile * TL + w * (64 * SROUNDS) + lane;
+    uint64_t key[SROUNDS];
+    int32_t val[SROUNDS];
+#pragma unroll
+    for (int r = 0; r < SROUNDS; ++r) {
+        const int i = base + r * 64;
+        key[r] = i < n ? kin[i] : 0ull;
+        if constexpr (VALS) val[r] = i < n ? vin[i] : 0;
+    }
     if (next_hist)
-        for (int i = threadIdx.x; i < tiles * RADIX; i += WG) nh[i] = 0;
+        for (int i = threadIdx.x; i < tiles * RADIX; i += T) nh[i] = 0;
     // this tile's offsets: digits before d over all tiles, then digit d in
     // the tiles before this one (hist is digit-major: hist[d * tiles + t])
-    {
-        const int d = threadIdx.x;
-        int32_t row = 0, before = 0;
-        for (int t = 0; t < tiles; ++t) {
-            const int32_t x = hist[d * tiles + t];
-            before += t < tile ? x : 0;
-            row += x;
-        }
-        int32_t total;
-        offs[d] = wg_scan_excl<int32_t>(row, OpSum(), 0, sh, &total) + before;
-    }
-    __syncthreads();
-    const int base = tile * TILE + w * (64 * ROUNDS);
-    uint64_t key[ROUNDS];
-    int32_t val[ROUNDS];
-    int dig[ROUNDS], rnk[ROUNDS];
+    int32_t row = 0, before = 0;
+    if (threadIdx.x < RADIX) {
+        int32_t x[FUSED_TILES];
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
-        const int i = base + r * 64 + lane;
-        const bool ok = i < n;
-        key[r] = ok ? kin[i] : 0ull;
-        if constexpr (VALS) val[r] = ok ? vin[i] : 0;
-        const int d = ok ? digit_of(key[r], shift, bits) : 0;
-        uint64_t peers = __ballot(ok);
-        for (int b = 0; b < bits; ++b) {
-            const uint64_t bal = __ballot((d >> b) & 1);
-            peers &= ((d >> b) & 1) ? bal : ~bal;
-        }
-        const int below = __popcll(peers & lanemask_lt());
-        int r0 = 0;
-        if (ok) r0 = run[w][d];
-        if (ok && below == 0) run[w][d] = r0 + __popcll(peers);
-        dig[r] = ok ? d : -1;
-        rnk[r] = r0 + below;
-    }
-    __syncthreads();
-    {
-        const int d = threadIdx.x;
-        int32_t c = 0;
+        for (int t = 0; t < FUSED_TILES; ++t) x[t] = t < tiles ? hist[threadIdx.x * tiles + t] : 0;
 #pragma unroll
-        for (int i = 0; i < NWAVE; ++i) {
-            const int32_t x = run[i][d];
-            run[i][d] = c;
-            c += x;
+        for (int t = 0; t < FUSED_TILES; ++t) {
+            before += t < tile ? x[t] : 0;
+            row += x[t];
         }
-        int32_t total;
-        start[d] = wg_scan_excl<int32_t>(c, OpSum(), 0, sh, &total);
     }
-    __syncthreads();
+    const int32_t off = prefix256(row, psh) + before;
+    if (threadIdx.x < RADIX) offs[threadIdx.x] = off;
+    int pos[SROUNDS], dig[SROUNDS];
+    rank_tile(S, key, [&](int r) { return base + r * 64 < n; }, dg, pos, dig);
 #pragma unroll
-    for (int r = 0; r < ROUNDS; ++r) {
+    for (int r = 0; r < SROUNDS; ++r) {
         if (dig[r] >= 0) {
-            const int p = start[dig[r]] + run[w][dig[r]] + rnk[r];
-            sk[p] = key[r];
-            if constexpr (VALS) sv[p] = val[r];
+            sk[pos[r]] = key[r];
+            if constexpr (VALS) sv[pos[r]] = val[r];
         }
     }
     __syncthreads();
-    const int cnt = min(TILE, n - tile * TILE);
-    for (int p = threadIdx.x; p < cnt; p += WG) {
+    const int cnt = min(TL, n - tile * TL);
+#pragma unroll
+    for (int r = 0; r < SROUNDS; ++r) {
+        const int p = r * T + threadIdx.x;
+        if (p >= cnt) break;
         const uint64_t k = sk[p];
-        const int dd = digit_of(k, shift, bits);
-        const int o = offs[dd] + (p - start[dd]);
+        const int dd = dg.of(k);
+        const int o = offs[dd] + (p - S.start[dd]);
         kout[o] = k;
         if constexpr (VALS) vout[o] = sv[p];
-        if (next_hist) atomicAdd(&nh[(o / TILE) * RADIX + digit_of(k, next_shift, next_bits)], 1);
+        if (next_hist) atomicAdd(&nh[(o / TL) * RADIX + ndg.of(k)], 1);
     }
     if (next_hist) {
         __syncthreads();
-        for (int i = threadIdx.x; i < tiles * RADIX; i += WG) {
+        for (int i = threadIdx.x; i < tiles * RADIX; i += T) {
             const int32_t c = nh[i];
             if (c) atomicAdd(&next_hist[(i % RADIX) * tiles + i / RADIX], c);
         }
@@ -459,9 +510,11 @@ __global__ __launch_bounds__(WG) void k_scan_totals(int32_t *__restrict__ totals
 }
 
 // Tile scan: elements staged in LDS, each thread scans 16 consecutive ones.
+// totals: of every tile (direct), or the tiles' offsets.
 template <typename In, typename Op, bool EXCL>
 __global__ __launch_bounds__(WG) void k_scan_tile(const In *__restrict__ in, int32_t *__restrict__ out, int64_t n,
-                                                  const int32_t *__restrict__ offsets, const int *__restrict__ skip) {
+                                                  const int32_t *__restrict__ totals, bool direct,
+                                                  const int *__restrict__ skip) {
     if (skip && *skip) return;  // the caller's flag: this sort is not wanted
     __shared__ int32_t s[TILE + TILE / 32];  // one pad word per 32 to spread the banks
     __shared__ int32_t sh[NWAVE];
@@ -480,8 +533,16 @@ __global__ __launch_bounds__(WG) void k_scan_tile(const In *__restrict__ in, int
         v[j] = s[at(threadIdx.x * ROUNDS + j)];
         acc = op(acc, v[j]);
     }
-    int32_t total;
-    int32_t run = op(offsets[blockIdx.x], wg_scan_excl<int32_t>(acc, op, Op::id, sh, &total));
+    int32_t total, offset;
+    if (direct) {
+        int32_t t = Op::id;
+        for (int i = threadIdx.x; i < (int)blockIdx.x; i += WG) t = op(t, totals[i]);
+        (void)wg_scan_excl<int32_t>(t, op, Op::id, sh, &offset);
+        __syncthreads();
+    } else {
+        offset = totals[blockIdx.x];
+    }
+    int32_t run = op(offset, wg_scan_excl<int32_t>(acc, op, Op::id, sh, &total));
 #pragma unroll
     for (int j = 0; j < ROUNDS; ++j) {
         const int32_t next = op(run, v[j]);
@@ -554,80 +615,72 @@ int scan_with(const In *in, int32_t *out, int64_t n, int32_t *totals, hipStream_
     }
     const int tiles = tiles_of(n);
     hipLaunchKernelGGL((k_scan_reduce<In, Op>), dim3(tiles), dim3(WG), 0, st, in, n, totals, skip);
-    hipLaunchKernelGGL((k_scan_totals<Op>), dim3(1), dim3(WG), 0, st, totals, tiles, skip);
-    hipLaunchKernelGGL((k_scan_tile<In, Op, EXCL>), dim3(tiles), dim3(WG), 0, st, in, out, n, totals, skip);
+    const bool direct = tiles <= SCAN_DIRECT;
+    if (!direct) hipLaunchKernelGGL((k_scan_totals<Op>), dim3(1), dim3(WG), 0, st, totals, tiles, skip);
+    hipLaunchKernelGGL((k_scan_tile<In, Op, EXCL>), dim3(tiles), dim3(WG), 0, st, in, out, n, totals, direct, skip);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(VNM_E_HIP, "scan launch failed: %s", hipGetErrorString(e));
     return VNM_OK;
 }
 
+int passes_of(const KeyBits &b) { return (b.w0 + b.w1 + 7) / 8; }
+
 template <bool VALS>
-int radix_sort(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t *vout, int64_t n, int end_bit,
+int radix_sort(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t *vout, int64_t n, KeyBits b,
                hipStream_t st, const int *skip = nullptr) {
     if (n <= 0) return VNM_OK;
     if (n > (int64_t)INT32_MAX) return set_error(VNM_E_ARG, "radix sort of %lld keys", (long long)n);
-    end_bit = std::max(1, std::min(end_bit, 64));
+    const int total = b.w0 + b.w1, passes = passes_of(b);
+    const bool small = n <= FUSED_TILES * FWG * SROUNDS;  // 1,024-key tiles
+    const int tiles = small ? (int)((n + FWG * SROUNDS - 1) / (FWG * SROUNDS)) : tiles_of(n);
     if (n <= TILE) {
-        hipLaunchKernelGGL((k_radix_small<VALS>), dim3(1), dim3(WG), 0, st, kin, vin, kout, vout, (int)n, end_bit, skip);
+        hipLaunchKernelGGL((k_sort_one<VALS>), dim3(1), dim3(SWG), 0, st, kin, vin, kout, vout, (int)n, b, skip);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(VNM_E_HIP, "radix sort launch failed: %s", hipGetErrorString(e));
         return VNM_OK;
     }
-    const int passes = (end_bit + 7) / 8;
-    const int tiles = tiles_of(n);
-    if (tiles <= FUSED_TILES) {
-        // one count table per pass, zeroed up front; pass 0's by k_radix_hist,
-        // each later one by the pass before it
-        const size_t kb = align256((size_t)n * 8), vb = VALS ? align256((size_t)n * 4) : 0;
-        const int tab = RADIX * tiles;
-        int rc = g_tmp.ensure(kb + vb + align256((size_t)tab * passes * 4));
-        if (rc) return rc;
-        uint64_t *ktmp = (uint64_t *)g_tmp.p;
-        int32_t *vtmp = (int32_t *)((char *)g_tmp.p + kb);
-        int32_t *hists = (int32_t *)((char *)g_tmp.p + kb + vb);
-        hipLaunchKernelGGL(k_fill_zero_i32, dim3((tab * passes + 255) / 256), dim3(256), 0, st, hists, tab * passes, skip);
-        hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(WG), 0, st, kin, n, 0, std::min(8, end_bit), tiles, hists, skip);
-        const uint64_t *ks = kin;
-        const int32_t *vs = vin;
-        for (int p = 0; p < passes; ++p) {
-            const int shift = 8 * p, bits = std::min(8, end_bit - shift);
-            const bool last = p + 1 == passes;
-            uint64_t *kd = ((passes - 1 - p) % 2 == 0) ? kout : ktmp;
-            int32_t *vd = ((passes - 1 - p) % 2 == 0) ? vout : vtmp;
-            hipLaunchKernelGGL((k_radix_fused<VALS>), dim3(tiles), dim3(WG), 0, st, ks, vs, kd, vd, (int)n, shift, bits,
-                               tiles, hists + (size_t)tab * p, last ? 0 : shift + 8,
-                               last ? 1 : std::min(8, end_bit - shift - 8), last ? nullptr : hists + (size_t)tab * (p + 1), skip);
-            ks = kd;
-            vs = vd;
-        }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return set_error(VNM_E_HIP, "radix sort launch failed: %s", hipGetErrorString(e));
-        return VNM_OK;
-    }
-    const int64_t nh = (int64_t)RADIX * tiles;
-    // scratch: keys and values of the other buffer, digit counts, offsets,
-    // scan totals
+    // scratch: keys and values of the other buffer, then one count table per
+    // pass (fused) or one and its digits' totals
+    const bool fused = tiles <= FUSED_TILES;
     const size_t kb = align256((size_t)n * 8), vb = VALS ? align256((size_t)n * 4) : 0;
-    const size_t hb = align256((size_t)nh * 4), tb = align256((size_t)tiles_of(nh) * 4);
-    int rc = g_tmp.ensure(kb + vb + 2 * hb + tb);
+    const int64_t tab = (int64_t)RADIX * tiles;
+    int rc = g_tmp.ensure(kb + vb + align256((size_t)(fused ? tab * passes : tab + RADIX) * 4));
     if (rc) return rc;
-    char *base = (char *)g_tmp.p;
-    uint64_t *ktmp = (uint64_t *)base;
-    int32_t *vtmp = (int32_t *)(base + kb);
-    int32_t *hist = (int32_t *)(base + kb + vb);
-    int32_t *offs = (int32_t *)(base + kb + vb + hb);
-    int32_t *tot = (int32_t *)(base + kb + vb + 2 * hb);
+    uint64_t *ktmp = (uint64_t *)g_tmp.p;
+    int32_t *vtmp = (int32_t *)((char *)g_tmp.p + kb);
+    int32_t *hist = (int32_t *)((char *)g_tmp.p + kb + vb);
     const uint64_t *ks = kin;
     const int32_t *vs = vin;
+    int shift = 0;
     for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p, bits = std::min(8, end_bit - shift);
         // the last pass writes the output
         uint64_t *kd = ((passes - 1 - p) % 2 == 0) ? kout : ktmp;
         int32_t *vd = ((passes - 1 - p) % 2 == 0) ? vout : vtmp;
-        hipLaunchKernelGGL(k_radix_hist, dim3(tiles), dim3(WG), 0, st, ks, n, shift, bits, tiles, hist, skip);
-        if ((rc = scan_with<int32_t, OpSum, true>(hist, offs, nh, tot, st, skip))) return rc;
-        hipLaunchKernelGGL((k_radix_scatter<VALS>), dim3(tiles), dim3(WG), 0, st, ks, vs, kd, vd, n, shift, bits,
-                           tiles, offs, skip);
+        const Digit dg{b, shift, digit_bits(total, shift)};
+        shift += dg.bits;
+        if (fused) {
+            const bool last = p + 1 == passes;
+            int32_t *h = hist + tab * p;
+            const Digit ndg{b, shift, last ? 1 : digit_bits(total, shift)};
+            int32_t *nh = last ? nullptr : h + tab;
+            const int nz = (int)(tab * (passes - 1));
+            if (small) {
+                if (p == 0)  // the first table counted, the others cleared
+                    hipLaunchKernelGGL(k_radix_hist<FWG>, dim3(tiles), dim3(FWG), 0, st, ks, n, dg, tiles, h, h + tab, nz, skip);
+                hipLaunchKernelGGL((k_radix_fused<VALS, FWG>), dim3(tiles), dim3(FWG), 0, st, ks, vs, kd, vd, (int)n, dg,
+                                   tiles, h, ndg, nh, skip);
+            } else {
+                if (p == 0)
+                    hipLaunchKernelGGL(k_radix_hist<SWG>, dim3(tiles), dim3(SWG), 0, st, ks, n, dg, tiles, h, h + tab, nz, skip);
+                hipLaunchKernelGGL((k_radix_fused<VALS, SWG>), dim3(tiles), dim3(SWG), 0, st, ks, vs, kd, vd, (int)n, dg,
+                                   tiles, h, ndg, nh, skip);
+            }
+        } else {
+            hipLaunchKernelGGL(k_radix_hist<SWG>, dim3(tiles), dim3(SWG), 0, st, ks, n, dg, tiles, hist, nullptr, 0, skip);
+            hipLaunchKernelGGL(k_digit_scan, dim3(RADIX), dim3(SWG), 0, st, hist, tiles, hist + tab, skip);
+            hipLaunchKernelGGL((k_radix_scatter<VALS>), dim3(tiles), dim3(SWG), 0, st, ks, vs, kd, vd, n, dg, tiles, hist,
+                               hist + tab, skip);
+        }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return set_error(VNM_E_HIP, "radix sort launch failed: %s", hipGetErrorString(e));
         ks = kd;
@@ -638,12 +691,12 @@ int radix_sort(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t 
 
 }  // namespace
 
-int sort_keys_u64(const uint64_t *in, uint64_t *out, int64_t n, int end_bit, hipStream_t st) {
-    return radix_sort<false>(in, out, nullptr, nullptr, n, end_bit, st);
+int sort_keys_u64(const uint64_t *in, uint64_t *out, int64_t n, KeyBits bits, hipStream_t st) {
+    return radix_sort<false>(in, out, nullptr, nullptr, n, bits, st);
 }
 
-int sort_keys_u64_if(const uint64_t *in, uint64_t *out, int64_t n, int end_bit, hipStream_t st, const int *skip) {
-    return radix_sort<false>(in, out, nullptr, nullptr, n, end_bit, st, skip);
+int sort_keys_u64_if(const uint64_t *in, uint64_t *out, int64_t n, KeyBits bits, hipStream_t st, const int *skip) {
+    return radix_sort<false>(in, out, nullptr, nullptr, n, bits, st, skip);
 }
 
 int sort_scratch_slot(int slot) {
@@ -654,18 +707,14 @@ int sort_scratch_slot(int slot) {
 
 int sort_scratch_reserve(int64_t n) {
     if (n <= TILE) return VNM_OK;
-    // the larger of the two multi-tile paths' needs, keys and values, 8 passes
-    const int tiles = tiles_of(n);
-    const size_t kb = align256((size_t)n * 8), vb = align256((size_t)n * 4);
-    const size_t fused = kb + vb + align256((size_t)RADIX * tiles * 8 * 4);
-    const int64_t nh = (int64_t)RADIX * tiles;
-    const size_t multi = kb + vb + 2 * align256((size_t)nh * 4) + align256((size_t)tiles_of(nh) * 4);
-    return g_tmp.ensure(std::max(fused, multi));
+    // keys and values, count tables of 8 passes (fused) or one with its totals
+    const int64_t tab = (int64_t)RADIX * std::max<int64_t>(tiles_of(n), FUSED_TILES);
+    return g_tmp.ensure(align256((size_t)n * 8) + align256((size_t)n * 4) + align256((size_t)(tab * 8 + RADIX) * 4));
 }
 
 int sort_pairs_u64_i32(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t *vout, int64_t n,
-                       int end_bit, hipStream_t st) {
-    return radix_sort<true>(kin, kout, vin, vout, n, end_bit, st);
+                       KeyBits bits, hipStream_t st) {
+    return radix_sort<true>(kin, kout, vin, vout, n, bits, st);
 }
 
 int scan_excl_i32(const int32_t *in, int32_t *out, int64_t n, hipStream_t st) {
@@ -711,8 +760,9 @@ extern "C" int vnm_sort_pairs(vnm_ctx *ctx, const uint64_t *keys_in, uint64_t *k
         return vnm::set_error(VNM_E_ARG, "sort: values in and out must both be given or both be NULL");
     if (keys_in == keys_out || (vals_in && vals_in == vals_out))
         return vnm::set_error(VNM_E_ARG, "sort: output must not alias the input");
-    int rc = vals_in ? vnm::sort_pairs_u64_i32(keys_in, keys_out, vals_in, vals_out, n, end_bit, ctx->stream)
-                     : vnm::sort_keys_u64(keys_in, keys_out, n, end_bit, ctx->stream);
+    const vnm::KeyBits bits = vnm::key_range(0, end_bit);
+    int rc = vals_in ? vnm::sort_pairs_u64_i32(keys_in, keys_out, vals_in, vals_out, n, bits, ctx->stream)
+                     : vnm::sort_keys_u64(keys_in, keys_out, n, bits, ctx->stream);
     if (rc) return rc;
     ctx->launches += 5 * ((end_bit + 7) / 8);
     return VNM_OK;

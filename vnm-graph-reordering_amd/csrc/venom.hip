@@ -31,12 +31,6 @@ namespace vnm {
 
 namespace {
 
-int bits_for(int64_t x) {
-    int b = 1;
-    while ((1ll << b) <= x) ++b;
-    return b;
-}
-
 int grid_of(int64_t n, int block) {
     int64_t g = (n + block - 1) / block;
     return (int)std::max<int64_t>(1, std::min<int64_t>(g, 65535));
@@ -169,7 +163,7 @@ __global__ void k_ref_init(int32_t *order, int32_t *bstart, int32_t *act, int m)
 
 __global__ void k_ref_keys(const int32_t *__restrict__ act, int na, const int32_t *__restrict__ order,
                            const int32_t *__restrict__ bstart, const int32_t *__restrict__ rptr,
-                           const int32_t *__restrict__ tok, int level,
+                           const int32_t *__restrict__ tok, int level, uint32_t bias,
                            uint64_t *__restrict__ kk, int32_t *__restrict__ vv) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < na) {
@@ -177,7 +171,7 @@ __global__ void k_ref_keys(const int32_t *__restrict__ act, int na, const int32_
         const int row = order[p];
         const int beg = rptr[row], n = rptr[row + 1] - beg;
         const int t = level < n ? tok[beg + level] : 0;  // 0 = end of the list
-        kk[i] = ((uint64_t)(uint32_t)bstart[p] << 32) | (uint32_t)(t ^ (int)0x80000000);
+        kk[i] = ((uint64_t)(uint32_t)bstart[p] << 32) | ((uint32_t)t + bias);
         vv[i] = row;
     }
 }
@@ -193,13 +187,13 @@ __global__ void k_ref_apply(const int32_t *__restrict__ act, int na, const uint6
 }
 
 __global__ void k_ref_next(const int32_t *__restrict__ act, int na, const uint64_t *__restrict__ kk,
-                           const int32_t *__restrict__ bpos, int32_t *__restrict__ bstart,
+                           const int32_t *__restrict__ bpos, uint32_t bias, int32_t *__restrict__ bstart,
                            uint8_t *__restrict__ flags) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < na) {
         bstart[act[i]] = bpos[i];
         const bool tied = (i > 0 && kk[i] == kk[i - 1]) || (i + 1 < na && kk[i + 1] == kk[i]);
-        const bool ended = (uint32_t)kk[i] == 0x80000000u;
+        const bool ended = (uint32_t)kk[i] == bias;
         flags[i] = tied && !ended;
     }
 }
@@ -294,7 +288,7 @@ struct VenomWork {
         }
         const int gb = grid_of(nnz, 256);
         hipLaunchKernelGGL(k_pos_keys, dim3(gb), dim3(256), 0, st, row, col, nnz, keys.p);
-        int rc = sort_keys_u64(keys.p, keys2.p, nnz, 32 + bits_for(m), st);
+        int rc = sort_keys_u64(keys.p, keys2.p, nnz, key_halves(bits_for(std::max(m, n)), bits_for(m)), st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_run_heads, dim3(gb), dim3(256), 0, st, keys2.p, nnz, M, head.p);
         if ((rc = scan_excl_i32(head.p, excl.p, nnz, st))) return rc;
@@ -328,25 +322,28 @@ struct VenomWork {
     int sort_rows() {
         hipStream_t st = g->ctx->stream;
         int rc;
+        const int scale = M <= 8 ? 512 : 1 << 17;
         VNM_HIP_TRY(hipMemsetAsync(rcnt.p, 0, (size_t)(m + 1) * 4, st));
         if (U > 0)
             hipLaunchKernelGGL(k_tokens, dim3(grid_of(U, 256)), dim3(256), 0, st, rrow.p, rseg.p,
-                               bits.p, U, S, M <= 8 ? 512 : (1 << 17), tok.p, rcnt.p);
+                               bits.p, U, S, scale, tok.p, rcnt.p);
         if ((rc = scan_excl_i32(rcnt.p, rptr.p, m + 1, st))) return rc;
         hipLaunchKernelGGL(k_ref_init, dim3((m + 255) / 256), dim3(256), 0, st, order.p, bstart.p,
                            act.p, m);
         g->ctx->launches += 2;
         int na = m;
-        const int end_bit = 32 + bits_for(m);
+        // tokens are of either sign within +-S * scale (k_tokens), 0 the end mark
+        const int tbits = std::min(32, bits_for(2 * ((int64_t)S + 1) * scale));
+        const uint32_t bias = 1u << (tbits - 1);  // token + bias orders as the signed token
         for (int level = 0; na > 1; ++level) {
             const int gb = (na + 255) / 256;
             hipLaunchKernelGGL(k_ref_keys, dim3(gb), dim3(256), 0, st, act.p, na, order.p,
-                               bstart.p, rptr.p, tok.p, level, kk.p, vv.p);
-            if ((rc = sort_pairs_u64_i32(kk.p, kk2.p, vv.p, vv2.p, na, end_bit, st))) return rc;
+                               bstart.p, rptr.p, tok.p, level, bias, kk.p, vv.p);
+            if ((rc = sort_pairs_u64_i32(kk.p, kk2.p, vv.p, vv2.p, na, key_halves(tbits, bits_for(m)), st))) return rc;
             hipLaunchKernelGGL(k_ref_apply, dim3(gb), dim3(256), 0, st, act.p, na, kk2.p, vv2.p,
                                order.p, headpos.p);
             if ((rc = scan_incl_max_i32(headpos.p, bpos.p, na, st))) return rc;
-            hipLaunchKernelGGL(k_ref_next, dim3(gb), dim3(256), 0, st, act.p, na, kk2.p, bpos.p,
+            hipLaunchKernelGGL(k_ref_next, dim3(gb), dim3(256), 0, st, act.p, na, kk2.p, bpos.p, bias,
                                bstart.p, flags.p);
             if ((rc = select_flagged_i32(act.p, flags.p, act2.p, cnt2.p + 2, na, st))) return rc;
             g->ctx->launches += 6;
@@ -425,7 +422,8 @@ int reload_sort(vnm_graph *g, bool quantize) {
     const int gb = grid_of(nnz, 256);
     hipLaunchKernelGGL(k_pos_keys, dim3(gb), dim3(256), 0, st, g->row.p, g->col.p, nnz, k1.p);
     hipLaunchKernelGGL(k_iota64, dim3(gb), dim3(256), 0, st, i1.p, nnz);
-    if ((rc = sort_pairs_u64_i32(k1.p, k2.p, i1.p, i2.p, nnz, 64, st))) return rc;
+    const int ib = bits_for(std::max(g->nrows, g->ncols));  // ids are below both after any relabel
+    if ((rc = sort_pairs_u64_i32(k1.p, k2.p, i1.p, i2.p, nnz, key_halves(ib, ib), st))) return rc;
     if (g->col_overflow)
         return set_error(VNM_E_ARG, "entries lie past the padded column count; the reference's "
                                     "coo_matrix(shape=(n, n)) raises here");
