@@ -27,9 +27,9 @@
 //                          or touched segments) from an LDS row hash or LDS
 //                          row tiles, segments taken from a work counter
 //   k_lp_features        : 16 input features per node
-//   k_lp_agg_*           : neighbour mean (and its transpose for backward),
-//                          one wave per node, long lists split into chunks
-//                          summed in a fixed order (bit-reproducible)
+//   k_lp_agg(_combine)   : neighbour mean (and its transpose for backward),
+//                          short lists four to a wave, the longest split into
+//                          chunks, all summed in a fixed order (bit-reproducible)
 //   k_lp_dense_mfma      : [H, Agg] W + b with v_mfma_f32_16x16x16_bf16
 //   k_lp_dense_f32       : the same on VALU in FP32
 //   k_lp_pair_loss, k_lp_bwd_in, k_lp_wgrad(+reduce), k_lp_adam
@@ -157,7 +157,7 @@ __global__ void k_lp_inv_deg(int R, const int32_t *__restrict__ ptr, float *__re
 
 // ------------------------------------------------------------ segment statistics
 
-constexpr int SS_T = 256;
+constexpr int SS_T = 512;
 constexpr int TB = SS_T / 8;  // row tiles whose ends one pass of binary searches finds
 constexpr int PB = 256 / 16;   // the same for the pair scorer (2M <= 16 columns)
 constexpr int PAIR_TILE_ROWS = TILE_ROWS / 2;  // rows of a pair tile (16 bits per row)
@@ -209,7 +209,8 @@ __global__ __launch_bounds__(SS_T) void k_lp_seg_stats(
             if ((bits >> (M - 1 - t)) == 1u) atomicAdd(&segc[k], 1);
         };
         if (total <= HASH_MAX) {
-            hash_scatter(L.h, M, cols, pre, M, total, idx);
+            const int hb = hash_bits(total);
+            hash_scatter(L.h, hb, M, cols, pre, M, total, idx);
             __syncthreads();
             // TAB_U entries per thread resolved before their loads are issued
             for (int e0 = tid; e0 < total; e0 += SS_T * TAB_U) {
@@ -217,10 +218,10 @@ __global__ __launch_bounds__(SS_T) void k_lp_seg_stats(
                 table_entries(cols, pre, M, total, idx, e0, SS_T, t, r);
 #pragma unroll
                 for (int u = 0; u < TAB_U; ++u)
-                    if (t[u] >= 0) count(t[u], hash_get(L.h, (uint32_t)r[u]) & 0xFFu);
+                    if (t[u] >= 0) count(t[u], hash_get(L.h, hb, (uint32_t)r[u]) & 0xFFu);
             }
             __syncthreads();
-            hash_reset(L.h);
+            hash_reset(L.h, hb);
         } else {
             // rows [r0, r0 + TILE_ROWS) at a time in an LDS byte tile: the
             // column lists are sorted by row, so each column's entries of a
@@ -239,8 +240,9 @@ __global__ __launch_bounds__(SS_T) void k_lp_seg_stats(
             for (int g0 = 0; g0 < ntile; g0 += TB) {
                 if (tid < M * TB) {  // end of tile g0 + j in column t
                     const int t = tid / TB, j = tid % TB;
-                    const int64_t r1 = min((int64_t)R, (int64_t)(g0 + j + 1) * TILE_ROWS);
+                    const int64_t r1 = (int64_t)(g0 + j + 1) * TILE_ROWS;
                     int lo = cols[t].start, hi = cols[t].start + cols[t].len;
+                    if (r1 >= R) lo = hi;  // the last tile: no search
                     while (lo < hi) {
                         const int mid = (lo + hi) >> 1;
                         if (idx[mid] < r1) lo = mid + 1;
@@ -261,19 +263,17 @@ __global__ __launch_bounds__(SS_T) void k_lp_seg_stats(
                     __syncthreads();
                     const int tt = tpre[M];
                     if (tt > 0) {  // uniform
-                        for (int e0 = tid; e0 < tt; e0 += SS_T * TAB_U) {
-                            int t[TAB_U], r[TAB_U];
+                        // column by column: no search for an entry's column
+                        for (int t = 0; t < M; ++t) {
+                            const int hi = thi[t];
+                            for (int e0 = tlo[t] + tid; e0 < hi; e0 += SS_T * TAB_U) {
+                                int r[TAB_U];
 #pragma unroll
-                            for (int u = 0; u < TAB_U; ++u) {
-                                const int e = e0 + u * SS_T;
-                                t[u] = e < tt ? entry_col(tpre, M, e) : -1;
+                                for (int u = 0; u < TAB_U; ++u) r[u] = e0 + u * SS_T < hi ? idx[e0 + u * SS_T] - r0 : -1;
+#pragma unroll
+                                for (int u = 0; u < TAB_U; ++u)
+                                    if (r[u] >= 0) atomicOr(&L.tile[r[u] >> 2], (1u << (M - 1 - t)) << (8 * (r[u] & 3)));
                             }
-#pragma unroll
-                            for (int u = 0; u < TAB_U; ++u)
-                                r[u] = t[u] >= 0 ? idx[tlo[t[u]] + (e0 + u * SS_T - tpre[t[u]])] - r0 : 0;
-#pragma unroll
-                            for (int u = 0; u < TAB_U; ++u)
-                                if (t[u] >= 0) atomicOr(&L.tile[r[u] >> 2], (1u << (M - 1 - t[u])) << (8 * (r[u] & 3)));
                         }
                         __syncthreads();
                         // every row of the tile once: its bitmap's class,
@@ -396,70 +396,147 @@ __global__ void k_lp_features(int R, int M, const int32_t *__restrict__ perm,
 
 // Forward (BWD = false): out[u] = inv_deg[u] * sum_{j in list(u)} H[j].
 // Transpose (BWD = true): out[u] += sum_{j in tlist(u)} inv_deg[j] * H[j].
-// One wave per node: F/4 lanes cover a row (4 values each), 256/F rows in
-// flight; the partial sums of the row slots are combined by a fixed xor tree.
+// F/4 lanes cover a row of H (4 values each).  A sum has NS = 256/F slots: slot s
+// takes the rows s, s + NS, ... of its list in order, and the slots are added
+// pairwise (s with s ^ 1, then s ^ 2, ...), whichever lanes hold them, so every
+// path below gives the same bits.
+//
+// What bounds the sums is the latency of a list's loads (its node's range, its
+// members, their rows), not their bytes: a wave per list with 4 rows per slot in
+// flight left a list of 1,024 members 41 us long and ran 65,536 short lists
+// in 8 waves' worth of round trips (64 us a call at R-MAT 65,536, F = 64, and 41
+// more for the chunks of longer lists in a launch of their own).  One launch now
+// takes the chunks and the long lists first, a wave each with AGG_DEEP rows per slot in
+// flight, then the lists of at most AGG_LIGHT members, four to a wave.
+constexpr int AGG_LIGHT = 64;
+
+template <typename TI>
+constexpr int agg_deep() { return sizeof(TI) == 2 ? 16 : 8; }
+
+template <typename TI, int F, bool BWD>
+__device__ __forceinline__ float4 agg_row(const float *__restrict__ inv_deg, const TI *__restrict__ H, int v, int gq) {
+    float4 h = Act<TI>::load4(H + (size_t)v * F + gq * 4);
+    if (BWD) {
+        const float f = inv_deg[v];
+        h.x *= f; h.y *= f; h.z *= f; h.w *= f;
+    }
+    return h;
+}
+
+__device__ __forceinline__ void add4(float4 &a, const float4 &b) {
+    a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w;
+}
+
+// a += b where ok (a select, not a branch).
+__device__ __forceinline__ void add4_if(float4 &a, const float4 &b, bool ok) {
+    a.x = ok ? a.x + b.x : a.x;
+    a.y = ok ? a.y + b.y : a.y;
+    a.z = ok ? a.z + b.z : a.z;
+    a.w = ok ? a.w + b.w : a.w;
+}
+
+// a plus the same lanes' a at distance `off`.
+__device__ __forceinline__ void add_xor(float4 &a, int off) {
+    a.x += __shfl_xor(a.x, off);
+    a.y += __shfl_xor(a.y, off);
+    a.z += __shfl_xor(a.z, off);
+    a.w += __shfl_xor(a.w, off);
+}
+
+// One list [b, e), a wave: lane group s (F/4 lanes) holds slot s.
 template <typename TI, int F, bool BWD>
 __device__ __forceinline__ float4 agg_range(int b, int e, const int32_t *__restrict__ idx,
                                             const float *__restrict__ inv_deg, const TI *__restrict__ H) {
-    constexpr int LPR = F / 4, NS = 64 / LPR;
+    constexpr int LPR = F / 4, NS = 64 / LPR, UN = agg_deep<TI>();
     const int lane = threadIdx.x & 63;
     const int gq = lane % LPR, slot = lane / LPR;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    // four rows per slot in flight; each slot still sums its rows in list
-    // order, so the result does not depend on the unrolling
-    constexpr int UN = 4;
-    int j = b + slot;
-    for (; j + (UN - 1) * NS < e; j += UN * NS) {
-        int v[UN];
+    // no branches around the loads, so that they stay in flight together: past
+    // the list's end they repeat its last member, which is not added
+    int v[UN];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) v[u] = idx[j + u * NS];
+    for (int u = 0; u < UN; ++u) v[u] = idx[min(b + slot + u * NS, e - 1)];
+    for (int j = b + slot; j - slot < e; j += UN * NS) {
         float4 h[UN];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) h[u] = Act<TI>::load4(H + (size_t)v[u] * F + gq * 4);
+        for (int u = 0; u < UN; ++u) h[u] = agg_row<TI, F, BWD>(inv_deg, H, v[u], gq);
+        // the next members, while the rows are on their way
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            if (BWD) {
-                const float f = inv_deg[v[u]];
-                h[u].x *= f; h[u].y *= f; h[u].z *= f; h[u].w *= f;
-            }
-            acc.x += h[u].x; acc.y += h[u].y; acc.z += h[u].z; acc.w += h[u].w;
-        }
-    }
-    for (; j < e; j += NS) {
-        const int v = idx[j];
-        float4 h = Act<TI>::load4(H + (size_t)v * F + gq * 4);
-        if (BWD) {
-            const float f = inv_deg[v];
-            h.x *= f; h.y *= f; h.z *= f; h.w *= f;
-        }
-        acc.x += h.x; acc.y += h.y; acc.z += h.z; acc.w += h.w;
+        for (int u = 0; u < UN; ++u) v[u] = idx[min(j + (UN + u) * NS, e - 1)];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) add4_if(acc, h[u], j + u * NS < e);
     }
 #pragma unroll
-    for (int off = LPR; off < 64; off <<= 1) {
-        acc.x += __shfl_xor(acc.x, off);
-        acc.y += __shfl_xor(acc.y, off);
-        acc.z += __shfl_xor(acc.z, off);
-        acc.w += __shfl_xor(acc.w, off);
-    }
+    for (int off = LPR; off < 64; off <<= 1) add_xor(acc, off);
     return acc;
 }
 
-template <typename TI, typename TO, int F, bool BWD>
-__global__ __launch_bounds__(256) void k_lp_agg_nodes(int R, const int32_t *__restrict__ ptr,
-                                                      const int32_t *__restrict__ idx,
-                                                      const float *__restrict__ inv_deg,
-                                                      const TI *__restrict__ H, TO *__restrict__ out, const int *__restrict__ skip) {
-    if (skip && *skip) return;  // not wanted this iteration (a device-side flag)
+// One list of at most AGG_LIGHT members, 16 lanes: lane group q of Q = 64/F
+// (F/4 lanes) holds slots q, q + Q, q + 2 Q, q + 3 Q.  Valid in every lane group.
+template <typename TI, int F, bool BWD>
+__device__ __forceinline__ float4 agg_light(int b, int e, const int32_t *__restrict__ idx,
+                                            const float *__restrict__ inv_deg, const TI *__restrict__ H) {
+    constexpr int LPR = F / 4, Q = 16 / LPR;
+    const int l = threadIdx.x & 15, gq = l % LPR, q = l / LPR;
+    float4 acc[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    constexpr int UN = 8;  // rows per lane group in flight
+    for (int j = b + q; j - q < e; j += UN * Q) {
+        int v[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) v[u] = idx[min(j + u * Q, e - 1)];
+        float4 h[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) h[u] = agg_row<TI, F, BWD>(inv_deg, H, v[u], gq);
+#pragma unroll
+        for (int u = 0; u < UN; ++u) add4_if(acc[u % 4], h[u], j + u * Q < e);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int off = LPR; off < 16; off <<= 1) add_xor(acc[k], off);
+    add4(acc[0], acc[1]);
+    add4(acc[2], acc[3]);
+    add4(acc[0], acc[2]);
+    return acc[0];
+}
 
-    const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (u >= R) return;
-    const int b = ptr[u], e = ptr[u + 1];
-    if (e - b > AGG_CH) return;  // split into chunks
-    const float4 acc = agg_range<TI, F, BWD>(b, e, idx, inv_deg, H);
+// The chunks [0, nch) of lists of more than AGG_CH members (partial sums, added
+// by k_lp_agg_combine), the nlong lists of more than AGG_LIGHT, then every
+// node's list if it is shorter.
+template <typename TI, typename TO, int F, bool BWD>
+__global__ __launch_bounds__(256) void k_lp_agg(int R, int nch, const int32_t *__restrict__ ch_beg,
+                                                const int32_t *__restrict__ ch_end, int nlong,
+                                                const int32_t *__restrict__ longs, const int32_t *__restrict__ ptr,
+                                                const int32_t *__restrict__ idx, const float *__restrict__ inv_deg,
+                                                const TI *__restrict__ H, float *__restrict__ part,
+                                                TO *__restrict__ out, const int *__restrict__ skip) {
+    if (skip && *skip) return;  // not wanted this iteration (a device-side flag)
     constexpr int LPR = F / 4;
     const int lane = threadIdx.x & 63;
-    if (lane < LPR) {
-        TO *o = out + (size_t)u * F + lane * 4;
+    const int w = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    int u, l;
+    float4 acc;
+    if (w < nch) {
+        acc = agg_range<TI, F, BWD>(ch_beg[w], ch_end[w], idx, inv_deg, H);
+        if (lane < LPR) *(float4 *)&part[(size_t)w * F + lane * 4] = acc;
+        return;
+    }
+    if (w < nch + nlong) {
+        u = longs[w - nch];
+        l = lane;
+        acc = agg_range<TI, F, BWD>(ptr[u], ptr[u + 1], idx, inv_deg, H);
+    } else {
+        u = (w - nch - nlong) * 4 + (lane >> 4);
+        if (u >= R) return;
+        l = lane & 15;
+        const int b = ptr[u], e = ptr[u + 1];
+        if (e - b > AGG_LIGHT) return;  // a long list
+        acc = agg_light<TI, F, BWD>(b, e, idx, inv_deg, H);
+    }
+    if (l < LPR) {
+        TO *o = out + (size_t)u * F + l * 4;
         if (BWD) {
             o[0] += acc.x; o[1] += acc.y; o[2] += acc.z; o[3] += acc.w;
         } else {
@@ -470,21 +547,6 @@ __global__ __launch_bounds__(256) void k_lp_agg_nodes(int R, const int32_t *__re
             Act<TO>::put(o + 3, acc.w * f);
         }
     }
-}
-
-template <typename TI, int F, bool BWD>
-__global__ __launch_bounds__(256) void k_lp_agg_chunks(int nch, const int32_t *__restrict__ ch_beg,
-                                                       const int32_t *__restrict__ ch_end,
-                                                       const int32_t *__restrict__ idx,
-                                                       const float *__restrict__ inv_deg,
-                                                       const TI *__restrict__ H, float *__restrict__ part, const int *__restrict__ skip) {
-    if (skip && *skip) return;  // not wanted this iteration (a device-side flag)
-
-    const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (c >= nch) return;
-    const float4 acc = agg_range<TI, F, BWD>(ch_beg[c], ch_end[c], idx, inv_deg, H);
-    const int lane = threadIdx.x & 63;
-    if (lane < F / 4) *(float4 *)&part[(size_t)c * F + lane * 4] = acc;
 }
 
 template <typename TO, int F, bool BWD>
@@ -1039,9 +1101,10 @@ __global__ __launch_bounds__(256) void k_lp_pair_gain(const int *__restrict__ d_
         }
     };
     if (total <= HASH_MAX) {
-        hash_reset(L.h);
+        const int hb = hash_bits(total);
+        hash_reset(L.h, hb);
         __syncthreads();
-        hash_scatter(L.h, M, cols, pre, 2 * M, total, idx);
+        hash_scatter(L.h, hb, M, cols, pre, 2 * M, total, idx);
         __syncthreads();
         // TAB_U entries per thread resolved before their lookups
         for (int base = 0; base < total; base += 256 * TAB_U) {
@@ -1049,7 +1112,7 @@ __global__ __launch_bounds__(256) void k_lp_pair_gain(const int *__restrict__ d_
             table_entries(cols, pre, 2 * M, total, idx, base + tid, 256, tt, rw);
 #pragma unroll
             for (int u = 0; u < TAB_U; ++u) {
-                const uint32_t h = tt[u] >= 0 ? hash_get(L.h, (uint32_t)rw[u]) : 0u;
+                const uint32_t h = tt[u] >= 0 ? hash_get(L.h, hb, (uint32_t)rw[u]) : 0u;
                 fold(tt[u], h & 0xFFu, (h >> 8) & 0xFFu);
             }
         }
@@ -1322,8 +1385,9 @@ __global__ void k_lp_swap(const LPCtl *__restrict__ ctl, int M, const int32_t *_
 // ------------------------------------------------------------ host: cache
 
 struct AggPlan {
-    int nheavy = 0, nch = 0;
-    DBuf<int32_t> heavy, ch0, beg, end;
+    int nheavy = 0, nch = 0, nlong = 0;
+    DBuf<int32_t> heavy, ch0, beg, end;  // lists of more than AGG_CH members and their chunks
+    DBuf<int32_t> longs;                 // the other lists of more than AGG_LIGHT
     DBuf<float> part;  // nch x 64
 };
 
@@ -1345,11 +1409,15 @@ struct LPCache {
 static void lp_cache_free(void *p) { delete (LPCache *)p; }
 
 static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P) {
-    std::vector<int32_t> heavy, ch0{0}, beg, end;
+    std::vector<int32_t> heavy, ch0{0}, beg, end, longs;
     const int R = (int)hptr.size() - 1;
     for (int u = 0; u < R; ++u) {
         const int b = hptr[u], e = hptr[u + 1];
-        if (e - b <= AGG_CH) continue;
+        if (e - b <= AGG_LIGHT) continue;
+        if (e - b <= AGG_CH) {
+            longs.push_back(u);
+            continue;
+        }
         heavy.push_back(u);
         for (int s = b; s < e; s += AGG_CH) {
             beg.push_back(s);
@@ -1359,11 +1427,15 @@ static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P) {
     }
     P.nheavy = (int)heavy.size();
     P.nch = (int)beg.size();
+    P.nlong = (int)longs.size();
+    // the longest first: they end last
+    std::stable_sort(longs.begin(), longs.end(), [&](int x, int y) { return hptr[x + 1] - hptr[x] > hptr[y + 1] - hptr[y]; });
     int rc;
     if ((rc = P.heavy.alloc(std::max(1, P.nheavy))) || (rc = P.ch0.alloc(P.nheavy + 1)) ||
         (rc = P.beg.alloc(std::max(1, P.nch))) || (rc = P.end.alloc(std::max(1, P.nch))) ||
-        (rc = P.part.alloc((size_t)std::max(1, P.nch) * 64)))
+        (rc = P.part.alloc((size_t)std::max(1, P.nch) * 64)) || (rc = P.longs.alloc(std::max(1, P.nlong))))
         return rc;
+    if (P.nlong) VNM_HIP_TRY(hipMemcpy(P.longs.p, longs.data(), longs.size() * 4, hipMemcpyHostToDevice));
     if (P.nheavy) {
         VNM_HIP_TRY(hipMemcpy(P.heavy.p, heavy.data(), heavy.size() * 4, hipMemcpyHostToDevice));
         VNM_HIP_TRY(hipMemcpy(P.beg.p, beg.data(), beg.size() * 4, hipMemcpyHostToDevice));
@@ -1500,15 +1572,14 @@ static int lp_aggregate(vnm_graph *g, LPCache *c, const TI *H, TO *out, const in
     const AggPlan &P = BWD ? c->bwd : c->fwd;
     const int32_t *ptr = BWD ? c->tptr.p : c->ptr.p;
     const int32_t *idx = BWD ? c->tidx.p : c->idx.p;
-    hipLaunchKernelGGL((k_lp_agg_nodes<TI, TO, F, BWD>), dim3((R + 3) / 4), dim3(256), 0, st, R, ptr, idx,
-                       c->inv_deg.p, H, out, skip);
+    const int waves = P.nch + P.nlong + (R + 3) / 4;
+    hipLaunchKernelGGL((k_lp_agg<TI, TO, F, BWD>), dim3((waves + 3) / 4), dim3(256), 0, st, R, P.nch, P.beg.p, P.end.p,
+                       P.nlong, P.longs.p, ptr, idx, c->inv_deg.p, H, P.part.p, out, skip);
     g->ctx->launches++;
     if (P.nch) {
-        hipLaunchKernelGGL((k_lp_agg_chunks<TI, F, BWD>), dim3((P.nch + 3) / 4), dim3(256), 0, st, P.nch,
-                           P.beg.p, P.end.p, idx, c->inv_deg.p, H, P.part.p, skip);
         hipLaunchKernelGGL((k_lp_agg_combine<TO, F, BWD>), dim3(grid_of((int64_t)P.nheavy * F, 256)),
                            dim3(256), 0, st, P.nheavy, P.heavy.p, P.ch0.p, P.part.p, c->inv_deg.p, out, skip);
-        g->ctx->launches += 2;
+        g->ctx->launches++;
     }
     VNM_LAUNCH_CHECK("k_lp_agg");
     return VNM_OK;

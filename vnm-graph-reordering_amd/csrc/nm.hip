@@ -157,7 +157,8 @@ __global__ __launch_bounds__(LOC_T) void k_locate_all(
         int total = table_columns(sel, 1, M, inv, cptr, cols, pre);
         // row bitmaps: the LDS hash for small segments, the global slot else
         const bool small = total <= HASH_MAX;
-        if (small) hash_scatter(H, M, cols, pre, M, total, crow);
+        const int hb = hash_bits(min(total, HASH_MAX));
+        if (small) hash_scatter(H, hb, M, cols, pre, M, total, crow);
         else table_scatter(slot, M, R, cols, pre, M, total, crow);
         __syncthreads();
         int my_inv = 0, my_nz = 0;
@@ -168,7 +169,7 @@ __global__ __launch_bounds__(LOC_T) void k_locate_all(
             table_entries(cols, pre, M, total, crow, e0, blockDim.x, t, r);
 #pragma unroll
             for (int u = 0; u < TAB_U; ++u)
-                bits[u] = t[u] < 0 ? 0u : small ? (hash_get(H, (uint32_t)r[u]) & 0xFFu) : slot_byte(slot, 0, R, r[u]);
+                bits[u] = t[u] < 0 ? 0u : small ? (hash_get(H, hb, (uint32_t)r[u]) & 0xFFu) : slot_byte(slot, 0, R, r[u]);
 #pragma unroll
             for (int u = 0; u < TAB_U; ++u)
                 if (t[u] >= 0 && (bits[u] >> (M - 1 - t[u])) == 1u) {  // leading bit: the row's owner
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(LOC_T) void k_locate_all(
         if (my_inv) atomicAdd(&c_inv, my_inv);
         if (my_nz) atomicAdd(&c_nz, my_nz);
         __syncthreads();
-        if (small) hash_reset(H);
+        if (small) hash_reset(H, hb);
         else table_clear(slot, M, R, cols, pre, M, total, crow);
         if (threadIdx.x == 0) { cnt[s] = c_inv; nzr[s] = c_nz; }
         __syncthreads();

@@ -115,12 +115,16 @@ __device__ inline void table_pass(uint32_t *tab, int slot0, int M, int R, const 
 // atomic, read and clear per entry in a table far larger than the L2; a set
 // of a few thousand entries touches at most that many rows, which an
 // open-addressing hash in LDS holds instead: key = row, value = the row's
-// bitmaps (byte j = slot j, as in the global slots).  Probes are bounded by
-// the capacity, so every loop ends.
+// bitmaps (byte j = slot j, as in the global slots).  A set uses the first 2^bits
+// slots, the smallest power of two that its entries fill by half at most:
+// most segments of a sparse graph have around a hundred entries, and clearing
+// 4,096 slots for each cost more than filling them.  Slots are empty between
+// uses.  Probes are bounded by the capacity, so every loop ends.
 
 constexpr int HASH_BITS = 12;
 constexpr int HASH_CAP = 1 << HASH_BITS;  // slots (32 KiB of LDS with the values)
 constexpr int HASH_MAX = HASH_CAP / 2;    // entries of a set that uses the hash
+constexpr int HASH_MIN_BITS = 6;
 constexpr uint32_t HASH_EMPTY = 0xFFFFFFFFu;
 constexpr int TILE_ROWS = HASH_CAP * 8;    // rows of an LDS byte tile in the hash's storage
 
@@ -129,49 +133,54 @@ struct RowHash {
     uint32_t val[HASH_CAP];
 };
 
-__device__ __forceinline__ uint32_t hash_home(uint32_t r) { return (r * 0x9E3779B1u) >> (32 - HASH_BITS); }
+// Slots (as their log) for a set of `total` <= HASH_MAX entries.
+__device__ __forceinline__ int hash_bits(int total) {
+    return max(HASH_MIN_BITS, 32 - __builtin_clz(2 * max(total, 1) - 1));
+}
 
-// All slots empty; call with every thread, synchronise before use.
-__device__ inline void hash_reset(RowHash &H) {
-    for (int i = threadIdx.x; i < HASH_CAP; i += blockDim.x) {
+__device__ __forceinline__ uint32_t hash_home(uint32_t r, int bits) { return (r * 0x9E3779B1u) >> (32 - bits); }
+
+// The first 2^bits slots empty; call with every thread, synchronise before use.
+__device__ inline void hash_reset(RowHash &H, int bits = HASH_BITS) {
+    for (int i = threadIdx.x; i < (1 << bits); i += blockDim.x) {
         H.key[i] = HASH_EMPTY;
         H.val[i] = 0u;
     }
 }
 
-__device__ __forceinline__ void hash_or(RowHash &H, uint32_t r, uint32_t bits) {
-    uint32_t h = hash_home(r);
-    for (int p = 0; p < HASH_CAP; ++p) {
+__device__ __forceinline__ void hash_or(RowHash &H, int bits, uint32_t r, uint32_t v) {
+    uint32_t h = hash_home(r, bits);
+    for (int p = 0; p < (1 << bits); ++p) {
         const uint32_t k = atomicCAS(&H.key[h], HASH_EMPTY, r);
         if (k == HASH_EMPTY || k == r) {
-            atomicOr(&H.val[h], bits);
+            atomicOr(&H.val[h], v);
             return;
         }
-        h = (h + 1) & (HASH_CAP - 1);
+        h = (h + 1) & ((1u << bits) - 1);
     }
 }
 
 // Bitmaps of row r (inserted before the last barrier).
-__device__ __forceinline__ uint32_t hash_get(const RowHash &H, uint32_t r) {
-    uint32_t h = hash_home(r);
-    for (int p = 0; p < HASH_CAP; ++p) {
+__device__ __forceinline__ uint32_t hash_get(const RowHash &H, int bits, uint32_t r) {
+    uint32_t h = hash_home(r, bits);
+    for (int p = 0; p < (1 << bits); ++p) {
         const uint32_t k = H.key[h];
         if (k == r) return H.val[h];
         if (k == HASH_EMPTY) return 0u;
-        h = (h + 1) & (HASH_CAP - 1);
+        h = (h + 1) & ((1u << bits) - 1);
     }
     return 0u;
 }
 
 // Insert the entries of nc columns (slot t / M, bit t % M) into the hash.
-__device__ inline void hash_scatter(RowHash &H, int M, const ColSpan *cols, const int *pre, int nc, int total,
+__device__ inline void hash_scatter(RowHash &H, int bits, int M, const ColSpan *cols, const int *pre, int nc, int total,
                                     const int32_t *crow) {
     for (int e0 = threadIdx.x; e0 < total; e0 += blockDim.x * TAB_U) {
         int t[TAB_U], r[TAB_U];
         table_entries(cols, pre, nc, total, crow, e0, blockDim.x, t, r);
 #pragma unroll
         for (int u = 0; u < TAB_U; ++u)
-            if (t[u] >= 0) hash_or(H, (uint32_t)r[u], (1u << (M - 1 - t[u] % M)) << (8 * (t[u] / M)));
+            if (t[u] >= 0) hash_or(H, bits, (uint32_t)r[u], (1u << (M - 1 - t[u] % M)) << (8 * (t[u] / M)));
     }
 }
 
