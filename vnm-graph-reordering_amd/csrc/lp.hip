@@ -32,7 +32,8 @@
 //                          chunks, all summed in a fixed order (bit-reproducible)
 //   k_lp_dense_mfma      : [H, Agg] W + b with v_mfma_f32_16x16x16_bf16
 //   k_lp_dense_f32       : the same on VALU in FP32
-//   k_lp_pair_loss, k_lp_bwd_in, k_lp_wgrad(+reduce), k_lp_adam
+//   k_lp_pair_loss, k_lp_bwd_in, k_lp_wgrad(+reduce), k_lp_adam: the products on
+//                          v_mfma_f32_16x16x4_f32
 //   k_lp_pick/match      : donor and acceptor per segment, candidate pairs
 //   k_lp_pair_gain       : exact M x M gain matrix of a segment pair from the
 //                          entries of its two segments (ballot bit planes)
@@ -656,133 +657,212 @@ __global__ __launch_bounds__(256) void k_lp_dense_f32(int R, const float *__rest
 
 // ------------------------------------------------------------ loss and backward
 
-__global__ __launch_bounds__(256) void k_lp_pair_loss(int count, const int32_t *__restrict__ pairs,
-                                                      const float *__restrict__ target,
-                                                      const float *__restrict__ Y, float *__restrict__ dY,
-                                                      float *__restrict__ part) {
-    __shared__ float red[256];
-    const int i = blockIdx.x * 256 + threadIdx.x;
+// Pair scores, the loss's partial sums and dY.  16 lanes per pair, one of the 16
+// products each, so the rows' loads and the atomics cover whole 64-byte pieces (a
+// thread per pair walked 34 scattered atomics: 44 us at 16,384 pairs, 13 now); a
+// workgroup takes LOSS_PAIRS pairs.
+constexpr int LOSS_T = 1024, LOSS_PAIRS = 256;
+__global__ __launch_bounds__(LOSS_T) void k_lp_pair_loss(int count, const int32_t *__restrict__ pairs,
+                                                         const float *__restrict__ target,
+                                                         const float *__restrict__ Y, float *__restrict__ dY,
+                                                         float *__restrict__ part) {
+    __shared__ float red[LOSS_T / 64];
+    const int lane = threadIdx.x & 63, j = lane & 15;
     float l = 0.f;
-    if (i < count) {
+    for (int p = threadIdx.x >> 4; p < LOSS_PAIRS; p += LOSS_T / 16) {
+        const int i = blockIdx.x * LOSS_PAIRS + p;
+        if (i >= count) break;
         const int u = pairs[2 * i], v = pairs[2 * i + 1];
         const float *yu = Y + (size_t)u * LP_HD, *yv = Y + (size_t)v * LP_HD;
-        float s = yu[0] + yv[1];
-        for (int j = 0; j < LP_PQ; ++j) s += yu[2 + j] * yv[2 + LP_PQ + j];
-        const float d = s - target[i];
-        l = d * d;
+        const float pu = yu[2 + j], qv = yv[2 + LP_PQ + j];
+        float s = pu * qv;
+#pragma unroll
+        for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+        const float d = (yu[0] + yv[1] + s) - target[i];
         const float ds = 2.0f * d / (float)count;
-        atomicAdd(&dY[(size_t)u * LP_HD + 0], ds);
-        atomicAdd(&dY[(size_t)v * LP_HD + 1], ds);
-        for (int j = 0; j < LP_PQ; ++j) {
-            atomicAdd(&dY[(size_t)u * LP_HD + 2 + j], ds * yv[2 + LP_PQ + j]);
-            atomicAdd(&dY[(size_t)v * LP_HD + 2 + LP_PQ + j], ds * yu[2 + j]);
+        float *du = dY + (size_t)u * LP_HD, *dv = dY + (size_t)v * LP_HD;
+        atomicAdd(&du[2 + j], ds * qv);
+        atomicAdd(&dv[2 + LP_PQ + j], ds * pu);
+        if (j == 0) {
+            l += d * d;
+            atomicAdd(&du[0], ds);
+            atomicAdd(&dv[1], ds);
         }
     }
-    red[threadIdx.x] = l;
+    for (int o = 32; o >= 1; o >>= 1) l += __shfl_xor(l, o, 64);
+    if (lane == 0) red[threadIdx.x >> 6] = l;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
+    if (threadIdx.x == 0) {
+        float s = 0.f;
+        for (int w = 0; w < LOSS_T / 64; ++w) s += red[w];
+        part[blockIdx.x] = s;
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = red[0];
+}
+
+// The backward products run on v_mfma_f32_16x16x4_f32: FP32 operands, FP32
+// accumulation, as the vector FMAs they replace.  Lane l of an operand holds row
+// (A) or column (B) l % 16 at contraction index l / 16, of the result column l %
+// 16 in rows 4 (l / 16) .. + 3.
+
+// 16 values of dPre = dOut * [Hout > 0] (MASK) or dOut from p on.
+template <typename T, bool MASK>
+__device__ __forceinline__ void load_dpre(const float *__restrict__ dOut, const T *__restrict__ Hout, size_t p,
+                                          float (&d)[16]) {
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) {
+        const float4 x = *(const float4 *)(dOut + p + i);
+        d[i] = x.x; d[i + 1] = x.y; d[i + 2] = x.z; d[i + 3] = x.w;
+        if constexpr (MASK) {
+            const float4 h = Act<T>::load4(Hout + p + i);
+            if (!(h.x > 0.f)) d[i] = 0.f;
+            if (!(h.y > 0.f)) d[i + 1] = 0.f;
+            if (!(h.z > 0.f)) d[i + 2] = 0.f;
+            if (!(h.w > 0.f)) d[i + 3] = 0.f;
+        }
+    }
 }
 
 // dA = dPre W[:KA]^T, dB = dPre W[KA:]^T with dPre = dOut * [Hout > 0] (MASK)
-// or dOut.  Four rows per step; W staged transposed so lanes read
-// consecutive k.
+// or dOut.  A wave takes 16 rows: lane group g = l / 16 contracts columns 16 g ..
+// 16 g + 15 of dPre, so both operands are runs of 16 values read as they lie
+// (W's rows stay in L2: no LDS).  64 -> 128 columns, 16,384 rows: 71 us with FMAs
+// on W in LDS (its transposing store and its reads bound by bank conflicts), 9 now.
 template <typename T, int KA, int KB, bool MASK>
 __global__ __launch_bounds__(256) void k_lp_bwd_in(int R, const float *__restrict__ dOut,
                                                    const T *__restrict__ Hout,
                                                    const float *__restrict__ W,
                                                    float *__restrict__ dA, float *__restrict__ dB) {
-    constexpr int K = KA + KB;
-    __shared__ float wt[64 * K];
-    __shared__ float d[4][64];
-    for (int i = threadIdx.x; i < K * 64; i += 256) {
-        const int k = i / 64, n = i % 64;
-        wt[n * K + k] = W[i];
-    }
-    for (int r0 = blockIdx.x * 4; r0 < R; r0 += gridDim.x * 4) {
-        __syncthreads();
-        {
-            const int q = threadIdx.x >> 6, n = threadIdx.x & 63, rr = r0 + q;
-            float gv = 0.f;
-            if (rr < R) {
-                gv = dOut[(size_t)rr * 64 + n];
-                if (MASK && !(Act<T>::get(Hout + (size_t)rr * 64 + n) > 0.f)) gv = 0.f;
+    constexpr int KT = (KA + KB) / 16, TW = 2;  // 16-column result tiles, TW at a time
+    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
+    const int r0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+    if (r0 >= R) return;
+    float d[16];
+    load_dpre<T, MASK>(dOut, Hout, (size_t)min(r0 + m, R - 1) * 64 + 16 * g, d);
+#pragma unroll
+    for (int kt = 0; kt < KT; kt += TW) {
+        float w[TW][16];
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+#pragma unroll
+            for (int i = 0; i < 16; i += 4) {
+                const float4 x = *(const float4 *)(W + (size_t)((kt + t) * 16 + m) * 64 + 16 * g + i);
+                w[t][i] = x.x; w[t][i + 1] = x.y; w[t][i + 2] = x.z; w[t][i + 3] = x.w;
             }
-            d[q][n] = gv;
-        }
-        __syncthreads();
-        for (int o = threadIdx.x; o < 4 * K; o += 256) {
-            const int q = o / K, k = o % K, rr = r0 + q;
-            if (rr >= R) continue;
-            float s = 0.f;
-#pragma unroll 8
-            for (int n = 0; n < 64; ++n) s += d[q][n] * wt[n * K + k];
-            if (k < KA) dA[(size_t)rr * KA + k] = s;
-            else dB[(size_t)rr * KB + (k - KA)] = s;
+        f32x4_t acc[TW];
+#pragma unroll
+        for (int t = 0; t < TW; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int t = 0; t < TW; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[i], w[t][i], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int k = (kt + t) * 16 + m;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int rr = r0 + 4 * g + i;
+                if (rr >= R) continue;
+                if ((kt + t) * 16 < KA) dA[(size_t)rr * KA + k] = acc[t][i];
+                else dB[(size_t)rr * KB + (k - KA)] = acc[t][i];
+            }
         }
     }
 }
 
-// Partial weight and bias gradients of one layer over a strided share of
-// the rows: part[blk][k*64 + n] = sum_r [A|B][r][k] dPre[r][n], then the 64
-// bias sums.  k_lp_wgrad_reduce adds the partials in block order.
+// Partial weight and bias gradients of one layer over a share of the rows:
+// part[blk][k*64 + n] = sum_r [A|B][r][k] dPre[r][n], then the 64 bias sums.
+// k_lp_wgrad_reduce adds the partials.  Contraction over rows, 4 a step; the
+// K/16 x 4 result tiles go round the workgroup's 4 waves.  128 x 64 outputs,
+// 16,384 rows: 32 us with FMAs from LDS, 20 now.
 template <typename T, int KA, int KB, bool MASK>
 __global__ __launch_bounds__(256) void k_lp_wgrad(int R, const T *__restrict__ A, const T *__restrict__ B,
                                                   const float *__restrict__ dOut,
                                                   const T *__restrict__ Hout, float *__restrict__ part) {
-    // thread (kb, n) owns outputs k = kb + 4j of column n, j < K/4, and, for
-    // kb == 0, the bias of column n
-    constexpr int K = KA + KB, RW = 16, NOUT = K * 64 + 64, NJ = K / 4;
-    __shared__ float cin[RW][K];
-    __shared__ float d[RW][64];
-    const int n = threadIdx.x & 63, kb = threadIdx.x >> 6;
-    float acc[NJ];
+    constexpr int K = KA + KB, NOUT = K * 64 + 64;
+    constexpr int KW = K >= 64 ? K / 64 : 1;  // 16-row tiles of a wave
+    constexpr int NW = K >= 64 ? 4 : 2;       // its 16-column tiles
+    constexpr int UN = 4;                     // steps whose loads go out together
+    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4, wv = threadIdx.x >> 6;
+    const int k0 = (K >= 64 ? wv * KW : wv / 2) * 16, n0 = K >= 64 ? 0 : (wv & 1) * 32;
+    const int rows = ((R + gridDim.x - 1) / gridDim.x + 3) / 4 * 4;  // of a workgroup
+    const int rb = blockIdx.x * rows, re = min(R, rb + rows);
+    f32x4_t acc[KW][NW];
+    float bias[NW];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = 0.f;
-    float accb = 0.f;
-    for (int r0 = blockIdx.x * RW; r0 < R; r0 += gridDim.x * RW) {
-        __syncthreads();
-        for (int i = threadIdx.x; i < RW * K; i += 256) {
-            const int q = i / K, k = i % K, rr = r0 + q;
-            float x = 0.f;
-            if (rr < R) x = k < KA ? Act<T>::get(A + (size_t)rr * KA + k) : Act<T>::get(B + (size_t)rr * KB + (k - KA));
-            cin[q][k] = x;
-        }
-        for (int i = threadIdx.x; i < RW * 64; i += 256) {
-            const int q = i / 64, c = i % 64, rr = r0 + q;
-            float gv = 0.f;
-            if (rr < R) {
-                gv = dOut[(size_t)rr * 64 + c];
-                if (MASK && !(Act<T>::get(Hout + (size_t)rr * 64 + c) > 0.f)) gv = 0.f;
+    for (int t = 0; t < NW; ++t) {
+        bias[t] = 0.f;
+#pragma unroll
+        for (int q = 0; q < KW; ++q) acc[q][t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    for (int r = rb; r < re; r += 4 * UN) {
+        float a[UN][KW], d[UN][NW];
+#pragma unroll
+        for (int s = 0; s < UN; ++s) {
+            const int rr = r + 4 * s + g;
+            const bool in = rr < re;
+            const size_t rc = (size_t)min(rr, R - 1);
+#pragma unroll
+            for (int q = 0; q < KW; ++q) {
+                const int k = k0 + q * 16 + m;
+                const float x = k < KA ? Act<T>::get(A + rc * KA + k) : Act<T>::get(B + rc * KB + (k - KA));
+                a[s][q] = in ? x : 0.f;
             }
-            d[q][c] = gv;
-        }
-        __syncthreads();
-        for (int q = 0; q < RW; ++q) {
-            const float dq = d[q][n];
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[j] += cin[q][kb + 4 * j] * dq;
-            accb += dq;
+            for (int t = 0; t < NW; ++t) {
+                const size_t p = rc * 64 + n0 + t * 16 + m;
+                const float x = dOut[p];
+                d[s][t] = in && (!MASK || Act<T>::get(Hout + p) > 0.f) ? x : 0.f;
+            }
         }
+#pragma unroll
+        for (int s = 0; s < UN; ++s)
+#pragma unroll
+            for (int t = 0; t < NW; ++t) {
+                bias[t] += d[s][t];
+#pragma unroll
+                for (int q = 0; q < KW; ++q)
+                    acc[q][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][q], d[s][t], acc[q][t], 0, 0, 0);
+            }
     }
     float *o = part + (size_t)blockIdx.x * NOUT;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) o[(kb + 4 * j) * 64 + n] = acc[j];
-    if (kb == 0) o[K * 64 + n] = accb;
+    for (int t = 0; t < NW; ++t) {
+#pragma unroll
+        for (int q = 0; q < KW; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[(k0 + q * 16 + 4 * g + i) * 64 + n0 + t * 16 + m] = acc[q][t][i];
+        if (k0 == 0) {
+            float b = bias[t];
+            b += __shfl_xor(b, 16, 64);
+            b += __shfl_xor(b, 32, 64);
+            if (g == 0) o[K * 64 + n0 + t * 16 + m] = b;
+        }
+    }
 }
 
-__global__ void k_lp_wgrad_reduce(int nblk, int K, const float *__restrict__ part,
-                                  float *__restrict__ gw, float *__restrict__ gb) {
-    const int nout = K * 64 + 64;
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= nout) return;
+// Sums of the nblk partials, 64 outputs a workgroup: wave w adds partials w,
+// w + 16, ..., then the waves' sums in order.  (One thread per output walking
+// all 256 partials: 61 us for 8,256 outputs; 5 now.)
+constexpr int WR_T = 1024;
+__global__ __launch_bounds__(WR_T) void k_lp_wgrad_reduce(int nblk, int K, const float *__restrict__ part,
+                                                          float *__restrict__ gw, float *__restrict__ gb) {
+    constexpr int W = WR_T / 64;
+    __shared__ float sum[W][64];
+    const int nout = K * 64 + 64;  // a multiple of 64
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int o = blockIdx.x * 64 + lane;
     float s = 0.f;
-    for (int b = 0; b < nblk; ++b) s += part[(size_t)b * nout + o];
-    if (o < K * 64) gw[o] = s;
-    else gb[o - K * 64] = s;
+#pragma unroll 16
+    for (int b = w; b < nblk; b += W) s += part[(size_t)b * nout + o];
+    sum[w][lane] = s;
+    __syncthreads();
+    if (w == 0) {
+        s = 0.f;
+#pragma unroll
+        for (int i = 0; i < W; ++i) s += sum[i][lane];
+        if (o < K * 64) gw[o] = s;
+        else gb[o - K * 64] = s;
+    }
 }
 
 __global__ void k_lp_adam(int n, float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
@@ -1643,19 +1723,19 @@ static int lp_backward_t(vnm_graph *g, LPCache *c, vnm_lp_model *m) {
     const T *H3 = (const T *)c->H3.p;
     float *G = m->g.p;
     const int gb = std::min(WG_GRID, std::max(1, (R + 15) / 16));
-    const int gi = grid_of(R, 4, 4096);
+    const int gi = (R + 63) / 64;
     int rc;
     // head: dY -> dWh, dbh, dH3
     hipLaunchKernelGGL((k_lp_wgrad<T, 64, 0, false>), dim3(gb), dim3(256), 0, st, R, H3, (const T *)nullptr,
                        c->dY.p, (const T *)nullptr, c->part.p);
-    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(grid_of(64 * 64 + 64, 256)), dim3(256), 0, st, gb, 64,
+    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(65), dim3(WR_T), 0, st, gb, 64,
                        c->part.p, G + LP_OFF_WH, G + LP_OFF_BH);
     hipLaunchKernelGGL((k_lp_bwd_in<T, 64, 0, false>), dim3(gi), dim3(256), 0, st, R, c->dY.p,
                        (const T *)nullptr, m->w.p + LP_OFF_WH, c->dH.p, (float *)nullptr);
     // layer 2: dH = dH3
     hipLaunchKernelGGL((k_lp_wgrad<T, 64, 64, true>), dim3(gb), dim3(256), 0, st, R, H2, A2, c->dH.p, H3,
                        c->part.p);
-    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(grid_of(128 * 64 + 64, 256)), dim3(256), 0, st, gb, 128,
+    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(129), dim3(WR_T), 0, st, gb, 128,
                        c->part.p, G + LP_OFF_W[2], G + LP_OFF_B[2]);
     hipLaunchKernelGGL((k_lp_bwd_in<T, 64, 64, true>), dim3(gi), dim3(256), 0, st, R, c->dH.p, H3,
                        m->w.p + LP_OFF_W[2], c->dIn.p, c->dAg.p);
@@ -1663,7 +1743,7 @@ static int lp_backward_t(vnm_graph *g, LPCache *c, vnm_lp_model *m) {
     // layer 1: dH2 in dIn
     hipLaunchKernelGGL((k_lp_wgrad<T, 64, 64, true>), dim3(gb), dim3(256), 0, st, R, H1, A1, c->dIn.p, H2,
                        c->part.p);
-    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(grid_of(128 * 64 + 64, 256)), dim3(256), 0, st, gb, 128,
+    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(129), dim3(WR_T), 0, st, gb, 128,
                        c->part.p, G + LP_OFF_W[1], G + LP_OFF_B[1]);
     hipLaunchKernelGGL((k_lp_bwd_in<T, 64, 64, true>), dim3(gi), dim3(256), 0, st, R, c->dIn.p, H2,
                        m->w.p + LP_OFF_W[1], c->dH.p, c->dAg.p);
@@ -1671,7 +1751,7 @@ static int lp_backward_t(vnm_graph *g, LPCache *c, vnm_lp_model *m) {
     // layer 0: dH1 in dH (input features need no gradient)
     hipLaunchKernelGGL((k_lp_wgrad<T, 16, 16, true>), dim3(gb), dim3(256), 0, st, R, X, A0, c->dH.p, H1,
                        c->part.p);
-    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(grid_of(32 * 64 + 64, 256)), dim3(256), 0, st, gb, 32,
+    hipLaunchKernelGGL(k_lp_wgrad_reduce, dim3(33), dim3(WR_T), 0, st, gb, 32,
                        c->part.p, G + LP_OFF_W[0], G + LP_OFF_B[0]);
     g->ctx->launches += 13;
     VNM_LAUNCH_CHECK("lp_backward");
@@ -1698,7 +1778,7 @@ static int lp_loss_grad(vnm_graph *g, LPCache *c, vnm_lp_model *m, int bf16, con
             (rc = c->lpart.alloc(65536)))
             return rc;
     }
-    const int nb = (count + 255) / 256;
+    const int nb = (count + LOSS_PAIRS - 1) / LOSS_PAIRS;
     if (nb > 65536) return set_error(VNM_E_ARG, "too many training pairs (%d)", count);
     if (count) {
         VNM_HIP_TRY(hipMemcpyAsync(c->pairs.p, pairs, (size_t)count * 8, hipMemcpyHostToDevice, st));
@@ -1706,7 +1786,7 @@ static int lp_loss_grad(vnm_graph *g, LPCache *c, vnm_lp_model *m, int bf16, con
     }
     VNM_HIP_TRY(hipMemsetAsync(c->dY.p, 0, (size_t)R * 64 * 4, st));
     if (count)
-        hipLaunchKernelGGL(k_lp_pair_loss, dim3(nb), dim3(256), 0, st, count, c->pairs.p, c->target.p, c->Y.p,
+        hipLaunchKernelGGL(k_lp_pair_loss, dim3(nb), dim3(LOSS_T), 0, st, count, c->pairs.p, c->target.p, c->Y.p,
                            c->dY.p, c->lpart.p);
     g->ctx->launches++;
     VNM_LAUNCH_CHECK("k_lp_pair_loss");
