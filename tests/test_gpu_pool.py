@@ -1,0 +1,56 @@
+"""The device memory that a context keeps between its calls (GPU): results on
+reused buffers equal those on fresh ones, over calls of growing and shrinking
+size, with objects that outlive their call, and with two contexts in threads."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+import vnm
+
+pytestmark = pytest.mark.gpu
+SIZES = [(300, 4), (4096, 12), (900, 6), (5000, 9), (300, 4), (4096, 12)]
+
+
+def product(ctx, p, n, B):
+    C = torch.full((n, 64), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    p.spmm(B.data_ptr(), 64, 64, vnm.DT_F32, C.data_ptr(), 64)
+    torch.cuda.synchronize()
+    return C.cpu().numpy()
+
+
+def call(ctx, n, deg, keep):
+    rng = np.random.default_rng(n)
+    r = rng.integers(0, n, n * deg).astype(np.int32)
+    c = rng.integers(0, n, n * deg).astype(np.int32)
+    m = vnm.coo_from_tuples(n, n, r, c, rng.uniform(-1, 1, n * deg).astype(np.float32), 8)
+    B = torch.from_numpy(rng.standard_normal((n, 64)).astype(np.float32)).cuda()
+    g = vnm.Graph(ctx, m, 8)
+    g.lp_reorder(None, 2, mode=vnm.LP_EXHAUSTIVE, maxiter=3)
+    p = g.pack(64, vnm.DT_F32)
+    out = product(ctx, p, n, B)
+    keep.append((g, p, n, B, out))
+    return out, g.perm()
+
+
+def series(ctx, out):
+    keep = []
+    out.extend(call(ctx, n, d, keep) for n, d in SIZES)
+    for g, p, n, B, ref in keep[::-1]:  # objects still whole after the later calls
+        assert np.array_equal(product(ctx, p, n, B), ref)
+
+
+def test_reused_buffers():
+    fresh = [call(vnm.Context(0), n, d, []) for n, d in SIZES]
+    got = [[], []]
+    ts = [threading.Thread(target=series, args=(vnm.Context(0), got[i])) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for res in got:
+        assert len(res) == len(fresh)
+        for (a, pa), (b, pb) in zip(res, fresh):
+            assert np.array_equal(a, b) and np.array_equal(pa, pb)

@@ -472,5 +472,6 @@ using namespace vnm;
 
 extern "C" int vnm_nm_reorder_allpairs(vnm_graph *g, int N, int sched, int maxiter, int clean, vnm_nm_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     return nm_reorder_allpairs(g, N, sched, maxiter, clean, st);
 }

@@ -128,6 +128,7 @@ int vnm_ctx_create(int device, vnm_ctx **out) {
     VNM_HIP_TRY(hipSetDevice(device));
     vnm_ctx *c = new vnm_ctx();
     c->device = device;
+    c->pool = std::make_shared<DevPool>();
     int rc = noalloc_setup(device, &c->noalloc_slots);
     if (rc) {
         delete c;
@@ -168,6 +169,7 @@ int vnm_graph_create(vnm_ctx *ctx, const vnm_coo *coo, int M, vnm_graph **out) {
             coo->col[i] >= coo->ncols)
             return set_error(VNM_E_ARG, "entry %lld out of range", (long long)i);
     VNM_HIP_TRY(hipSetDevice(ctx->device));
+    PoolScope pool(ctx->pool);
     vnm_graph *g = new vnm_graph();
     g->ctx = ctx;
     g->nrows = coo->nrows;

@@ -437,6 +437,7 @@ extern "C" {
 int vnm_batch_create(vnm_ctx *ctx, vnm_packed *const *ps, int count, const void *const *B, const int32_t *ldb,
                      int n, int b_dtype, const float *const *b_scales, float *const *C, const int32_t *ldc,
                      const float *const *bias, int cols_per_lane, vnm_batch **out) {
+    PoolScope pool(ctx ? ctx->pool : nullptr);
     return batch_create(ctx, ps, count, B, ldb, n, b_dtype, b_scales, C, ldc, bias, cols_per_lane, out);
 }
 
@@ -466,6 +467,7 @@ void vnm_batch_destroy(vnm_batch *b) {
 
 int vnm_gcn_layer(vnm_packed *p, const uint16_t *X, int ldx, int K, const uint16_t *W, int N, const float *bias,
                   float *Y, int ldy) {
+    PoolScope pool(p ? p->ctx->pool : nullptr);
     return gcn_layer(p, X, ldx, K, W, N, bias, Y, ldy);
 }
 

@@ -178,7 +178,10 @@ int build_dense(vnm_packed *p, int dense_min, int U, int nb, int nblk, const int
     p->nmulti = (int)multi.size();
     p->ndslots = nds;
     VNM_HIP_TRY(hipMemcpyAsync(dmap.p, hmap.data(), hmap.size() * 4, hipMemcpyHostToDevice, st));
-    if (nch == 0) return VNM_OK;
+    if (nch == 0) {
+        VNM_HIP_TRY(hipStreamSynchronize(st));  // the copy reads this frame's vector
+        return VNM_OK;
+    }
     const size_t nf = (size_t)nch * S * 64;
     if ((rc = p->dgrp.alloc(grp.size())) || (rc = p->dcol.alloc(col.size())) || (rc = p->dfrag.alloc(nf * 4)) ||
         (rc = p->didx.alloc(nf)) || (rc = p->dvb.alloc(nblk)) || (rc = p->dmulti.alloc(std::max<size_t>(multi.size(), 1))))

@@ -6,6 +6,8 @@
 #include "vnm_internal.h"
 
 #include <map>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -16,9 +18,91 @@ struct vnm_timer_pending {
     hipEvent_t a, b;
 };
 
+namespace vnm {
+
+// Idle device memory of one context, for its next calls: packing takes 60
+// buffers and a learned reorder 45, and hipMalloc and hipFree (which waits for the
+// whole device) were most of such a call's time (packing R-MAT 65,536 took 7.6 ms,
+// of it 0.9 in kernels, and 1.27 from the pool; its learned reorder 8.1 ms and 5.8).  A block given back may still be read by
+// work enqueued on the context's stream; the next owner's work is enqueued behind
+// it, on the same stream, so nothing waits.  (Host copies into a block go through
+// the stream as well.)  At most POOL_IDLE bytes stay idle; the context and its
+// objects share the pool, and the last of them frees it.
+constexpr size_t POOL_IDLE = (size_t)2 << 30;
+constexpr size_t POOL_GRAIN = 4096;
+
+class DevPool {
+public:
+    // A block of at least `bytes`; *cap its size.
+    hipError_t take(size_t bytes, void **p, size_t *cap) {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            auto it = idle.lower_bound(bytes);
+            if (it != idle.end() && it->first <= 2 * bytes + POOL_GRAIN) {
+                *p = it->second;
+                *cap = it->first;
+                idle_bytes -= it->first;
+                idle.erase(it);
+                return hipSuccess;
+            }
+        }
+        // rounded up to an eighth of its size, so that a little growth still fits
+        size_t grain = POOL_GRAIN;
+        while (grain * 16 <= bytes) grain *= 2;
+        const size_t want = (bytes + grain - 1) / grain * grain;
+        hipError_t e = hipMalloc(p, want);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            flush();
+            e = hipMalloc(p, want);
+        }
+        *cap = want;
+        return e;
+    }
+    void give(void *p, size_t cap) noexcept {
+        try {
+            std::lock_guard<std::mutex> lk(mu);
+            if (idle_bytes + cap <= POOL_IDLE) {
+                idle.emplace(cap, p);
+                idle_bytes += cap;
+                return;
+            }
+        } catch (...) {  // no memory for the entry
+        }
+        (void)hipFree(p);
+    }
+    void flush() {
+        std::lock_guard<std::mutex> lk(mu);
+        for (auto &b : idle) (void)hipFree(b.second);
+        idle.clear();
+        idle_bytes = 0;
+    }
+    ~DevPool() { flush(); }
+
+private:
+    std::mutex mu;
+    std::multimap<size_t, void *> idle;
+    size_t idle_bytes = 0;
+};
+
+// The pool that this host thread's allocations come from, for the length of a
+// scope: each entry point opens one for its context.
+inline thread_local std::shared_ptr<DevPool> t_pool;
+
+struct PoolScope {
+    std::shared_ptr<DevPool> prev;
+    explicit PoolScope(const std::shared_ptr<DevPool> &p) : prev(t_pool) { t_pool = p; }
+    ~PoolScope() { t_pool = prev; }
+    PoolScope(const PoolScope &) = delete;
+    PoolScope &operator=(const PoolScope &) = delete;
+};
+
+}  // namespace vnm
+
 struct vnm_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    std::shared_ptr<vnm::DevPool> pool;
     float *noalloc_slots = nullptr;  // device address of the static SpMM slot array on `device`
     int64_t launches = 0;
     bool timing = false;
@@ -28,7 +112,7 @@ struct vnm_ctx {
 
 namespace vnm {
 
-// A device buffer owned by a graph.
+// A device buffer, from the pool of the scope it was allocated in.
 template <typename T>
 struct DBuf {
     T *p = nullptr;
@@ -36,25 +120,42 @@ struct DBuf {
     int alloc(size_t count) {
         release();
         if (count == 0) count = 1;
-        hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+        hipError_t e;
+        if (t_pool) e = t_pool->take(count * sizeof(T), (void **)&p, &cap);
+        else e = hipMalloc((void **)&p, count * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
             (void)hipGetLastError();
             return set_error(e == hipErrorOutOfMemory ? VNM_E_OOM : VNM_E_HIP,
                              "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
         }
+        pool = t_pool;
         n = count;
         return VNM_OK;
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (pool) pool->give(p, cap);
+            else (void)hipFree(p);
+        }
+        pool.reset();
         p = nullptr;
         n = 0;
+    }
+    void swap(DBuf &o) {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        std::swap(cap, o.cap);
+        pool.swap(o.pool);
     }
     DBuf() = default;
     DBuf(const DBuf &) = delete;
     DBuf &operator=(const DBuf &) = delete;
     ~DBuf() { release(); }
+
+private:
+    size_t cap = 0;
+    std::shared_ptr<DevPool> pool;
 };
 
 }  // namespace vnm

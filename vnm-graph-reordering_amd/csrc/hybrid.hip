@@ -132,6 +132,7 @@ extern "C" {
 
 int vnm_hybrid(vnm_graph *g, int N, int V, int rounds, int sched, vnm_hybrid_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     if (V <= 0) return set_error(VNM_E_ARG, "V must be positive (got %d)", V);
     if (rounds < 0) return set_error(VNM_E_ARG, "rounds must be >= 0");
     return hybrid(g, N, V, rounds, sched, st);
@@ -140,6 +141,7 @@ int vnm_hybrid(vnm_graph *g, int N, int V, int rounds, int sched, vnm_hybrid_sta
 int vnm_hybrid_learned(vnm_graph *g, const vnm_lp_model *m, int N, int V, int rounds, int mode, int topk,
                        int window, int maxiter, vnm_hybrid_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     if (V <= 0) return set_error(VNM_E_ARG, "V must be positive (got %d)", V);
     if (rounds < 0) return set_error(VNM_E_ARG, "rounds must be >= 0");
     return hybrid_learned(g, m, N, V, rounds, mode, topk, window, maxiter, st);
@@ -147,12 +149,14 @@ int vnm_hybrid_learned(vnm_graph *g, const vnm_lp_model *m, int N, int V, int ro
 
 int vnm_graph_clone(vnm_graph *g, vnm_graph **out) {
     if (!g || !out) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     return graph_clone(g, out);
 }
 
 int vnm_find_best_sched(vnm_graph *g, int N, int nsched, int32_t *best) {
     if (!g || !best || nsched < 1 || nsched > 4)
         return set_error(VNM_E_ARG, "find_best: nsched must be 1..4");
+    PoolScope pool(g->ctx->pool);
     return find_best_sched(g, N, nsched, best);
 }
 

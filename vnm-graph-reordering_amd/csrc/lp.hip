@@ -1488,7 +1488,7 @@ struct LPCache {
 
 static void lp_cache_free(void *p) { delete (LPCache *)p; }
 
-static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P) {
+static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P, hipStream_t st) {
     std::vector<int32_t> heavy, ch0{0}, beg, end, longs;
     const int R = (int)hptr.size() - 1;
     for (int u = 0; u < R; ++u) {
@@ -1515,13 +1515,14 @@ static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P) {
         (rc = P.beg.alloc(std::max(1, P.nch))) || (rc = P.end.alloc(std::max(1, P.nch))) ||
         (rc = P.part.alloc((size_t)std::max(1, P.nch) * 64)) || (rc = P.longs.alloc(std::max(1, P.nlong))))
         return rc;
-    if (P.nlong) VNM_HIP_TRY(hipMemcpy(P.longs.p, longs.data(), longs.size() * 4, hipMemcpyHostToDevice));
+    if (P.nlong) VNM_HIP_TRY(hipMemcpyAsync(P.longs.p, longs.data(), longs.size() * 4, hipMemcpyHostToDevice, st));
     if (P.nheavy) {
-        VNM_HIP_TRY(hipMemcpy(P.heavy.p, heavy.data(), heavy.size() * 4, hipMemcpyHostToDevice));
-        VNM_HIP_TRY(hipMemcpy(P.beg.p, beg.data(), beg.size() * 4, hipMemcpyHostToDevice));
-        VNM_HIP_TRY(hipMemcpy(P.end.p, end.data(), end.size() * 4, hipMemcpyHostToDevice));
+        VNM_HIP_TRY(hipMemcpyAsync(P.heavy.p, heavy.data(), heavy.size() * 4, hipMemcpyHostToDevice, st));
+        VNM_HIP_TRY(hipMemcpyAsync(P.beg.p, beg.data(), beg.size() * 4, hipMemcpyHostToDevice, st));
+        VNM_HIP_TRY(hipMemcpyAsync(P.end.p, end.data(), end.size() * 4, hipMemcpyHostToDevice, st));
     }
-    VNM_HIP_TRY(hipMemcpy(P.ch0.p, ch0.data(), ch0.size() * 4, hipMemcpyHostToDevice));
+    VNM_HIP_TRY(hipMemcpyAsync(P.ch0.p, ch0.data(), ch0.size() * 4, hipMemcpyHostToDevice, st));
+    VNM_HIP_TRY(hipStreamSynchronize(st));  // the copies read this frame's vectors
     return VNM_OK;
 }
 
@@ -1583,7 +1584,7 @@ static int lp_prepare(vnm_graph *g, LPCache **out) {
     if ((rc = build_lists(g, kc.p, tmp.p, nnz, nvalid, c->ptr, c->idx, hp))) return rc;
     if ((rc = c->inv_deg.alloc(R))) return rc;
     hipLaunchKernelGGL(k_lp_inv_deg, dim3(grid_of(R, 256)), dim3(256), 0, st, R, c->ptr.p, c->inv_deg.p);
-    if ((rc = agg_plan(hp, c->fwd))) return rc;
+    if ((rc = agg_plan(hp, c->fwd, st))) return rc;
     const int ns = c->nseg;
     if ((rc = c->ccls.alloc((size_t)R * 4)) || (rc = c->segcls.alloc((size_t)ns * 4)) ||
         (rc = c->segnnz.alloc(ns)) || (rc = c->tot.alloc(4)))
@@ -1636,7 +1637,7 @@ static int lp_prepare_bwd(vnm_graph *g, LPCache *c) {
     VNM_LAUNCH_CHECK("k_lp_adj_keys");
     std::vector<int32_t> htp;
     if ((rc = build_lists(g, kt.p, tmp.p, nnz, c->nadj, c->tptr, c->tidx, htp))) return rc;
-    if ((rc = agg_plan(htp, c->bwd))) return rc;
+    if ((rc = agg_plan(htp, c->bwd, st))) return rc;
     c->has_bwd = true;
     return VNM_OK;
 }
@@ -2212,6 +2213,7 @@ extern "C" {
 
 int vnm_lp_model_create(vnm_ctx *ctx, const float *params, uint64_t seed, vnm_lp_model **out) {
     if (!ctx || !out) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(ctx->pool);
     VNM_HIP_TRY(hipSetDevice(ctx->device));
     vnm_lp_model *m = new vnm_lp_model();
     m->ctx = ctx;
@@ -2269,6 +2271,7 @@ int vnm_lp_model_get(const vnm_lp_model *m, float *params) {
 
 int vnm_lp_features(vnm_graph *g, int N, float *X) {
     if (!g || !X) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     LPCache *c;
     int rc = lp_begin(g, N, &c);
     if (rc) return rc;
@@ -2284,6 +2287,7 @@ int vnm_lp_features(vnm_graph *g, int N, float *X) {
 
 int vnm_lp_forward(vnm_lp_model *m, vnm_graph *g, int N, int bf16, float *head) {
     if (!m || !g || !head || m->ctx != g->ctx) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     LPCache *c;
     int rc = lp_begin(g, N, &c);
     if (rc) return rc;
@@ -2298,6 +2302,7 @@ int vnm_lp_loss_grad(vnm_lp_model *m, vnm_graph *g, int N, int bf16, const int32
                      const float *target, int count, float *loss, float *grad) {
     if (!m || !g || count < 0 || (count > 0 && (!pairs || !target)) || m->ctx != g->ctx)
         return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     for (int i = 0; i < 2 * count; ++i)
         if (pairs[i] < 0 || pairs[i] >= g->nrows) return set_error(VNM_E_ARG, "pair id out of range");
     LPCache *c;
@@ -2316,6 +2321,7 @@ int vnm_lp_train_step(vnm_lp_model *m, vnm_graph *g, int N, const int32_t *pairs
                       int count, float lr, float *loss) {
     if (!m || !g || count < 1 || !pairs || !target || !(lr > 0.f) || m->ctx != g->ctx)
         return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     for (int i = 0; i < 2 * count; ++i)
         if (pairs[i] < 0 || pairs[i] >= g->nrows) return set_error(VNM_E_ARG, "pair id out of range");
     LPCache *c;
@@ -2337,6 +2343,7 @@ int vnm_lp_train_step(vnm_lp_model *m, vnm_graph *g, int N, const int32_t *pairs
 
 int vnm_pair_score(vnm_graph *g, int N, const int32_t *segp, const int32_t *segq, int count, int32_t *scores) {
     if (!g || count < 0 || (count > 0 && (!segp || !segq || !scores))) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     LPCache *c;
     int rc = lp_check(g, N);
     if (rc) return rc;
@@ -2366,12 +2373,14 @@ int vnm_pair_score(vnm_graph *g, int N, const int32_t *segp, const int32_t *segq
 int vnm_lp_reorder(vnm_graph *g, const vnm_lp_model *m, int N, int mode, int topk, int window, int maxiter,
                    uint64_t seed, vnm_lp_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     return lp_reorder(g, m, N, mode, topk, window, maxiter, seed, st);
 }
 
 int vnm_lp_reorder_batch(vnm_graph *const *graphs, int count, const vnm_lp_model *m, int N, int mode, int topk,
                          int window, int maxiter, uint64_t seed, vnm_lp_stats *st) {
     if (!graphs || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(count > 0 && graphs[0] ? graphs[0]->ctx->pool : nullptr);
     return lp_reorder_batch(graphs, count, m, N, mode, topk, window, maxiter, seed, st);
 }
 

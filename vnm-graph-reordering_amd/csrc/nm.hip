@@ -1767,6 +1767,7 @@ extern "C" {
 
 int vnm_locate(vnm_graph *g, int N, int32_t *cnt, int32_t *zero) {
     if (!g) return set_error(VNM_E_ARG, "null graph");
+    PoolScope pool(g->ctx->pool);
     int rc = check_nm_args(g, N);
     if (rc) return rc;
     if ((rc = build_csc(g))) return rc;
@@ -1784,6 +1785,7 @@ int vnm_locate(vnm_graph *g, int N, int32_t *cnt, int32_t *zero) {
 
 int vnm_swap_score(vnm_graph *g, int N, int seg1, const int32_t *seg2, int count, int32_t *scores) {
     if (!g || count < 0 || (count > 0 && (!seg2 || !scores))) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     int rc = check_nm_args(g, N);
     if (rc) return rc;
     const int ns = g->nseg(), M = g->M;
@@ -1817,13 +1819,14 @@ int vnm_swap_score(vnm_graph *g, int N, int seg1, const int32_t *seg2, int count
         VNM_LAUNCH_CHECK("k_score_rows");
         VNM_HIP_TRY(hipMemcpyAsync(scores + (size_t)base * 2 * M * M, dsc.p,
                                    (size_t)n * 2 * M * M * 4, hipMemcpyDeviceToHost, st));
+        VNM_HIP_TRY(hipStreamSynchronize(st));  // the copy reads this block's vector
     }
-    VNM_HIP_TRY(hipStreamSynchronize(st));
     return VNM_OK;
 }
 
 int vnm_pq_pop_order(vnm_ctx *ctx, const int32_t *scores, int count, int M, int32_t *order) {
     if (!ctx || count < 0 || M < 1 || M > 8) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(ctx->pool);
     if (count == 0) return VNM_OK;
     const int MM = M * M;
     DBuf<int32_t> ds, dord;
@@ -1843,18 +1846,21 @@ int vnm_pq_pop_order(vnm_ctx *ctx, const int32_t *scores, int count, int M, int3
 
 int vnm_nm_reorder(vnm_graph *g, int N, int sched, int maxiter, vnm_nm_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     return nm_reorder(g, N, sched, maxiter, st);
 }
 
 int vnm_nm_reorder_batch(vnm_graph *const *graphs, int count, int N, const int32_t *sched, int maxiter,
                          vnm_nm_stats *st) {
     if (!graphs || !sched || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(count > 0 && graphs[0] ? graphs[0]->ctx->pool : nullptr);
     return nm_reorder_batch(graphs, count, N, sched, maxiter, st);
 }
 
 int vnm_nm_trace(vnm_graph *g, int N, int sched, int maxiter, int round_cap, int32_t *rec,
                  int64_t cap, int64_t *count, vnm_nm_stats *st) {
     if (!g || !st || cap < 0 || (cap > 0 && !rec)) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(g->ctx->pool);
     if (cap > ((int64_t)1 << 31) / 9) return set_error(VNM_E_ARG, "trace capacity too large");
     DBuf<int32_t> d;
     int rc;

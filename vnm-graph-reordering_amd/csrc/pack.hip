@@ -1040,17 +1040,20 @@ extern "C" {
 
 int vnm_retained_nnz(vnm_graph *g, int V, int N, int64_t *out) {
     if (!g || !out) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     if (N != 2) return set_error(VNM_E_ARG, "the V:N:M format keeps N = 2 per row (got %d)", N);
     return pack(g, V, VNM_DT_F32, 0, nullptr, out);
 }
 
 int vnm_pack(vnm_graph *g, int V, int dtype, vnm_packed **out) {
     if (!g || !out) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     return pack(g, V, dtype, 0, out, nullptr);
 }
 
 int vnm_pack_ex(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out) {
     if (!g || !out) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     return pack(g, V, dtype, dense_min, out, nullptr);
 }
 
@@ -1091,6 +1094,7 @@ void vnm_packed_destroy(vnm_packed *p) {
 
 int vnm_spmm(vnm_packed *p, const void *B, int ldb, int n, int b_dtype, const float *b_scales,
              float *C, int ldc) {
+    PoolScope pool(p ? p->ctx->pool : nullptr);
     return spmm(p, B, ldb, n, b_dtype, b_scales, C, ldc, nullptr);
 }
 

@@ -36,6 +36,7 @@
 // SCAN_DIRECT tiles one workgroup scans the totals first, k_scan_totals).  Sum and
 // max, int32 or uint8 input; at most one tile in one launch (k_scan_small).
 // Compaction: exclusive sum of the flags, then a scatter of flagged items.
+#include "graph.h"
 #include "sortlib.h"
 
 #include <algorithm>
@@ -65,8 +66,15 @@ struct TempBuf {
         if (p) (void)hipFree(p);  // waits for the device, so no kernel still reads it
         p = nullptr;
         bytes = 0;
-        if (hipMalloc(&p, need ? need : 1) != hipSuccess) {
+        hipError_t e = hipMalloc(&p, need ? need : 1);
+        if (e != hipSuccess && t_pool) {
             (void)hipGetLastError();
+            t_pool->flush();
+            e = hipMalloc(&p, need ? need : 1);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
             return set_error(VNM_E_OOM, "scratch allocation of %zu bytes failed", need);
         }
         bytes = need;
@@ -750,7 +758,6 @@ int select_flagged_i32(const int32_t *in, const uint8_t *flags, int32_t *out, in
 
 }  // namespace vnm
 
-#include "graph.h"
 
 extern "C" int vnm_sort_pairs(vnm_ctx *ctx, const uint64_t *keys_in, uint64_t *keys_out, const int32_t *vals_in,
                               int32_t *vals_out, int64_t n, int end_bit) {

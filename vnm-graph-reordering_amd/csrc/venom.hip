@@ -352,7 +352,7 @@ struct VenomWork {
             VNM_HIP_TRY(hipMemcpyAsync(&nn, cnt2.p + 2, 4, hipMemcpyDeviceToHost, st));
             VNM_HIP_TRY(hipStreamSynchronize(st));
             na = nn;
-            std::swap(act.p, act2.p);
+            act.swap(act2);
         }
         return VNM_OK;
     }
@@ -445,13 +445,14 @@ int reload_sort(vnm_graph *g, bool quantize) {
         VNM_HIP_TRY(hipStreamSynchronize(st));
         quantize_values(v);
         VNM_HIP_TRY(hipMemcpyAsync(g->val.p, v.data(), nnz * 4, hipMemcpyHostToDevice, st));
+        VNM_HIP_TRY(hipStreamSynchronize(st));  // the copy reads this block's vector
     }
     VNM_HIP_TRY(hipMemsetAsync(dup.p, 0, 4, st));
     hipLaunchKernelGGL(k_unpack_sorted, dim3(gb), dim3(256), 0, st, k2.p, i2.p, g->val.p, nnz,
                        g->row.p, g->col.p, v2.p, dup.p);
     g->ctx->launches += 3;
     VNM_LAUNCH_CHECK("reload sort");
-    std::swap(g->val.p, v2.p);
+    g->val.swap(v2);
     int32_t ndup = 0;
     VNM_HIP_TRY(hipMemcpyAsync(&ndup, dup.p, 4, hipMemcpyDeviceToHost, st));
     VNM_HIP_TRY(hipStreamSynchronize(st));
@@ -567,6 +568,7 @@ extern "C" {
 
 int vnm_venom_eval(vnm_graph *g, int V, int32_t *inv, int32_t *inv_strict) {
     if (!g || !inv || !inv_strict) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     int rc = check_venom_args(g, V);
     if (rc) return rc;
     return venom_eval(g, V, inv, inv_strict);
@@ -574,6 +576,7 @@ int vnm_venom_eval(vnm_graph *g, int V, int32_t *inv, int32_t *inv_strict) {
 
 int vnm_venom_reorder(vnm_graph *g, int V, int maxiter, vnm_venom_stats *st) {
     if (!g || !st) return set_error(VNM_E_ARG, "null argument");
+    PoolScope pool(g->ctx->pool);
     int rc = check_venom_args(g, V);
     if (rc) return rc;
     if ((rc = venom_reorder(g, V, maxiter, st))) return rc;
