@@ -151,6 +151,91 @@ __host__ __device__ __forceinline__ uint32_t heap_pop(HeapRef &H) {
     return top_el;
 }
 
+// A value that is the same in every lane, in a scalar register: loops and
+// branches on it are scalar.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Rank of each lane's key among the first n lanes' (the number of strictly
+// smaller ones); n <= 64.
+__device__ __forceinline__ int wave_rank(int64_t key, int n) {
+    const int lo = (int)(uint32_t)key, hi = (int)(key >> 32);
+    n = uniform(n);
+    int rank = 0;
+    for (int j = 0; j < n; ++j) {
+        const int64_t k = ((int64_t)__builtin_amdgcn_readlane(hi, j) << 32) |
+                          (uint32_t)__builtin_amdgcn_readlane(lo, j);
+        rank += k < key;
+    }
+    return rank;
+}
+
+// The same pop order by a whole wave, of the entries of lanes 0..n-1 pushed in
+// that order; n <= 64.  Lane k returns the element popped k-th.
+//
+// The wave holds the heap: lane i has the entry at 1-based position i (parent
+// i / 2, root 1; -1, below every rank, where there is none), and position 64,
+// which exists only until the first pop, a scalar.  Ranks never grow along a
+// path down, so the passed and kept positions of a path split at one depth:
+// - A push at position i goes up past the ancestors with rank <= its own: it
+//   lands c levels below the root, with c the number of ancestors of a larger
+//   rank, and the path's positions below that take their parents' entries.
+// - A pop's hole goes down to the bottom, at each position to the left child
+//   when rank(right) <= rank(left), then the last entry goes up from there.
+//   What that moves up past goes back to where it was, so the last entry lands
+//   c levels below the root, with c the number of the path's positions
+//   (without the root) of a larger rank, and those above take their child's.
+// Each is a comparison of all positions at once, one lane exchange and scalar
+// arithmetic on the masks.  A position is on the pop's path when the turn taken
+// at each of its ancestors (bit a of `rights`) is the one that leads to it.
+__device__ __forceinline__ int wave_pop_order(int entry, int n) {
+    const int lane = threadIdx.x & 63;
+    n = uniform(n);
+    // position `lane`: its depth, its ancestors and those it lies right of
+    // (lane 0 is no position: off every path, as it asks for an unset bit 0)
+    const int depth = lane ? 31 - __builtin_clz(lane) : 31;
+    const int pos = lane ? lane : -1;
+    uint32_t anc = lane ? 0u : 1u, want = lane ? 0u : 1u;
+    for (int a = lane; a > 1; a >>= 1) {
+        anc |= 1u << (a >> 1);
+        want |= (uint32_t)(a & 1) << (a >> 1);
+    }
+    int v = -1, v64 = -1;
+    for (int e = 0; e < n; ++e) {
+        const int i = e + 1;
+        const int val = __builtin_amdgcn_readlane(entry, e);
+        const int di = 31 - __builtin_clz(i);
+        const bool path = (int)((uint32_t)i >> ((di - depth) & 31)) == pos;
+        const int c = __popcll(__builtin_amdgcn_ballot_w64(path) & __builtin_amdgcn_ballot_w64(v > (val | 0xFF)));
+        if (c < di) {
+            const int up = __builtin_amdgcn_ds_bpermute((lane >> 1) * 4, v);
+            if (i == 64) v64 = __builtin_amdgcn_readlane(v, 32);
+            v = path && depth > c ? up : v;
+            v = path && depth == c ? val : v;
+        } else if (i == 64) {
+            v64 = val;
+        } else {
+            v = lane == i ? val : v;
+        }
+    }
+    int order = 0;
+    for (int k = 0; k < n; ++k) {
+        const int m = n - k;  // entries in the heap
+        order = lane == k ? __builtin_amdgcn_readlane(v, 1) : order;
+        if (m == 1) break;
+        const int last = m == 64 ? v64 : __builtin_amdgcn_readlane(v, m & 63);
+        v = lane == m ? -1 : v;
+        const int l = __builtin_amdgcn_ds_bpermute(lane * 8, v);  // lanes 1..31 have children
+        const int r = __builtin_amdgcn_ds_bpermute(lane * 8 + 4, v);
+        const bool right = r > (l | 0xFF);
+        const uint32_t rights = (uint32_t)__builtin_amdgcn_ballot_w64(right) & ~1u;
+        const bool path = ((rights ^ want) & anc) == 0;
+        const int c = __popcll(__builtin_amdgcn_ballot_w64(path) & __builtin_amdgcn_ballot_w64(v > (last | 0xFF)) & ~2ull);
+        v = path && depth < c ? (right ? r : l) : v;
+        v = path && depth == c ? last : v;
+    }
+    return order & 0xFF;
+}
+
 // BF16 storage codec: round to nearest even, NaN kept quiet.
 __host__ __device__ inline uint16_t f32_to_bf16(float f) {
     uint32_t u;

@@ -267,8 +267,8 @@ __global__ __launch_bounds__(SC_ROWS) void k_score_rows(int R, int M, int N, int
 
 // ------------------------------------------------------------ heap pop order
 
-// One thread per list: dense ranks of the list's M*M keys, then the same
-// heap code as the greedy pushes every pair and pops them all.
+// One thread per list: dense ranks of the list's M*M keys, then every pair
+// pushed and all popped.
 __global__ void k_pq_pop_order(const int32_t *__restrict__ scores, int count, int M,
                                int32_t *__restrict__ order) {
     extern __shared__ uint32_t hsm[];  // thread t's heap at [t * HEAP_WORDS, (t + 1) * HEAP_WORDS)
@@ -284,6 +284,19 @@ __global__ void k_pq_pop_order(const int32_t *__restrict__ scores, int count, in
         heap_push(H, (uint32_t)((r << 8) | i));
     }
     for (int k = 0; k < MM; ++k) order[(size_t)q * MM + k] = (int32_t)(heap_pop(H) & 0xFFu);
+}
+
+constexpr int PQ_WAVES = 4096;  // lists that a wave each takes
+
+// One wave per list, with the greedy's own ranks and queue.
+__global__ __launch_bounds__(64) void k_pq_pop_order_wave(const int32_t *__restrict__ scores, int M,
+                                                     int32_t *__restrict__ order) {
+    const int MM = M * M, lane = threadIdx.x;
+    const size_t q = blockIdx.x;
+    const int32_t *sc = scores + q * 2 * MM;
+    const int64_t key = lane < MM ? swap_key(sc[2 * lane], sc[2 * lane + 1]) : 0;
+    const int e = wave_pop_order((wave_rank(key, MM) << 8) | lane, MM);
+    if (lane < MM) order[q * MM + lane] = e;
 }
 
 // ------------------------------------------------------------ relabel
@@ -333,8 +346,9 @@ __global__ void k_compose(int32_t *__restrict__ total, int64_t n, const int32_t 
 //                                 choose the round's segments, their columns
 //   k_gr_fill_a   (grid)          clear records B (last recount), fill A
 //   k_gr_score    (grid)          gains of every pair from records A
-//   k_gr_greedy   (1 workgroup)   priority queues, sequential greedy, commit
-//                                 to perm/inv, columns after the commit
+//   k_gr_queues   (a wave a pair) pop order of every ordered pair's queue
+//   k_gr_greedy   (1 workgroup)   sequential greedy over the pop orders,
+//                                 commit to perm/inv, columns after it
 //   k_gr_fill_b   (grid)          clear records A, fill B
 //   k_gr_count    (grid)          cnt / nzr of the round's segments from B
 //
@@ -354,8 +368,6 @@ constexpr int KMAX = 9;          // primary + up to M targets (M <= 8)
 constexpr int MMAX = 8;
 constexpr int NPAIR_T = KMAX * (KMAX - 1) / 2 + 1;  // unordered pairs + one self pair
 constexpr int NQ = (KMAX - 1) * (KMAX - 1);         // ordered pairs the greedy can visit
-constexpr int POPP = 16;                            // fewest pops precomputed per ordered pair
-static_assert(NQ <= 64, "one heap thread per ordered pair, all in wave 0");
 constexpr int NACC = KMAX * MMAX + NPAIR_T * 2 * MMAX * MMAX;  // E and both, flattened
 
 // The columns of one set of records: slot j, bit b = column j*M + b.
@@ -374,7 +386,6 @@ struct GreedyState {
     int32_t *trace;  // optional: 9 ints per swap
     // run state
     int round, L, totcnt, maxiter, init_size, init_cnt, status, done, pending;
-    int npre;  // pops to precompute per ordered pair this round (from the last round's need)
     int K, self_pair, size1;
     int sel[KMAX], selcnt[KMAX];
     int64_t trace_len, work;
@@ -384,42 +395,48 @@ struct GreedyState {
     uint64_t clk[16];
 };
 
+// The round's queues: of ordered pair q the pop order, element and gains.
+struct PopOrders {
+    int lg[NQ][MMAX * MMAX], rg[NQ][MMAX * MMAX];
+    uint8_t e[NQ][MMAX * MMAX];
+};
+
 // Arguments of the round kernels for one graph: pointers fixed for the
 // graph.  The kernels take graph 0's by value and an array of all of them in
 // device memory, and serve graph blockIdx.y, so one launch chain runs the
 // greedy of many graphs at once (a single graph reads no argument memory).
 struct NMArgs {
     GreedyState *st;
+    PopOrders *pops;
     const int32_t *cptr, *crow;
     int32_t *perm, *inv, *cnt, *nzr;
     uint32_t *rta, *rtb;
 };
 
-// LDS of the single-workgroup kernels.
-struct GreedyShared {
+constexpr int SEL_KEYS = 1024;  // keys that k_gr_select ranks in LDS
+
+// LDS of k_gr_select.
+struct SelectShared {
     int sel[KMAX];
     int selcnt[KMAX];
     int K, self_pair, size1, cont, status, L;
     ColSet cs;
-    int E[KMAX][MMAX];
-    // per unordered pair (j < j2) and one self pair: the "both rows" sums
-    //   Bl[b1*M+b2] = sum over rows in both of y_b2 * (x_b1 ? A : B)
-    //   Br[b1*M+b2] = sum over rows in both of x_b1 * (y_b2 ? D : C)
-    int both[NPAIR_T][2][MMAX * MMAX];
-    // per ordered pair q: the heap, its first
-    // npre pops, the next of those not yet consumed, and the heap's size
-    uint32_t heap[NQ][HEAP_WORDS];
-    uint8_t popped[MMAX * MMAX][NQ];
-    int qcur[NQ];
-    int heapn[NQ];
-    int npre, heap_pops;  // pops precomputed this round; pops the greedy took from heaps
-    int maxk;             // precomputed pops the greedy used, most over the ordered pairs
-    int swv1[64], swv2[64], swlg[64], swrg[64], swp[64], swt[64], swpc[64], swtc[64];
-    int nsw;
-    uint64_t wbest[NW];
+    uint64_t wbest[NW], wtop[NW];
     uint64_t topk[KMAX + 1];
-    int selthr[KMAX + 1], nselthr;  // threads whose segments hold the round's top keys
-    int64_t wkeys[NW][64];
+    int nkeys;
+    uint64_t keys[SEL_KEYS];
+};
+
+// LDS of k_gr_greedy.
+struct GreedyShared {
+    int sel[KMAX];
+    int selcnt[KMAX];
+    int K, self_pair, size1, cont, status;
+    ColSet cs;
+    PopOrders pops;
+    int sww[64];  // per swap: slot a | slot b << 8 | element << 16
+    int swlg[64], swrg[64], swpc[64], swtc[64];
+    int nsw, trace;
 };
 
 __device__ __forceinline__ uint64_t key_fwd(int s, int c) {
@@ -461,49 +478,12 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
     return ((uint64_t)hi << 32) | lo;
 }
 
-// Top k (k <= KMAX + 1) of n keys in LDS (0 = none) into S.topk, by wave 0
-// alone: each lane keeps a descending list of its keys (j = lane, lane + 64,
-// ...), then k wave maxima merge the lists.  The other waves skip it (one
-// wave's short chains instead of sixteen waves sharing four SIMDs).
-__device__ __forceinline__ void wave0_topk(const uint64_t *keys, int n, int k, GreedyShared &S) {
-    const int lane = threadIdx.x & 63;
-    if (threadIdx.x >= 64) return;
-    uint64_t lst[KMAX + 1];
-#pragma unroll
-    for (int i = 0; i <= KMAX; ++i) lst[i] = 0;
-    for (int j = lane; j < n; j += 64) {
-        uint64_t x = keys[j];
-        if (x <= lst[KMAX]) continue;
-#pragma unroll
-        for (int i = 0; i <= KMAX; ++i) {
-            const uint64_t hi = lst[i] > x ? lst[i] : x;
-            x = lst[i] > x ? x : lst[i];
-            lst[i] = hi;
-        }
-    }
-    for (int it = 0; it < k; ++it) {
-        const uint64_t m = wave_max_u64(lst[0]);
-        if (m != 0 && lst[0] == m) {
-#pragma unroll
-            for (int i = 0; i < KMAX; ++i) lst[i] = lst[i + 1];
-            lst[KMAX] = 0;
-        }
-        if (lane == 0) S.topk[it] = m;
-    }
-}
-
-__device__ __forceinline__ uint64_t block_max_u64(uint64_t v, GreedyShared &S) {
+__device__ __forceinline__ uint64_t block_max_u64(uint64_t v, uint64_t *wbest) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     v = wave_max_u64(v);
-    if (lane == 0) S.wbest[w] = v;
+    if (lane == 0) wbest[w] = v;
     __syncthreads();
-    if (w == 0) {
-        uint64_t x = lane < NW ? S.wbest[lane] : 0ull;
-        x = wave_max_u64(x);
-        if (lane == 0) S.wbest[0] = x;
-    }
-    __syncthreads();
-    uint64_t r = S.wbest[0];
+    const uint64_t r = wave_max_u64(wbest[lane & (NW - 1)]);
     __syncthreads();
     return r;
 }
@@ -516,22 +496,18 @@ __device__ __forceinline__ int tri_index(int a, int b, int K) {
 // lgain/rgain of element e = b1*M + b2 of ordered pair (a, b) of slots:
 //   score(a, b)[b1][b2] = (E_a[b1] - Bl(a,b)[b1][b2], E_b[b2] - Br(a,b)[b1][b2])
 // and score(b, a) is score(a, b) transposed with the two gains exchanged.
-__device__ __forceinline__ void pair_gain(const GreedyShared &S, int K, int M, int a, int b, int e,
-                                          int &lg, int &rg) {
+// acc: the sums of k_gr_score, E[KMAX][MMAX] and then per unordered pair (and
+// one self pair) the "both rows" sums, Bl and Br of M*M each:
+//   Bl[b1*M+b2] = sum over rows in both of y_b2 * (x_b1 ? A : B)
+//   Br[b1*M+b2] = sum over rows in both of x_b1 * (y_b2 ? D : C)
+__device__ __forceinline__ void pair_gain(const int *acc, int K, int M, int a, int b, int e, int &lg, int &rg) {
     const int b1 = e / M, b2 = e % M;
-    if (a == b) {
-        lg = S.E[a][b1] - S.both[NPAIR_T - 1][0][e];
-        rg = S.E[a][b2] - S.both[NPAIR_T - 1][1][e];
-    } else if (a < b) {
-        const int pi = tri_index(a, b, K);
-        lg = S.E[a][b1] - S.both[pi][0][e];
-        rg = S.E[b][b2] - S.both[pi][1][e];
-    } else {
-        const int pi = tri_index(b, a, K);
-        const int t = b2 * M + b1;
-        lg = S.E[a][b1] - S.both[pi][1][t];
-        rg = S.E[b][b2] - S.both[pi][0][t];
-    }
+    const int *both = acc + KMAX * MMAX;
+    const int pi = a == b ? NPAIR_T - 1 : a < b ? tri_index(a, b, K) : tri_index(b, a, K);
+    const int *Bl = both + (2 * pi + (a > b)) * MMAX * MMAX, *Br = both + (2 * pi + (a <= b)) * MMAX * MMAX;
+    const int t = a > b ? b2 * M + b1 : e;
+    lg = acc[a * MMAX + b1] - Bl[t];
+    rg = acc[b * MMAX + b2] - Br[t];
 }
 
 // Ordered pair index of (a, b): (0, t) -> t-1; (i, j) with i, j >= 1 -> after.
@@ -804,134 +780,106 @@ __global__ __launch_bounds__(PT) void k_gr_count(NMArgs a0, const NMArgs *__rest
     clock_add(st, 5, t0);
 }
 
-// Visited vertices of a round: bit a*M + v for vertex v of slot a (< 72).
-struct Visited {
-    uint64_t lo = 0, hi = 0;
-    __device__ __forceinline__ bool has(int i) const {
-        return ((i < 64 ? lo >> i : hi >> (i - 64)) & 1ull) != 0;
-    }
-    __device__ __forceinline__ void set(int i) {
-        if (i < 64) lo |= 1ull << i;
-        else hi |= 1ull << (i - 64);
-    }
-    // every vertex of slot a (M divides 64, so a slot's bits share a word)
-    __device__ __forceinline__ bool full(int a, int M) const {
-        const int i = a * M;
-        const uint64_t m = (1ull << M) - 1;
-        return (((i < 64 ? lo >> i : hi >> (i - 64))) & m) == m;
-    }
-};
-
-// First element of ordered pair q (slots a -> b) in pop order whose two
-// vertices are unvisited; -1 when the queue runs empty.  Skipped pops are
-// consumed (a visited vertex stays visited for the round), so each queue
-// resumes where its last search stopped: first the precomputed pops, one
-// per lane and a ballot, then the heap itself.  Called by a whole wave with
-// the same arguments in every lane.
-__device__ __forceinline__ int first_free(GreedyShared &S, int q, int a, int b, int M, const Visited &vis) {
-    const int lane = threadIdx.x & 63;
-    const int npre = S.npre;  // <= 64
-    const int k0 = S.qcur[q];
-    if (k0 < npre) {
-        const int k = k0 + lane;
-        const int e = k < npre ? (int)S.popped[k][q] : 0;
-        const bool ok = k < npre && !vis.has(a * M + e / M) && !vis.has(b * M + e % M);
-        const uint64_t m = __ballot(ok);
-        if (m) {
-            const int i = __builtin_ctzll(m);
-            S.qcur[q] = k0 + i;
-            if (lane == 0) S.maxk = max(S.maxk, k0 + i + 1);  // precomputed pops this round used
-            return __builtin_amdgcn_readlane(e, i);
-        }
-        S.qcur[q] = npre;
-    }
-    HeapRef H{reinterpret_cast<uint16_t *>(S.heap[q]), S.heapn[q]};
-    while (H.n > 0) {
-        const int e = (int)(heap_pop(H) & 0xFFu);
-        S.heap_pops += 1;
-        if (!vis.has(a * M + e / M) && !vis.has(b * M + e % M)) {
-            S.heapn[q] = H.n;
-            return e;
-        }
-    }
-    S.heapn[q] = 0;
-    return -1;
-}
-
-__device__ __forceinline__ bool list_before(int sa, int ca, int sb, int cb, bool rev) {
-    // true when (sa, ca) is nearer the top of the invalid list than (sb, cb)
-    if (!rev) return ca != cb ? ca > cb : sa < sb;
-    return ca != cb ? ca < cb : sa > sb;
-}
-
 // The sequential part of one round (reorder/reorder.h:1837-1932), run by one
-// wave in lockstep: every lane holds the same values and writes the same
-// LDS words, and first_free spreads its search over the lanes.  Returns the
-// number of swaps.
+// wave.  Lane s holds slot s's visited vertices and lane i the i-th target of
+// the current segment's turn; the rest is uniform.  A queue's next pair is its
+// first, in pop order, whose two vertices are unvisited: the lanes hold the pop
+// order of one queue (read while the swap before is chosen), so a swap is a
+// ballot and a few lane reads.  The loops stay rolled: a round runs this once on
+// some CU, and unrolled over the targets most of its time went into fetching
+// its instructions (R-MAT 16,384, 34 swaps a round: 15.6 us a round; 11.4
+// now, and 45 with targets, counts and queue positions in scratch and LDS).
+// Returns the number of swaps.
 template <int M>  // 4 or 8: the per-element divisions by M become shifts
 __device__ __forceinline__ int greedy_apply(GreedyShared &S, bool rev, bool drain) {
-    const int K = S.K;
+    constexpr int MM = M * M, FULL = (1 << M) - 1;
+    const int lane = threadIdx.x & 63;
+    const int K = uniform(S.K);
+    const bool trace = uniform(S.trace) != 0;
     int nsw = 0;
-    Visited vis;
     auto add_swap = [&](int a, int b, int e, int lg, int rg, int pc, int tc) {
         const int n = nsw++;
-        S.swv1[n] = S.sel[a] * M + e / M;
-        S.swv2[n] = S.sel[b] * M + e % M;
-        S.swlg[n] = lg; S.swrg[n] = rg;
-        S.swp[n] = S.sel[a]; S.swt[n] = S.sel[b];
-        S.swpc[n] = pc; S.swtc[n] = tc;
+        S.sww[n] = a | b << 8 | e << 16;
+        if (trace) {
+            S.swlg[n] = lg; S.swrg[n] = rg;
+            S.swpc[n] = pc; S.swtc[n] = tc;
+        }
     };
     if (S.size1) {
         // one invalid segment: swap the top pair with the emptiest segment, no
         // visited filter (reorder/reorder.h:1837-1860)
-        const int b = S.self_pair ? 0 : 1;
-        const int e = S.popped[0][0];  // first pop of list 0
-        int lg, rg;
-        pair_gain(S, K, M, 0, b, e, lg, rg);
-        add_swap(0, b, e, lg, rg, 0, 0);
+        add_swap(0, S.self_pair ? 0 : 1, S.pops.e[0][0], S.pops.lg[0][0], S.pops.rg[0][0], 0, 0);
         return nsw;
     }
-    int cur = 0, pc = S.selcnt[0];
-    int tgt[KMAX], tcnt[KMAX], nt = K - 1;
-    for (int i = 0; i < nt; ++i) { tgt[i] = i + 1; tcnt[i] = S.selcnt[i + 1]; }
+    const int *el = &S.pops.lg[0][0] + (lane < MM ? lane : 0);
+    const int *er = &S.pops.rg[0][0] + (lane < MM ? lane : 0);
+    const uint8_t *ee = &S.pops.e[0][0] + (lane < MM ? lane : 0);
+    const int selv = lane < K ? S.sel[lane] : 0;
+    int vis = 0;  // slot `lane`: its visited vertices
+    int cur = 0, nt = K - 1, pc = uniform(S.selcnt[0]);
+    // target `lane` of the turn: its slot, and its count (after its swap, if any)
+    int tslot = lane + 1, tcnt = lane < nt ? S.selcnt[lane + 1] : 0;
     while (true) {
-        int upd[KMAX], ucnt[KMAX], nu = 0;
+        const int qv = lane < nt ? q_index(cur, tslot, K) * (MMAX * MMAX) : 0;
+        int vc = __builtin_amdgcn_readlane(vis, cur);
+        uint32_t alive = 0;  // targets that stay in the list
+        bool empty = false;  // a queue without a free pair
+        int q = __builtin_amdgcn_readlane(qv, 0);
+        int pe = ee[q], pl = el[q], pr = er[q];
+#pragma unroll 1
         for (int i = 0; i < nt; ++i) {
-            if (pc <= 0 || vis.full(cur, M)) break;  // reorder/reorder.h:1878
-            const int t = tgt[i];
-            const int q = q_index(cur, t, K);
-            int e = first_free(S, q, cur, t, M, vis);
-            if (e < 0) {
-                // top() of an empty queue: the reference would read the last
-                // popped pair, which has a visited endpoint (:1908)
-                S.status = VNM_E_UB_PATH;
-                return nsw;
-            }
-            int lg, rg;
-            pair_gain(S, K, M, cur, t, e, lg, rg);
-            vis.set(cur * M + e / M);
-            vis.set(t * M + e % M);
+            pc = uniform(pc);
+            vc = uniform(vc);
+            if (pc <= 0 || vc == FULL) break;  // reorder/reorder.h:1878
+            q = __builtin_amdgcn_readlane(qv, i + 1);  // (the last target's successor reads queue 0)
+            const int ne = ee[q], nl = el[q], nr = er[q];
+            const int t = __builtin_amdgcn_readlane(tslot, i);
+            const int vt = __builtin_amdgcn_readlane(vis, t);
+            // bit 0 of `used`: either vertex visited
+            const uint32_t used = (uint32_t)vc >> ((uint32_t)pe / M) | (uint32_t)vt >> ((uint32_t)pe % M);
+            const uint64_t m = __builtin_amdgcn_ballot_w64((used & 1) == 0) & (MM == 64 ? ~0ull : (1ull << (MM & 63)) - 1);
+            empty = m == 0;
+            if (empty) break;
+            const int k = __builtin_ctzll(m);
+            const uint32_t e = (uint32_t)__builtin_amdgcn_readlane(pe, k);
+            const int lg = __builtin_amdgcn_readlane(pl, k), rg = __builtin_amdgcn_readlane(pr, k);
+            vc |= 1 << (e / M);
+            vis = lane == t ? vt | 1 << (e % M) : vis;
             pc -= lg;
-            int tc = tcnt[i] - rg;
-            add_swap(cur, t, e, lg, rg, pc, tc);
-            if (tc > 0) { upd[nu] = t; ucnt[nu] = tc; ++nu; }
+            const int c = __builtin_amdgcn_readlane(tcnt, i) - rg;
+            tcnt = lane == i ? c : tcnt;
+            add_swap(cur, t, (int)e, lg, rg, pc, c);
+            alive |= (uint32_t)(c > 0) << i;
+            pe = ne; pl = nl; pr = nr;
         }
+        if (empty) {
+            // top() of an empty queue: the reference would read the last
+            // popped pair, which has a visited endpoint (:1908)
+            S.status = VNM_E_UB_PATH;
+            break;
+        }
+        vis = lane == cur ? vc : vis;
+        const int nu = __popc(alive);
         if (nu < 2) break;  // while (inv_seg_list.size() >= 2)
-        for (int i = 1; i < nu; ++i) {
-            int s = upd[i], c = ucnt[i], k = i - 1;
-            while (k >= 0 && list_before(S.sel[s], c, S.sel[upd[k]], ucnt[k], rev)) {
-                upd[k + 1] = upd[k]; ucnt[k + 1] = ucnt[k]; --k;
-            }
-            upd[k + 1] = s; ucnt[k + 1] = c;
+        // each remaining target's place in the list (segments are distinct):
+        // the first is the next turn's segment, the others its targets
+        const bool al = lane < M && ((alive >> lane) & 1);
+        const int tseg = __shfl(selv, tslot, 64);
+        const uint64_t key = rev ? key_rev(tseg, tcnt) : key_fwd(tseg, tcnt);
+        int place = 0;
+        for (uint32_t r = alive; r; r &= r - 1) {
+            const int j = __builtin_ctz(r);
+            const uint64_t kj = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(key >> 32), j) << 32 |
+                                (uint32_t)__builtin_amdgcn_readlane((int)key, j);
+            place += kj > key;
         }
-        cur = upd[0];
-        pc = ucnt[0];
+        const int first = __builtin_ctzll(__builtin_amdgcn_ballot_w64(place == 0) & alive);
+        cur = __builtin_amdgcn_readlane(tslot, first);
+        pc = __builtin_amdgcn_readlane(tcnt, first);
         nt = nu - 1;
-        for (int i = 0; i < nt; ++i) {
-            int src = drain ? (nu - 1 - i) : (i + 1);
-            tgt[i] = upd[src];
-            tcnt[i] = ucnt[src];
-        }
+        const int to = al && place > 0 ? (drain ? nt - place : place - 1) : 63;
+        tslot = __builtin_amdgcn_ds_permute(to * 4, tslot);
+        tcnt = __builtin_amdgcn_ds_permute(to * 4, tcnt);
     }
     return nsw;
 }
@@ -942,45 +890,46 @@ __device__ __forceinline__ int greedy_apply(GreedyShared &S, bool rev, bool drai
 // the round's segments and their columns.
 __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__restrict__ args) {
     const NMArgs A = blockIdx.y == 0 ? a0 : args[blockIdx.y];
-    __shared__ GreedyShared S;
+    __shared__ SelectShared S;
     GreedyState *st = A.st;
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-    if (tid == 0) S.cont = !st->done;
-    __syncthreads();
-    if (!S.cont) return;
-    const int M = st->M, R = st->R, nseg = st->nseg, MM = M * M;
+    const int M = st->M, R = st->R, nseg = st->nseg, K0 = st->K, pending = st->pending;
+    const int psel = tid < KMAX ? st->sel[tid] : 0, pcnt = tid < KMAX ? st->newcnt[tid] : 0,
+              pnzr = tid < KMAX ? st->newnzr[tid] : 0;
+    int round = st->round, L = st->L;
+    const int maxiter = st->maxiter, round_cap = st->round_cap, totcnt = st->totcnt, status = st->status;
+    if (st->done) return;
     const bool plain = st->sched >= 8;
     const bool rev = (st->sched == 2 || st->sched == 3);
     const bool drain = (st->sched == 1 || st->sched == 3);
     const bool tfwd = drain ? rev : !rev;  // traversal order uses the forward key
     const int min_size = plain ? 2 : 1;
-    (void)lane; (void)w; (void)MM;
     // the last round's segments (distinct), one thread each
     if (tid == 0) { S.K = 0; S.L = 0; S.status = 0; }
     __syncthreads();
-    const int pending = st->pending;
-    if (pending && tid < st->K) {
-        const int s = st->sel[tid];
-        const int oc = ld_l2(&A.cnt[s]), nc = st->newcnt[tid];
+    if (pending && tid < K0) {
+        const int s = psel, nc = pcnt;
+        const int oc = ld_l2(&A.cnt[s]);
         st_l2(&A.cnt[s], nc);
-        st_l2(&A.nzr[s], st->newnzr[tid]);
+        st_l2(&A.nzr[s], pnzr);
         atomicAdd(&S.L, (nc != 0) - (oc != 0));
         atomicAdd(&S.status, nc - oc);
     }
     __syncthreads();
     if (tid == 0) {
         if (pending) {
-            st->L += S.L;
-            st->totcnt += S.status;
-            st->round += 1;
+            L += S.L;
+            round += 1;
+            st->L = L;
+            st->totcnt = totcnt + S.status;
+            st->round = round;
             st->pending = 0;
         }
-        S.cont = st->round <= st->maxiter && st->round <= st->round_cap && st->L >= min_size &&
-                 st->status == 0;
+        S.cont = round <= maxiter && round <= round_cap && L >= min_size && status == 0;
         if (!S.cont) st->done = 1;
-        S.L = st->L;
+        S.L = L;
     }
     __syncthreads();
     if (!S.cont) return;
@@ -998,8 +947,8 @@ __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__res
             uint64_t z = ((uint64_t)(uint32_t)(R - ld_l2(&A.nzr[s])) << 32) | (uint32_t)s;
             best_z = z > best_z ? z : best_z;
         }
-        uint64_t bl = block_max_u64(best_l, S);
-        uint64_t bz = block_max_u64(best_z, S);
+        uint64_t bl = block_max_u64(best_l, S.wbest);
+        uint64_t bz = block_max_u64(best_z, S.wbest);
         if (tid == 0) {
             int top = (int)(uint32_t)bl, minseg = (int)(uint32_t)bz;
             S.size1 = 1;
@@ -1011,94 +960,104 @@ __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__res
         __syncthreads();
     } else {
         const int k = min(M, Lr - 1) + 1;  // targets + the primary itself
-        // Top-k traversal keys in three steps.  Thread t scans the segments
-        // s = t (mod GT) and keeps only its largest key; keys are distinct
-        // (they hold s), so every key of the top k lies in a thread whose own
-        // maximum is among the k largest thread maxima.  Those threads'
-        // segments are then scored again, spread over the workgroup, and the
-        // top k of them is the top k of all.
-        uint64_t tk[KMAX + 1];
+        // The k largest traversal keys (keys are distinct, they hold the
+        // segment) and the largest list key.  The k-th largest of the waves'
+        // largest keys bounds the k-th largest of all from below, so only keys
+        // from there on are ranked against each other, in LDS.  Segment s goes
+        // to wave s mod 16: of counts that fall with s, as where hubs come
+        // first, each wave has its share, and about k keys pass.  (R-MAT
+        // 16,384, 2,048 segments: 10.7 us a round with the top k by insertion
+        // into sorted lists of one wave; 4.3 now.)
+        const int s1 = lane * NW + w;
+        auto key_of = [&](int seg, int c) { return tfwd ? key_fwd(seg, c) : key_rev(seg, c); };
+        uint64_t best_l = 0, best_t = 0;
+        int cv[4];  // four loads in flight per thread; the first four stay
+        for (int s0 = s1; s0 < nseg; s0 += GT * 4) {
+            int cu[4];
 #pragma unroll
-        for (int i = 0; i <= KMAX; ++i) tk[i] = 0;
-        uint64_t best_l = 0;
-        for (int s0 = tid; s0 < nseg; s0 += GT * 4) {
-            int cv[4];  // four loads in flight per thread
-#pragma unroll
-            for (int u = 0; u < 4; ++u) cv[u] = s0 + u * GT < nseg ? ld_l2(&A.cnt[s0 + u * GT]) : 0;
+            for (int u = 0; u < 4; ++u) cu[u] = s0 + u * GT < nseg ? ld_l2(&A.cnt[s0 + u * GT]) : 0;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const int c = cv[u], s = s0 + u * GT;
-                if (c == 0) continue;
-                uint64_t lk = rev ? key_rev(s, c) : key_fwd(s, c);
+                if (s0 == s1) cv[u] = cu[u];
+                const uint64_t lk = rev ? key_rev(s0 + u * GT, cu[u]) : key_fwd(s0 + u * GT, cu[u]);
+                const uint64_t x = key_of(s0 + u * GT, cu[u]);
                 best_l = lk > best_l ? lk : best_l;
-                const uint64_t x = tfwd ? key_fwd(s, c) : key_rev(s, c);
-                tk[0] = x > tk[0] ? x : tk[0];
+                best_t = x > best_t ? x : best_t;
             }
         }
-        uint64_t bl = block_max_u64(best_l, S);
-        // the k largest thread maxima (one key per thread in LDS)
-        uint64_t *keys = (uint64_t *)&S.wkeys[0][0];
-        keys[tid] = tk[0];
-        __syncthreads();
-        wave0_topk(keys, GT, k, S);
-        __syncthreads();
-        if (tid == 0) {
-            int n = 0;
-            for (int i = 0; i < k; ++i)
-                if (S.topk[i] != 0) S.selthr[n++] = seg_of_key(S.topk[i], tfwd) % GT;
-            S.nselthr = n;
+        best_l = wave_max_u64(best_l);
+        best_t = wave_max_u64(best_t);
+        if (lane == 0) {
+            S.wbest[w] = best_l;
+            S.wtop[w] = best_t;
         }
+        if (tid == 0) S.nkeys = 0;
+        if (tid <= KMAX) S.topk[tid] = 0;
         __syncthreads();
-        // those threads' segments scored again by wave 0, then their top k
-        const int per = (nseg + GT - 1) / GT;  // segments per thread, at most
-        const int ncand = S.nselthr * per;
-        if (tid < 64) {
-            uint64_t lst[KMAX + 1];
+        uint64_t bound = 0;  // k-th largest wave maximum (0: fewer have any)
+        {
+            const uint64_t x = S.wtop[lane & (NW - 1)];
+            int above = 0;
 #pragma unroll
-            for (int i = 0; i <= KMAX; ++i) lst[i] = 0;
-            for (int j = tid; j < ncand; j += 64) {
-                const int s = S.selthr[j / per] + (j % per) * GT;
-                const int c = s < nseg ? ld_l2(&A.cnt[s]) : 0;
-                if (c == 0) continue;
-                uint64_t x = tfwd ? key_fwd(s, c) : key_rev(s, c);
+            for (int j = 0; j < NW; ++j) above += S.wtop[j] > x;
+            bound = wave_max_u64(above >= k - 1 ? x : 0);
+        }
+        for (int s0 = s1; s0 < nseg; s0 += GT * 4) {
 #pragma unroll
-                for (int i = 0; i <= KMAX; ++i) {
-                    const uint64_t hi = lst[i] > x ? lst[i] : x;
-                    x = lst[i] > x ? x : lst[i];
-                    lst[i] = hi;
+            for (int u = 0; u < 4; ++u) {
+                const int seg = s0 + u * GT;
+                const int c = s0 == s1 ? cv[u] : seg < nseg ? ld_l2(&A.cnt[seg]) : 0;
+                const uint64_t x = seg < nseg ? key_of(seg, c) : 0;
+                if (x != 0 && x >= bound) {
+                    const int n = atomicAdd(&S.nkeys, 1);
+                    if (n < SEL_KEYS) S.keys[n] = x;
                 }
             }
-            for (int it = 0; it < k; ++it) {
-                const uint64_t m = wave_max_u64(lst[0]);
-                if (m != 0 && lst[0] == m) {
-#pragma unroll
-                    for (int i = 0; i < KMAX; ++i) lst[i] = lst[i + 1];
-                    lst[KMAX] = 0;
+        }
+        __syncthreads();
+        const int nk = S.nkeys;
+        if (nk <= SEL_KEYS) {
+            if (tid < nk) {
+                const uint64_t x = S.keys[tid];
+                int above = 0;
+#pragma unroll 4
+                for (int j = 0; j < nk; ++j) above += S.keys[j] > x;
+                if (above < k) S.topk[above] = x;
+            }
+        } else {  // too many in the waves that hold any: one key after the other
+            uint64_t last = ~0ull;
+            for (int i = 0; i < k && last; ++i) {
+                uint64_t best = 0;
+                for (int seg = tid; seg < nseg; seg += GT) {
+                    const uint64_t x = key_of(seg, ld_l2(&A.cnt[seg]));
+                    if (x < last && x > best) best = x;
                 }
-                if (tid == 0) S.topk[it] = m;
+                last = block_max_u64(best, S.keys);
+                if (tid == 0) S.topk[i] = last;
             }
         }
         __syncthreads();
-        if (tid == 0) {
-            int primary = seg_of_key(bl, !rev);
-            S.size1 = 0;
-            S.self_pair = 0;
-            S.sel[0] = primary;
-            S.selcnt[0] = cnt_of_key(bl, !rev);
-            int K = 1;
-            for (int i = 0; i < k && K < k; ++i) {
-                if (S.topk[i] == 0) break;
-                int s = seg_of_key(S.topk[i], tfwd);
-                if (s == primary) continue;
-                S.sel[K] = s;
-                S.selcnt[K] = cnt_of_key(S.topk[i], tfwd);
-                ++K;
+        if (w == 0) {
+            const uint64_t bl = wave_max_u64(S.wbest[lane & (NW - 1)]);
+            const int primary = seg_of_key(bl, !rev);
+            const uint64_t x = lane < k ? S.topk[lane] : 0;
+            const int seg = seg_of_key(x, tfwd);
+            const uint64_t m = __ballot(x != 0 && seg != primary);
+            const int at = 1 + __popcll(m & ((1ull << lane) - 1));
+            if (((m >> lane) & 1) && at < k) {
+                S.sel[at] = seg;
+                S.selcnt[at] = cnt_of_key(x, tfwd);
             }
-            S.K = K;
+            if (lane == 0) {
+                S.size1 = 0;
+                S.self_pair = 0;
+                S.sel[0] = primary;
+                S.selcnt[0] = cnt_of_key(bl, !rev);
+                S.K = min(k, 1 + (int)__popcll(m));
+            }
         }
         __syncthreads();
     }
-
 
     const uint64_t tB = __builtin_amdgcn_s_memrealtime();
     const int K = S.K;
@@ -1124,9 +1083,42 @@ __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__res
     clock_add(st, 0, t0);
 }
 
-// The round's sequential part: priority queues of every ordered pair of the
-// round's segments, the greedy (reorder/reorder.h:1837-1932), the commit to
-// perm/inv, and the columns of the segments after the commit.
+// Pop order of every ordered pair's queue (ordered pair blockIdx.x), one wave
+// each: dense ranks of its M*M swaps, then the queue (wave_pop_order), then
+// element and gains in pop order for k_gr_greedy.  A queue's pushes and pops are
+// a serial chain of 2 M*M steps, so the queues run side by side on as many
+// CUs (R-MAT 16,384: 55 us a round with a thread per queue in one wave of
+// k_gr_greedy, bound by that wave's instruction issue).
+__global__ __launch_bounds__(64) void k_gr_queues(NMArgs a0, const NMArgs *__restrict__ args) {
+    const NMArgs A = blockIdx.y == 0 ? a0 : args[blockIdx.y];
+    const GreedyState *st = A.st;
+    const int lane = threadIdx.x, q = blockIdx.x;
+    const int done = uniform(st->done), size1 = uniform(st->size1), self_pair = uniform(st->self_pair);
+    const int K = uniform(st->K), M = uniform(st->M), MM = M * M;
+    if (done) return;
+    int a = 0, b = self_pair ? 0 : 1;
+    if (size1) {
+        if (q > 0) return;
+    } else {
+        if (q >= (K - 1) * (K - 1)) return;
+        q_pair(q, K, a, b);
+    }
+    int lg = 0, rg = 0;
+    if (lane < MM) pair_gain(st->acc, K, M, a, b, lane, lg, rg);
+    const int rank = wave_rank(swap_key(lg, rg), MM);
+    const int e = wave_pop_order((rank << 8) | lane, MM);
+    lg = __shfl(lg, e, 64);
+    rg = __shfl(rg, e, 64);
+    if (lane < MM) {
+        A.pops->e[q][lane] = (uint8_t)e;
+        A.pops->lg[q][lane] = lg;
+        A.pops->rg[q][lane] = rg;
+    }
+}
+
+// The round's sequential part: the greedy (reorder/reorder.h:1837-1932) over
+// the pop orders, the commit to perm/inv, and the columns of the segments
+// after the commit.
 __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__restrict__ args) {
     const NMArgs A = blockIdx.y == 0 ? a0 : args[blockIdx.y];
     __shared__ GreedyShared S;
@@ -1134,16 +1126,10 @@ __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__res
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
     const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-    if (tid == 0) S.cont = !st->done;
-    __syncthreads();
-    if (!S.cont) return;
-    const int M = st->M, R = st->R, nseg = st->nseg, MM = M * M;
-    const bool plain = st->sched >= 8;
-    const bool rev = (st->sched == 2 || st->sched == 3);
-    const bool drain = (st->sched == 1 || st->sched == 3);
-    const bool tfwd = drain ? rev : !rev;  // traversal order uses the forward key
-    const int min_size = plain ? 2 : 1;
-    (void)R; (void)nseg; (void)plain; (void)tfwd; (void)min_size;
+    if (st->done) return;
+    const int M = st->M, K = st->K;
+    const int sched = uniform(st->sched);
+    const bool rev = sched == 2 || sched == 3, drain = sched == 1 || sched == 3;
     if (tid < KMAX) {
         S.sel[tid] = st->sel[tid];
         S.selcnt[tid] = st->selcnt[tid];
@@ -1152,84 +1138,28 @@ __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__res
         S.K = st->K;
         S.size1 = st->size1;
         S.self_pair = st->self_pair;
+        S.trace = st->trace != nullptr;
         S.status = 0;
     }
-    // the pair gains summed by k_gr_score; zeroed for the next round
-    for (int t = tid; t < NACC; t += GT) {
-        const int v = st->acc[t];
-        st->acc[t] = 0;
-        if (t < KMAX * MMAX) (&S.E[0][0])[t] = v;
-        else (&S.both[0][0][0])[t - KMAX * MMAX] = v;
+    // the pair gains summed by k_gr_score are used up: zero for the next round
+    for (int t = tid; t < NACC; t += GT) st->acc[t] = 0;
+    const int nq = st->size1 ? 1 : (K - 1) * (K - 1);
+    const int words = nq * MMAX * MMAX;
+    for (int t = tid * 4; t < words; t += GT * 4) {
+        *(int4 *)(&S.pops.lg[0][0] + t) = *(const int4 *)(&A.pops->lg[0][0] + t);
+        *(int4 *)(&S.pops.rg[0][0] + t) = *(const int4 *)(&A.pops->rg[0][0] + t);
+        *(uint32_t *)(&S.pops.e[0][0] + t) = *(const uint32_t *)(&A.pops->e[0][0] + t);
     }
     __syncthreads();
 
-    const uint64_t tD = __builtin_amdgcn_s_memrealtime();
-    // ---- phase D: priority queues: dense ranks (one wave per list), then one
-    // thread per list pushes all pairs and pops the first POPP (all of them
-    // after a round whose greedy popped the heaps often)
-    {
-        const int K = S.K;
-        const int nq = S.size1 ? 1 : (K - 1) * (K - 1);
-        for (int q = w; q < nq; q += NW) {
-            int a, b;
-            if (S.size1) { a = 0; b = S.self_pair ? 0 : 1; }
-            else q_pair(q, K, a, b);
-            int64_t key = 0;
-            if (lane < MM) {
-                int lg, rg;
-                pair_gain(S, K, M, a, b, lane, lg, rg);
-                key = swap_key(lg, rg);
-                S.wkeys[w][lane] = key;
-            }
-            __builtin_amdgcn_wave_barrier();
-            int rnk = 0;
-            if (lane < MM) {
-                // independent broadcast reads: unrolled so they issue back to
-                // back instead of one LDS round trip per key
-#pragma unroll 16
-                for (int j = 0; j < MM; ++j) rnk += S.wkeys[w][j] < key;
-            }
-            // the push order is element order: stage entry e in slot e
-            if (lane < MM) {
-                HeapRef Hq{reinterpret_cast<uint16_t *>(S.heap[q]), 0};
-                hset(Hq, lane, (uint32_t)((rnk << 8) | lane));
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        __syncthreads();
-        if (tid == 0) st->clk[11] += __builtin_amdgcn_s_memrealtime() - tD;
-        // one thread per list, all in wave 0: the heap steps are bound by
-        // instruction issue, so 64 lists share every instruction
-        const int npre = min(st->npre, MM);
-        if (tid == 0) {
-            S.npre = npre;
-            S.heap_pops = 0;
-            S.maxk = 0;
-        }
-        if (tid < nq) {
-            HeapRef H{reinterpret_cast<uint16_t *>(S.heap[tid]), 0};
-            for (int e = 0; e < MM; ++e) heap_push(H, hget(H, e));
-            for (int k = 0; k < npre; ++k) S.popped[k][tid] = (uint8_t)(heap_pop(H) & 0xFFu);
-            S.heapn[tid] = H.n;
-            S.qcur[tid] = 0;
-        }
-        __syncthreads();
-    }
-
     const uint64_t tE = __builtin_amdgcn_s_memrealtime();
-    // ---- phase E: the sequential greedy (wave 0 in lockstep)
+    // ---- the sequential greedy (wave 0)
     if (w == 0) {
         const int nsw = M == 8 ? greedy_apply<8>(S, rev, drain) : greedy_apply<4>(S, rev, drain);
         if (lane == 0) {
             S.nsw = nsw;
-            st->clk[12] += nsw;           // swaps
-            st->clk[13] += S.heap_pops;   // pops taken from heaps by the greedy
-            st->clk[14] += S.npre;        // pops precomputed per ordered pair
-            // the next round precomputes what this one used, plus 8: a
-            // round that had to pop heaps precomputes whole pop orders next
-            st->npre = S.heap_pops > 0 ? MM : max(POPP, min(MM, (S.maxk + 15) / 8 * 8));
+            st->clk[12] += nsw;  // swaps
             const uint64_t t1 = __builtin_amdgcn_s_memrealtime();
-            st->clk[6] += tE - tD;
             st->clk[7] += t1 - tE;
         }
     }
@@ -1242,9 +1172,10 @@ __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__res
         return;
     }
 
-    // ---- phase F: commit the swaps to perm/inv (reorder(), :392-418)
+    // ---- commit the swaps to perm/inv (reorder(), :392-418)
     if (tid < S.nsw) {
-        int v1 = S.swv1[tid], v2 = S.swv2[tid];
+        const int sw = S.sww[tid], a = sw & 0xFF, b = (sw >> 8) & 0xFF, e = sw >> 16;
+        const int v1 = S.sel[a] * M + e / M, v2 = S.sel[b] * M + e % M;
         if (v1 != v2) {
             int b1 = ld_l2(&A.inv[v1]), b2 = ld_l2(&A.inv[v2]);
             st_l2(&A.inv[v1], b2);
@@ -1256,7 +1187,7 @@ __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__res
             int64_t n = st->trace_len + tid;
             if (n < st->trace_cap) {
                 int32_t *t = st->trace + n * 9;
-                t[0] = st->round; t[1] = S.swp[tid]; t[2] = S.swt[tid];
+                t[0] = st->round; t[1] = S.sel[a]; t[2] = S.sel[b];
                 t[3] = v1; t[4] = v2; t[5] = S.swlg[tid]; t[6] = S.swrg[tid];
                 t[7] = S.swpc[tid]; t[8] = S.swtc[tid];
             }
@@ -1264,11 +1195,7 @@ __global__ __launch_bounds__(GT) void k_gr_greedy(NMArgs a0, const NMArgs *__res
     }
     __syncthreads();
     if (tid == 0) st->trace_len += S.nsw;
-
-
-    __syncthreads();
     // columns of the round's segments after the commit, for the recount
-    const int K = S.K;
     const int total = table_columns(S.sel, K, M, A.inv, A.cptr, S.cs.cols, S.cs.pre);
     if (tid == 0) S.cs.total = total;
     chunk_table(S.cs, K, M);
@@ -1310,7 +1237,7 @@ __global__ __launch_bounds__(GT) void k_gr_init(NMArgs A, int R, int M, int N, i
         st->round = 1; st->L = sL; st->totcnt = sC;
         st->init_size = sL; st->init_cnt = sC;
         st->maxiter = maxiter > sL ? maxiter : sL;
-        st->status = 0; st->done = 0; st->pending = 0; st->npre = POPP;
+        st->status = 0; st->done = 0; st->pending = 0;
         st->K = 0; st->self_pair = 0; st->size1 = 0;
         st->trace_len = 0; st->work = 0;
         st->S.K = 0; st->S.total = 0; st->S.cb[0] = 0;
@@ -1536,7 +1463,7 @@ __global__ __launch_bounds__(64) void k_gr_alldone(const NMArgs *__restrict__ ar
     if (threadIdx.x == 0) *flag = b == 0;
 }
 
-// Capture ROUND_BATCH rounds (six kernels each, grid y = the G graphs) and
+// Capture ROUND_BATCH rounds (seven kernels each, grid y = the G graphs) and
 // the all-done test on the context stream.
 static int capture_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args, int G, int gpx,
                           int32_t *d_flag, hipGraph_t *graph_out, hipGraphExec_t *exec_out) {
@@ -1545,6 +1472,7 @@ static int capture_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args
         hipLaunchKernelGGL(k_gr_select, dim3(1, G), dim3(GT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_fill_a, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_score, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
+        hipLaunchKernelGGL(k_gr_queues, dim3(NQ, G), dim3(64), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_greedy, dim3(1, G), dim3(GT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_fill_b, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_count, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
@@ -1577,9 +1505,10 @@ static int pass_grid(vnm_ctx *ctx, int G) {
     return std::max(16, std::min(2 * ncu, 8 * ncu / G));
 }
 
-// Bytes of the greedy state of a graph, then its one-graph argument block
-// and all-done flag.
-constexpr size_t GST_STATE = (sizeof(GreedyState) + 255) / 256 * 256;
+// Bytes of the greedy state and pop orders of a graph, then its one-graph
+// argument block and all-done flag.
+constexpr size_t GST_POPS = (sizeof(GreedyState) + 255) / 256 * 256;
+constexpr size_t GST_STATE = GST_POPS + (sizeof(PopOrders) + 255) / 256 * 256;
 constexpr size_t GST_BYTES = GST_STATE + (sizeof(NMArgs) + 63) / 64 * 64 + 64;
 
 // Per-graph state of a run: CSC, counts, records, greedy state and the
@@ -1596,6 +1525,7 @@ static int greedy_prepare(vnm_graph *g, int N, NMArgs *A) {
         VNM_HIP_TRY(hipMemsetAsync(g->rt.p, 0, (size_t)g->nrows * 32, st));
     }
     A->st = (GreedyState *)g->gst.p;
+    A->pops = (PopOrders *)((char *)g->gst.p + GST_POPS);
     A->cptr = g->cptr.p; A->crow = g->crow.p; A->perm = g->perm.p; A->inv = g->inv.p;
     A->cnt = g->cnt.p; A->nzr = g->nzr.p;
     A->rta = g->rt.p; A->rtb = g->rt.p + (size_t)g->nrows * 4;
@@ -1604,18 +1534,15 @@ static int greedy_prepare(vnm_graph *g, int N, NMArgs *A) {
 
 static void debug_print(int i, const GreedyState &h) {
     fprintf(stderr, "[vnm] greedy%s%d rounds=%d entries=%lld kernel_us select=%llu fill_a=%llu score=%llu "
-                    "greedy=%llu (heaps %llu, sequential %llu) fill_b=%llu count=%llu\n",
+                    "greedy=%llu (sequential %llu) fill_b=%llu count=%llu\n",
             i < 0 ? "" : " graph ", i < 0 ? 0 : i,
             h.round - 1, (long long)h.work, (unsigned long long)(h.clk[0] / 100),
             (unsigned long long)(h.clk[1] / 100), (unsigned long long)(h.clk[2] / 100),
-            (unsigned long long)(h.clk[3] / 100), (unsigned long long)(h.clk[6] / 100),
-            (unsigned long long)(h.clk[7] / 100), (unsigned long long)(h.clk[4] / 100),
+            (unsigned long long)(h.clk[3] / 100), (unsigned long long)(h.clk[7] / 100), (unsigned long long)(h.clk[4] / 100),
             (unsigned long long)(h.clk[5] / 100));
-    fprintf(stderr, "[vnm]   select: commit %llu, segments %llu, columns %llu; heaps: ranks %llu\n",
+    fprintf(stderr, "[vnm]   select: commit %llu, segments %llu, columns %llu; swaps %llu\n",
             (unsigned long long)(h.clk[8] / 100), (unsigned long long)(h.clk[9] / 100),
-            (unsigned long long)(h.clk[10] / 100), (unsigned long long)(h.clk[11] / 100));
-    fprintf(stderr, "[vnm]   greedy: swaps %llu, heap pops %llu, precomputed pops per pair (sum) %llu\n",
-            (unsigned long long)h.clk[12], (unsigned long long)h.clk[13], (unsigned long long)h.clk[14]);
+            (unsigned long long)(h.clk[10] / 100), (unsigned long long)h.clk[12]);
 }
 
 // The greedy of G graphs (schedules 0-3 or >= 8 each) as one chain of round
@@ -1690,7 +1617,7 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
     int32_t done = 0;
     while (!done) {
         VNM_HIP_TRY(hipGraphLaunch(exec, st));
-        ctx->launches += 6 * ROUND_BATCH + 1;
+        ctx->launches += 7 * ROUND_BATCH + 1;
         VNM_HIP_TRY(hipMemcpyAsync(&done, d_flag, 4, hipMemcpyDeviceToHost, st));
         VNM_HIP_TRY(hipStreamSynchronize(st));
     }
@@ -1834,9 +1761,13 @@ int vnm_pq_pop_order(vnm_ctx *ctx, const int32_t *scores, int count, int M, int3
     if ((rc = ds.alloc((size_t)count * 2 * MM)) || (rc = dord.alloc((size_t)count * MM))) return rc;
     hipStream_t st = ctx->stream;
     VNM_HIP_TRY(hipMemcpyAsync(ds.p, scores, (size_t)count * 2 * MM * 4, hipMemcpyHostToDevice, st));
-    const int bt = 64;
-    hipLaunchKernelGGL(k_pq_pop_order, dim3((count + bt - 1) / bt), dim3(bt), (size_t)bt * HEAP_WORDS * 4, st, ds.p,
-                       count, M, dord.p);
+    // a wave per list while the chip holds them all at once; beyond, a thread
+    // per list
+    if (count <= PQ_WAVES)
+        hipLaunchKernelGGL(k_pq_pop_order_wave, dim3(count), dim3(64), 0, st, ds.p, M, dord.p);
+    else
+        hipLaunchKernelGGL(k_pq_pop_order, dim3((count + 63) / 64), dim3(64), (size_t)64 * HEAP_WORDS * 4, st, ds.p,
+                           count, M, dord.p);
     ctx->launches++;
     VNM_LAUNCH_CHECK("k_pq_pop_order");
     VNM_HIP_TRY(hipMemcpyAsync(order, dord.p, (size_t)count * MM * 4, hipMemcpyDeviceToHost, st));
