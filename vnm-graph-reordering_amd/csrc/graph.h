@@ -23,11 +23,12 @@ namespace vnm {
 // Idle device memory of one context, for its next calls: packing takes 60
 // buffers and a learned reorder 45, and hipMalloc and hipFree (which waits for the
 // whole device) were most of such a call's time (packing R-MAT 65,536 took 7.6 ms,
-// of it 0.9 in kernels, and 1.27 from the pool; its learned reorder 8.1 ms and 5.8).  A block given back may still be read by
-// work enqueued on the context's stream; the next owner's work is enqueued behind
-// it, on the same stream, so nothing waits.  (Host copies into a block go through
-// the stream as well.)  At most POOL_IDLE bytes stay idle; the context and its
-// objects share the pool, and the last of them frees it.
+// of it 0.9 in kernels, and 1.27 from the pool; its learned reorder 8.1 ms and 5.8).
+// A block given back may still be read by work enqueued on the context's stream;
+// the next owner's work is enqueued behind it, on the same stream, so nothing
+// waits.  (Host copies into a block go through the stream as well.)  At most
+// POOL_IDLE bytes stay idle; the context and its objects share the pool, and the
+// last of them frees it.
 constexpr size_t POOL_IDLE = (size_t)2 << 30;
 constexpr size_t POOL_GRAIN = 4096;
 

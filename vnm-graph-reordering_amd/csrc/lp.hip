@@ -117,6 +117,9 @@ __global__ void k_lp_adj_keys(const int32_t *__restrict__ row, const int32_t *__
                               const float *__restrict__ val, int64_t nnz, int R,
                               uint64_t *__restrict__ kc, uint64_t *__restrict__ kt,
                               int32_t *__restrict__ nvalid) {
+    __shared__ int sum;
+    if (threadIdx.x == 0) sum = 0;
+    __syncthreads();
     int local = 0;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nnz;
          i += (int64_t)gridDim.x * blockDim.x) {
@@ -126,7 +129,11 @@ __global__ void k_lp_adj_keys(const int32_t *__restrict__ row, const int32_t *__
         kt[i] = ok ? ((uint64_t)(uint32_t)r << 32) | (uint32_t)c : (uint64_t)(uint32_t)R << 32;
         local += ok;
     }
-    if (local) atomicAdd(nvalid, local);
+    // one device atomic a workgroup (one a thread: 193 us for 1.0 M entries; 52)
+    for (int o = 32; o > 0; o >>= 1) local += __shfl_xor(local, o);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&sum, local);
+    __syncthreads();
+    if (threadIdx.x == 0 && sum) atomicAdd(nvalid, sum);
 }
 
 // Sorted keys (node << 32 | neighbour), n of them valid: idx[i] = neighbour,
@@ -331,17 +338,48 @@ __global__ __launch_bounds__(SS_T) void k_lp_seg_stats(
     }
 }
 
+// Device-side control of one learned run.  The host enqueues iterations
+// without reading anything back; the control kernels take the decisions of
+// the iteration loop (stop, fall back to the exhaustive window, sizes), and
+// every kernel of an iteration reads its counts and its skip flag here.
+struct LPCtl {
+    int done;       // the run has ended (converged, no donors, nothing to apply)
+    int exh;        // this iteration scores every window entry exactly
+    int skip_fwd;   // no forward pass this iteration
+    int skip_norm;  // no sort of the one-per-donor candidates (done || exh)
+    int skip_exh;   // no sort of the window candidates (done || !exh)
+    int skip_swap;  // no swaps to apply (done || none accepted)
+    int it;         // iterations run (the proposals' seeds follow it)
+    int ndonor;     // donors counted by k_lp_pick
+    int nd, nc, stride;
+    int nacc, gain;  // accepted swaps and their summed gain (k_lp_select)
+    int nsel;        // segments the accepted swaps touched
+    int fallbacks, swaps;
+    long long gain_total, exact_pairs;
+};
+
+// The start of an iteration: donors counted from 0, and whether it has a
+// forward pass.
+__device__ __forceinline__ void ctl_begin(LPCtl *ctl, int done, int exh, int mode) {
+    ctl->ndonor = 0;
+    ctl->skip_fwd = done || exh || mode != 0;
+}
+
 // tot[0] = sum over segments of rows with more than N ones, tot[1] = number
-// of segments with at least one such row.
+// of segments with at least one such row.  At the end of a run's iteration
+// (ctl): not when no swap was applied; the run is over when nothing is invalid.
 __global__ __launch_bounds__(1024) void k_lp_totals(int nseg, const int32_t *__restrict__ segcls,
-                                                     int32_t *__restrict__ tot, const int *__restrict__ skip) {
-    if (skip && *skip) return;
+                                                     int32_t *__restrict__ tot, LPCtl *ctl, int mode) {
+    if (ctl && ctl->skip_swap) {
+        if (threadIdx.x == 0) ctl_begin(ctl, ctl->done, ctl->exh, mode);
+        return;
+    }
     __shared__ int sc[16], ss[16];
     int c = 0, s = 0;
     for (int i = threadIdx.x; i < nseg; i += 1024) {
-        int v = segcls[i * 4 + 2] + segcls[i * 4 + 3];
-        c += v;
-        s += v != 0;
+        const int2 v = *(const int2 *)&segcls[i * 4 + 2];
+        c += v.x + v.y;
+        s += v.x + v.y != 0;
     }
     for (int o = 32; o > 0; o >>= 1) {
         c += __shfl_xor(c, o);
@@ -354,6 +392,11 @@ __global__ __launch_bounds__(1024) void k_lp_totals(int nseg, const int32_t *__r
         for (int w = 0; w < 16; ++w) { a += sc[w]; b += ss[w]; }
         tot[0] = a;
         tot[1] = b;
+        if (ctl) {
+            const int done = ctl->done || a <= 0;
+            ctl->done = done;
+            ctl_begin(ctl, done, ctl->exh, mode);
+        }
     }
 }
 
@@ -891,26 +934,6 @@ __global__ void k_lp_wt(const float *__restrict__ w, uint16_t *__restrict__ wt) 
 
 // ------------------------------------------------------------ candidates
 
-// Device-side control of one learned run.  The host enqueues iterations
-// without reading anything back; the control kernels take the decisions of
-// the iteration loop (stop, fall back to the exhaustive window, sizes), and
-// every kernel of an iteration reads its counts and its skip flag here.
-struct LPCtl {
-    int done;       // the run has ended (converged, no donors, nothing to apply)
-    int exh;        // this iteration scores every window entry exactly
-    int skip_fwd;   // no forward pass this iteration
-    int skip_norm;  // no sort of the one-per-donor candidates (done || exh)
-    int skip_exh;   // no sort of the window candidates (done || !exh)
-    int skip_swap;  // no swaps to apply (done || none accepted)
-    int it;         // iterations run (the proposals' seeds follow it)
-    int ndonor;     // donors counted by k_lp_pick
-    int nd, nc, stride;
-    int nacc, gain;  // accepted swaps and their summed gain (k_lp_select)
-    int nsel;        // segments the accepted swaps touched
-    int fallbacks, swaps;
-    long long gain_total, exact_pairs;
-};
-
 // A run starts at iteration 0, in the exhaustive mode for mode 2, and is
 // over at once when no segment is invalid.
 __global__ void k_lp_ctl_init(LPCtl *ctl, const int32_t *__restrict__ tot, int mode) {
@@ -919,19 +942,12 @@ __global__ void k_lp_ctl_init(LPCtl *ctl, const int32_t *__restrict__ tot, int m
     z.exh = mode == 2;
     z.done = tot[0] <= 0;
     *ctl = z;
-}
-
-__global__ void k_lp_ctl_begin(LPCtl *ctl, int mode) {
-    if (threadIdx.x != 0) return;
-    ctl->ndonor = 0;
-    ctl->skip_fwd = ctl->done || ctl->exh || mode != 0;
+    ctl_begin(ctl, z.done, z.exh, mode);
 }
 
 // After the donors are counted: this iteration's sizes, or the end of the run
 // when there is no donor.
-__global__ void k_lp_ctl_mid(LPCtl *ctl, int topk, int W, int nseg) {
-    if (threadIdx.x != 0) return;
-    LPCtl c = *ctl;
+__device__ __forceinline__ void ctl_sizes(LPCtl &c, int topk, int W, int nseg) {
     c.nd = min(topk, c.ndonor);
     if (!c.done && c.nd == 0) c.done = 1;
     if (c.done) {
@@ -944,18 +960,17 @@ __global__ void k_lp_ctl_mid(LPCtl *ctl, int topk, int W, int nseg) {
         c.skip_norm = c.exh;
         c.skip_exh = !c.exh;
     }
-    *ctl = c;
 }
 
 // After the selection: nothing accepted falls back to the exhaustive window
 // once (mode 0) or ends the run; otherwise the swaps are applied and the
 // next iteration proposes again.
-__global__ void k_lp_ctl_after(LPCtl *ctl, int mode, int32_t *__restrict__ queue) {
-    if (threadIdx.x != 0) return;
+__device__ __forceinline__ void ctl_accept(LPCtl *ctl, int nacc, int gain, int mode, int32_t *queue) {
     LPCtl c = *ctl;
-    if (c.done) return;
+    c.nacc = nacc;
+    c.gain = gain;
     c.it++;
-    if (c.nacc == 0) {
+    if (nacc == 0) {
         c.skip_swap = 1;
         c.nsel = 0;
         if (mode == 0 && !c.exh) {
@@ -966,18 +981,13 @@ __global__ void k_lp_ctl_after(LPCtl *ctl, int mode, int32_t *__restrict__ queue
         }
     } else {
         c.skip_swap = 0;
-        c.nsel = 2 * c.nacc;
-        c.swaps += c.nacc;
-        c.gain_total += c.gain;
+        c.nsel = 2 * nacc;
+        c.swaps += nacc;
+        c.gain_total += gain;
         if (mode == 0) c.exh = 0;
         *queue = 0;  // k_lp_seg_stats' work counter
     }
     *ctl = c;
-}
-
-// After the touched segments are recounted: over when nothing is invalid.
-__global__ void k_lp_ctl_end(LPCtl *ctl, const int32_t *__restrict__ tot) {
-    if (threadIdx.x == 0 && !ctl->done && !ctl->skip_swap && tot[0] <= 0) ctl->done = 1;
 }
 
 // The done flags of a batch's runs, in one array the host reads.
@@ -1043,28 +1053,48 @@ struct Cand { int p, q, bu, bv; };
 // Donor i (in donor order) looks at the acceptors ranked (i*stride + w) mod
 // nseg, w < W.  all == 0: one candidate per donor, the window entry with the
 // best pair score (network: Y0[u] + Y1[v] + P[u].Q[v]; hash in mode 1; the
-// first in mode 2); all == 1: every window entry is a candidate.
-__global__ void k_lp_match(const LPCtl *__restrict__ ctl, int W, int nseg, int M, int mode0, uint64_t seed0,
-                           const uint64_t *__restrict__ sdkey, const uint64_t *__restrict__ sakey,
-                           const int8_t *__restrict__ dbest, const int8_t *__restrict__ abest,
-                           const int32_t *__restrict__ inv, const float *__restrict__ Y,
-                           Cand *__restrict__ cand, uint64_t smask) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ctl->done || i >= ctl->nd) return;
-    const int stride = ctl->stride, all = ctl->exh, mode = ctl->exh ? 2 : mode0;
-    const uint64_t seed = seed0 ^ ((uint64_t)ctl->it << 20);
+// first in mode 2), the first of equal ones; all == 1: every window entry is a
+// candidate.  MATCH_L lanes share a donor's window, an entry each, so that the
+// chain from ranks to segments to nodes to rows of Y is walked once (a thread a
+// donor walked it W times: 28 us for 4,096 donors).  The first thread also
+// writes the iteration's sizes, which every thread works out for itself.
+constexpr int MATCH_L = 16;
+
+__global__ __launch_bounds__(256) void k_lp_match(LPCtl *ctl, int topk, int W, int nseg, int M, int mode0,
+                                                  uint64_t seed0, const uint64_t *__restrict__ sdkey,
+                                                  const uint64_t *__restrict__ sakey, const int8_t *__restrict__ dbest,
+                                                  const int8_t *__restrict__ abest, const int32_t *__restrict__ inv,
+                                                  const float *__restrict__ Y, Cand *__restrict__ cand,
+                                                  uint64_t smask) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = t / MATCH_L, l = t % MATCH_L;
+    LPCtl c = *ctl;  // (the fields written here are not read, or come out the same)
+    const uint64_t seed = seed0 ^ ((uint64_t)c.it << 20);
+    const int all = c.exh, mode = c.exh ? 2 : mode0;
+    ctl_sizes(c, topk, W, nseg);
+    if (t == 0) {
+        ctl->done = c.done;
+        ctl->nd = c.nd; ctl->nc = c.nc; ctl->stride = c.stride;
+        ctl->exact_pairs = c.exact_pairs;
+        ctl->skip_norm = c.skip_norm; ctl->skip_exh = c.skip_exh;
+        if (c.done) ctl->skip_swap = 1;
+    }
+    if (c.done || i >= c.nd) return;
     const int p = (int)(sdkey[i] & smask);
     const int bu = dbest[p];
     const int u = inv[p * M + bu];
+    const uint32_t j0 = (uint32_t)i * (uint32_t)c.stride;  // below nseg
+    // the best of the lane's entries; the first one of another segment, and
+    // whether its score is not a number
     float best = 0.f;
-    int bw = -1;
-    for (int w = 0; w < W; ++w) {
-        const int j = (int)(((int64_t)i * stride + w) % nseg);
+    int bw = -1, first = 0x7FFFFFFF;
+    bool fnan = false;
+    for (int w = l; w < W; w += MATCH_L) {
+        const int j = (int)((j0 + (uint32_t)w) % (uint32_t)nseg);
         const int q = (int)(sakey[j] & smask);
         const int bv = abest[q];
-        Cand c{p, q == p ? -1 : q, bu, bv};
         if (all) {
-            cand[(size_t)i * W + w] = c;
+            cand[(size_t)i * W + w] = Cand{p, q == p ? -1 : q, bu, bv};
             continue;
         }
         if (q == p) continue;
@@ -1079,14 +1109,36 @@ __global__ void k_lp_match(const LPCtl *__restrict__ ctl, int W, int nseg, int M
         } else {
             sc = -(float)w;
         }
-        if (bw < 0 || sc > best) { best = sc; bw = w; }
+        if (bw < 0) {
+            first = w;
+            fnan = sc != sc;
+        }
+        if (bw < 0 || sc > best || best != best) { best = sc; bw = w; }
     }
-    if (!all) {
+    if (all) return;
+    auto better = [](float a, int aw, float b, int bw) {
+        if (aw < 0 || bw < 0) return bw < 0;
+        if (a != a || b != b) return a == a || (b != b && aw < bw);
+        return a > b || (a == b && aw < bw);
+    };
+    for (int o = 1; o < MATCH_L; o <<= 1) {
+        const float ob = __shfl_xor(best, o);
+        const int ow = __shfl_xor(bw, o);
+        if (!better(best, bw, ob, ow)) { best = ob; bw = ow; }
+    }
+    // a score that is not a number wins as the window's first, which nothing
+    // compares greater than, and only then
+    for (int o = 1; o < MATCH_L; o <<= 1) {
+        const int of = __shfl_xor(first, o);
+        const int on = __shfl_xor((int)fnan, o);
+        if (of < first) { first = of; fnan = on != 0; }
+    }
+    if (fnan) bw = first;
+    if (l == 0) {
         if (bw < 0) {
             cand[i] = Cand{p, -1, bu, 0};
         } else {
-            const int j = (int)(((int64_t)i * stride + bw) % nseg);
-            const int q = (int)(sakey[j] & smask);
+            const int q = (int)(sakey[(j0 + (uint32_t)bw) % (uint32_t)nseg] & smask);
             cand[i] = Cand{p, q, bu, abest[q]};
         }
     }
@@ -1105,12 +1157,29 @@ __global__ void k_lp_match(const LPCtl *__restrict__ ctl, int W, int nseg, int M
 // Writes the best pair (max lgain + rgain, then max rgain, then the lower
 // index b1*M+b2) and, when full != nullptr, the whole matrix in the layout
 // of vnm_swap_score.
-__global__ __launch_bounds__(256) void k_lp_pair_gain(const int *__restrict__ d_nc, int R, int M, int N,
+// In a run (gk.ctl) the candidates' number is the control block's, and each
+// one's sort key is written too: (gain descending, candidate) in gbits + ibits
+// bits, ibits the bits of the largest candidate index, gmax = 2^gbits - 1 at
+// least the largest gain (a gain counts rows of the pair's two segments, each row
+// at most once per segment, so it is at most twice the row count).  Slots past
+// the candidates, up to the size of the sort that follows, get ~0, which sorts
+// last.  A workgroup takes candidates blockIdx.x, + gridDim.x, ...: one each
+// but in the exhaustive mode.
+struct GainKeys {
+    const LPCtl *ctl;
+    int nnorm, nexh;  // keys of the two sorts
+    uint64_t *keys;
+    int ibits;
+    uint32_t gmax;
+};
+
+__global__ __launch_bounds__(256) void k_lp_pair_gain(int nc, int R, int M, int N,
                                                       const Cand *__restrict__ cand,
                                                       const int32_t *__restrict__ inv,
                                                       const int32_t *__restrict__ ptr,
                                                       const int32_t *__restrict__ idx,
-                                                      int4 *__restrict__ best, int32_t *__restrict__ full) {
+                                                      int4 *__restrict__ best, int32_t *__restrict__ full,
+                                                      GainKeys gk) {
     __shared__ ColSpan cols[16];
     __shared__ int pre[17];
     __shared__ int sel[2];
@@ -1124,200 +1193,195 @@ __global__ __launch_bounds__(256) void k_lp_pair_gain(const int *__restrict__ d_
         RowHash h;
         uint32_t tile[PAIR_TILE_ROWS / 2];
     } L;
-    const int i = blockIdx.x;
-    if (d_nc && i >= *d_nc) return;  // past this iteration's candidates (device count)
-    const Cand c = cand[i];
     const int tid = threadIdx.x, lane = tid & 63;
     const int MM = M * M;
-    if (c.q < 0) {
-        if (tid == 0) best[i] = make_int4(0, 0, -0x40000000, 0);
-        return;
+    if (gk.ctl) {
+        if (gk.ctl->done) return;
+        nc = gk.ctl->nc;
+        const int nkeys = gk.ctl->exh ? gk.nexh : gk.nnorm;
+        for (int j = nc + blockIdx.x * 256 + tid; j < nkeys; j += gridDim.x * 256) gk.keys[j] = ~0ull;
     }
-    if (tid == 0) { sel[0] = c.p; sel[1] = c.q; }
-    if (tid < 64) { sBl[tid] = 0; sBr[tid] = 0; }
-    if (tid < 8) { sEp[tid] = 0; sEq[tid] = 0; }
-    __syncthreads();
-    const int total = table_columns(sel, 2, M, inv, ptr, cols, pre);
-    const int b1 = lane / M, b2 = lane % M;
-    int aBl = 0, aBr = 0, aEp = 0, aEq = 0;
-    // one entry per lane (t = its column, -1 for none; lv / rv = its row's
-    // bitmaps in p and q), folded into the gain sums with wave ballots; the
-    // sums count each row once, through its owner (leading-bit) entries
-    auto fold = [&](int t, uint32_t lv, uint32_t rv) {
-        bool isP = false, isQ = false;
-        uint32_t l = 0, rr = 0;
-        if (t >= 0) {
-            if (t < M) {
-                l = lv;
-                isP = (l >> (M - 1 - t)) == 1u;  // the row's owner entry in p
-                if (isP) rr = rv;
-            } else {
-                rr = rv;
-                isQ = (rr >> (M - 1 - (t - M))) == 1u;
+    for (int i = blockIdx.x; i < nc; i += gridDim.x) {
+        const Cand c = cand[i];
+        if (c.q < 0) {
+            if (tid == 0) {
+                best[i] = make_int4(0, 0, -0x40000000, 0);
+                if (gk.ctl) gk.keys[i] = ~0ull;
+            }
+            continue;
+        }
+        __syncthreads();  // the last candidate's sums are read
+        if (tid == 0) { sel[0] = c.p; sel[1] = c.q; }
+        if (tid < 64) { sBl[tid] = 0; sBr[tid] = 0; }
+        if (tid < 8) { sEp[tid] = 0; sEq[tid] = 0; }
+        __syncthreads();
+        const int total = table_columns(sel, 2, M, inv, ptr, cols, pre);
+        const int b1 = lane / M, b2 = lane % M;
+        int aBl = 0, aBr = 0, aEp = 0, aEq = 0;
+        // one entry per lane (t = its column, -1 for none; lv / rv = its row's
+        // bitmaps in p and q), folded into the gain sums with wave ballots; the
+        // sums count each row once, through its owner (leading-bit) entries
+        auto fold = [&](int t, uint32_t lv, uint32_t rv) {
+            bool isP = false, isQ = false;
+            uint32_t l = 0, rr = 0;
+            if (t >= 0) {
+                if (t < M) {
+                    l = lv;
+                    isP = (l >> (M - 1 - t)) == 1u;  // the row's owner entry in p
+                    if (isP) rr = rv;
+                } else {
+                    rr = rv;
+                    isQ = (rr >> (M - 1 - (t - M))) == 1u;
+                }
+            }
+            const int pl = popc32(l), pr = popc32(rr);
+            const bool both = isP && rr != 0;
+            const uint64_t Ap = __ballot(isP && pl == N + 1);
+            const uint64_t Dq = __ballot(isQ && pr == N + 1);
+            const uint64_t A = __ballot(both && pl == N + 1), B = __ballot(both && pl == N);
+            const uint64_t C = __ballot(both && pr == N), D = __ballot(both && pr == N + 1);
+            uint64_t Lb = 0, Rb = 0, Lown = 0, Rown = 0;
+            for (int b = 0; b < M; ++b) {
+                const uint64_t lm = __ballot(isP && ((l >> (M - 1 - b)) & 1u));
+                const uint64_t rb = __ballot(both && ((rr >> (M - 1 - b)) & 1u));
+                const uint64_t rq = __ballot(isQ && ((rr >> (M - 1 - b)) & 1u));
+                if (b == b1) Lb = lm;
+                if (b == b2) Rb = rb;
+                if (b == lane) { Lown = lm; Rown = rq; }
+            }
+            if (lane < MM && (A | B | C | D)) {
+                aBl += __popcll(Rb & ((Lb & A) | (~Lb & B)));
+                aBr += __popcll(Lb & ((Rb & D) | (~Rb & C)));
+            }
+            if (lane < M) {
+                aEp += __popcll(Lown & Ap);
+                aEq += __popcll(Rown & Dq);
+            }
+        };
+        if (total <= HASH_MAX) {
+            const int hb = hash_bits(total);
+            hash_reset(L.h, hb);
+            __syncthreads();
+            hash_scatter(L.h, hb, M, cols, pre, 2 * M, total, idx);
+            __syncthreads();
+            // TAB_U entries per thread resolved before their lookups
+            for (int base = 0; base < total; base += 256 * TAB_U) {
+                int tt[TAB_U], rw[TAB_U];
+                table_entries(cols, pre, 2 * M, total, idx, base + tid, 256, tt, rw);
+    #pragma unroll
+                for (int u = 0; u < TAB_U; ++u) {
+                    const uint32_t h = tt[u] >= 0 ? hash_get(L.h, hb, (uint32_t)rw[u]) : 0u;
+                    fold(tt[u], h & 0xFFu, (h >> 8) & 0xFFu);
+                }
+            }
+        } else {
+            // rows [r0, r0 + PAIR_TILE_ROWS) at a time: each column's entries of
+            // a tile are one range of its row-sorted list; the ends of PB tiles
+            // of all 2M columns come from one round of binary searches
+            const int nc = 2 * M;
+            for (int w = tid; w < PAIR_TILE_ROWS / 2; w += 256) L.tile[w] = 0u;
+            if (tid < nc) tlo[tid] = cols[tid].start;
+            const int ntile = (R + PAIR_TILE_ROWS - 1) / PAIR_TILE_ROWS;
+            for (int g0 = 0; g0 < ntile; g0 += PB) {
+                if (tid < nc * PB) {
+                    const int t = tid / PB, j = tid % PB;
+                    const int64_t r1 = min((int64_t)R, (int64_t)(g0 + j + 1) * PAIR_TILE_ROWS);
+                    int lo = cols[t].start, hi = cols[t].start + cols[t].len;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (idx[mid] < r1) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    tend[t][j] = lo;
+                }
+                __syncthreads();
+                for (int j = 0; j < PB && g0 + j < ntile; ++j) {
+                    const int r0 = (g0 + j) * PAIR_TILE_ROWS;
+                    if (tid == 0) {
+                        tpre[0] = 0;
+                        for (int t = 0; t < nc; ++t) {
+                            thi[t] = tend[t][j];
+                            tpre[t + 1] = tpre[t] + thi[t] - tlo[t];
+                        }
+                    }
+                    __syncthreads();
+                    const int tt = tpre[nc];
+                    if (tt > 0) {  // uniform
+                        // TAB_U entries per thread resolved before their loads
+                        auto entries = [&](int e0, int (&t)[TAB_U], int (&r)[TAB_U]) {
+    #pragma unroll
+                            for (int u = 0; u < TAB_U; ++u) {
+                                const int e = e0 + u * 256;
+                                t[u] = e < tt ? entry_col(tpre, nc, e) : -1;
+                            }
+    #pragma unroll
+                            for (int u = 0; u < TAB_U; ++u)
+                                r[u] = t[u] >= 0 ? idx[tlo[t[u]] + (e0 + u * 256 - tpre[t[u]])] - r0 : 0;
+                        };
+                        for (int e0 = tid; e0 < tt; e0 += 256 * TAB_U) {
+                            int t[TAB_U], r[TAB_U];
+                            entries(e0, t, r);
+    #pragma unroll
+                            for (int u = 0; u < TAB_U; ++u)
+                                if (t[u] >= 0)
+                                    atomicOr(&L.tile[r[u] >> 1],
+                                             ((1u << (M - 1 - t[u] % M)) << (8 * (t[u] / M))) << (16 * (r[u] & 1)));
+                        }
+                        __syncthreads();
+                        for (int base = 0; base < tt; base += 256 * TAB_U) {
+                            int t[TAB_U], r[TAB_U];
+                            entries(base + tid, t, r);
+    #pragma unroll
+                            for (int u = 0; u < TAB_U; ++u) {
+                                const uint32_t h = t[u] >= 0 ? (L.tile[r[u] >> 1] >> (16 * (r[u] & 1))) & 0xFFFFu : 0u;
+                                fold(t[u], h & 0xFFu, h >> 8);
+                            }
+                        }
+                        __syncthreads();
+                        for (int w = tid; w < PAIR_TILE_ROWS / 2; w += 256) L.tile[w] = 0u;
+                    }
+                    if (tid < nc) tlo[tid] = thi[tid];
+                    __syncthreads();
+                }
             }
         }
-        const int pl = popc32(l), pr = popc32(rr);
-        const bool both = isP && rr != 0;
-        const uint64_t Ap = __ballot(isP && pl == N + 1);
-        const uint64_t Dq = __ballot(isQ && pr == N + 1);
-        const uint64_t A = __ballot(both && pl == N + 1), B = __ballot(both && pl == N);
-        const uint64_t C = __ballot(both && pr == N), D = __ballot(both && pr == N + 1);
-        uint64_t Lb = 0, Rb = 0, Lown = 0, Rown = 0;
-        for (int b = 0; b < M; ++b) {
-            const uint64_t lm = __ballot(isP && ((l >> (M - 1 - b)) & 1u));
-            const uint64_t rb = __ballot(both && ((rr >> (M - 1 - b)) & 1u));
-            const uint64_t rq = __ballot(isQ && ((rr >> (M - 1 - b)) & 1u));
-            if (b == b1) Lb = lm;
-            if (b == b2) Rb = rb;
-            if (b == lane) { Lown = lm; Rown = rq; }
-        }
-        if (lane < MM && (A | B | C | D)) {
-            aBl += __popcll(Rb & ((Lb & A) | (~Lb & B)));
-            aBr += __popcll(Lb & ((Rb & D) | (~Rb & C)));
+        if (lane < MM) {
+            if (aBl) atomicAdd(&sBl[lane], aBl);
+            if (aBr) atomicAdd(&sBr[lane], aBr);
         }
         if (lane < M) {
-            aEp += __popcll(Lown & Ap);
-            aEq += __popcll(Rown & Dq);
+            if (aEp) atomicAdd(&sEp[lane], aEp);
+            if (aEq) atomicAdd(&sEq[lane], aEq);
         }
-    };
-    if (total <= HASH_MAX) {
-        const int hb = hash_bits(total);
-        hash_reset(L.h, hb);
         __syncthreads();
-        hash_scatter(L.h, hb, M, cols, pre, 2 * M, total, idx);
-        __syncthreads();
-        // TAB_U entries per thread resolved before their lookups
-        for (int base = 0; base < total; base += 256 * TAB_U) {
-            int tt[TAB_U], rw[TAB_U];
-            table_entries(cols, pre, 2 * M, total, idx, base + tid, 256, tt, rw);
-#pragma unroll
-            for (int u = 0; u < TAB_U; ++u) {
-                const uint32_t h = tt[u] >= 0 ? hash_get(L.h, hb, (uint32_t)rw[u]) : 0u;
-                fold(tt[u], h & 0xFFu, (h >> 8) & 0xFFu);
-            }
-        }
-    } else {
-        // rows [r0, r0 + PAIR_TILE_ROWS) at a time: each column's entries of
-        // a tile are one range of its row-sorted list; the ends of PB tiles
-        // of all 2M columns come from one round of binary searches
-        const int nc = 2 * M;
-        for (int w = tid; w < PAIR_TILE_ROWS / 2; w += 256) L.tile[w] = 0u;
-        if (tid < nc) tlo[tid] = cols[tid].start;
-        const int ntile = (R + PAIR_TILE_ROWS - 1) / PAIR_TILE_ROWS;
-        for (int g0 = 0; g0 < ntile; g0 += PB) {
-            if (tid < nc * PB) {
-                const int t = tid / PB, j = tid % PB;
-                const int64_t r1 = min((int64_t)R, (int64_t)(g0 + j + 1) * PAIR_TILE_ROWS);
-                int lo = cols[t].start, hi = cols[t].start + cols[t].len;
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (idx[mid] < r1) lo = mid + 1;
-                    else hi = mid;
+        if (tid < 64) {
+            int lg = -0x40000000, rg = 0, j = tid;
+            if (tid < MM) {
+                lg = sEp[b1] - sBl[tid];
+                rg = sEq[b2] - sBr[tid];
+                if (full) {
+                    full[(size_t)i * 2 * MM + tid * 2 + 0] = lg;
+                    full[(size_t)i * 2 * MM + tid * 2 + 1] = rg;
                 }
-                tend[t][j] = lo;
             }
-            __syncthreads();
-            for (int j = 0; j < PB && g0 + j < ntile; ++j) {
-                const int r0 = (g0 + j) * PAIR_TILE_ROWS;
-                if (tid == 0) {
-                    tpre[0] = 0;
-                    for (int t = 0; t < nc; ++t) {
-                        thi[t] = tend[t][j];
-                        tpre[t + 1] = tpre[t] + thi[t] - tlo[t];
-                    }
-                }
-                __syncthreads();
-                const int tt = tpre[nc];
-                if (tt > 0) {  // uniform
-                    // TAB_U entries per thread resolved before their loads
-                    auto entries = [&](int e0, int (&t)[TAB_U], int (&r)[TAB_U]) {
-#pragma unroll
-                        for (int u = 0; u < TAB_U; ++u) {
-                            const int e = e0 + u * 256;
-                            t[u] = e < tt ? entry_col(tpre, nc, e) : -1;
-                        }
-#pragma unroll
-                        for (int u = 0; u < TAB_U; ++u)
-                            r[u] = t[u] >= 0 ? idx[tlo[t[u]] + (e0 + u * 256 - tpre[t[u]])] - r0 : 0;
-                    };
-                    for (int e0 = tid; e0 < tt; e0 += 256 * TAB_U) {
-                        int t[TAB_U], r[TAB_U];
-                        entries(e0, t, r);
-#pragma unroll
-                        for (int u = 0; u < TAB_U; ++u)
-                            if (t[u] >= 0)
-                                atomicOr(&L.tile[r[u] >> 1],
-                                         ((1u << (M - 1 - t[u] % M)) << (8 * (t[u] / M))) << (16 * (r[u] & 1)));
-                    }
-                    __syncthreads();
-                    for (int base = 0; base < tt; base += 256 * TAB_U) {
-                        int t[TAB_U], r[TAB_U];
-                        entries(base + tid, t, r);
-#pragma unroll
-                        for (int u = 0; u < TAB_U; ++u) {
-                            const uint32_t h = t[u] >= 0 ? (L.tile[r[u] >> 1] >> (16 * (r[u] & 1))) & 0xFFFFu : 0u;
-                            fold(t[u], h & 0xFFu, h >> 8);
-                        }
-                    }
-                    __syncthreads();
-                    for (int w = tid; w < PAIR_TILE_ROWS / 2; w += 256) L.tile[w] = 0u;
-                }
-                if (tid < nc) tlo[tid] = thi[tid];
-                __syncthreads();
+            int sum = lg + rg;
+            for (int off = 1; off < 64; off <<= 1) {
+                const int os = __shfl_xor(sum, off), org = __shfl_xor(rg, off), oj = __shfl_xor(j, off);
+                const int olg = __shfl_xor(lg, off);
+                const bool take = os > sum || (os == sum && (org > rg || (org == rg && oj < j)));
+                if (take) { sum = os; rg = org; j = oj; lg = olg; }
+            }
+            if (tid == 0) {
+                best[i] = make_int4(j / M, j % M, lg, rg);
+                const int gain = lg + rg;
+                if (gk.ctl)
+                    gk.keys[i] = gain > 0 ? ((uint64_t)(gk.gmax - (uint32_t)gain) << gk.ibits) | (uint32_t)i : ~0ull;
             }
         }
-    }
-    if (lane < MM) {
-        if (aBl) atomicAdd(&sBl[lane], aBl);
-        if (aBr) atomicAdd(&sBr[lane], aBr);
-    }
-    if (lane < M) {
-        if (aEp) atomicAdd(&sEp[lane], aEp);
-        if (aEq) atomicAdd(&sEq[lane], aEq);
-    }
-    __syncthreads();
-    if (tid < 64) {
-        int lg = -0x40000000, rg = 0, j = tid;
-        if (tid < MM) {
-            lg = sEp[b1] - sBl[tid];
-            rg = sEq[b2] - sBr[tid];
-            if (full) {
-                full[(size_t)i * 2 * MM + tid * 2 + 0] = lg;
-                full[(size_t)i * 2 * MM + tid * 2 + 1] = rg;
-            }
-        }
-        int sum = lg + rg;
-        for (int off = 1; off < 64; off <<= 1) {
-            const int os = __shfl_xor(sum, off), org = __shfl_xor(rg, off), oj = __shfl_xor(j, off);
-            const int olg = __shfl_xor(lg, off);
-            const bool take = os > sum || (os == sum && (org > rg || (org == rg && oj < j)));
-            if (take) { sum = os; rg = org; j = oj; lg = olg; }
-        }
-        if (tid == 0) best[i] = make_int4(j / M, j % M, lg, rg);
     }
 }
 
 // ------------------------------------------------------------ selection
-
-// (gain descending, candidate) in gbits + ibits bits: ibits the bits of the
-// largest candidate index, gmax = 2^gbits - 1 at least the largest gain (a
-// gain counts rows of the pair's two segments, each row at most once per
-// segment, so it is at most twice the row count)
-// Keys for the first nkeys slots; slots past this iteration's candidates get
-// the sentinel ~0 (it sorts last), so the sort runs at a size fixed ahead.
-__global__ void k_lp_gain_keys(const LPCtl *__restrict__ ctl, int nkeys, const Cand *__restrict__ cand,
-                               const int4 *__restrict__ best, uint64_t *__restrict__ keys, int ibits,
-                               uint32_t gmax) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nkeys || ctl->done) return;
-    uint64_t key = ~0ull;
-    if (i < ctl->nc) {
-        const int4 b = best[i];
-        const int gain = b.z + b.w;
-        if (cand[i].q >= 0 && gain > 0) key = ((uint64_t)(gmax - (uint32_t)gain) << ibits) | (uint32_t)i;
-    }
-    keys[i] = key;
-}
 
 constexpr int SEL_T = 1024, SEL_B = 1024;
 constexpr int SEL_ROUNDS = 24;                 // parallel rounds before the sequential finish
@@ -1337,7 +1401,8 @@ constexpr int32_t OWNER_NONE = 0x7F7F7F7F;    // empty owner (bytes 0x7F, set by
 __global__ __launch_bounds__(SEL_T) void k_lp_select(LPCtl *ctl, int nseg, const uint64_t *__restrict__ skeys,
                                                      const Cand *__restrict__ cand,
                                                      const int4 *__restrict__ best, int32_t *__restrict__ acc,
-                                                     int32_t *owner, uint64_t imask) {
+                                                     int32_t *owner, uint64_t imask, int mode,
+                                                     int32_t *__restrict__ queue) {
     if (ctl->done) return;
     const int nc = ctl->nc;
     extern __shared__ uint32_t used[];
@@ -1436,10 +1501,7 @@ __global__ __launch_bounds__(SEL_T) void k_lp_select(LPCtl *ctl, int nseg, const
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        ctl->nacc = nacc;
-        ctl->gain = gsum;
-    }
+    if (tid == 0) ctl_accept(ctl, nacc, gsum, mode, queue);
 }
 
 // Apply the accepted swaps (segment-disjoint, so in parallel) and list the
@@ -1572,7 +1634,7 @@ static int lp_prepare(vnm_graph *g, LPCache **out) {
         return rc;
     VNM_HIP_TRY(hipMemsetAsync(nv.p, 0, 4, st));
     if (nnz)
-        hipLaunchKernelGGL(k_lp_adj_keys, dim3(grid_of(nnz, 256, 4096)), dim3(256), 0, st, g->row.p,
+        hipLaunchKernelGGL(k_lp_adj_keys, dim3(grid_of(nnz, 256, 1024)), dim3(256), 0, st, g->row.p,
                            g->col.p, g->val.p, nnz, R, kc.p, kt.p, nv.p);
     g->ctx->launches++;
     VNM_LAUNCH_CHECK("k_lp_adj_keys");
@@ -1611,7 +1673,7 @@ static int lp_stats(vnm_graph *g, LPCache *c, int N, const int32_t *segs, int ns
     hipLaunchKernelGGL(k_lp_seg_stats, dim3(grid), dim3(SS_T), 0, st, g->nrows, g->M, N, c->nseg, segs, nsel,
                        g->inv.p, c->ptr.p, c->idx.p, c->ccls.p, c->segcls.p, c->segnnz.p, g->queue.p, nullptr,
                        nullptr);
-    hipLaunchKernelGGL(k_lp_totals, dim3(1), dim3(1024), 0, st, c->nseg, c->segcls.p, c->tot.p, nullptr);
+    hipLaunchKernelGGL(k_lp_totals, dim3(1), dim3(1024), 0, st, c->nseg, c->segcls.p, c->tot.p, nullptr, 0);
     g->ctx->launches += 2;
     VNM_LAUNCH_CHECK("k_lp_seg_stats");
     return VNM_OK;
@@ -1631,7 +1693,7 @@ static int lp_prepare_bwd(vnm_graph *g, LPCache *c) {
         return rc;
     VNM_HIP_TRY(hipMemsetAsync(nv.p, 0, 4, st));
     if (nnz)
-        hipLaunchKernelGGL(k_lp_adj_keys, dim3(grid_of(nnz, 256, 4096)), dim3(256), 0, st, g->row.p,
+        hipLaunchKernelGGL(k_lp_adj_keys, dim3(grid_of(nnz, 256, 1024)), dim3(256), 0, st, g->row.p,
                            g->col.p, g->val.p, nnz, c->R, kc.p, kt.p, nv.p);
     g->ctx->launches++;
     VNM_LAUNCH_CHECK("k_lp_adj_keys");
@@ -1841,12 +1903,15 @@ struct LPRound {
 
 // Score candidates [0, nc) exactly: a workgroup per candidate.
 // nc candidates, or (d_nc given) the first *d_nc of nc launched blocks.
+constexpr int PAIR_GRID = 4096;  // workgroups of a run's pair scores, at least
+
 static int lp_score_cands(vnm_graph *g, LPCache *c, int N, Cand *cand, int4 *best, int nc, int32_t *full,
-                          const int *d_nc = nullptr) {
+                          const GainKeys &gk = GainKeys{}) {
     if (nc <= 0) return VNM_OK;
+    const int grid = gk.ctl ? std::min(nc, std::max(gk.nnorm, PAIR_GRID)) : nc;
     KernelTimer kt(g->ctx, "k_lp_pair_gain");
-    hipLaunchKernelGGL(k_lp_pair_gain, dim3(nc), dim3(256), 0, g->ctx->stream, d_nc, g->nrows, g->M, N, cand,
-                       g->inv.p, c->ptr.p, c->idx.p, best, full);
+    hipLaunchKernelGGL(k_lp_pair_gain, dim3(grid), dim3(256), 0, g->ctx->stream, nc, g->nrows, g->M, N, cand,
+                       g->inv.p, c->ptr.p, c->idx.p, best, full, gk);
     kt.stop();
     g->ctx->launches++;
     VNM_LAUNCH_CHECK("k_lp_pair_gain");
@@ -1930,7 +1995,9 @@ static int lp_run_begin(LPRun &r, vnm_graph *g, const vnm_lp_model *m, int N, in
 
 // Enqueue one iteration; every kernel reads its sizes and flags from the
 // control block, so nothing here waits for the device.
-static int lp_run_iter(LPRun &r) {
+// exh: the iteration's mode where the host has read it (the other mode's sort,
+// and the exhaustive mode's forward pass, are not enqueued), -1 where it has not.
+static int lp_run_iter(LPRun &r, int exh) {
     vnm_graph *g = r.g;
     LPCache *c = r.c;
     LPRound &w = r.w;
@@ -1938,49 +2005,50 @@ static int lp_run_iter(LPRun &r) {
     hipStream_t st = g->ctx->stream;
     const int ns = r.ns, M = r.M;
     int rc;
-    hipLaunchKernelGGL(k_lp_ctl_begin, dim3(1), dim3(64), 0, st, ctl, r.mode);
-    if (r.mode == 0 && (rc = lp_forward(g, c, r.m, 1, &ctl->skip_fwd))) return rc;
+    if (r.mode == 0 && exh != 1 && (rc = lp_forward(g, c, r.m, 1, &ctl->skip_fwd))) return rc;
     hipLaunchKernelGGL(k_lp_pick, dim3(grid_of(ns, 256)), dim3(256), 0, st, ctl, ns, M, r.mode, r.seed, g->inv.p,
                        c->ptr.p, c->ccls.p, c->segcls.p, c->Y.p, w.dkey.p, w.dkey.p + ns, w.dbest.p, w.abest.p,
                        r.sbits);
     VNM_LAUNCH_CHECK("k_lp_pick");
     if ((rc = sort_keys_u64_if(w.dkey.p, w.sdkey.p, 2 * (int64_t)ns, key_range(r.sbits, 33 + r.sbits), st,
                                &ctl->done))) return rc;
-    hipLaunchKernelGGL(k_lp_ctl_mid, dim3(1), dim3(64), 0, st, ctl, r.topk, r.window, ns);
-    hipLaunchKernelGGL(k_lp_match, dim3(grid_of(r.nnorm, 256)), dim3(256), 0, st, ctl, r.window, ns, M, r.mode,
-                       r.seed, w.sdkey.p, w.sdkey.p + ns, w.dbest.p, w.abest.p, g->inv.p, c->Y.p, w.cand.p, r.smask);
+    hipLaunchKernelGGL(k_lp_match, dim3(grid_of((int64_t)r.nnorm * MATCH_L, 256, 1 << 30)), dim3(256), 0, st, ctl,
+                       r.topk, r.window, ns, M, r.mode, r.seed, w.sdkey.p, w.sdkey.p + ns, w.dbest.p, w.abest.p,
+                       g->inv.p, c->Y.p, w.cand.p, r.smask);
     VNM_LAUNCH_CHECK("k_lp_match");
-    if ((rc = lp_score_cands(g, c, r.N, w.cand.p, w.best.p, r.ncap, nullptr, &ctl->nc))) return rc;
-    hipLaunchKernelGGL(k_lp_gain_keys, dim3(grid_of(r.ncap, 256)), dim3(256), 0, st, ctl, r.ncap, w.cand.p,
-                       w.best.p, w.gkey.p, r.ibits, r.gmax);
+    if ((rc = lp_score_cands(g, c, r.N, w.cand.p, w.best.p, r.ncap, nullptr,
+                             GainKeys{ctl, r.nnorm, r.ncap, w.gkey.p, r.ibits, r.gmax})))
+        return rc;
     // one candidate per donor: the first nnorm keys; the whole window: ncap
     // keys come in candidate order, so the sort leaves their low ibits alone
     const KeyBits kbits = key_range(r.ibits, r.gbits + r.ibits);
-    if (r.mode != 2 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.nnorm, kbits, st, &ctl->skip_norm))) return rc;
-    if (r.mode != 1 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.ncap, kbits, st, &ctl->skip_exh))) return rc;
+    if (r.mode != 2 && exh != 1 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.nnorm, kbits, st, &ctl->skip_norm)))
+        return rc;
+    if (r.mode != 1 && exh != 0 && (rc = sort_keys_u64_if(w.gkey.p, w.sgkey.p, r.ncap, kbits, st, &ctl->skip_exh)))
+        return rc;
     const size_t shm = (size_t)((ns + 31) / 32) * 4;
     hipLaunchKernelGGL(k_lp_select, dim3(1), dim3(SEL_T), shm, st, ctl, ns, w.sgkey.p, w.cand.p, w.best.p,
-                       w.acc.p, w.owner.p, r.imask);
+                       w.acc.p, w.owner.p, r.imask, r.mode, g->queue.p);
     VNM_LAUNCH_CHECK("k_lp_select");
-    hipLaunchKernelGGL(k_lp_ctl_after, dim3(1), dim3(64), 0, st, ctl, r.mode, g->queue.p);
     const int maxsw = std::min(r.ncap, ns);
     hipLaunchKernelGGL(k_lp_swap, dim3(grid_of(maxsw, 256)), dim3(256), 0, st, ctl, M, w.acc.p, w.cand.p,
                        w.best.p, g->perm.p, g->inv.p, w.touched.p);
     hipLaunchKernelGGL(k_lp_seg_stats, dim3(std::max(1, std::min(2 * maxsw, 1024))), dim3(SS_T), 0, st, g->nrows,
                        M, r.N, ns, w.touched.p, 0, g->inv.p, c->ptr.p, c->idx.p, c->ccls.p, c->segcls.p,
                        c->segnnz.p, g->queue.p, &ctl->nsel, &ctl->skip_swap);
-    hipLaunchKernelGGL(k_lp_totals, dim3(1), dim3(1024), 0, st, ns, c->segcls.p, c->tot.p, &ctl->skip_swap);
-    hipLaunchKernelGGL(k_lp_ctl_end, dim3(1), dim3(64), 0, st, ctl, c->tot.p);
-    g->ctx->launches += 11;
-    VNM_LAUNCH_CHECK("k_lp_ctl_end");
+    hipLaunchKernelGGL(k_lp_totals, dim3(1), dim3(1024), 0, st, ns, c->segcls.p, c->tot.p, ctl, r.mode);
+    g->ctx->launches += 6;
+    VNM_LAUNCH_CHECK("k_lp_totals");
     return VNM_OK;
 }
 
-static int lp_run_done(LPRun &r, bool *done) {
-    int32_t d = 0;
-    VNM_HIP_TRY(hipMemcpyAsync(&d, &r.ctl.p->done, 4, hipMemcpyDeviceToHost, r.g->ctx->stream));
+static int lp_run_state(LPRun &r, bool *done, int *exh) {
+    static_assert(offsetof(LPCtl, exh) == offsetof(LPCtl, done) + 4, "read together");
+    int32_t d[2] = {0, 0};
+    VNM_HIP_TRY(hipMemcpyAsync(d, &r.ctl.p->done, 8, hipMemcpyDeviceToHost, r.g->ctx->stream));
     VNM_HIP_TRY(hipStreamSynchronize(r.g->ctx->stream));
-    *done = d != 0;
+    *done = d[0] != 0;
+    *exh = d[1] != 0;
     return VNM_OK;
 }
 
@@ -2019,10 +2087,11 @@ static int lp_reorder_run(vnm_graph *g, const vnm_lp_model *m, int N, int mode, 
     int rc = lp_run_begin(r, g, m, N, mode, topk, window, seed);
     if (rc) return rc;
     bool done = false;
-    if ((rc = lp_run_done(r, &done))) return rc;
+    int exh = 0;
+    if ((rc = lp_run_state(r, &done, &exh))) return rc;
     for (int it = 0; it < maxiter && !done; ++it) {
-        if ((rc = lp_run_iter(r))) return rc;
-        if ((rc = lp_run_done(r, &done))) return rc;
+        if ((rc = lp_run_iter(r, exh))) return rc;
+        if ((rc = lp_run_state(r, &done, &exh))) return rc;
     }
     return lp_run_end(r, stats);
 }
@@ -2034,15 +2103,15 @@ int lp_reorder(vnm_graph *g, const vnm_lp_model *m, int N, int mode, int topk, i
     return lp_reorder_run(g, m, N, mode, topk, window, maxiter, seed, stats);
 }
 
-// The learned reorder of many graphs of one context as one launch chain:
-// one iteration of every graph is captured as a HIP graph -- LP_BRANCHES
-// parallel branches (forked from the context stream inside the capture),
-// the graphs dealt round-robin over them, each branch with its own sort
-// scratch; every kernel reads its sizes and flags from its graph's control
-// block -- and the graph is replayed until every run is over or maxiter
-// iterations have run; the host reads the runs' done flags after each
-// replay and captures again with the running graphs once at most half of
-// the captured ones still run.  A graph's
+// The learned reorder of many graphs of one context: the graphs are dealt
+// round-robin over LP_BRANCHES streams, each with its own sort scratch, and one
+// iteration of a stream's graphs is captured as a HIP graph; every kernel reads
+// its sizes and flags from its graph's control block.  The streams' graphs are
+// replayed side by side until every run is over or maxiter iterations have run;
+// the host reads the runs' done flags after each replay and captures a stream
+// again with its running graphs once at most half of the captured ones still
+// run.  (Each capture is of one stream.  One capture of all, forked over the
+// streams and joined, has ended in a segmentation fault of the host.)  A graph's
 // result is the one lp_reorder makes alone with the same seed: the same
 // kernels take the same decisions.
 constexpr int LP_BRANCHES = 8;
@@ -2063,13 +2132,24 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
     }
     hipStream_t st = ctx->stream;
     const int B = std::min(LP_BRANCHES, count);
-    // branch streams (default priority) and fork/join events, released on
-    // every path; the graphs get their context back on every path
-    struct Res {
-        std::vector<vnm_ctx> aux;
-        std::vector<hipEvent_t> ev;
+    // branch streams (default priority) and their captured iterations, released
+    // on every path; the graphs get their context back on every path
+    struct Branch {
+        vnm_ctx aux;
+        std::vector<int> act;  // its graphs that still run
+        size_t captured = 0;   // and how many the captured iteration holds
+        int off = 0, n = 0;    // its graphs' control blocks and flags
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
+        void drop() {
+            if (exec) (void)hipGraphExecDestroy(exec);
+            if (graph) (void)hipGraphDestroy(graph);
+            exec = nullptr;
+            graph = nullptr;
+        }
+    };
+    struct Res {
+        std::vector<Branch> br;
         vnm_graph *const *gs = nullptr;
         int count = 0;
         vnm_ctx *ctx = nullptr;
@@ -2077,44 +2157,47 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
         ~Res() {
             for (int i = 0; i < count; ++i) gs[i]->ctx = ctx;
             (void)sort_scratch_slot(slot);
-            if (exec) (void)hipGraphExecDestroy(exec);
-            if (graph) (void)hipGraphDestroy(graph);
-            for (auto e : ev) (void)hipEventDestroy(e);
-            for (auto &x : aux)
-                if (x.stream) {
-                    (void)hipStreamSynchronize(x.stream);
-                    (void)hipStreamDestroy(x.stream);
-                }
+            for (auto &b : br)
+                if (b.aux.stream) (void)hipStreamSynchronize(b.aux.stream);
+            for (auto &b : br) {
+                b.drop();
+                if (b.aux.stream) (void)hipStreamDestroy(b.aux.stream);
+            }
         }
     } res;
     res.gs = gs;
     res.count = count;
     res.ctx = ctx;
     res.slot = sort_scratch_slot(0);
-    res.aux.resize(B);
-    for (int b = 0; b < B; ++b) {
-        res.aux[b].device = ctx->device;
-        hipError_t e = hipStreamCreateWithFlags(&res.aux[b].stream, hipStreamNonBlocking);
+    res.br.resize(B);
+    for (auto &b : res.br) {
+        b.aux.device = ctx->device;
+        hipError_t e = hipStreamCreateWithFlags(&b.aux.stream, hipStreamNonBlocking);
         if (e != hipSuccess) {
-            res.aux[b].stream = nullptr;
+            b.aux.stream = nullptr;
             return set_error(VNM_E_HIP, "hipStreamCreate failed: %s", hipGetErrorString(e));
         }
-    }
-    for (int k = 0; k < B + 1; ++k) {
-        hipEvent_t e = nullptr;
-        VNM_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        res.ev.push_back(e);
     }
     // per graph: cache, buffers, control block (on the context stream), sort
     // scratch reserved in its branch's slot
     std::vector<LPRun> runs(count);
-    std::vector<LPCtl *> hctl(count);
     int rc;
     for (int i = 0; i < count; ++i) {
         (void)sort_scratch_slot(i % B);
         if ((rc = lp_run_begin(runs[i], gs[i], m, N, mode, topk, window, seed)))
             return set_error(rc, "graph %d: %s", i, last_error());
-        hctl[i] = runs[i].ctl.p;
+        res.br[i % B].act.push_back(i);
+    }
+    // control blocks and flags, branch by branch: graph i is entry at[i]
+    std::vector<LPCtl *> hctl;
+    std::vector<int> at(count);
+    for (auto &b : res.br) {
+        b.off = (int)hctl.size();
+        b.n = (int)b.act.size();
+        for (int i : b.act) {
+            at[i] = (int)hctl.size();
+            hctl.push_back(runs[i].ctl.p);
+        }
     }
     DBuf<LPCtl *> dctl;
     DBuf<int32_t> dflags;
@@ -2122,80 +2205,72 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
     VNM_HIP_TRY(hipMemcpyAsync(dctl.p, hctl.data(), count * sizeof(LPCtl *), hipMemcpyHostToDevice, st));
     std::vector<int32_t> done(count, 0);
     VNM_HIP_TRY(hipStreamSynchronize(st));
-    // capture one iteration of the graphs in `act` (no event timing inside)
-    auto capture = [&](const std::vector<int> &act) -> int {
-        if (res.exec) (void)hipGraphExecDestroy(res.exec);
-        if (res.graph) (void)hipGraphDestroy(res.graph);
-        res.exec = nullptr;
-        res.graph = nullptr;
-        const bool timing = ctx->timing;
-        ctx->timing = false;
-        hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-        if (e != hipSuccess) {
-            ctx->timing = timing;
+    // capture one iteration of a branch's running graphs and their flags
+    auto capture = [&](int bi) -> int {
+        Branch &b = res.br[bi];
+        b.drop();
+        hipError_t e = hipStreamBeginCapture(b.aux.stream, hipStreamCaptureModeThreadLocal);
+        if (e != hipSuccess)
             return set_error(VNM_E_HIP, "capture of the learned iteration failed: %s", hipGetErrorString(e));
-        }
         int rc = VNM_OK;
-        // the branches the running graphs use join the capture (a stream
-        // that did not would run its kernels at once instead of recording)
-        std::vector<char> used(B, 0);
-        for (int i : act) used[i % B] = 1;
-        if (hipEventRecord(res.ev[B], st) != hipSuccess) rc = set_error(VNM_E_HIP, "fork event failed");
-        for (int b = 0; b < B && rc == VNM_OK; ++b)
-            if (used[b] && hipStreamWaitEvent(res.aux[b].stream, res.ev[B], 0) != hipSuccess)
-                rc = set_error(VNM_E_HIP, "fork failed");
-        for (size_t k = 0; k < act.size() && rc == VNM_OK; ++k) {
-            const int i = act[k], b = i % B;  // a graph keeps its branch: its sort scratch slot
-            (void)sort_scratch_slot(b);
-            gs[i]->ctx = &res.aux[b];
-            rc = lp_run_iter(runs[i]);
+        (void)sort_scratch_slot(bi);
+        for (size_t k = 0; k < b.act.size() && rc == VNM_OK; ++k) {
+            const int i = b.act[k];
+            gs[i]->ctx = &b.aux;  // no event timing inside
+            rc = lp_run_iter(runs[i], -1);
             gs[i]->ctx = ctx;
-            ctx->launches += res.aux[b].launches;
-            res.aux[b].launches = 0;
         }
-        for (int b = 0; b < B && rc == VNM_OK; ++b)
-            if (used[b] && (hipEventRecord(res.ev[b], res.aux[b].stream) != hipSuccess ||
-                            hipStreamWaitEvent(st, res.ev[b], 0) != hipSuccess))
-                rc = set_error(VNM_E_HIP, "join failed");
-        if (rc == VNM_OK) hipLaunchKernelGGL(k_lp_done_flags, dim3(1), dim3(256), 0, st, dctl.p, count, dflags.p);
-        e = hipStreamEndCapture(st, &res.graph);
-        ctx->timing = timing;
+        ctx->launches += b.aux.launches;
+        b.aux.launches = 0;
+        if (rc == VNM_OK)
+            hipLaunchKernelGGL(k_lp_done_flags, dim3(1), dim3(256), 0, b.aux.stream, dctl.p + b.off, b.n,
+                               dflags.p + b.off);
+        e = hipStreamEndCapture(b.aux.stream, &b.graph);
         if (rc) return rc;
         if (e != hipSuccess)
             return set_error(VNM_E_HIP, "capture of the learned iteration failed: %s", hipGetErrorString(e));
-        e = hipGraphInstantiate(&res.exec, res.graph, nullptr, nullptr, 0);
+        e = hipGraphInstantiate(&b.exec, b.graph, nullptr, nullptr, 0);
         if (e != hipSuccess)
             return set_error(VNM_E_HIP, "instantiating the learned iteration failed: %s", hipGetErrorString(e));
+        b.captured = b.act.size();
         return VNM_OK;
     };
-    // replay; once at most half of the captured graphs still run, capture
-    // again with those only (a finished graph's kernels would all return at
+    // replay; once at most half of a branch's captured graphs still run, capture
+    // it again with those only (a finished graph's kernels would all return at
     // once, but each still costs a launch)
-    std::vector<int> act;
-    for (int i = 0; i < count; ++i) act.push_back(i);
-    size_t captured = 0;
     const bool dbg = getenv("VNM_DEBUG") != nullptr;
     auto tnow = [] { return std::chrono::steady_clock::now(); };
     auto tms = [](std::chrono::steady_clock::time_point a, std::chrono::steady_clock::time_point b) {
         return std::chrono::duration<double, std::milli>(b - a).count();
     };
     auto tb = tnow();
-    for (int it = 0; it < maxiter && !act.empty(); ++it) {
-        if (2 * act.size() <= captured || captured == 0) {
-            auto tc = tnow();
-            if ((rc = capture(act))) return rc;
-            captured = act.size();
-            if (dbg)
-                fprintf(stderr, "[vnm] lp batch: iteration %d, capture of %zu graphs %.2f ms (%.2f ms so far)\n", it,
-                        captured, tms(tc, tnow()), tms(tb, tnow()));
+    for (int it = 0; it < maxiter; ++it) {
+        bool any = false;
+        for (int bi = 0; bi < B; ++bi) {
+            Branch &b = res.br[bi];
+            if (b.act.empty()) continue;
+            any = true;
+            if (2 * b.act.size() <= b.captured || !b.exec) {
+                if ((rc = capture(bi))) return rc;
+                if (dbg)
+                    fprintf(stderr, "[vnm] lp batch: iteration %d, branch %d captured with %zu graphs (%.2f ms so far)\n",
+                            it, bi, b.captured, tms(tb, tnow()));
+            }
+            VNM_HIP_TRY(hipGraphLaunch(b.exec, b.aux.stream));
         }
-        VNM_HIP_TRY(hipGraphLaunch(res.exec, st));
-        VNM_HIP_TRY(hipMemcpyAsync(done.data(), dflags.p, count * 4, hipMemcpyDeviceToHost, st));
-        VNM_HIP_TRY(hipStreamSynchronize(st));
-        std::vector<int> next;
-        for (int i : act)
-            if (!done[i]) next.push_back(i);
-        act.swap(next);
+        if (!any) break;
+        for (auto &b : res.br)
+            if (!b.act.empty())
+                VNM_HIP_TRY(hipMemcpyAsync(done.data() + b.off, dflags.p + b.off, b.n * 4, hipMemcpyDeviceToHost,
+                                           b.aux.stream));
+        for (auto &b : res.br) {
+            if (b.act.empty()) continue;
+            VNM_HIP_TRY(hipStreamSynchronize(b.aux.stream));
+            std::vector<int> next;
+            for (int i : b.act)
+                if (!done[at[i]]) next.push_back(i);
+            b.act.swap(next);
+        }
     }
     if (dbg) fprintf(stderr, "[vnm] lp batch: iterations done %.2f ms\n", tms(tb, tnow()));
     for (int i = 0; i < count; ++i)
@@ -2380,7 +2455,6 @@ int vnm_lp_reorder(vnm_graph *g, const vnm_lp_model *m, int N, int mode, int top
 int vnm_lp_reorder_batch(vnm_graph *const *graphs, int count, const vnm_lp_model *m, int N, int mode, int topk,
                          int window, int maxiter, uint64_t seed, vnm_lp_stats *st) {
     if (!graphs || !st) return set_error(VNM_E_ARG, "bad arguments");
-    PoolScope pool(count > 0 && graphs[0] ? graphs[0]->ctx->pool : nullptr);
     return lp_reorder_batch(graphs, count, m, N, mode, topk, window, maxiter, seed, st);
 }
 
