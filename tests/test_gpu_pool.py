@@ -15,9 +15,9 @@ SIZES = [(300, 4), (4096, 12), (900, 6), (5000, 9), (300, 4), (4096, 12)]
 
 def product(ctx, p, n, B):
     C = torch.full((n, 64), float("nan"), device="cuda")
-    torch.cuda.synchronize()
+    torch.cuda.current_stream().synchronize()
     p.spmm(B.data_ptr(), 64, 64, vnm.DT_F32, C.data_ptr(), 64)
-    torch.cuda.synchronize()
+    torch.cuda.ExternalStream(ctx.stream).synchronize()
     return C.cpu().numpy()
 
 
@@ -26,6 +26,7 @@ def call(ctx, n, deg, keep):
     r = rng.integers(0, n, n * deg).astype(np.int32)
     c = rng.integers(0, n, n * deg).astype(np.int32)
     m = vnm.coo_from_tuples(n, n, r, c, rng.uniform(-1, 1, n * deg).astype(np.float32), 8)
+    n = -(-n // 8) * 8  # the operand and the result have the padded rows
     B = torch.from_numpy(rng.standard_normal((n, 64)).astype(np.float32)).cuda()
     g = vnm.Graph(ctx, m, 8)
     g.lp_reorder(None, 2, mode=vnm.LP_EXHAUSTIVE, maxiter=3)
