@@ -234,46 +234,6 @@ static int batch_create(vnm_ctx *ctx, vnm_packed *const *ps, int count, const vo
 
 // ------------------------------------------------------------ GCN layer
 
-// Wt[N x K] = W[K x N]^T (BF16), so that the GEMM's LDS stage is a plain
-// 16-byte copy.  Tiles of 64 x 64 through LDS, both sides coalesced.
-__global__ __launch_bounds__(256) void k_transpose_w(int K, int N, const uint16_t *__restrict__ W,
-                                                     uint16_t *__restrict__ Wt) {
-    __shared__ uint16_t t[64][65];
-    const int k0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int r = i / 64, c = i % 64;
-        if (k0 + r < K && n0 + c < N) t[r][c] = W[(size_t)(k0 + r) * N + n0 + c];
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 64 * 64; i += 256) {
-        const int r = i / 64, c = i % 64;  // r: column of W, c: k
-        if (n0 + r < N && k0 + c < K) Wt[(size_t)(n0 + r) * K + k0 + c] = t[c][r];
-    }
-}
-
-// H[R x N] (BF16) = X[R x K] (BF16, leading dimension ldx) W[K x N], with
-// W given transposed (Wt, N x K); K a multiple of 16, N of 64.  A workgroup
-// takes RT row tiles of 128 rows of one XCD for one 64-column panel; a wave
-// computes 32 rows x 64 columns of each (two row fragments share every W
-// fragment), GK k at a time.  Wt's 64-row panel is staged in LDS (rows
-// padded by 16 bytes, so the 16 lanes reading one k range hit different
-// banks), once per workgroup when K <= GK.  gfx950's v_mfma_f32_16x16x32_bf16
-// takes the W fragment as its first operand (lane l: column n = l%16 of the
-// panel, k 8(l/16)..+7) and the X fragment as its second (row l%16, the same
-// k), so it produces H transposed: lane l ends with 4 consecutive columns of
-// one row, stored as 8 bytes.  In step s lane group g = l/16 takes k
-// 32s + 8g .. +7, so one load covers 64 contiguous bytes of each of 16 rows;
-// a tile's loads are all issued before its first MFMA, and the X loads of
-// the first tile are in flight while the panel is staged (the barriers wait
-// for LDS only).  Groups past the stage's k count (a K that is an odd
-// multiple of 16) hold zeros in both operands.  The N/64 column panels of
-// a row tile are consecutive workgroups of one XCD, so the X tile is fetched
-// from HBM once and hit in that XCD's L2 by the other panels.
-constexpr int GK = 256;
-constexpr int GKP = GK + 8;
-constexpr int GS = GK / 32;  // MFMA steps of a full stage
-constexpr int GCP = 64 * (GK / 8) / 256;  // 16-byte panel copies per thread and stage
-
 // A barrier for LDS data only: pending global loads stay in flight.
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -288,107 +248,162 @@ __device__ __forceinline__ uint32_t bf16_bits(float f) {
     return (u & 0x7FFFFFFFu) > 0x7F800000u ? ((u >> 16) | 0x40u) : r;
 }
 
-__global__ __launch_bounds__(256) void k_gemm_xw(int R, int K, int N, const uint16_t *__restrict__ X, int ldx,
-                                                 const uint16_t *__restrict__ Wt, uint16_t *__restrict__ H,
-                                                 int RT) {
-    typedef short bf16x4_t __attribute__((ext_vector_type(4)));
+// H[R x N] (BF16) = X[R x K] (BF16, leading dimension ldx) W[K x N]; K a multiple
+// of 16, N of 64.  A workgroup of four waves takes a tile of 64 HF rows, 16 HF a
+// wave, and 64-column panels of W: blockIdx.y, + gridDim.y, ...  With K <= GKT
+// (every row of X fits the wave's registers) X is read once for all of them.
+// Bound by X and H in memory (R 65,536, K = N = 256: 67 MB in 22.3 us, 3.0 TB/s of
+// a copy's 4.9: reading, then multiplying and writing, in step over the chip; 30 us
+// with X read once a panel and W transposed by a launch of its own, 7.5 us).
+//
+// The panel lies transposed in LDS, K-contiguous per column, for 16-byte reads of
+// 8 k: a thread loads two columns' 8 k as eight words, straight from W, and packs
+// them into two 16-byte writes; the next panel's words are in flight while the
+// current one is multiplied, and go to the other half of the LDS buffer.
+// gfx950's v_mfma_f32_16x16x32_bf16 takes the W fragment as its first operand
+// (lane l: row l%16 of the fragment, k 8(l/16)..+7) and the X fragment as its
+// second (row l%16, the same k), so it produces H transposed: lane l holds rows
+// 4(l/16)..+3 of the W fragment for one row of X.  Row 4g + i of fragment nt is
+// column 16g + 4nt + i of the panel, so that a lane's four fragments are 16
+// consecutive columns, stored as two 16-byte pieces.  LDS rows are padded by 16
+// bytes and the 16-byte chunks of fragment nt's rows exchanged by 4nt, which keeps
+// both the fragment reads and the transposing writes off each other's banks.
+// In step s lane group g = l/16 takes k 32s + 8g .. +7; where K is an odd
+// multiple of 16, the last step's upper groups hold zeros in both operands.
+constexpr int GEMM_WG = 256;
+constexpr int GEMM_K = 256;  // k of a stage
+
+template <int GKT>
+struct GemmStage {  // two columns x 8 k each, of up to GKT k
+    static constexpr int PT = (GKT / 8) * 32 / GEMM_WG;
+    uint32_t r[PT][8];
+    __device__ __forceinline__ void load(const uint16_t *__restrict__ W, int N, int n0, int kn) {
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const int i = threadIdx.x + GEMM_WG * j, c = i % 32, k = min(i / 32 * 8, kn - 8);
+#pragma unroll
+            for (int q = 0; q < 8; ++q)  // W may be 2-byte aligned
+                __builtin_memcpy(&r[j][q], W + (size_t)(k + q) * N + n0 + 2 * c, 4);
+        }
+    }
+    __device__ __forceinline__ void store(uint16_t *w, int kn) const {
+        const int kr = (kn + 31) / 32 * 32;  // zeros up to the last step's end
+#pragma unroll
+        for (int j = 0; j < PT; ++j) {
+            const int i = threadIdx.x + GEMM_WG * j, c = i % 32 * 2, kb = i / 32;
+            if (kb * 8 >= kr) continue;
+            const bool live = kb * 8 < kn;
+            uint32_t lo[4], hi[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                lo[q] = live ? __builtin_amdgcn_perm(r[j][2 * q + 1], r[j][2 * q], 0x05040100u) : 0u;
+                hi[q] = live ? __builtin_amdgcn_perm(r[j][2 * q + 1], r[j][2 * q], 0x07060302u) : 0u;
+            }
+            const int nt = (c >> 2) & 3, row = nt * 16 + (c >> 4) * 4 + (c & 3);
+            uint16_t *d = w + row * (GKT + 8) + ((kb ^ (4 * nt)) * 8);
+            *(uint4 *)d = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            *(uint4 *)(d + GKT + 8) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+        }
+    }
+};
+
+template <int HF, int GKT>
+__global__ __launch_bounds__(GEMM_WG) void k_gemm_xw(int R, int K, int N, const uint16_t *__restrict__ X, int ldx,
+                                                     const uint16_t *__restrict__ W, uint16_t *__restrict__ H) {
     typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
     typedef float f32x4_t __attribute__((ext_vector_type(4)));
-    __shared__ __align__(16) uint16_t w[64 * GKP];
+    constexpr int GS = GKT / 32, BUF = 64 * (GKT + 8);
+    __shared__ __align__(16) uint16_t w[2 * BUF];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // workgroups are dealt round-robin over the 8 XCDs: b -> XCD b % 8
-    const int P = N / 64;
-    const int xcd = blockIdx.x % 8, jx = blockIdx.x / 8;
-    const int panel = jx % P, tgroup = jx / P;
-    const int n0 = panel * 64;
     const int m = lane & 15, g = lane >> 4;
-    const bool once = K <= GK;  // the whole panel fits one stage: staged once
-    if (once) {
-        if (K == GK) {  // every copy's load issued first
-            uint4 cp[GCP];
+    const int r0 = (blockIdx.x * 4 + wv) * 16 * HF;
+    const int P = N / 64;
+    const bool once = K <= GKT;
+    bf16x8_t a[HF][GS];
+    auto load_x = [&](int kc, int kn) {
 #pragma unroll
-            for (int j = 0; j < GCP; ++j) {
-                const int i = threadIdx.x + 256 * j;
-                cp[j] = *(const uint4 *)(Wt + (size_t)(n0 + i / (GK / 8)) * K + (i % (GK / 8)) * 8);
-            }
+        for (int h = 0; h < HF; ++h) {
+            const uint16_t *xp = X + (size_t)min(r0 + h * 16 + m, R - 1) * ldx + kc;
 #pragma unroll
-            for (int j = 0; j < GCP; ++j) {
-                const int i = threadIdx.x + 256 * j;
-                *(uint4 *)&w[(i / (GK / 8)) * GKP + (i % (GK / 8)) * 8] = cp[j];
+            for (int st = 0; st < GS; ++st) {
+                if (32 * st >= kn) break;
+                const int k0 = 32 * st + 8 * g;
+                uint4 v;
+                __builtin_memcpy(&v, __builtin_assume_aligned(xp + min(k0, kn - 8), 8), 16);
+                if (k0 >= kn) v = make_uint4(0u, 0u, 0u, 0u);
+                a[h][st] = __builtin_bit_cast(bf16x8_t, v);
             }
-        } else {
-            const int per_row = K / 8;
-            for (int i = threadIdx.x; i < 64 * per_row; i += 256)
-                *(uint4 *)&w[(i / per_row) * GKP + (i % per_row) * 8] =
-                    *(const uint4 *)(Wt + (size_t)(n0 + i / per_row) * K + (i % per_row) * 8);
         }
-        lds_barrier();
-    }
-    for (int t = 0; t < RT; ++t) {
-        const int tile = (tgroup * RT + t) * 8 + xcd;
-        const int r0 = (tile * 4 + wv) * 32;
-        if (once && (tile * 4) * 32 >= R) break;  // workgroup-uniform: no later tile has rows
-        f32x4_t acc[2][4];
+    };
+    f32x4_t acc[HF][4];
+    auto clear = [&] {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < HF; ++h)
 #pragma unroll
             for (int nt = 0; nt < 4; ++nt) acc[h][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        for (int kc = 0; kc < K; kc += GK) {
-            const int kn = min(GK, K - kc);  // a multiple of 16
-            const int S = (kn + 31) / 32;    // steps of 32 k
-            bf16x8_t a[2][GS];
+    };
+    auto multiply = [&](const uint16_t *wb, int kn) {
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int row = r0 + h * 16 + m;
+        for (int st = 0; st < GS; ++st) {
+            if (32 * st >= kn) break;
 #pragma unroll
-                for (int st = 0; st < GS; ++st) {
-                    bf16x4_t lo = bf16x4_t{0, 0, 0, 0}, hi = bf16x4_t{0, 0, 0, 0};
-                    const int k0 = 32 * st + 8 * g;
-                    if (st < S && k0 < kn && row < R) {
-                        const uint16_t *xp = X + (size_t)row * ldx + kc + k0;
-                        lo = *(const bf16x4_t *)xp;  // ldx % 4 == 0: 8-byte aligned
-                        hi = *(const bf16x4_t *)(xp + 4);
-                    }
-                    a[h][st] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                }
-            }
-            if (!once) {  // this chunk of the panel, after its earlier readers
-                const int per_row = kn / 8;
-                lds_barrier();
-                for (int i = threadIdx.x; i < 64 * per_row; i += 256)
-                    *(uint4 *)&w[(i / per_row) * GKP + (i % per_row) * 8] =
-                        *(const uint4 *)(Wt + (size_t)(n0 + i / per_row) * K + kc + (i % per_row) * 8);
-                lds_barrier();
-            }
-            if (r0 < R) {
+            for (int nt = 0; nt < 4; ++nt) {
+                const bf16x8_t b = *(const bf16x8_t *)&wb[(nt * 16 + m) * (GKT + 8) + ((4 * st + g) ^ (4 * nt)) * 8];
 #pragma unroll
-                for (int st = 0; st < GS; ++st) {
-                    if (st >= S) break;
-                    const int k0 = 32 * st + 8 * g;
-                    const bool live = k0 < kn;
-#pragma unroll
-                    for (int nt = 0; nt < 4; ++nt) {
-                        bf16x8_t bb = bf16x8_t{};
-                        if (live) bb = *(const bf16x8_t *)&w[(nt * 16 + m) * GKP + k0];
-#pragma unroll
-                        for (int h = 0; h < 2; ++h)
-                            acc[h][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bb, a[h][st], acc[h][nt], 0, 0, 0);
-                    }
-                }
+                for (int h = 0; h < HF; ++h)
+                    acc[h][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[h][st], acc[h][nt], 0, 0, 0);
             }
         }
-        // lane (m, g): row r0 + 16h + m, columns n0 + 16nt + 4g .. +3
+    };
+    // lane (m, g): row r0 + 16h + m, columns n0 + 16g .. +15
+    auto store_h = [&](int n0) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < HF; ++h) {
             const int rr = r0 + h * 16 + m;
-            if (rr < R) {
+            if (rr >= R) continue;
+            uint32_t v[8];
 #pragma unroll
-                for (int nt = 0; nt < 4; ++nt) {
-                    const uint2 v = make_uint2(bf16_bits(acc[h][nt][0]) | (bf16_bits(acc[h][nt][1]) << 16),
-                                               bf16_bits(acc[h][nt][2]) | (bf16_bits(acc[h][nt][3]) << 16));
-                    *(uint2 *)(H + (size_t)rr * N + n0 + nt * 16 + g * 4) = v;
-                }
+            for (int nt = 0; nt < 4; ++nt) {
+                v[2 * nt] = bf16_bits(acc[h][nt][0]) | (bf16_bits(acc[h][nt][1]) << 16);
+                v[2 * nt + 1] = bf16_bits(acc[h][nt][2]) | (bf16_bits(acc[h][nt][3]) << 16);
             }
+            uint4 *d = (uint4 *)(H + (size_t)rr * N + n0 + 16 * g);
+            d[0] = make_uint4(v[0], v[1], v[2], v[3]);
+            d[1] = make_uint4(v[4], v[5], v[6], v[7]);
+        }
+    };
+    GemmStage<GKT> sg;
+    if (once) {
+        int p = blockIdx.y, cur = 0;
+        sg.load(W, N, p * 64, K);
+        load_x(0, K);
+        sg.store(w, K);
+        lds_barrier();
+        for (; p < P; p += gridDim.y) {
+            const int np = p + gridDim.y;
+            if (np < P) sg.load(W, N, np * 64, K);
+            clear();
+            multiply(w + cur * BUF, K);
+            store_h(p * 64);
+            if (np < P) {
+                cur ^= 1;
+                sg.store(w + cur * BUF, K);
+                lds_barrier();
+            }
+        }
+    } else {
+        for (int p = blockIdx.y; p < P; p += gridDim.y) {
+            clear();
+            for (int kc = 0; kc < K; kc += GKT) {
+                const int kn = min(GKT, K - kc);  // a multiple of 16
+                sg.load(W + (size_t)kc * N, N, p * 64, kn);
+                load_x(kc, kn);
+                lds_barrier();  // the chunk before has been read
+                sg.store(w, kn);
+                lds_barrier();
+                multiply(w, kn);
+            }
+            store_h(p * 64);
         }
     }
 }
@@ -403,25 +418,26 @@ static int gcn_layer(vnm_packed *p, const uint16_t *X, int ldx, int K, const uin
     const int R = p->ncols;  // X W has one row per column of A
     hipStream_t st = p->ctx->stream;
     int rc;
-    if (p->gcn_h.n < (size_t)R * N + (size_t)K * N) {  // X W, then W transposed
+    if (p->gcn_h.n < (size_t)R * N) {
         p->gcn_h.release();
-        if ((rc = p->gcn_h.alloc((size_t)R * N + (size_t)K * N))) return rc;
+        if ((rc = p->gcn_h.alloc((size_t)R * N))) return rc;
     }
-    uint16_t *Wt = p->gcn_h.p + (size_t)R * N;  // 16-byte aligned: R * N is a multiple of 64
-    hipLaunchKernelGGL(k_transpose_w, dim3((K + 63) / 64, N / 64), dim3(256), 0, st, K, N, W, Wt);
-    p->ctx->launches++;
-    VNM_LAUNCH_CHECK("k_transpose_w");
     KernelTimer kt(p->ctx, "k_gemm_xw");
-    // row tiles of 128 per XCD, RT of them per workgroup and column panel:
-    // about 4 workgroups per CU, so each stages its W panel once for RT tiles
+    // Tiles of 128 rows share every W fragment between two X fragments; 64-row ones
+    // where 128-row tiles and panels are fewer workgroups than CUs (R 3,008, N 256:
+    // 6.0 us against 7.2; equal at 8,192).  A workgroup takes every panel, X read
+    // once, where the row tiles alone give each CU one (R 65,536: 22.3 us against
+    // 33.2 with a panel each; 32,768: 18.6 against 23.1; 16,384: 18.0 against 14.2).
     int ncu = 0;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, p->ctx->device) != hipSuccess || ncu < 8)
         ncu = 8;
-    const int P = N / 64;
-    const int tiles_x = ((R + 127) / 128 + 7) / 8;  // row tiles per XCD
-    const int RT = K <= GK ? std::max(1, std::min(tiles_x, tiles_x * P * 8 / (4 * ncu))) : 1;
-    const int groups = (tiles_x + RT - 1) / RT;
-    hipLaunchKernelGGL(k_gemm_xw, dim3(8 * P * groups), dim3(256), 0, st, R, K, N, X, ldx, Wt, p->gcn_h.p, RT);
+    const int P = N / 64, tiles = (R + 127) / 128;
+    if ((int64_t)tiles * P < ncu)
+        hipLaunchKernelGGL((k_gemm_xw<1, GEMM_K>), dim3((R + 63) / 64, P), dim3(GEMM_WG), 0, st, R, K, N, X, ldx, W,
+                           p->gcn_h.p);
+    else
+        hipLaunchKernelGGL((k_gemm_xw<2, GEMM_K>), dim3(tiles, K <= GEMM_K && tiles >= ncu ? 1 : P), dim3(GEMM_WG), 0,
+                           st, R, K, N, X, ldx, W, p->gcn_h.p);
     kt.stop();
     p->ctx->launches++;
     VNM_LAUNCH_CHECK("k_gemm_xw");
