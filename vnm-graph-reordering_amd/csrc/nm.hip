@@ -1237,7 +1237,9 @@ __global__ __launch_bounds__(GT) void k_gr_init(NMArgs A, int R, int M, int N, i
         st->round = 1; st->L = sL; st->totcnt = sC;
         st->init_size = sL; st->init_cnt = sC;
         st->maxiter = maxiter > sL ? maxiter : sL;
-        st->status = 0; st->done = 0; st->pending = 0;
+        // a run whose list is too short for a first round is over (k_gr_select's rule)
+        st->status = 0; st->pending = 0;
+        st->done = !(1 <= max(maxiter, sL) && 1 <= round_cap && sL >= (sched >= 8 ? 2 : 1));
         st->K = 0; st->self_pair = 0; st->size1 = 0;
         st->trace_len = 0; st->work = 0;
         st->S.K = 0; st->S.total = 0; st->S.cb[0] = 0;
@@ -1581,11 +1583,24 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
     }
     ctx->launches += G;
     VNM_LAUNCH_CHECK("k_gr_init");
-    // rounds run in captured batches of ROUND_BATCH; the kernels of rounds
-    // past a graph's end return at entry
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    if (G == 1) {
+    // Rounds run in captured batches of ROUND_BATCH; the kernels of rounds past a
+    // graph's end return at entry.  Many runs have no round at all (the later
+    // steps of the hybrid find nothing invalid): those are seen before the first
+    // batch, whose 112 launches they paid for nothing.
+    struct Drop {
+        hipGraph_t g = nullptr;
+        hipGraphExec_t e = nullptr;
+        ~Drop() {
+            if (e) (void)hipGraphExecDestroy(e);
+            if (g) (void)hipGraphDestroy(g);
+        }
+    } drop;
+    auto rounds = [&](hipGraphExec_t *exec) -> int {
+        if (G > 1) {
+            const int rc = capture_rounds(st, hargs[0], d_args, G, gpx, d_flag, &drop.g, &drop.e);
+            *exec = drop.e;
+            return rc;
+        }
         // the captured rounds hold the arguments by value: capture again when
         // they changed (a reload that shrinks the rows moves records B)
         vnm_graph *g0 = gs[0];
@@ -1598,23 +1613,21 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
             g0->nm_graph = nullptr;
         }
         if (!g0->nm_exec) {
-            if ((rc = capture_rounds(st, hargs[0], d_args, 1, gpx, d_flag, &g0->nm_graph, &g0->nm_exec)))
-                return rc;
+            const int rc = capture_rounds(st, hargs[0], d_args, 1, gpx, d_flag, &g0->nm_graph, &g0->nm_exec);
+            if (rc) return rc;
             g0->nm_key.assign(key, key + sizeof(NMArgs));
         }
-        exec = g0->nm_exec;
-    } else if ((rc = capture_rounds(st, hargs[0], d_args, G, gpx, d_flag, &graph, &exec))) {
-        return rc;
-    }
-    struct Drop {
-        hipGraph_t g;
-        hipGraphExec_t e;
-        ~Drop() {
-            if (e) (void)hipGraphExecDestroy(e);
-            if (g) (void)hipGraphDestroy(g);
-        }
-    } drop{graph, G == 1 ? nullptr : exec};
+        *exec = g0->nm_exec;
+        return VNM_OK;
+    };
+    hipLaunchKernelGGL(k_gr_alldone, dim3(1), dim3(64), 0, st, d_args, G, d_flag);
+    ctx->launches++;
+    VNM_LAUNCH_CHECK("k_gr_alldone");
     int32_t done = 0;
+    VNM_HIP_TRY(hipMemcpyAsync(&done, d_flag, 4, hipMemcpyDeviceToHost, st));
+    VNM_HIP_TRY(hipStreamSynchronize(st));
+    hipGraphExec_t exec = nullptr;
+    if (!done && (rc = rounds(&exec))) return rc;
     while (!done) {
         VNM_HIP_TRY(hipGraphLaunch(exec, st));
         ctx->launches += 7 * ROUND_BATCH + 1;

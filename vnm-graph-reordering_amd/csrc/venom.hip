@@ -61,7 +61,7 @@ __global__ void k_run_heads(const uint64_t *__restrict__ k, int64_t nnz, int M,
 __global__ void k_run_fill(const uint64_t *__restrict__ k, const int32_t *__restrict__ head,
                            const int32_t *__restrict__ excl, int64_t nnz, int M,
                            uint32_t *__restrict__ bits, int32_t *__restrict__ rrow,
-                           int32_t *__restrict__ rseg) {
+                           int32_t *__restrict__ rseg, int32_t *__restrict__ runs) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < nnz; i += (int64_t)gridDim.x * blockDim.x) {
         const uint64_t key = k[i];
@@ -72,12 +72,14 @@ __global__ void k_run_fill(const uint64_t *__restrict__ k, const int32_t *__rest
             rrow[u] = (int32_t)(key >> 32);
             rseg[u] = (int32_t)(c / M);
         }
+        if (i == nnz - 1) *runs = u + 1;
     }
 }
 
 __global__ void k_cells_or(const int32_t *__restrict__ rrow, const int32_t *__restrict__ rseg,
-                           const uint32_t *__restrict__ bits, int U, int V, int nblk,
+                           const uint32_t *__restrict__ bits, const int32_t *__restrict__ runs, int V, int nblk,
                            uint32_t *__restrict__ cells) {
+    const int U = *runs;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < U; i += gridDim.x * blockDim.x) {
         const uint32_t b = bits[i];
@@ -87,8 +89,9 @@ __global__ void k_cells_or(const int32_t *__restrict__ rrow, const int32_t *__re
 }
 
 __global__ void k_cells_count(const int32_t *__restrict__ rrow, const int32_t *__restrict__ rseg,
-                              int U, int V, int nblk, uint32_t *__restrict__ cells,
+                              const int32_t *__restrict__ runs, int V, int nblk, uint32_t *__restrict__ cells,
                               int32_t *__restrict__ out) {
+    const int U = *runs;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     int a = 0, b = 0;
     for (; i < U; i += gridDim.x * blockDim.x) {
@@ -111,7 +114,8 @@ __global__ void k_cells_count(const int32_t *__restrict__ rrow, const int32_t *_
 }
 
 __global__ void k_cells_clear(const int32_t *__restrict__ rrow, const int32_t *__restrict__ rseg,
-                              int U, int V, int nblk, uint32_t *__restrict__ cells) {
+                              const int32_t *__restrict__ runs, int V, int nblk, uint32_t *__restrict__ cells) {
+    const int U = *runs;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < U; i += gridDim.x * blockDim.x) cells[(size_t)rseg[i] * nblk + rrow[i] / V] = 0u;
 }
@@ -292,26 +296,22 @@ struct VenomWork {
         if (rc) return rc;
         hipLaunchKernelGGL(k_run_heads, dim3(gb), dim3(256), 0, st, keys2.p, nnz, M, head.p);
         if ((rc = scan_excl_i32(head.p, excl.p, nnz, st))) return rc;
-        int32_t last[2];
-        VNM_HIP_TRY(hipMemcpyAsync(&last[0], excl.p + nnz - 1, 4, hipMemcpyDeviceToHost, st));
-        VNM_HIP_TRY(hipMemcpyAsync(&last[1], head.p + nnz - 1, 4, hipMemcpyDeviceToHost, st));
+        // the number of runs stays on the device: one host read, at the end
         VNM_HIP_TRY(hipMemsetAsync(bits.p, 0, (size_t)nnz * 4, st));
         hipLaunchKernelGGL(k_run_fill, dim3(gb), dim3(256), 0, st, keys2.p, head.p, excl.p, nnz, M,
-                           bits.p, rrow.p, rseg.p);
-        VNM_HIP_TRY(hipStreamSynchronize(st));
-        U = last[0] + last[1];
-        const int gu = grid_of(U, 256);
-        hipLaunchKernelGGL(k_cells_or, dim3(gu), dim3(256), 0, st, rrow.p, rseg.p, bits.p, U, V,
+                           bits.p, rrow.p, rseg.p, cnt2.p + 3);
+        hipLaunchKernelGGL(k_cells_or, dim3(gb), dim3(256), 0, st, rrow.p, rseg.p, bits.p, cnt2.p + 3, V,
                            nblk, cells.p);
-        hipLaunchKernelGGL(k_cells_count, dim3(gu), dim3(256), 0, st, rrow.p, rseg.p, U, V, nblk,
+        hipLaunchKernelGGL(k_cells_count, dim3(gb), dim3(256), 0, st, rrow.p, rseg.p, cnt2.p + 3, V, nblk,
                            cells.p, cnt2.p);
-        hipLaunchKernelGGL(k_cells_clear, dim3(gu), dim3(256), 0, st, rrow.p, rseg.p, U, V, nblk,
+        hipLaunchKernelGGL(k_cells_clear, dim3(gb), dim3(256), 0, st, rrow.p, rseg.p, cnt2.p + 3, V, nblk,
                            cells.p);
         g->ctx->launches += 7;
         VNM_LAUNCH_CHECK("venom count");
-        int32_t h[2];
-        VNM_HIP_TRY(hipMemcpyAsync(h, cnt2.p, 8, hipMemcpyDeviceToHost, st));
+        int32_t h[4];
+        VNM_HIP_TRY(hipMemcpyAsync(h, cnt2.p, 16, hipMemcpyDeviceToHost, st));
         VNM_HIP_TRY(hipStreamSynchronize(st));
+        U = h[3];
         *inv = h[0];
         *strict = h[1];
         return VNM_OK;
