@@ -24,7 +24,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <unordered_map>
 #include <vector>
 
 namespace vnm {
@@ -217,15 +216,46 @@ __global__ void k_iota64(int32_t *p, int64_t n) {
     for (; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = (int32_t)i;
 }
 
+// Values of magnitude 2^24 or more and those that are not finite are left to the
+// host's printf (long_value), the others rounded where they are (text_value).
+__host__ __device__ __forceinline__ bool long_value(float v) { return !(fabsf(v) < 16777216.0f); }
+
+// A float (not a long one) after "%.2f" -> strtod -> "%.1e" -> strtof, exactly.
+// v * 100 is exact in double, and printf rounds the exact value half to even, as
+// rint does: q hundredths, read back as the double d = q / 100.  "%.1e" rounds
+// d, not q / 100, to two digits: where q is just between two of those, the sign
+// of d - q / 100 decides (an fma's d * 100 - q, exact), and the even digit where d
+// is exact.  (m t) / 100 as a float is what strtof reads: checked over every
+// number of hundredths below 30,000 and millions of floats against the library.
+__host__ __device__ __forceinline__ float text_value(float v) {
+    const double qd = rint((double)v * 100.0), d = qd / 100.0, aq = fabs(qd);
+    const int64_t q = (int64_t)aq;
+    int64_t t = 1;
+    while (q >= 100 * t) t *= 10;  // q / t: the first two digits
+    int64_t m = q / t;
+    if (t > 1) {
+        const int64_t r2 = 2 * (q % t);
+        const double e = fma(fabs(d), 100.0, -aq);
+        m += r2 > t || (r2 == t && (e > 0 || (e == 0 && (m & 1))));
+    }
+    return (float)copysign((double)(m * t) / 100.0, d);
+}
+
+// quantize: values through the text; dup[1] set when a long one is among them.
 __global__ void k_unpack_sorted(const uint64_t *__restrict__ k, const int32_t *__restrict__ idx,
-                                const float *__restrict__ vin, int64_t nnz,
+                                const float *__restrict__ vin, int64_t nnz, bool quantize,
                                 int32_t *__restrict__ row, int32_t *__restrict__ col,
                                 float *__restrict__ vout, int32_t *__restrict__ dup) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < nnz; i += (int64_t)gridDim.x * blockDim.x) {
         row[i] = (int32_t)(k[i] >> 32);
         col[i] = (int32_t)(uint32_t)k[i];
-        vout[i] = vin[idx[i]];
+        float v = vin[idx[i]];
+        if (quantize) {
+            if (long_value(v)) dup[1] = 1;
+            else v = text_value(v);
+        }
+        vout[i] = v;
         if (i > 0 && k[i] == k[i - 1]) atomicAdd(dup, 1);
     }
 }
@@ -369,32 +399,14 @@ int venom_eval(vnm_graph *g, int V, int32_t *inv, int32_t *inv_strict) {
     return VNM_OK;
 }
 
-// Exact value of a float after "%.2f" -> strtod -> "%.1e" -> strtof.  The
-// "%.2f" step is done exactly (v * 100 is exact in double; printf rounds the
-// exact value half-to-even, as nearbyint does); the "%.1e" step goes through
-// snprintf once per distinct intermediate value.
-static void quantize_values(std::vector<float> &vals) {
-    std::unordered_map<uint64_t, float> memo;
+// The long values after "%.2f" -> strtod -> "%.1e" -> strtof ("%.2f" prints them
+// exactly: they are integral).
+static void quantize_long_values(std::vector<float> &vals) {
     for (float &v : vals) {
-        double d;
-        if (std::fabs(v) >= 16777216.0f || !std::isfinite(v)) {
-            d = (double)v;  // integral: "%.2f" prints it exactly
-        } else {
-            const double q = std::nearbyint((double)v * 100.0);
-            d = q / 100.0;
-        }
-        uint64_t key;
-        memcpy(&key, &d, 8);
-        auto it = memo.find(key);
-        if (it != memo.end()) {
-            v = it->second;
-            continue;
-        }
+        if (!long_value(v)) continue;
         char buf[64];
-        snprintf(buf, sizeof buf, "%.1e", d);
-        float r = strtof(buf, nullptr);
-        memo.emplace(key, r);
-        v = r;
+        snprintf(buf, sizeof buf, "%.1e", (double)v);
+        v = strtof(buf, nullptr);
     }
 }
 
@@ -417,7 +429,7 @@ int reload_sort(vnm_graph *g, bool quantize) {
     DBuf<int32_t> i1, i2, dup;
     DBuf<float> v2;
     if ((rc = k1.alloc(nnz)) || (rc = k2.alloc(nnz)) || (rc = i1.alloc(nnz)) ||
-        (rc = i2.alloc(nnz)) || (rc = v2.alloc(nnz)) || (rc = dup.alloc(1)))
+        (rc = i2.alloc(nnz)) || (rc = v2.alloc(nnz)) || (rc = dup.alloc(2)))
         return rc;
     const int gb = grid_of(nnz, 256);
     hipLaunchKernelGGL(k_pos_keys, dim3(gb), dim3(256), 0, st, g->row.p, g->col.p, nnz, k1.p);
@@ -439,23 +451,24 @@ int reload_sort(vnm_graph *g, bool quantize) {
     }
     g->nrows = n;
     g->ncols = n;
-    if (quantize) {
-        std::vector<float> v(nnz);
-        VNM_HIP_TRY(hipMemcpyAsync(v.data(), g->val.p, nnz * 4, hipMemcpyDeviceToHost, st));
-        VNM_HIP_TRY(hipStreamSynchronize(st));
-        quantize_values(v);
-        VNM_HIP_TRY(hipMemcpyAsync(g->val.p, v.data(), nnz * 4, hipMemcpyHostToDevice, st));
-        VNM_HIP_TRY(hipStreamSynchronize(st));  // the copy reads this block's vector
-    }
-    VNM_HIP_TRY(hipMemsetAsync(dup.p, 0, 4, st));
-    hipLaunchKernelGGL(k_unpack_sorted, dim3(gb), dim3(256), 0, st, k2.p, i2.p, g->val.p, nnz,
+    VNM_HIP_TRY(hipMemsetAsync(dup.p, 0, 8, st));
+    hipLaunchKernelGGL(k_unpack_sorted, dim3(gb), dim3(256), 0, st, k2.p, i2.p, g->val.p, nnz, quantize,
                        g->row.p, g->col.p, v2.p, dup.p);
     g->ctx->launches += 3;
     VNM_LAUNCH_CHECK("reload sort");
     g->val.swap(v2);
-    int32_t ndup = 0;
-    VNM_HIP_TRY(hipMemcpyAsync(&ndup, dup.p, 4, hipMemcpyDeviceToHost, st));
+    int32_t found[2] = {0, 0};
+    VNM_HIP_TRY(hipMemcpyAsync(found, dup.p, 8, hipMemcpyDeviceToHost, st));
     VNM_HIP_TRY(hipStreamSynchronize(st));
+    const int32_t ndup = found[0];
+    if (found[1]) {
+        std::vector<float> v(nnz);
+        VNM_HIP_TRY(hipMemcpyAsync(v.data(), g->val.p, nnz * 4, hipMemcpyDeviceToHost, st));
+        VNM_HIP_TRY(hipStreamSynchronize(st));
+        quantize_long_values(v);
+        VNM_HIP_TRY(hipMemcpyAsync(g->val.p, v.data(), nnz * 4, hipMemcpyHostToDevice, st));
+        VNM_HIP_TRY(hipStreamSynchronize(st));  // the copy reads this block's vector
+    }
     if (ndup > 0) {
         // repeated positions only follow a relabel that was not one-to-one:
         // apply the loader's exact duplicate rule on the host
