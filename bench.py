@@ -713,7 +713,7 @@ def main():
 
     if a.copy_calib:
         copy_calibration(dev)
-    vec32 = p32.get_shape(vnm.DT_F32, NCOLS)  # the launch shape the tuner chose
+    vec32 = p32.get_shape(vnm.DT_F32, NCOLS)  # the launch shape of the rule
     traffic = measured_traffic("k_spmm_rmat65536_V128_traffic.json", "k_spmm_f32", vec32)
 
     res = {

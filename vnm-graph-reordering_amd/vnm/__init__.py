@@ -654,7 +654,7 @@ class Packed:
         _check(lib().vnm_spmm_noalloc(self.h, B_ptr, ldb, n, b_dtype, b_scales_ptr, C_ptr, ldc))
 
     def set_shape(self, b_dtype, n, cols_per_lane):
-        """Fix the SpMM launch shape for (b_dtype, n); 0 re-enables tuning."""
+        """Fix the SpMM launch shape for (b_dtype, n); 0 returns to the rule."""
         _check(lib().vnm_spmm_set_shape(self.h, b_dtype, n, cols_per_lane))
 
     def get_shape(self, b_dtype, n):
