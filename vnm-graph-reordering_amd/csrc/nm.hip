@@ -1453,6 +1453,12 @@ static int check_nm_args(vnm_graph *g, int N) {
     return VNM_OK;
 }
 
+// The first rounds of a run are launched as they are, the later ones in captured
+// batches.  Rounds past a run's end still cost their launches (2 us each), and
+// capturing a batch 0.3 ms, which a run on a new graph pays: a run of a sparse
+// matrix has a few rounds (ER 3,787 nodes, degree 12: 650 us with a captured batch,
+// SHORT_US now).
+constexpr int ROUND_FIRST = 4;   // greedy rounds launched one by one
 constexpr int ROUND_BATCH = 16;  // greedy rounds per captured graph launch
 constexpr int MAX_BATCH = 4096;  // graphs per batched run
 
@@ -1465,12 +1471,11 @@ __global__ __launch_bounds__(64) void k_gr_alldone(const NMArgs *__restrict__ ar
     if (threadIdx.x == 0) *flag = b == 0;
 }
 
-// Capture ROUND_BATCH rounds (seven kernels each, grid y = the G graphs) and
-// the all-done test on the context stream.
-static int capture_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args, int G, int gpx,
-                          int32_t *d_flag, hipGraph_t *graph_out, hipGraphExec_t *exec_out) {
-    VNM_HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    for (int b = 0; b < ROUND_BATCH; ++b) {
+// Enqueue `rounds` rounds (seven kernels each, grid y = the G graphs) and the
+// all-done test on the context stream.
+static void enqueue_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args, int G, int gpx, int rounds,
+                           int32_t *d_flag) {
+    for (int b = 0; b < rounds; ++b) {
         hipLaunchKernelGGL(k_gr_select, dim3(1, G), dim3(GT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_fill_a, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
         hipLaunchKernelGGL(k_gr_score, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
@@ -1480,6 +1485,13 @@ static int capture_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args
         hipLaunchKernelGGL(k_gr_count, dim3(gpx, G), dim3(PT), 0, st, a0, d_args);
     }
     hipLaunchKernelGGL(k_gr_alldone, dim3(1), dim3(64), 0, st, d_args, G, d_flag);
+}
+
+// Capture ROUND_BATCH rounds.
+static int capture_rounds(hipStream_t st, const NMArgs &a0, const NMArgs *d_args, int G, int gpx,
+                          int32_t *d_flag, hipGraph_t *graph_out, hipGraphExec_t *exec_out) {
+    VNM_HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    enqueue_rounds(st, a0, d_args, G, gpx, ROUND_BATCH, d_flag);
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(st, &graph);
     if (e != hipSuccess) {
@@ -1583,10 +1595,9 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
     }
     ctx->launches += G;
     VNM_LAUNCH_CHECK("k_gr_init");
-    // Rounds run in captured batches of ROUND_BATCH; the kernels of rounds past a
-    // graph's end return at entry.  Many runs have no round at all (the later
-    // steps of the hybrid find nothing invalid): those are seen before the first
-    // batch, whose 112 launches they paid for nothing.
+    // The kernels of rounds past a graph's end return at entry.  Many runs have no
+    // round at all (the later steps of the hybrid find nothing invalid): those are
+    // seen before the first.
     struct Drop {
         hipGraph_t g = nullptr;
         hipGraphExec_t e = nullptr;
@@ -1595,14 +1606,15 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
             if (g) (void)hipGraphDestroy(g);
         }
     } drop;
-    auto rounds = [&](hipGraphExec_t *exec) -> int {
+    auto batch = [&](hipGraphExec_t *exec) -> int {
         if (G > 1) {
-            const int rc = capture_rounds(st, hargs[0], d_args, G, gpx, d_flag, &drop.g, &drop.e);
+            const int rc = drop.e ? VNM_OK : capture_rounds(st, hargs[0], d_args, G, gpx, d_flag, &drop.g, &drop.e);
             *exec = drop.e;
             return rc;
         }
-        // the captured rounds hold the arguments by value: capture again when
-        // they changed (a reload that shrinks the rows moves records B)
+        // one graph's captured rounds stay with it and hold the arguments by
+        // value: captured again when they changed (a reload that shrinks the rows
+        // moves records B)
         vnm_graph *g0 = gs[0];
         const uint8_t *key = (const uint8_t *)&hargs[0];
         if (g0->nm_exec && (g0->nm_key.size() != sizeof(NMArgs) ||
@@ -1620,19 +1632,24 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
         *exec = g0->nm_exec;
         return VNM_OK;
     };
-    hipLaunchKernelGGL(k_gr_alldone, dim3(1), dim3(64), 0, st, d_args, G, d_flag);
-    ctx->launches++;
-    VNM_LAUNCH_CHECK("k_gr_alldone");
     int32_t done = 0;
-    VNM_HIP_TRY(hipMemcpyAsync(&done, d_flag, 4, hipMemcpyDeviceToHost, st));
-    VNM_HIP_TRY(hipStreamSynchronize(st));
-    hipGraphExec_t exec = nullptr;
-    if (!done && (rc = rounds(&exec))) return rc;
-    while (!done) {
-        VNM_HIP_TRY(hipGraphLaunch(exec, st));
-        ctx->launches += 7 * ROUND_BATCH + 1;
+    for (int k = 0;; ++k) {
+        if (k == 0) {
+            enqueue_rounds(st, hargs[0], d_args, G, gpx, 0, d_flag);
+            ctx->launches++;
+        } else if (k == 1) {
+            enqueue_rounds(st, hargs[0], d_args, G, gpx, ROUND_FIRST, d_flag);
+            ctx->launches += 7 * ROUND_FIRST + 1;
+        } else {
+            hipGraphExec_t exec = nullptr;
+            if ((rc = batch(&exec))) return rc;
+            VNM_HIP_TRY(hipGraphLaunch(exec, st));
+            ctx->launches += 7 * ROUND_BATCH + 1;
+        }
+        VNM_LAUNCH_CHECK("greedy rounds");
         VNM_HIP_TRY(hipMemcpyAsync(&done, d_flag, 4, hipMemcpyDeviceToHost, st));
         VNM_HIP_TRY(hipStreamSynchronize(st));
+        if (done) break;
     }
     for (int i = 0; i < G; ++i)
         hipLaunchKernelGGL(k_gr_cleanup, dim3(gpx), dim3(PT), 0, st, hargs[i], d_args + i);
