@@ -1456,8 +1456,8 @@ static int check_nm_args(vnm_graph *g, int N) {
 // The first rounds of a run are launched as they are, the later ones in captured
 // batches.  Rounds past a run's end still cost their launches (2 us each), and
 // capturing a batch 0.3 ms, which a run on a new graph pays: a run of a sparse
-// matrix has a few rounds (ER 3,787 nodes, degree 12: 650 us with a captured batch,
-// SHORT_US now).
+// matrix has a few rounds (ER 3,787 nodes, degree 12: 650 us with a captured
+// batch, 330 now).
 constexpr int ROUND_FIRST = 4;   // greedy rounds launched one by one
 constexpr int ROUND_BATCH = 16;  // greedy rounds per captured graph launch
 constexpr int MAX_BATCH = 4096;  // graphs per batched run
