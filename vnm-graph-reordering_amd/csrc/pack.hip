@@ -843,8 +843,11 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
     if ((rc = scan_excl_i32(nv.p, voff.p, (int64_t)E + 1, st))) { delete p; return rc; }
     hipLaunchKernelGGL(k_vrowptr, dim3(grid_of((int64_t)R + 1, 256)), dim3(256), 0, st, p->rowptr.p, voff.p, R,
                        vrp.p);
-    // the sparse-MFMA part's values are not in the row entries
-    const int64_t values = std::min<int64_t>(p->retained, 2 * (int64_t)E);
+    // the most values the row entries hold: two each, and every kept value is an
+    // entry of its own.  (The retained count is no bound: it counts positions, and a
+    // relabel that is not one-to-one leaves a position's entries side by side, of
+    // which a row entry keeps two.)
+    const int64_t values = std::min<int64_t>(nz, 2 * (int64_t)E);
     PieceBufs P;
     if ((rc = p->vrec.alloc(std::max<int64_t>(values, 1))) || (rc = build_items(p, vrp.p, values, P))) {
         delete p;
