@@ -1034,13 +1034,14 @@ __global__ void k_lp_pick(LPCtl *ctl, int nseg, int M, int mode0, uint64_t seed0
     dbest[s] = (int8_t)bdi;
     abest[s] = (int8_t)bai;
     // (score descending, segment) in 32 + sbits bits, sbits the bits of the
-    // largest segment index.  One array for one sort: donors first, acceptors after
-    // them (bit 32 + sbits set), a segment without a donor the last of the
-    // donors.  Each half is in segment order already, so the (stable) sort compares
-    // the score and the bit above it only.
-    const uint64_t low = (1ull << (32 + sbits)) - 1;
-    dkey[s] = bdi >= 0 ? ((uint64_t)(~ord_f32(bd)) << sbits) | (uint32_t)s : low;
-    akey[s] = (low + 1) | ((uint64_t)(~ord_f32(ba)) << sbits) | (uint32_t)s;
+    // largest segment index.  One array for one sort: donors first, then (bit 32 +
+    // sbits) the segments without a donor, then (the bit above) the acceptors.  Each
+    // kind is in segment order already, so the (stable) sort compares the score and
+    // the two bits above it only.  A score may be any 32 bits, NaNs among them, so no
+    // score stands for "no donor".
+    const uint64_t none = 1ull << (32 + sbits);
+    dkey[s] = bdi >= 0 ? ((uint64_t)(~ord_f32(bd)) << sbits) | (uint32_t)s : none | (uint32_t)s;
+    akey[s] = (none << 1) | ((uint64_t)(~ord_f32(ba)) << sbits) | (uint32_t)s;
     // donors counted once per wave (lanes past nseg have returned)
     const uint64_t dm = __ballot(bdi >= 0);
     const uint64_t live = __ballot(1);
@@ -2010,7 +2011,7 @@ static int lp_run_iter(LPRun &r, int exh) {
                        c->ptr.p, c->ccls.p, c->segcls.p, c->Y.p, w.dkey.p, w.dkey.p + ns, w.dbest.p, w.abest.p,
                        r.sbits);
     VNM_LAUNCH_CHECK("k_lp_pick");
-    if ((rc = sort_keys_u64_if(w.dkey.p, w.sdkey.p, 2 * (int64_t)ns, key_range(r.sbits, 33 + r.sbits), st,
+    if ((rc = sort_keys_u64_if(w.dkey.p, w.sdkey.p, 2 * (int64_t)ns, key_range(r.sbits, 34 + r.sbits), st,
                                &ctl->done))) return rc;
     hipLaunchKernelGGL(k_lp_match, dim3(grid_of((int64_t)r.nnorm * MATCH_L, 256, 1 << 30)), dim3(256), 0, st, ctl,
                        r.topk, r.window, ns, M, r.mode, r.seed, w.sdkey.p, w.sdkey.p + ns, w.dbest.p, w.abest.p,
