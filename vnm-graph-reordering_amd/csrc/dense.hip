@@ -61,9 +61,9 @@ __global__ void k_blk_kept(const int32_t *__restrict__ run_blk, const int32_t *_
 }
 
 __global__ void k_blk_vb(const int32_t *__restrict__ blk_first, const uint64_t *__restrict__ bkey, int nb,
-                         int nblk, int32_t *__restrict__ blk_vb) {
+                         int V, int32_t *__restrict__ blk_vb) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < nb) blk_vb[b] = (int32_t)((bkey[blk_first[b]] >> 32) % (uint64_t)nblk);
+    if (b < nb) blk_vb[b] = (int32_t)((uint32_t)bkey[blk_first[b]] / (uint32_t)V);
 }
 
 // One run (a row of a block) of a dense block: its kept values into the
@@ -123,7 +123,7 @@ int build_dense(vnm_packed *p, int dense_min, int U, int nb, int nblk, const int
     if ((rc = kept.alloc(std::max(nb, 1))) || (rc = vb.alloc(std::max(nb, 1)))) return rc;
     VNM_HIP_TRY(hipMemsetAsync(kept.p, 0, (size_t)std::max(nb, 1) * 4, st));
     if (U > 0) hipLaunchKernelGGL(k_blk_kept, dim3((U + 255) / 256), dim3(256), 0, st, run_blk, nkeep, U, kept.p);
-    if (nb > 0) hipLaunchKernelGGL(k_blk_vb, dim3((nb + 255) / 256), dim3(256), 0, st, blk_first, bkey, nb, nblk, vb.p);
+    if (nb > 0) hipLaunchKernelGGL(k_blk_vb, dim3((nb + 255) / 256), dim3(256), 0, st, blk_first, bkey, nb, V, vb.p);
     VNM_LAUNCH_CHECK("dense block counts");
     std::vector<int32_t> hk(nb), hv(nb), hs(nb);
     std::vector<uint16_t> hsel(nb);

@@ -102,9 +102,8 @@ __global__ void k_pk_total(const int32_t *__restrict__ excl, const int32_t *__re
 }
 
 __global__ void k_pk_runs(const uint64_t *__restrict__ k, const int32_t *__restrict__ head,
-                          const int32_t *__restrict__ excl, int64_t n, int M, int V, int nblk,
-                          uint32_t *__restrict__ bits, int32_t *__restrict__ rstart,
-                          int32_t *__restrict__ rlen, uint64_t *__restrict__ bkey,
+                          const int32_t *__restrict__ excl, int64_t n, int M, uint32_t *__restrict__ bits,
+                          int32_t *__restrict__ rstart, int32_t *__restrict__ rlen, uint64_t *__restrict__ bkey,
                           int32_t *__restrict__ rid) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     for (; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -115,16 +114,18 @@ __global__ void k_pk_runs(const uint64_t *__restrict__ k, const int32_t *__restr
         atomicAdd(&rlen[u], 1);
         if (head[i]) {
             rstart[u] = (int32_t)i;
-            // block key: (segment, row / V), then the row (stable order)
-            bkey[u] = ((uint64_t)((uint64_t)(c / M) * nblk + r / V) << 32) | r;
+            // (segment, row): a block's runs, rows r / V of one segment, lie together
+            bkey[u] = ((uint64_t)(c / M) << 32) | r;
             rid[u] = u;
         }
     }
 }
 
-__global__ void k_blk_heads(const uint64_t *__restrict__ bk, int U, int32_t *__restrict__ head) {
+__global__ void k_blk_heads(const uint64_t *__restrict__ bk, int U, int V, int32_t *__restrict__ head) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < U) head[i] = (i == 0) || ((bk[i] >> 32) != (bk[i - 1] >> 32));
+    if (i < U)
+        head[i] = (i == 0) || ((bk[i] >> 32) != (bk[i - 1] >> 32)) ||
+                  (uint32_t)bk[i] / (uint32_t)V != (uint32_t)bk[i - 1] / (uint32_t)V;
 }
 
 // The selected subset's 4 column offsets (ascending), 4 bits each.
@@ -144,7 +145,7 @@ constexpr int LANE_RUNS = 8;  // runs of a block that one lane scores
 // smallest), the order k_blk_select's argmax yields.  Longer blocks are
 // listed for k_blk_select.
 __global__ __launch_bounds__(256) void k_blk_select_lane(
-    const uint64_t *__restrict__ bk, const int32_t *__restrict__ rid_sorted, int U, int nb, int M, int nblk,
+    const uint64_t *__restrict__ bk, const int32_t *__restrict__ rid_sorted, int U, int nb, int M,
     const uint32_t *__restrict__ bits, const uint32_t *__restrict__ subs, int nsub,
     const int32_t *__restrict__ blk_first, int32_t *__restrict__ blk_seg, uint16_t *__restrict__ blk_sel,
     uint32_t *__restrict__ blk_mask, int32_t *__restrict__ run_blk, unsigned long long *__restrict__ retained,
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(256) void k_blk_select_lane(
                 }
             }
             const uint32_t S = subs[best_idx];
-            blk_seg[b] = (int32_t)((bk[first] >> 32) / (uint64_t)nblk);
+            blk_seg[b] = (int32_t)(bk[first] >> 32);
             blk_sel[b] = subset_sel(S, M);
             blk_mask[b] = S;
             kept += best_score;
@@ -194,7 +195,7 @@ __global__ __launch_bounds__(256) void k_blk_select_lane(
 // One wave per listed block: best 4-column subset (lexicographic order of
 // ascending column tuples; ties to the smallest).  nsub = C(M, 4) <= 70.
 __global__ __launch_bounds__(256) void k_blk_select(const uint64_t *__restrict__ bk, const int32_t *__restrict__ rid_sorted,
-                             int U, int nb, int M, int nblk, const uint32_t *__restrict__ bits,
+                             int U, int nb, int M, const uint32_t *__restrict__ bits,
                              const uint32_t *__restrict__ subs, int nsub,
                              const int32_t *__restrict__ blk_first, int32_t *__restrict__ blk_seg,
                              uint16_t *__restrict__ blk_sel, uint32_t *__restrict__ blk_mask,
@@ -242,8 +243,7 @@ __global__ __launch_bounds__(256) void k_blk_select(const uint64_t *__restrict__
         }
         const uint32_t S = subs[best_idx];
         if (lane == 0) {
-            const uint64_t key = bk[first] >> 32;
-            blk_seg[b] = (int32_t)(key / (uint64_t)nblk);
+            blk_seg[b] = (int32_t)(bk[first] >> 32);
             blk_sel[b] = subset_sel(S, M);
             blk_mask[b] = S;
             kept += (unsigned long long)best_score;
@@ -745,11 +745,11 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
         VNM_HIP_TRY(hipMemsetAsync(bits.p, 0, (size_t)U * 4, st));
         VNM_HIP_TRY(hipMemsetAsync(rlen.p, 0, (size_t)U * 4, st));
         hipLaunchKernelGGL(k_pk_runs, dim3(grid_of(nz, 256)), dim3(256), 0, st, keys2.p, head.p,
-                           excl.p, nz, M, V, nblk, bits.p, rstart.p, rlen.p, bkey.p, rid.p);
+                           excl.p, nz, M, bits.p, rstart.p, rlen.p, bkey.p, rid.p);
         if ((rc = sort_pairs_u64_i32(bkey.p, bkey2.p, rid.p, rid2.p, U,
-                                     key_halves(bits_for(R - 1), bits_for((int64_t)nseg * nblk)), st)))
+                                     key_halves(bits_for(R - 1), bits_for(nseg - 1)), st)))
             return rc;
-        hipLaunchKernelGGL(k_blk_heads, dim3(grid_of(U, 256)), dim3(256), 0, st, bkey2.p, U, bhead.p);
+        hipLaunchKernelGGL(k_blk_heads, dim3(grid_of(U, 256)), dim3(256), 0, st, bkey2.p, U, V, bhead.p);
         if ((rc = scan_excl_i32(bhead.p, bexcl.p, U, st))) return rc;
         hipLaunchKernelGGL(k_pk_total, dim3(1), dim3(1), 0, st, bexcl.p, bhead.p, (int64_t)U, cnt.p + 2);
         VNM_HIP_TRY(hipMemcpyAsync(&nb, cnt.p + 2, 4, hipMemcpyDeviceToHost, st));
@@ -775,10 +775,10 @@ int pack(vnm_graph *g, int V, int dtype, int dense_min, vnm_packed **out, int64_
         }
         VNM_HIP_TRY(hipMemsetAsync(nlong.p, 0, 4, st));
         hipLaunchKernelGGL(k_blk_select_lane, dim3(std::min(grid_of(nb, 256), 2048)), dim3(256), 0, st, bkey2.p, rid2.p, U, nb,
-                           M, nblk, bits.p, dsubs.p, (int)subs.size(), blk_first.p, p->blk_seg.p, p->blk_sel.p,
+                           M, bits.p, dsubs.p, (int)subs.size(), blk_first.p, p->blk_seg.p, p->blk_sel.p,
                            blk_mask.p, run_blk.p, dret.p, longb.p, nlong.p);
         hipLaunchKernelGGL(k_blk_select, dim3(std::min((nb + 3) / 4, 4096)), dim3(256), 0, st, bkey2.p, rid2.p,
-                           U, nb, M, nblk, bits.p, dsubs.p, (int)subs.size(), blk_first.p, p->blk_seg.p,
+                           U, nb, M, bits.p, dsubs.p, (int)subs.size(), blk_first.p, p->blk_seg.p,
                            p->blk_sel.p, blk_mask.p, run_blk.p, dret.p, longb.p, nlong.p);
         VNM_HIP_TRY(hipMemsetAsync(absmax.p, 0, (size_t)nb * 4, st));
         hipLaunchKernelGGL(k_run_keep, dim3(grid_of(U, 256)), dim3(256), 0, st, keys2.p, idx2.p,
