@@ -107,6 +107,12 @@ int  vnm_ctx_create(int device, vnm_ctx **out);
 /* Destroy every graph, packed matrix, model and batch created on the
  * context first: their destroy calls wait on the context's stream. */
 void vnm_ctx_destroy(vnm_ctx *ctx);
+/* A context keeps the device memory that its calls and objects have freed for
+ * its next ones: at most 2 GiB, until it and its objects are gone, or until an
+ * allocation of any context of the process fails without it.  Memory kept so is
+ * not seen by other allocators of the process; vnm_ctx_trim waits for the
+ * context's stream and gives it back. */
+int vnm_ctx_trim(vnm_ctx *ctx);
 /* The context's hipStream_t, for event timing by the caller. */
 void *vnm_ctx_stream(vnm_ctx *ctx);
 /* Number of kernels launched on the context so far. */

@@ -55,3 +55,14 @@ def test_reused_buffers():
         assert len(res) == len(fresh)
         for (a, pa), (b, pb) in zip(res, fresh):
             assert np.array_equal(a, b) and np.array_equal(pa, pb)
+
+
+def test_trim_gives_idle_memory_back():
+    ctx = vnm.Context(0)
+    first = call(ctx, 65536, 16, [])  # its graph and packed matrix are gone
+    torch.cuda.synchronize()
+    idle = torch.cuda.mem_get_info()[0]
+    ctx.trim()
+    assert torch.cuda.mem_get_info()[0] >= idle + (32 << 20)
+    again = call(ctx, 65536, 16, [])
+    assert all(np.array_equal(a, b) for a, b in zip(first, again))

@@ -153,6 +153,13 @@ void vnm_ctx_destroy(vnm_ctx *c) {
     delete c;
 }
 
+int vnm_ctx_trim(vnm_ctx *c) {
+    if (!c) return set_error(VNM_E_ARG, "null context");
+    VNM_HIP_TRY(hipStreamSynchronize(c->stream));
+    c->pool->trim();
+    return VNM_OK;
+}
+
 void *vnm_ctx_stream(vnm_ctx *c) { return c ? (void *)c->stream : nullptr; }
 
 int64_t vnm_ctx_launches(vnm_ctx *c) { return c ? c->launches : 0; }

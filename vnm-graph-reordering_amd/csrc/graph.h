@@ -5,9 +5,11 @@
 
 #include "vnm_internal.h"
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -26,15 +28,64 @@ namespace vnm {
 // of it 0.9 in kernels, and 1.27 from the pool; its learned reorder 8.1 ms and 5.8).
 // A block given back may still be read by work enqueued on the context's stream;
 // the next owner's work is enqueued behind it, on the same stream, so nothing
-// waits.  (Host copies into a block go through the stream as well.)  At most
-// POOL_IDLE bytes stay idle; the context and its objects share the pool, and the
-// last of them frees it.
+// waits.  (Host copies into a block go through the stream as well.  Work on
+// another stream must have ended before its buffers are released.)  At most
+// POOL_IDLE bytes stay idle, until vnm_ctx_trim, an allocation of any context that
+// fails without them, or the end of the context and of its objects, which share
+// the pool.
 constexpr size_t POOL_IDLE = (size_t)2 << 30;
 constexpr size_t POOL_GRAIN = 4096;
 
+class DevPool;
+
+// The process's pools.  (Never destroyed: a context may be left to process exit.)
+struct PoolList {
+    std::mutex mu;
+    std::set<DevPool *> pools;
+    std::atomic<int> wanted{0};  // allocations that failed and try again: nothing more goes idle
+    static PoolList &all() {
+        static PoolList *l = new PoolList();
+        return *l;
+    }
+    inline void flush();
+};
+
+// hipMalloc; where it fails, every pool's idle blocks are freed first.
+inline hipError_t device_alloc(void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        PoolList &l = PoolList::all();
+        l.wanted++;
+        l.flush();
+        e = hipMalloc(p, bytes);
+        l.wanted--;
+        if (e != hipSuccess) (void)hipGetLastError();
+    }
+    return e;
+}
+
 class DevPool {
 public:
-    // A block of at least `bytes`; *cap its size.
+    DevPool() {
+        PoolList &l = PoolList::all();
+        std::lock_guard<std::mutex> lk(l.mu);
+        l.pools.insert(this);
+    }
+    ~DevPool() {
+        PoolList &l = PoolList::all();
+        std::lock_guard<std::mutex> lk(l.mu);
+        l.pools.erase(this);
+        flush();
+    }
+    // Free the idle blocks.
+    void trim() {
+        std::lock_guard<std::mutex> lk(PoolList::all().mu);
+        flush();
+    }
+    DevPool(const DevPool &) = delete;
+    DevPool &operator=(const DevPool &) = delete;
+    // A block of at least `bytes` (> 0); *cap its size.
     hipError_t take(size_t bytes, void **p, size_t *cap) {
         {
             std::lock_guard<std::mutex> lk(mu);
@@ -47,23 +98,22 @@ public:
                 return hipSuccess;
             }
         }
-        // rounded up to an eighth of its size, so that a little growth still fits
+        // rounded up to an eighth of its size, so that a little growth still fits;
+        // just its size where memory is short
         size_t grain = POOL_GRAIN;
         while (grain * 16 <= bytes) grain *= 2;
-        const size_t want = (bytes + grain - 1) / grain * grain;
-        hipError_t e = hipMalloc(p, want);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            flush();
-            e = hipMalloc(p, want);
+        *cap = (bytes + grain - 1) / grain * grain;
+        hipError_t e = device_alloc(p, *cap);
+        if (e != hipSuccess && *cap > bytes) {
+            *cap = bytes;
+            e = device_alloc(p, bytes);
         }
-        *cap = want;
         return e;
     }
     void give(void *p, size_t cap) noexcept {
         try {
             std::lock_guard<std::mutex> lk(mu);
-            if (idle_bytes + cap <= POOL_IDLE) {
+            if (idle_bytes + cap <= POOL_IDLE && PoolList::all().wanted == 0) {
                 idle.emplace(cap, p);
                 idle_bytes += cap;
                 return;
@@ -72,19 +122,29 @@ public:
         }
         (void)hipFree(p);
     }
-    void flush() {
-        std::lock_guard<std::mutex> lk(mu);
-        for (auto &b : idle) (void)hipFree(b.second);
-        idle.clear();
-        idle_bytes = 0;
-    }
-    ~DevPool() { flush(); }
 
 private:
+    friend struct PoolList;
+    // Under PoolList::mu, so that an allocation that failed finds these blocks freed
+    // when its own turn to flush comes.
+    void flush() {
+        std::multimap<size_t, void *> blocks;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            blocks.swap(idle);
+            idle_bytes = 0;
+        }
+        for (auto &b : blocks) (void)hipFree(b.second);  // waits for the device
+    }
     std::mutex mu;
     std::multimap<size_t, void *> idle;
     size_t idle_bytes = 0;
 };
+
+inline void PoolList::flush() {
+    std::lock_guard<std::mutex> lk(mu);
+    for (DevPool *p : pools) p->flush();
+}
 
 // The pool that this host thread's allocations come from, for the length of a
 // scope: each entry point opens one for its context.
@@ -123,10 +183,9 @@ struct DBuf {
         if (count == 0) count = 1;
         hipError_t e;
         if (t_pool) e = t_pool->take(count * sizeof(T), (void **)&p, &cap);
-        else e = hipMalloc((void **)&p, count * sizeof(T));
+        else e = device_alloc((void **)&p, count * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
-            (void)hipGetLastError();
             return set_error(e == hipErrorOutOfMemory ? VNM_E_OOM : VNM_E_HIP,
                              "hipMalloc of %zu bytes failed: %s", count * sizeof(T), hipGetErrorString(e));
         }

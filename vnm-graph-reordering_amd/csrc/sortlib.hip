@@ -66,14 +66,7 @@ struct TempBuf {
         if (p) (void)hipFree(p);  // waits for the device, so no kernel still reads it
         p = nullptr;
         bytes = 0;
-        hipError_t e = hipMalloc(&p, need ? need : 1);
-        if (e != hipSuccess && t_pool) {
-            (void)hipGetLastError();
-            t_pool->flush();
-            e = hipMalloc(&p, need ? need : 1);
-        }
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
+        if (device_alloc(&p, need ? need : 1) != hipSuccess) {
             p = nullptr;
             return set_error(VNM_E_OOM, "scratch allocation of %zu bytes failed", need);
         }
