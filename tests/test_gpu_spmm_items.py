@@ -3,11 +3,12 @@
 Rows of every length around the item and block sizes (1 to 66 values, whole
 chunks, chunks with a remainder, a hub row of more than 16 chunks), rows without
 values before the first row, in runs of 8 and 9, after a cut row and at the end,
-and column counts that take every tile width, among them FP8 rows of an odd number
-of 64-column groups.  Every entry is kept (one per 4-column segment, V = 1), so
-the reference is the plain product in FP64; an output of L terms in FP32 may be off by
-(L + 3) 2^-24 times the sum of the terms' magnitudes (one rounding per FMA, one for
-the weight's scale, and the chunk sums).
+and column counts of one to eight 64-column groups, among them FP8 rows of an odd
+number of those, at the width that the rule takes and at every other one.  Every
+entry is kept (one per 4-column segment, V = 1), so the reference is the plain product
+in FP64; an output of L terms in FP32 may be off by (L + 3) 2^-24 times the sum of the
+terms' magnitudes (one rounding per FMA, one for the weight's scale, and the chunk
+sums).
 """
 import numpy as np
 import pytest
@@ -50,10 +51,8 @@ def _reference(m, B):
     return (A @ B).numpy(), (mag @ B.abs()).numpy(), np.bincount(m.row, minlength=m.nrows)
 
 
-@pytest.mark.parametrize("dt", [vnm.DT_F32, vnm.DT_BF16, vnm.DT_FP8])
-@pytest.mark.parametrize("n", [64, 128, 192, 320, 512])
-def test_items_and_tiles_at_their_edges(matrix, dt, n):
-    m, g, p = matrix
+def _operand(m, dt, n):
+    """(B on the device, its scales, B in FP64)."""
     gen = torch.Generator().manual_seed(n)
     B = torch.randn(m.ncols, n, generator=gen)
     scales = None
@@ -67,14 +66,57 @@ def test_items_and_tiles_at_their_edges(matrix, dt, n):
     else:
         dev = B
         B = B.double()
-    dev = dev.cuda()
-    sc = scales.cuda() if scales is not None else None
+    return dev.cuda(), scales.cuda() if scales is not None else None, B
+
+
+def _product(m, p, dt, n, dev, sc):
     C = torch.full((m.nrows, n), float("nan"), device="cuda")
     torch.cuda.synchronize()  # inputs made on torch's stream are complete
     p.spmm(dev.data_ptr(), n, n, dt, C.data_ptr(), n, sc.data_ptr() if sc is not None else None)
     torch.cuda.synchronize()
+    return C.cpu().numpy()
+
+
+@pytest.mark.parametrize("dt", [vnm.DT_F32, vnm.DT_BF16, vnm.DT_FP8])
+@pytest.mark.parametrize("n", [64, 128, 192, 320, 512])
+def test_items_and_tiles_at_their_edges(matrix, dt, n):
+    m, g, p = matrix
+    dev, sc, B = _operand(m, dt, n)
+    C = _product(m, p, dt, n, dev, sc)
     ref, mag, terms = _reference(m, B)
     bound = (terms[:, None] + 3) * 2.0 ** -24 * mag
-    off = np.abs(C.cpu().numpy() - ref) - bound
+    off = np.abs(C - ref) - bound
     assert not np.isnan(off).any()
     assert (off <= 0).all(), (dt, n, np.argwhere(off > 0)[:5])
+
+
+@pytest.mark.parametrize("dt,size", [(vnm.DT_F32, 4), (vnm.DT_BF16, 2), (vnm.DT_FP8, 1)])
+@pytest.mark.parametrize("n", [64, 192, 512, 1024])
+def test_every_width_gives_the_rule_s_bits(matrix, dt, size, n):
+    m, g, p = matrix
+    dev, sc, _ = _operand(m, dt, n)
+    p.set_shape(dt, n, 0)
+    C = _product(m, p, dt, n, dev, sc)
+    rule = p.get_shape(dt, n)
+    widths = [v for v in (1, 2, 4, 8, 16) if n % (64 * v) == 0 and 2 <= v * size <= 16] or [1]
+    assert rule in widths
+    for v in widths:
+        p.set_shape(dt, n, v)
+        assert p.get_shape(dt, n) == v
+        assert np.array_equal(_product(m, p, dt, n, dev, sc), C), v
+    # the batch takes the same widths, two matrices of a unit list
+    out = [torch.full((m.nrows, n), float("nan"), device="cuda") for _ in range(2)]
+    for v in [0] + widths:
+        b = vnm.Batch(g.ctx, [p, p], [dev.data_ptr()] * 2, [n] * 2, n, dt, [c.data_ptr() for c in out], [n] * 2,
+                      b_scales=[sc.data_ptr()] * 2 if sc is not None else None, cols_per_lane=v)
+        for c in out:
+            c.fill_(float("nan"))
+        torch.cuda.synchronize()
+        b.run()
+        torch.cuda.synchronize()
+        assert all(np.array_equal(c.cpu().numpy(), C) for c in out), v
+        b.close()
+    p.set_shape(dt, n, 0)
+    for v in {1, 2, 4, 8, 16, 3} - set(widths):  # what no product takes stays refused
+        with pytest.raises(vnm.VnmError):
+            p.set_shape(dt, n, v)

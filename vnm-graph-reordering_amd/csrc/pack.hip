@@ -888,11 +888,12 @@ int ensure_part(vnm_packed *p, int n) {
 int bsize_of(int bt) { return bt == VNM_DT_F32 ? 4 : bt == VNM_DT_BF16 ? 2 : 1; }
 
 // Column tiles of 64 * vec values usable for (bt, n): a tile is 128 to 1,024
-// bytes of a B row (8 to 64 lanes of 16 bytes) and divides n.
+// bytes of a B row (8 to 64 lanes of 16 bytes) and divides n; FP8 rows of an odd
+// number of 64-column groups, which have no such tile, take 64-byte ones (vec 1).
 bool vec_ok(int bt, int n, int vec) {
     if (vec != 1 && vec != 2 && vec != 4 && vec != 8 && vec != 16) return false;
     const int bytes = vec * bsize_of(bt);
-    return bytes >= 2 && bytes <= 16 && n % (64 * vec) == 0;
+    return (bytes >= 2 || n % 128 != 0) && bytes <= 16 && n % (64 * vec) == 0;
 }
 
 // The tile taken unless the caller fixes one: 256 bytes where they divide the
@@ -900,12 +901,11 @@ bool vec_ok(int bt, int n, int vec) {
 // up to 15 % slower (twice the item and value reads per byte), 1,024 20-30 %
 // (no slice of B stays with an XCD): us at 128 / 256 / 512 / 1,024 bytes, R-MAT
 // 65,536 n = 256 FP32 - / 76.3 / 76.4 / 98.7, BF16 54.4 / 49.0 / 52.5 / -;
-// R-MAT 131,072 n = 128 BF16 68.2 / 69.9.  FP8 rows of an odd number of
-// 64-column groups have no usable tile (vec_ok) and run as 64-byte tiles (vec 1).
+// R-MAT 131,072 n = 128 BF16 68.2 / 69.9.
 int default_vec(int bt, int n) {
-    for (int v = 4 / bsize_of(bt); v >= 1; v /= 2)
-        if (vec_ok(bt, n, v)) return v;
-    return 1;
+    int v = 4 / bsize_of(bt);
+    while (v > 1 && !vec_ok(bt, n, v)) v /= 2;
+    return v;
 }
 
 // Items one wave walks: 64 lanes over the lanes of a tile.
