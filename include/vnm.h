@@ -334,7 +334,8 @@ int vnm_spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int b_dtype,
  * lane; when the tile count divides 8, each tile runs on its own XCDs.  Not
  * in the reference (its kernels have fixed shapes).  Every shape gives the
  * same bits.  By default the first vnm_spmm call of a shape takes tiles of 256
- * bytes of a B row where they divide n, else narrower ones; set_shape with a
+ * bytes of a B row where they divide n, else narrower ones, or wider ones where
+ * that leaves more than 8 tiles; set_shape with a
  * value in {1, 2, 4, 8, 16} (cols_per_lane * sizeof(B value) of 2 to 16, or 1
  * where n is an odd multiple of 64, the shape such an FP8 product takes) fixes
  * it, 0 clears it; get_shape gives 0 when the shape has not been chosen yet. */

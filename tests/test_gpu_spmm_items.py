@@ -100,6 +100,7 @@ def test_every_width_gives_the_rule_s_bits(matrix, dt, size, n):
     rule = p.get_shape(dt, n)
     widths = [v for v in (1, 2, 4, 8, 16) if n % (64 * v) == 0 and 2 <= v * size <= 16] or [1]
     assert rule in widths
+    assert n // (64 * rule) <= 8 or rule == widths[-1]  # no more tiles than XCDs where a width allows
     for v in widths:
         p.set_shape(dt, n, v)
         assert p.get_shape(dt, n) == v

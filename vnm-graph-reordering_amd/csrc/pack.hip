@@ -897,14 +897,24 @@ bool vec_ok(int bt, int n, int vec) {
 }
 
 // The tile taken unless the caller fixes one: 256 bytes where they divide the
-// row, else 128.  Tiles of 256 and 512 bytes are within 3 % of each other, 128
-// up to 15 % slower (twice the item and value reads per byte), 1,024 20-30 %
-// (no slice of B stays with an XCD): us at 128 / 256 / 512 / 1,024 bytes, R-MAT
-// 65,536 n = 256 FP32 - / 76.3 / 76.4 / 98.7, BF16 54.4 / 49.0 / 52.5 / -;
-// R-MAT 131,072 n = 128 BF16 68.2 / 69.9.
+// row, else 128; wider where that leaves more than 8 tiles, which no longer have
+// XCDs of their own.  With 8 tiles or fewer, 256 and 512 bytes are within 3 % of
+// each other, 128 up to 15 % slower (twice the item and value reads per byte),
+// 1,024 20-30 % (no slice of B stays with an XCD): us at 128 / 256 / 512 / 1,024
+// bytes, R-MAT 65,536 n = 256 FP32 - / 76.3 / 76.4 / 98.7, BF16 54.4 / 49.0 / 52.5 /
+// -; R-MAT 131,072 n = 128 BF16 68.2 / 69.9.  Past 8 tiles of 256 bytes, at 256 /
+// 512 / 1,024 bytes: FP32 n = 1,024 (16 / 8 / 4 tiles) R-MAT 65,536 562 / 340 / 389,
+// ER 100,000 degree 10 582 / 598 / 607, 4,096 rows of 200 values 356 / 139 / 143; n =
+// 2,048 R-MAT 1,037 / 1,031 / 667.  Where the tile count does not divide 8 (n = 384:
+// 6 / 3 tiles, n = 768: 12 / 6 / 3), every XCD reads all of B and the widths are within
+// 10 % of each other: R-MAT 137 / 137 and 320 / 317 / 324, ER 227 / 233 and 435 / 461 /
+// 471, rows of 200 84 / 79 and 247 / 238 / 237.  (The width was timed per matrix before,
+// with one item a wave: such rows, all of them cut and B in L2, took 77 us at n = 384, 75
+// at 512, now 82, and 142 at 1,024; every other matrix here took longer than now.)
 int default_vec(int bt, int n) {
     int v = 4 / bsize_of(bt);
     while (v > 1 && !vec_ok(bt, n, v)) v /= 2;
+    while (n / (64 * v) > 8 && vec_ok(bt, n, 2 * v)) v *= 2;
     return v;
 }
 
