@@ -66,3 +66,22 @@ def test_trim_gives_idle_memory_back():
     assert torch.cuda.mem_get_info()[0] >= idle + (32 << 20)
     again = call(ctx, 65536, 16, [])
     assert all(np.array_equal(a, b) for a, b in zip(first, again))
+
+
+def test_batched_learned_reorder_on_reused_buffers():
+    M, N = 8, 2
+    rng = np.random.default_rng(8)
+    coos = [vnm.gen_chung_lu(int(n), 2.1, 12.0, 40 + i, M=M) for i, n in enumerate(rng.integers(300, 9000, 12))]
+    ctx = vnm.Context(0)
+    model = vnm.LPModel(ctx, seed=1)
+    fresh = vnm.Context(0)
+    fresh_model = vnm.LPModel(fresh, seed=1)
+    for order in (range(12), range(11, -1, -1), range(0, 12, 3)):
+        for mode, m in ((vnm.LP_LEARNED, model), (vnm.LP_EXHAUSTIVE, None)):
+            gs = [vnm.Graph(ctx, coos[i], M) for i in order]
+            vnm.Graph.lp_reorder_batch(gs, m, N, mode=mode, topk=512, window=8, maxiter=4, seed=3)
+            call(ctx, 900, 6, [])  # other calls take and give blocks of the same pool
+            for i, g in zip(order, gs):
+                alone = vnm.Graph(fresh, coos[i], M)
+                alone.lp_reorder(fresh_model if m else None, N, mode=mode, topk=512, window=8, maxiter=4, seed=3)
+                assert np.array_equal(g.perm(), alone.perm())

@@ -2133,6 +2133,12 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
     }
     hipStream_t st = ctx->stream;
     const int B = std::min(LP_BRANCHES, count);
+    // The runs' buffers go back to the context's pool, whose next owner's work is
+    // ordered behind the context's stream only: they are released after `res`, which
+    // waits for the branch streams on every path.
+    std::vector<LPRun> runs(count);
+    DBuf<LPCtl *> dctl;
+    DBuf<int32_t> dflags;
     // branch streams (default priority) and their captured iterations, released
     // on every path; the graphs get their context back on every path
     struct Branch {
@@ -2181,7 +2187,6 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
     }
     // per graph: cache, buffers, control block (on the context stream), sort
     // scratch reserved in its branch's slot
-    std::vector<LPRun> runs(count);
     int rc;
     for (int i = 0; i < count; ++i) {
         (void)sort_scratch_slot(i % B);
@@ -2200,8 +2205,6 @@ int lp_reorder_batch(vnm_graph *const *gs, int count, const vnm_lp_model *m, int
             hctl.push_back(runs[i].ctl.p);
         }
     }
-    DBuf<LPCtl *> dctl;
-    DBuf<int32_t> dflags;
     if ((rc = dctl.alloc(count)) || (rc = dflags.alloc(count))) return rc;
     VNM_HIP_TRY(hipMemcpyAsync(dctl.p, hctl.data(), count * sizeof(LPCtl *), hipMemcpyHostToDevice, st));
     std::vector<int32_t> done(count, 0);
@@ -2456,6 +2459,7 @@ int vnm_lp_reorder(vnm_graph *g, const vnm_lp_model *m, int N, int mode, int top
 int vnm_lp_reorder_batch(vnm_graph *const *graphs, int count, const vnm_lp_model *m, int N, int mode, int topk,
                          int window, int maxiter, uint64_t seed, vnm_lp_stats *st) {
     if (!graphs || !st) return set_error(VNM_E_ARG, "bad arguments");
+    PoolScope pool(count > 0 && graphs[0] ? graphs[0]->ctx->pool : nullptr);
     return lp_reorder_batch(graphs, count, m, N, mode, topk, window, maxiter, seed, st);
 }
 
