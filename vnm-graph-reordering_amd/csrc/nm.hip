@@ -396,7 +396,8 @@ struct GreedyState {
 };
 
 // The round's queues: of ordered pair q the pop order, element and gains.
-struct PopOrders {
+// (Copied to LDS 16 bytes at a time.)
+struct alignas(16) PopOrders {
     int lg[NQ][MMAX * MMAX], rg[NQ][MMAX * MMAX];
     uint8_t e[NQ][MMAX * MMAX];
 };
@@ -438,6 +439,7 @@ struct GreedyShared {
     int swlg[64], swrg[64], swpc[64], swtc[64];
     int nsw, trace;
 };
+static_assert(offsetof(GreedyShared, pops) % 16 == 0 && alignof(GreedyShared) >= 16, "pops is written 16 bytes at a time");
 
 __device__ __forceinline__ uint64_t key_fwd(int s, int c) {
     return c > 0 ? ((uint64_t)(uint32_t)c << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)s) : 0ull;
