@@ -26,6 +26,29 @@ inline int bits_for(int64_t x) {
     return b;
 }
 
+// The sorted bits of a key as one number: w0 bits from s0 on, then (w1 > 0) the
+// bits from s1 on (and whatever lies above them).
+__host__ __device__ __forceinline__ uint64_t sort_bits(const KeyBits &b, uint64_t k) {
+    uint64_t c = k >> b.s0;
+    if (b.w1) c = (c & ((1ull << b.w0) - 1)) | ((k >> b.s1) << b.w0);
+    return c;
+}
+
+// One pass's digit.
+struct Digit {
+    KeyBits b;
+    int shift, bits;
+    __host__ __device__ __forceinline__ int of(uint64_t k) const { return (int)((sort_bits(b, k) >> shift) & ((1u << bits) - 1u)); }
+};
+
+// A sort's passes, and the digit's width of the one that begins at `shift` of
+// `total` bits.
+inline int passes_of(const KeyBits &b) { return (b.w0 + b.w1 + 7) / 8; }
+__host__ __device__ inline int digit_bits(int total, int shift) {
+    const int left = total - shift;
+    return (left + (left + 7) / 8 - 1) / ((left + 7) / 8);
+}
+
 // Stable LSD radix sort on those bits (the input is not written; out must not
 // alias it).
 int sort_keys_u64(const uint64_t *in, uint64_t *out, int64_t n, KeyBits bits, hipStream_t st);

@@ -136,21 +136,6 @@ struct OpMax {
 
 // ------------------------------------------------------------ radix sort
 
-// The sorted bits of a key as one number: w0 bits from s0 on, then (w1 > 0) the
-// bits from s1 on.
-__device__ __forceinline__ uint64_t sort_bits(const KeyBits &b, uint64_t k) {
-    uint64_t c = k >> b.s0;
-    if (b.w1) c = (c & ((1ull << b.w0) - 1)) | ((k >> b.s1) << b.w0);
-    return c;
-}
-
-// One pass's digit.
-struct Digit {
-    KeyBits b;
-    int shift, bits;
-    __device__ __forceinline__ int of(uint64_t k) const { return (int)((sort_bits(b, k) >> shift) & ((1u << bits) - 1u)); }
-};
-
 // LDS of a tile's ranking.
 template <int T>
 struct RankShared {
@@ -325,12 +310,6 @@ __global__ __launch_bounds__(SWG) void k_radix_scatter(const uint64_t *__restric
         kout[o] = k;
         if constexpr (VALS) vout[o] = sv[p];
     }
-}
-
-// Digit widths of a sort of `total` bits in ceil(total / 8) passes.
-__host__ __device__ inline int digit_bits(int total, int shift) {
-    const int left = total - shift;
-    return (left + (left + 7) / 8 - 1) / ((left + 7) / 8);
 }
 
 // A whole sort of at most one tile in one workgroup: every pass ranks the
@@ -623,8 +602,6 @@ int scan_with(const In *in, int32_t *out, int64_t n, int32_t *totals, hipStream_
     if (e != hipSuccess) return set_error(VNM_E_HIP, "scan launch failed: %s", hipGetErrorString(e));
     return VNM_OK;
 }
-
-int passes_of(const KeyBits &b) { return (b.w0 + b.w1 + 7) / 8; }
 
 template <bool VALS>
 int radix_sort(const uint64_t *kin, uint64_t *kout, const int32_t *vin, int32_t *vout, int64_t n, KeyBits b,
