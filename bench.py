@@ -414,7 +414,7 @@ def copy_calibration(dev):
 
 
 def measured_traffic(fname, group, vec):
-    """HBM bytes per launch of a kernel variant (values per lane `vec`) from a
+    """HBM bytes per launch of a kernel variant (tiles of 64 `vec` columns) from a
     committed counter summary under profiles/ (rocprofv3 FETCH_SIZE +
     WRITE_SIZE per dispatch, calibrated), or None."""
     tpath = os.path.join(ROOT, "profiles", fname)
@@ -431,7 +431,7 @@ def bench_batch64(a):
     64 runs in one launch chain) and
     packed V:N:M = 64:2:8 in BF16; then the GCN sum aggregation Y_i = A_i X_i
     with X_i n_i x 256 BF16 N(0,1), all 64 products in one persistent
-    launch captured as a HIP graph (launch shape tuned on the batch).  Also
+    launch captured as a HIP graph.  Also
     timed: the same products as 64 separate vnm_spmm calls."""
     import numpy as np
     import torch
@@ -734,7 +734,7 @@ def main():
                    "hybrid_rounds": a.rounds, "sched": 0, "parallelism": "none (1 GPU)"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": f"k_spmm<f32 B, {vec32} columns per lane>", "kernel_ms": round(k_ms, 5),
+                     "kernel": f"k_spmm<f32 B, tiles of {64 * vec32} columns>", "kernel_ms": round(k_ms, 5),
                      "alg_bytes": int(alg_bytes), "a_read_bytes": int(a_bytes),
                      "a_packed_bytes": int(info.bytes)},
         "reorder": {"gpu_ms": round(reorder_wall_ms, 2), "hybrid_ms": round(hs.milliseconds, 2),

@@ -424,9 +424,12 @@ struct SelectShared {
     ColSet cs;
     uint64_t wbest[NW], wtop[NW];
     uint64_t topk[KMAX + 1];
-    int nkeys;
+    int thr[KMAX + 1];        // first segments of the threads that hold the top keys,
+    uint64_t tmax[KMAX + 1];  // and their largest keys, descending
+    int nthr, nkeys;
     uint64_t keys[SEL_KEYS];
 };
+static_assert(SEL_KEYS >= GT, "every thread's largest key fits");
 
 // LDS of k_gr_greedy.
 struct GreedyShared {
@@ -965,36 +968,51 @@ __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__res
         // The k largest traversal keys (keys are distinct, they hold the
         // segment) and the largest list key.  The k-th largest of the waves'
         // largest keys bounds the k-th largest of all from below, so only keys
-        // from there on are ranked against each other, in LDS.  Segment s goes
-        // to wave s mod 16: of counts that fall with s, as where hubs come
-        // first, each wave has its share, and about k keys pass.  (R-MAT
-        // 16,384, 2,048 segments: 10.7 us a round with the top k by insertion
-        // into sorted lists of one wave; 4.3 now.)
-        const int s1 = lane * NW + w;
+        // from there on are ranked against each other, in LDS.
+        // Up to 4 GT segments, a thread's counts stay in its registers, and
+        // segment s goes to wave s mod 16: of counts that fall with s, as where
+        // hubs come first, each wave has its share, and about k keys pass.
+        // (R-MAT 16,384, 2,048 segments: 10.7 us a round with the top k by
+        // insertion into sorted lists of one wave; 4.3 now.)
+        // More are read in runs of 16 (a wave's load of segments s mod 16 takes 64
+        // lines for 4), and once: the threads whose largest key passes are ranked
+        // by it, every key of the top k lies with one of the first k of them, and
+        // a wave each goes through those threads' segments again.  (200 rounds of
+        // R-MAT 2^18 / 2^20, schedule 1, 32,768 / 131,072 segments: 20.6 / 40.3 ms
+        // with all counts read twice in the first form, 16.7 / 23.1 now.)
+        const bool held = nseg <= 4 * GT;
+        const int s1 = held ? lane * NW + w : ((lane >> 4) * NW + w) * 16 + (lane & 15);
         auto key_of = [&](int seg, int c) { return tfwd ? key_fwd(seg, c) : key_rev(seg, c); };
         uint64_t best_l = 0, best_t = 0;
-        int cv[4];  // four loads in flight per thread; the first four stay
-        for (int s0 = s1; s0 < nseg; s0 += GT * 4) {
-            int cu[4];
+        auto see = [&](int seg, int c) {
+            const uint64_t lk = rev ? key_rev(seg, c) : key_fwd(seg, c);
+            const uint64_t x = key_of(seg, c);
+            best_l = lk > best_l ? lk : best_l;
+            best_t = x > best_t ? x : best_t;
+        };
+        int cv[4];
+        if (held) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) cu[u] = s0 + u * GT < nseg ? ld_l2(&A.cnt[s0 + u * GT]) : 0;
+            for (int u = 0; u < 4; ++u) cv[u] = s1 + u * GT < nseg ? ld_l2(&A.cnt[s1 + u * GT]) : 0;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (s0 == s1) cv[u] = cu[u];
-                const uint64_t lk = rev ? key_rev(s0 + u * GT, cu[u]) : key_fwd(s0 + u * GT, cu[u]);
-                const uint64_t x = key_of(s0 + u * GT, cu[u]);
-                best_l = lk > best_l ? lk : best_l;
-                best_t = x > best_t ? x : best_t;
+            for (int u = 0; u < 4; ++u) see(s1 + u * GT, cv[u]);
+        } else {
+            constexpr int UN = 8;  // loads in flight per thread
+            for (int s0 = s1; s0 < nseg; s0 += GT * UN) {
+                int cu[UN];
+#pragma unroll
+                for (int u = 0; u < UN; ++u) cu[u] = s0 + u * GT < nseg ? ld_l2(&A.cnt[s0 + u * GT]) : 0;
+#pragma unroll
+                for (int u = 0; u < UN; ++u) see(s0 + u * GT, cu[u]);
             }
         }
-        best_l = wave_max_u64(best_l);
-        best_t = wave_max_u64(best_t);
+        const uint64_t wave_l = wave_max_u64(best_l), wave_t = wave_max_u64(best_t);
         if (lane == 0) {
-            S.wbest[w] = best_l;
-            S.wtop[w] = best_t;
+            S.wbest[w] = wave_l;
+            S.wtop[w] = wave_t;
         }
-        if (tid == 0) S.nkeys = 0;
-        if (tid <= KMAX) S.topk[tid] = 0;
+        if (tid == 0) { S.nthr = 0; S.nkeys = 0; }
+        if (tid <= KMAX) { S.topk[tid] = 0; S.tmax[tid] = 0; }
         __syncthreads();
         uint64_t bound = 0;  // k-th largest wave maximum (0: fewer have any)
         {
@@ -1004,17 +1022,32 @@ __global__ __launch_bounds__(GT) void k_gr_select(NMArgs a0, const NMArgs *__res
             for (int j = 0; j < NW; ++j) above += S.wtop[j] > x;
             bound = wave_max_u64(above >= k - 1 ? x : 0);
         }
-        for (int s0 = s1; s0 < nseg; s0 += GT * 4) {
+        auto take = [&](int seg, int c) {
+            const uint64_t x = key_of(seg, c);
+            if (x != 0 && x >= bound) {
+                const int n = atomicAdd(&S.nkeys, 1);
+                if (n < SEL_KEYS) S.keys[n] = x;
+            }
+        };
+        if (held) {
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int seg = s0 + u * GT;
-                const int c = s0 == s1 ? cv[u] : seg < nseg ? ld_l2(&A.cnt[seg]) : 0;
-                const uint64_t x = seg < nseg ? key_of(seg, c) : 0;
-                if (x != 0 && x >= bound) {
-                    const int n = atomicAdd(&S.nkeys, 1);
-                    if (n < SEL_KEYS) S.keys[n] = x;
+            for (int u = 0; u < 4; ++u) take(s1 + u * GT, cv[u]);
+        } else {
+            const bool pass = best_t != 0 && best_t >= bound;
+            if (pass) S.keys[atomicAdd(&S.nthr, 1)] = best_t;  // at most one a thread
+            __syncthreads();
+            if (pass) {
+                int above = 0;
+                for (int j = 0; j < S.nthr; ++j) above += S.keys[j] > best_t;
+                if (above < k) {
+                    S.thr[above] = s1;
+                    S.tmax[above] = best_t;
                 }
             }
+            __syncthreads();  // the keys are read; theirs is the space of the next ones
+            bound = S.tmax[k - 1];
+            if (w < min(S.nthr, k))
+                for (int seg = S.thr[w] + lane * GT; seg < nseg; seg += 64 * GT) take(seg, ld_l2(&A.cnt[seg]));
         }
         __syncthreads();
         const int nk = S.nkeys;
