@@ -1571,8 +1571,14 @@ static int agg_plan(const std::vector<int32_t> &hptr, AggPlan &P, hipStream_t st
     P.nheavy = (int)heavy.size();
     P.nch = (int)beg.size();
     P.nlong = (int)longs.size();
-    // the longest first: they end last
-    std::stable_sort(longs.begin(), longs.end(), [&](int x, int y) { return hptr[x + 1] - hptr[x] > hptr[y + 1] - hptr[y]; });
+    // the longest first: they end last (a counting sort by length; a comparison sort
+    // was 2.8 of the 18.3 ms of five random iterations on R-MAT 2^20)
+    int at[AGG_CH + 2] = {};  // at[AGG_CH - length + 1]: lists that are longer, then the next place
+    for (int u : longs) at[AGG_CH - (hptr[u + 1] - hptr[u]) + 1]++;
+    for (int i = 1; i <= AGG_CH + 1; ++i) at[i] += at[i - 1];
+    std::vector<int32_t> sorted(longs.size());
+    for (int u : longs) sorted[at[AGG_CH - (hptr[u + 1] - hptr[u])]++] = u;
+    longs.swap(sorted);
     int rc;
     if ((rc = P.heavy.alloc(std::max(1, P.nheavy))) || (rc = P.ch0.alloc(P.nheavy + 1)) ||
         (rc = P.beg.alloc(std::max(1, P.nch))) || (rc = P.end.alloc(std::max(1, P.nch))) ||
