@@ -1164,8 +1164,7 @@ __global__ __launch_bounds__(256) void k_lp_match(LPCtl *ctl, int topk, int W, i
 // least the largest gain (a gain counts rows of the pair's two segments, each row
 // at most once per segment, so it is at most twice the row count).  Slots past
 // the candidates, up to the size of the sort that follows, get ~0, which sorts
-// last.  A workgroup takes candidates blockIdx.x, + gridDim.x, ...: one each
-// but in the exhaustive mode.
+// last.  A workgroup takes candidates blockIdx.x, + gridDim.x, ...
 struct GainKeys {
     const LPCtl *ctl;
     int nnorm, nexh;  // keys of the two sorts
@@ -1908,14 +1907,12 @@ struct LPRound {
     DBuf<int32_t> acc, out, touched, owner;
 };
 
-// Score candidates [0, nc) exactly: a workgroup per candidate.
-// nc candidates, or (d_nc given) the first *d_nc of nc launched blocks.
-constexpr int PAIR_GRID = 4096;  // workgroups of a run's pair scores, at least
-
+// Score candidates [0, nc) exactly; a run's number of them (gk.ctl) is on the
+// device, and `grid` workgroups share them.
 static int lp_score_cands(vnm_graph *g, LPCache *c, int N, Cand *cand, int4 *best, int nc, int32_t *full,
-                          const GainKeys &gk = GainKeys{}) {
+                          const GainKeys &gk = GainKeys{}, int grid = 0) {
     if (nc <= 0) return VNM_OK;
-    const int grid = gk.ctl ? std::min(nc, std::max(gk.nnorm, PAIR_GRID)) : nc;
+    if (grid <= 0) grid = nc;
     KernelTimer kt(g->ctx, "k_lp_pair_gain");
     hipLaunchKernelGGL(k_lp_pair_gain, dim3(grid), dim3(256), 0, g->ctx->stream, nc, g->nrows, g->M, N, cand,
                        g->inv.p, c->ptr.p, c->idx.p, best, full, gk);
@@ -2004,6 +2001,8 @@ static int lp_run_begin(LPRun &r, vnm_graph *g, const vnm_lp_model *m, int N, in
 // control block, so nothing here waits for the device.
 // exh: the iteration's mode where the host has read it (the other mode's sort,
 // and the exhaustive mode's forward pass, are not enqueued), -1 where it has not.
+constexpr int PAIR_GRID = 4096;  // workgroups of the pair scores of an iteration of unknown mode, at least
+
 static int lp_run_iter(LPRun &r, int exh) {
     vnm_graph *g = r.g;
     LPCache *c = r.c;
@@ -2023,8 +2022,15 @@ static int lp_run_iter(LPRun &r, int exh) {
                        r.topk, r.window, ns, M, r.mode, r.seed, w.sdkey.p, w.sdkey.p + ns, w.dbest.p, w.abest.p,
                        g->inv.p, c->Y.p, w.cand.p, r.smask);
     VNM_LAUNCH_CHECK("k_lp_match");
+    // A workgroup a candidate.  Where the mode is not known here (a batch's learned
+    // iterations), one for each donor, which then share the window's candidates if it
+    // is the exhaustive one: heavy pairs meet in one workgroup there (R-MAT 2^20, 65,536
+    // candidates: 6.8 ms in 4,096 workgroups, 6.1 in one each), but that is an
+    // iteration or two of a run, and a workgroup without a candidate costs in every one.
+    const bool window = r.mode == 2 || exh == 1;
+    const int grid = window ? r.ncap : exh == 0 || r.mode == 1 ? r.nnorm : std::min(r.ncap, std::max(r.nnorm, PAIR_GRID));
     if ((rc = lp_score_cands(g, c, r.N, w.cand.p, w.best.p, r.ncap, nullptr,
-                             GainKeys{ctl, r.nnorm, r.ncap, w.gkey.p, r.ibits, r.gmax})))
+                             GainKeys{ctl, r.nnorm, r.ncap, w.gkey.p, r.ibits, r.gmax}, grid)))
         return rc;
     // one candidate per donor: the first nnorm keys; the whole window: ncap
     // keys come in candidate order, so the sort leaves their low ibits alone
