@@ -1488,22 +1488,41 @@ static int check_nm_args(vnm_graph *g, int N) {
     return VNM_OK;
 }
 
-// The first rounds of a run are launched as they are, the later ones in captured
-// batches.  Rounds past a run's end still cost their launches (2 us each), and
-// capturing a batch 0.3 ms, which a run on a new graph pays: a run of a sparse
-// matrix has a few rounds (ER 3,787 nodes, degree 12: 650 us with a captured
-// batch, 330 now).
-constexpr int ROUND_FIRST = 4;   // greedy rounds launched one by one
+// The first rounds of a run are launched as they are, ROUND_FIRST at a time; a run
+// that is longer goes on in captured batches.  Capturing a batch takes 0.3 ms, which
+// a run on a new graph pays, a round launched as it is 10 us more than a captured
+// one, and a round past the run's end its seven launches (2 us each).  So a run is
+// captured once ROUND_DIRECT looks have not seen its end, or as soon as the invalid
+// segments left, at the rate they went so far, would take more than ROUND_LONG
+// rounds.  (us, all rounds captured, with the kernels before / four first / this rule:
+// ER 4,000 nodes, degree 12, 1-2 rounds 440 / 284 / 269; ER 256, degree 8, 6 rounds
+// 743 / 854 / 605; ER 1,000, degree 16, 18 rounds 1,743 / 1,506 / 1,501; Chung-Lu 700,
+// 51 rounds 6,404 / 4,056 / 4,019.)
+constexpr int ROUND_FIRST = 4;
+constexpr int ROUND_DIRECT = 8;
+constexpr int ROUND_LONG = 16;
 constexpr int ROUND_BATCH = 16;  // greedy rounds per captured graph launch
 constexpr int MAX_BATCH = 4096;  // graphs per batched run
 
-// 1 in *flag when every graph of the batch has finished.
+// flag[0]: every graph of the batch has finished; flag[1]: the rounds that the
+// others still take at the rate their invalid segments went so far, the most of them.
 __global__ __launch_bounds__(64) void k_gr_alldone(const NMArgs *__restrict__ args, int G,
                                                    int32_t *__restrict__ flag) {
-    int open = 0;
-    for (int i = threadIdx.x; i < G; i += 64) open |= args[i].st->done == 0;
+    int open = 0, left = 0;
+    for (int i = threadIdx.x; i < G; i += 64) {
+        const GreedyState *st = args[i].st;
+        if (st->done) continue;
+        open = 1;
+        const int gone = st->init_size - st->L;
+        const int64_t r = gone > 0 ? (int64_t)st->L * (st->round - 1) / gone : INT32_MAX;
+        left = max(left, (int)min(r, (int64_t)INT32_MAX));
+    }
     const uint64_t b = __ballot(open);
-    if (threadIdx.x == 0) *flag = b == 0;
+    for (int d = 32; d >= 1; d >>= 1) left = max(left, __shfl_xor(left, d, 64));
+    if (threadIdx.x == 0) {
+        flag[0] = b == 0;
+        flag[1] = left;
+    }
 }
 
 // Enqueue `rounds` rounds (seven kernels each, grid y = the G graphs) and the
@@ -1667,12 +1686,14 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
         *exec = g0->nm_exec;
         return VNM_OK;
     };
-    int32_t done = 0;
+    int32_t look[2] = {0, 0};
+    bool captured = false;
     for (int k = 0;; ++k) {
+        captured |= k > ROUND_DIRECT || (k > 1 && look[1] > ROUND_LONG);
         if (k == 0) {
             enqueue_rounds(st, hargs[0], d_args, G, gpx, 0, d_flag);
             ctx->launches++;
-        } else if (k == 1) {
+        } else if (!captured) {
             enqueue_rounds(st, hargs[0], d_args, G, gpx, ROUND_FIRST, d_flag);
             ctx->launches += 7 * ROUND_FIRST + 1;
         } else {
@@ -1682,9 +1703,9 @@ static int greedy_run(vnm_graph *const *gs, const int *scheds, int G, int N, int
             ctx->launches += 7 * ROUND_BATCH + 1;
         }
         VNM_LAUNCH_CHECK("greedy rounds");
-        VNM_HIP_TRY(hipMemcpyAsync(&done, d_flag, 4, hipMemcpyDeviceToHost, st));
+        VNM_HIP_TRY(hipMemcpyAsync(look, d_flag, 8, hipMemcpyDeviceToHost, st));
         VNM_HIP_TRY(hipStreamSynchronize(st));
-        if (done) break;
+        if (look[0]) break;
     }
     for (int i = 0; i < G; ++i)
         hipLaunchKernelGGL(k_gr_cleanup, dim3(gpx), dim3(PT), 0, st, hargs[i], d_args + i);
