@@ -335,10 +335,12 @@ int vnm_spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int b_dtype,
  * in the reference (its kernels have fixed shapes).  Every shape gives the
  * same bits.  By default the first vnm_spmm call of a shape takes tiles of 256
  * bytes of a B row where they divide n, else narrower ones, or wider ones where
- * that leaves more than 8 tiles; set_shape with a
- * value in {1, 2, 4, 8, 16} (cols_per_lane * sizeof(B value) of 2 to 16, or 1
- * where n is an odd multiple of 64, the shape such an FP8 product takes) fixes
- * it, 0 clears it; get_shape gives 0 when the shape has not been chosen yet. */
+ * that leaves more than 8 tiles, or B is of 512 MiB or more and few values
+ * lie in rows of more than 64; set_shape with a value in {1, 2, 4,
+ * 8, 16} (cols_per_lane * sizeof(B value) of 2 to 16, or 1 where n is an odd
+ * multiple of 64, the shape such an FP8 product takes) fixes it, 0 clears it;
+ * get_shape gives 0 when the shape has not been chosen yet.  A batch's
+ * cols_per_lane = 0 takes the rule without the last clause. */
 int vnm_spmm_set_shape(vnm_packed *p, int b_dtype, int n, int cols_per_lane);
 int vnm_spmm_get_shape(const vnm_packed *p, int b_dtype, int n, int32_t *cols_per_lane);
 
@@ -353,7 +355,7 @@ int vnm_gcn_layer(vnm_packed *p, const uint16_t *X, int ldx, int K, const uint16
 /* Batched SpMM: C_g = A_g B_g (+ bias_g) for `count` packed matrices of one
  * value dtype and uneven sizes, all with n output columns, in one persistent
  * launch captured with its row pre-fill as a HIP graph.  Not in the
- * reference.  cols_per_lane = 0 takes the shape vnm_spmm would choose.
+ * reference.  cols_per_lane = 0 takes the shape of vnm_spmm's rule.
  * The operand pointers are fixed at creation; vnm_batch_run replays the graph
  * on the context stream.  b_scales and bias may be NULL (per-entry NULLs
  * allowed for bias). */

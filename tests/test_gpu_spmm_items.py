@@ -121,3 +121,21 @@ def test_every_width_gives_the_rule_s_bits(matrix, dt, size, n):
     for v in {1, 2, 4, 8, 16, 3} - set(widths):  # what no product takes stays refused
         with pytest.raises(vnm.VnmError):
             p.set_shape(dt, n, v)
+
+
+@pytest.mark.parametrize("cut", [False, True])
+def test_width_for_a_far_operand(cut):
+    """512 MiB of B: the widest tile, unless many values lie in cut rows."""
+    rng = np.random.default_rng(6)
+    R, n = 1 << 20, 128
+    r, c = rng.integers(0, R, 3000), rng.integers(0, R, 3000)
+    if cut:
+        r, c = np.r_[r, np.full(300, 7)], np.r_[c, rng.choice(R // 4, 300, replace=False) * 4]
+    m = vnm.coo_from_tuples(R, R, r.astype(np.int32), c.astype(np.int32), rng.normal(size=len(r)).astype(np.float32), 4)
+    p = vnm.Graph(vnm.Context(0), m, 4).pack(1, vnm.DT_F32)
+    B = torch.randn(R, n, generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
+    C = _product(m, p, vnm.DT_F32, n, B, None)
+    assert p.get_shape(vnm.DT_F32, n) == (1 if cut else 2)
+    for v in (1, 2):
+        p.set_shape(vnm.DT_F32, n, v)
+        assert np.array_equal(_product(m, p, vnm.DT_F32, n, B, None), C)

@@ -56,7 +56,7 @@ static int spmm_noalloc(vnm_packed *p, const void *B, int ldb, int n, int bt, co
                          "(%zu floats); use vnm_spmm",
                          scratch_rows(p), n, scratch_rows(p) * (size_t)n, NOALLOC_FLOATS);
     auto it = p->shapes.find(shape_key(bt, n));
-    const int v = it != p->shapes.end() ? it->second : default_vec(bt, n);
+    const int v = it != p->shapes.end() ? it->second : shape_of(p, bt, n);
     return spmm_run(p, v, B, ldb, n, bt, bs, C, ldc, nullptr, p->ctx->noalloc_slots, false);
 }
 

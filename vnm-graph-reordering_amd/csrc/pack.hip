@@ -918,6 +918,20 @@ int default_vec(int bt, int n) {
     return v;
 }
 
+// default_vec for a matrix: the widest tile where B is far larger than the caches and
+// few values lie in cut rows.  Without hubs nothing of B is read again soon, so slices of
+// their own leave the XCDs nothing to keep, and a row of B in one piece is the better
+// access to memory: ER 2^20 at 256 / 512 / 1,024 bytes, FP32 n = 256 (1 GiB of B) 1,707 /
+// 1,636 / 1,583 us, n = 512 3,744 / 3,630 / 3,555; 2^18 (256 MiB) n = 256 331 / 340 / 337;
+// but R-MAT 2^20 n = 256 2,353 / 2,748 / 3,124.
+int shape_of(const vnm_packed *p, int bt, int n) {
+    constexpr uint64_t FAR_B = 512ull << 20;
+    int v = default_vec(bt, n);
+    if ((uint64_t)p->ncols * n * bsize_of(bt) >= FAR_B && (int64_t)p->nslots * ITEM * 16 <= p->nval)
+        while (vec_ok(bt, n, 2 * v)) v *= 2;
+    return v;
+}
+
 // Items one wave walks: 64 lanes over the lanes of a tile.
 int tile_items(int bt, int vec) {
     const int bytes = 64 * vec * bsize_of(bt);
@@ -1042,7 +1056,7 @@ int spmm(vnm_packed *p, const void *B, int ldb, int n, int bt, const float *bs, 
     int rc = spmm_check(p, B, ldb, n, bt, bs, C, ldc);
     if (rc) return rc;
     // the shape stays with the packed matrix: vnm_spmm_get_shape reports it
-    const int v = p->shapes.emplace(shape_key(bt, n), default_vec(bt, n)).first->second;
+    const int v = p->shapes.emplace(shape_key(bt, n), shape_of(p, bt, n)).first->second;
     return spmm_v(p, v, B, ldb, n, bt, bs, C, ldc, bias, true);
 }
 

@@ -400,6 +400,7 @@ size_t scratch_rows(const vnm_packed *p);
 int bsize_of(int bt);
 bool vec_ok(int bt, int n, int vec);
 int default_vec(int bt, int n);
+int shape_of(const vnm_packed *p, int bt, int n);
 int tile_items(int bt, int vec);
 SpmmArgs packed_args(const vnm_packed *p, const void *B, int ldb, const float *bs, float *C, int ldc,
                      const float *bias, float *part, int pn);
