@@ -353,8 +353,8 @@ int vnm_gcn_layer(vnm_packed *p, const uint16_t *X, int ldx, int K, const uint16
                   const float *bias, float *Y, int ldy);
 
 /* Batched SpMM: C_g = A_g B_g (+ bias_g) for `count` packed matrices of one
- * value dtype and uneven sizes, all with n output columns, in one persistent
- * launch captured with its row pre-fill as a HIP graph.  Not in the
+ * value dtype and uneven sizes, all with n output columns, as one persistent
+ * product kernel and one kernel for the cut rows, captured as a HIP graph.  Not in the
  * reference.  cols_per_lane = 0 takes the shape of vnm_spmm's rule.
  * The operand pointers are fixed at creation; vnm_batch_run replays the graph
  * on the context stream.  b_scales and bias may be NULL (per-entry NULLs
@@ -425,13 +425,13 @@ typedef struct {
 int vnm_lp_reorder(vnm_graph *g, const vnm_lp_model *m, int N, int mode, int topk, int window,
                    int maxiter, uint64_t seed, vnm_lp_stats *st);
 
-/* vnm_lp_reorder of count graphs of one context as one launch chain: one
- * iteration of every graph is captured as a HIP graph of 8 parallel branches
- * (every kernel reads its sizes and flags from its graph's device-side
- * control block) and replayed until every run is over or maxiter iterations
- * have run, with one host read of the runs' done flags per replay (and a new
- * capture of the running graphs once at most half of the captured ones
- * run).  st[i] and graph i's relabelling are those of vnm_lp_reorder on
+/* vnm_lp_reorder of count graphs of one context, side by side: the graphs are
+ * dealt to 8 streams, one iteration of a stream's graphs is captured as a HIP
+ * graph (every kernel reads its sizes and flags from its graph's device-side
+ * control block), and the 8 are replayed together until every run is over or
+ * maxiter iterations have run, with one host read of the runs' done flags per
+ * replay (and a new capture of a stream's running graphs once at most half of
+ * the captured ones run).  st[i] and graph i's relabelling are those of vnm_lp_reorder on
  * graph i alone with the same seed.  No counterpart in the reference; for
  * batches of graphs such as the inputs of one GCN training set. */
 int vnm_lp_reorder_batch(vnm_graph *const *graphs, int count, const vnm_lp_model *m, int N, int mode,

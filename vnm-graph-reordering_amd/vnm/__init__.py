@@ -524,8 +524,8 @@ class Graph:
 
     @staticmethod
     def lp_reorder_batch(graphs, model, N, mode=LP_LEARNED, topk=4096, window=16, maxiter=20, seed=1):
-        """lp_reorder of several graphs of one context as one launch chain (a
-        captured iteration of all graphs, replayed); each result is
+        """lp_reorder of several graphs of one context, side by side on 8 streams (a
+        captured iteration per stream, replayed); each result is
         lp_reorder's on the graph alone.  Returns the stats."""
         n = len(graphs)
         hs = (ctypes.c_void_p * n)(*[g.h for g in graphs])
